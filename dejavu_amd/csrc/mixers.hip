@@ -11,7 +11,7 @@
 #include "mix/delta_rule.hpp"
 #include "mix/hyper.hpp"
 #include "mix/linear_rows.hpp"
-#include "mix/linear_tiles.hpp"
+#include "mix/linear_stream.hpp"
 #include "mix/short_conv.hpp"
 #include "mix/ssd.hpp"
 #include "mix/stream.hpp"
@@ -48,6 +48,50 @@ int launch_lds(dim3 grid, dim3 block, size_t lds, hipStream_t s, A... args) {
   if (rc != DV_OK) return rc;
   hipLaunchKernelGGL(KERNEL, grid, block, lds, s, args...);
   return launched();
+}
+
+// ---- a portion's rows while the weight is the stream ------------------------
+struct StreamPlan {
+  int mb, nb;        // tile: rows of W, activation rows
+  int rows, cols;    // tiles
+  int splits;        // of K
+};
+
+// Tiles are as narrow as the rows allow; the taller one of 64 columns where it makes one round of workgroups of what would
+// be one and a half (22016 x 4096: 41 against 47 us with 47 rows, but 27.5 against 24.5 us at 4096 x 11008).  K is split until there are about as many
+// workgroups as compute units (4096 x 11008 with 47 rows: 1, 2, 4, 8 splits take 52, 32, 24.5, 27 us); the narrow tiles'
+// workgroups are small, so they go on to two per unit.  A split has at least 256 columns.
+StreamPlan plan_stream(int n, int M, int K) {
+  StreamPlan p;
+  p.nb = n <= 16 ? 16 : n <= 32 ? 32 : 64;
+  p.mb = p.nb == 16 ? 32 : p.nb == 64 && M >= 16384 ? 96 : 64;
+  p.rows = (M + p.mb - 1) / p.mb;
+  p.cols = (n + p.nb - 1) / p.nb;
+  const int64_t tiles = (int64_t)p.rows * p.cols;
+  int64_t s = p.nb == 16 ? (tiles >= 256 ? 1 : tiles >= 128 ? 4 : 8) : 288 / tiles;
+  if (s > K / 256) s = K / 256;
+  p.splits = (int)(s < 1 ? 1 : s > 8 ? 8 : s);
+  return p;
+}
+
+template <int AFTER, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W>
+int linear_stream_tiles(const StreamPlan& p, const TileArgs& a, void* workspace, hipStream_t s) {
+  float4_t* part = reinterpret_cast<float4_t*>(workspace);
+  const dim3 threads(WM * WN * 64);
+  const int rc = launch_lds<linear_stream_kernel<AFTER, MB, NB, KC, ST, WM, WN, NT_W>>(
+      dim3(p.rows, p.cols, p.splits), threads, (size_t)ST * (MB + NB) * KC * 2, s, a, part);
+  if (rc != DV_OK || p.splits == 1) return rc;
+  constexpr int values = (MB / WM / 16) * (NB / WN / 16);
+  hipLaunchKernelGGL((linear_stream_sum_kernel<AFTER, MB, NB, WM, WN>), dim3(p.rows, p.cols, values), threads, 0, s, a, part, p.splits);
+  return launched();
+}
+
+template <int AFTER>
+int linear_stream(const StreamPlan& p, const TileArgs& a, void* workspace, hipStream_t s) {
+  if (p.nb == 16) return linear_stream_tiles<AFTER, 32, 16, 128, 4, 2, 1, true>(p, a, workspace, s);
+  if (p.nb == 32) return linear_stream_tiles<AFTER, 64, 32, 64, 4, 4, 1, false>(p, a, workspace, s);
+  if (p.mb == 96) return linear_stream_tiles<AFTER, 96, 64, 64, 4, 2, 2, false>(p, a, workspace, s);
+  return linear_stream_tiles<AFTER, 64, 64, 64, 4, 2, 2, false>(p, a, workspace, s);
 }
 
 // ---- one row ---------------------------------------------------------------
@@ -418,30 +462,34 @@ int dv_mix_linear_row(int dtype, int before, int after, const dvRowArgs* a, void
                           : linear_row_any<float>(before, after, *a, st(stream));
 }
 
-int dv_mix_linear_tiles(int after, const dvTileArgs* a, void* stream) {
+size_t dv_mix_linear_tiles_workspace_bytes(int n, int M, int K) {
+  if (n < 1 || M < 1 || K < 8) return 0;
+  const StreamPlan p = plan_stream(n, M, K);
+  return p.splits > 1 ? (size_t)p.splits * p.rows * p.cols * p.mb * p.nb * sizeof(float) : 0;
+}
+
+int dv_mix_linear_tiles_ws(int after, const dvTileArgs* a, void* workspace, size_t workspace_bytes, void* stream) {
   if (!a || !a->x || !a->W || a->n < 1 || a->M < 1 || a->K < 8) return DV_ERR_INVALID_ARG;
-  if (a->K % 8 || a->ldw % 8 || a->ldx % 8 || !al16(a->W) || !al16(a->x)) return DV_ERR_ALIGNMENT;
+  if (a->K % 8 || a->ldw % 8 || a->ldx % 8 || !al16(a->W) || !al16(a->x) || !al16(workspace)) return DV_ERR_ALIGNMENT;
   if (after != DV_OUT_RESIDUAL && !a->out) return DV_ERR_INVALID_ARG;
   if (after == DV_OUT_GLU && a->M % 2) return DV_ERR_INVALID_ARG;
   if (after == DV_OUT_RESIDUAL && (!a->res.x || !a->res.post.w || (a->res.h && !a->res.pre.w))) return DV_ERR_INVALID_ARG;
-  const int nt = a->n <= 16 ? 1 : (a->n <= 32 ? 2 : 4);
-  const dim3 grid((a->M + 31) / 32, (a->n + 16 * nt - 1) / (16 * nt));
-  if (grid.y > 65535) return DV_ERR_UNSUPPORTED;
-#define DV_TILE(AFTER)                                                                                              \
-  do {                                                                                                              \
-    if (nt == 1) hipLaunchKernelGGL((linear_tiles_kernel<AFTER, 1>), grid, dim3(256), 0, st(stream), *a);            \
-    else if (nt == 2) hipLaunchKernelGGL((linear_tiles_kernel<AFTER, 2>), grid, dim3(256), 0, st(stream), *a);       \
-    else hipLaunchKernelGGL((linear_tiles_kernel<AFTER, 4>), grid, dim3(256), 0, st(stream), *a);                    \
-  } while (0)
+  StreamPlan p = plan_stream(a->n, a->M, a->K);
+  if (p.cols > 65535) return DV_ERR_UNSUPPORTED;
+  const size_t need = dv_mix_linear_tiles_workspace_bytes(a->n, a->M, a->K);
+  if (!workspace) p.splits = 1;
+  else if (workspace_bytes < need) return DV_ERR_WORKSPACE;
   switch (after) {
-    case DV_OUT_F32: DV_TILE(DV_OUT_F32); break;
-    case DV_OUT_T: DV_TILE(DV_OUT_T); break;
-    case DV_OUT_GLU: DV_TILE(DV_OUT_GLU); break;
-    case DV_OUT_RESIDUAL: DV_TILE(DV_OUT_RESIDUAL); break;
+    case DV_OUT_F32: return linear_stream<DV_OUT_F32>(p, *a, workspace, st(stream));
+    case DV_OUT_T: return linear_stream<DV_OUT_T>(p, *a, workspace, st(stream));
+    case DV_OUT_GLU: return linear_stream<DV_OUT_GLU>(p, *a, workspace, st(stream));
+    case DV_OUT_RESIDUAL: return linear_stream<DV_OUT_RESIDUAL>(p, *a, workspace, st(stream));
     default: return DV_ERR_UNSUPPORTED;
   }
-#undef DV_TILE
-  return launched();
+}
+
+int dv_mix_linear_tiles(int after, const dvTileArgs* a, void* stream) {
+  return dv_mix_linear_tiles_ws(after, a, nullptr, 0, stream);
 }
 
 int dv_mix_short_conv(int dtype, int out_f32, const dvConvArgs* a, void* stream) {

@@ -149,6 +149,13 @@ def _tile_args(x, W) -> L.TileArgs:
                       K=W.shape[1])
 
 
+def _tile_launch(after, a, device) -> None:
+    """The workspace is this call's own: calls on other streams have theirs, and a captured one is its graph's."""
+    nbytes = lib.dv_mix_linear_tiles_workspace_bytes(a.n, a.M, a.K)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+    check(lib.dv_mix_linear_tiles_ws(after, _ref(a), _ptr(ws), nbytes, _stream()), "dv_mix_linear_tiles_ws")
+
+
 def linear(x, W: torch.Tensor, bias: Optional[torch.Tensor] = None, f32: bool = False) -> torch.Tensor:
     """x (n, K) W (M, K)^T + bias -> (n, M) in x's type, or fp32."""
     n, M = x.shape[0], W.shape[0]
@@ -165,7 +172,7 @@ def linear(x, W: torch.Tensor, bias: Optional[torch.Tensor] = None, f32: bool = 
         out = torch.empty(n, M, dtype=out_t, device=x.device)
         a = _tile_args(x, W)
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
-        check(lib.dv_mix_linear_tiles(L.OUT_F32 if f32 else L.OUT_T, _ref(a), _stream()), "dv_mix_linear_tiles")
+        _tile_launch(L.OUT_F32 if f32 else L.OUT_T, a, x.device)
         return out
     return F.linear(x, W, bias)
 
@@ -183,7 +190,7 @@ def gated_unit(x, W: torch.Tensor, act: int, limit: float = 0.0) -> torch.Tensor
     if _tiles(x):
         a = _tile_args(x, W)
         a.out, a.ldo, a.act, a.limit = y.data_ptr(), M // 2, act, limit
-        check(lib.dv_mix_linear_tiles(L.OUT_GLU, _ref(a), _stream()), "dv_mix_linear_tiles")
+        _tile_launch(L.OUT_GLU, a, x.device)
     else:
         gu = F.linear(x, W)
         check(lib.dv_mix_glu(code, _ptr(gu), y.numel(), act, limit, _ptr(y), _stream()), "dv_mix_glu")
@@ -213,7 +220,7 @@ def linear_residual(x: torch.Tensor, W: torch.Tensor, stream: ResidualStream, po
     else:
         a = _tile_args(x, W)
         a.res = stream.args(post, pre, add_start, h)
-        check(lib.dv_mix_linear_tiles(L.OUT_RESIDUAL, _ref(a), _stream()), "dv_mix_linear_tiles")
+        _tile_launch(L.OUT_RESIDUAL, a, x.device)
     return h
 
 

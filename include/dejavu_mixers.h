@@ -288,7 +288,10 @@ DV_API int dv_mix_rms_rows(int dtype, const void* x, int64_t ldx, int64_t rows, 
 DV_API int dv_mix_gated_head_norm(int dtype, const float* o, const void* gate, int64_t ldg, int64_t rows, int heads,
                                   int vdim, int padded, const float* w, float eps, void* y, void* stream);
 DV_API int dv_mix_linear_row(int dtype, int before, int after, const dvRowArgs* args, void* stream);
+/* Without a workspace of dv_mix_linear_tiles_workspace_bytes (0: none is needed) K is not split over workgroups. */
 DV_API int dv_mix_linear_tiles(int after, const dvTileArgs* args, void* stream);
+DV_API size_t dv_mix_linear_tiles_workspace_bytes(int n, int M, int K);
+DV_API int dv_mix_linear_tiles_ws(int after, const dvTileArgs* args, void* workspace, size_t workspace_bytes, void* stream);
 DV_API int dv_mix_short_conv(int dtype, int out_f32, const dvConvArgs* args, void* stream);
 DV_API int dv_mix_conv_state(int dtype, const void* in, int64_t ldi, int n, int channels, int taps, float* state,
                              void* stream);

@@ -1,0 +1,68 @@
+"""Products of a portion's rows at the edges of their tiles, splits and dispatch rules, against float64 products of the
+same bf16 operands."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import vimulorn_oracle as V
+from tests.mixer_utils import OP_LIMIT, close, host
+from tests.test_gpu_vimulorn import _norm
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+# fp32 sums of K products of bf16 values: rounding stays below sqrt(K) 2^-24 of a row's rms (1e-5 up to K = 28000);
+# results in bf16: OP_LIMIT
+@pytest.mark.parametrize("n,K,M", [
+    (2, 8, 4),            # one piece of a chunk, one lane group of rows
+    (16, 520, 30),        # a tile of 32 rows that is not full, two splits, a last chunk of one piece
+    (15, 2048, 4100),     # 129 tiles, four splits
+    (13, 264, 8202),      # tiles enough for one split
+    (17, 2056, 66),       # 32 columns; a second tile of two rows; eight splits
+    (32, 136, 18440),     # one split
+    (33, 1096, 62),       # 64 columns, four splits
+    (64, 4104, 132),      # eight splits
+    (47, 264, 16388),     # the taller tile, the last one of four rows
+    (64, 72, 16384 + 96 * 3),
+])
+def test_edges(n, K, M):
+    from dejavu_amd import mixer_ops as ops
+
+    g = torch.Generator().manual_seed(n * 11 + M)
+    wide = torch.randn(n, K + 16, generator=g).to(BF16).cuda()
+    x = wide[:, 8:8 + K]  # rows further apart than they are long
+    W = (torch.randn(M, K, generator=g) * K ** -0.5).to(BF16).cuda()
+    bias = torch.randn(M, generator=g).to(BF16).cuda()
+    prod = host(x) @ host(W).T
+    close(ops.linear(x, W, f32=True), prod, 1e-5, f"{n}x{K}x{M}, fp32 result")
+    close(ops.linear(x, W, bias), prod + host(bias), OP_LIMIT[BF16], "with a bias")
+    gate, up = np.minimum(prod[:, 0::2], 0.75), np.clip(prod[:, 1::2], -0.75, 0.75)
+    close(ops.clamped_glu(x, W, 0.75), gate * V.sigmoid(1.702 * gate) * (up + 1), OP_LIMIT[BF16], "gated unit")
+    (post, f_post), (pre, f_pre) = _norm(M, 1), _norm(M, 2)
+    x0 = torch.randn(n, M, generator=g).cuda()
+    stream = ops.ResidualStream(x0.clone(), None, BF16)
+    h = ops.linear_residual(x, W, stream, post, pre)
+    want = host(x0) + f_post(prod)
+    close(stream.x, want, OP_LIMIT[BF16], "residual")
+    close(h, f_pre(want), OP_LIMIT[BF16], "next norm")
+
+
+def test_odd_places_of_the_result():
+    """Outputs whose rows do not start where four values can be stored at once."""
+    from dejavu_amd import _lib_mixers as L
+    from dejavu_amd import mixer_ops as ops
+
+    n, K, M = 19, 512, 70
+    g = torch.Generator().manual_seed(5)
+    x, W = torch.randn(n, K, generator=g).to(BF16).cuda(), torch.randn(M, K, generator=g).to(BF16).cuda()
+    prod = host(x) @ host(W).T
+    for after, dtype, ldo in ((L.OUT_T, BF16, 71), (L.OUT_T, BF16, 72), (L.OUT_F32, torch.float32, 73), (L.OUT_GLU, BF16, 37)):
+        out = torch.zeros(n * ldo + 1, dtype=dtype, device="cuda")
+        a = ops._tile_args(x, W)
+        a.out, a.ldo, a.act = out.data_ptr() + out.element_size(), ldo, L.GLU_RELU
+        ops._tile_launch(after, a, x.device)
+        got = out[1:].view(n, ldo)
+        want = np.maximum(prod[:, 0::2], 0) * prod[:, 1::2] if after == L.OUT_GLU else prod
+        close(got[:, :want.shape[1]], want, 1e-5 if dtype == torch.float32 else OP_LIMIT[BF16], f"after {after}, rows {ldo} apart")
+        assert not got[:, want.shape[1]:].any(), "stored past the end of a row"
