@@ -12,6 +12,7 @@ import ctypes
 
 import torch
 
+from . import ops
 from ._lib import check, lib
 
 _p = ctypes.c_void_p
@@ -53,8 +54,6 @@ _workspaces: dict = {}
 def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """Per-device scratch shared by all layers (they run one after the other).  A buffer that is
     outgrown stays allocated (captured HIP graphs may hold its address)."""
-    from . import ops
-
     return ops._grown(_workspaces, device, nbytes, 16 << 20)
 
 
@@ -168,7 +167,7 @@ def sparse_layer_decode(block, hidden_states, residual, head_idx, mlp_sp_logit, 
     nbytes = lib.dv_sparse_layer_workspace_bytes(ctypes.byref(a))
     ws = _workspace(hidden_out.device, nbytes)
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    check(lib.dv_sparse_layer_decode_f16(ctypes.byref(a), torch.cuda.current_stream().cuda_stream),
+    check(lib.dv_sparse_layer_decode_f16(ctypes.byref(a), ops._stream()),
           "dv_sparse_layer_decode_f16")
     _advance_window(block.mixer, flush)
     block.last_mlp_idx = mlp_idx_out
@@ -213,7 +212,7 @@ class LayerChain:
         arr = (SparseLayerArgs * n)(*self._args)
         ws = _workspace(self.outputs[0][0].device, self._nbytes)
         arr[0].workspace, arr[0].workspace_bytes = ws.data_ptr(), ws.numel()
-        check(lib.dv_sparse_layers_decode_f16(arr, n, torch.cuda.current_stream().cuda_stream),
+        check(lib.dv_sparse_layers_decode_f16(arr, n, ops._stream()),
               "dv_sparse_layers_decode_f16")
         return self.outputs[-1]
 

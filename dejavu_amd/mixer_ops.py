@@ -9,6 +9,7 @@ dense products of long prompts do elsewhere in this package.
 from __future__ import annotations
 
 import ctypes
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -39,7 +40,8 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """``torch.cuda.current_stream().cuda_stream`` without the Stream object (0.3 instead of 4 us a launch)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _f32(*tensors):
@@ -149,9 +151,12 @@ def _tile_args(x, W) -> L.TileArgs:
                       K=W.shape[1])
 
 
+_tile_workspace_bytes = lru_cache(maxsize=4096)(lib.dv_mix_linear_tiles_workspace_bytes)  # a function of the sizes alone
+
+
 def _tile_launch(after, a, device) -> None:
     """The workspace is this call's own: calls on other streams have theirs, and a captured one is its graph's."""
-    nbytes = lib.dv_mix_linear_tiles_workspace_bytes(a.n, a.M, a.K)
+    nbytes = _tile_workspace_bytes(a.n, a.M, a.K)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
     check(lib.dv_mix_linear_tiles_ws(after, _ref(a), _ptr(ws), nbytes, _stream()), "dv_mix_linear_tiles_ws")
 

@@ -524,7 +524,7 @@ class ParallelMHASparseAttMlp(_MHABase):
         nnz = head_idx.shape[0]
         nb = self.counter + 1
         batch_idx = torch.empty(nnz, nb, dtype=torch.int32, device=dev)
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = ops._stream()
         check(lib.dv_window_step_f16(x.data_ptr(), self.x_cache.data_ptr(), self.embed_dim, self.tracker.data_ptr(),
                                      head_idx.data_ptr(), nnz, H, self.counter, int(flush), batch_idx.data_ptr(),
                                      stream), "dv_window_step_f16")
@@ -586,7 +586,7 @@ class ParallelMHASparseAttMlp(_MHABase):
             batch_idx = torch.empty(nnz, nb, dtype=torch.int32, device=dev)
             check(lib.dv_window_step_f16(x.data_ptr(), self.x_cache_batch.data_ptr(), B * d, self.tracker.data_ptr(),
                                          head_idx.data_ptr(), nnz, H, self.counter, int(flush), batch_idx.data_ptr(),
-                                         torch.cuda.current_stream().cuda_stream), "dv_window_step_f16")
+                                         ops._stream()), "dv_window_step_f16")
         k_cache, v_cache = inference_params.key_value_memory_dict[self.layer_idx]
         b0 = inference_params.batch_size_offset
         kc, vc = k_cache[b0:b0 + B], v_cache[b0:b0 + B]

@@ -26,7 +26,12 @@ _ACT = {"id": _lib.DV_ACT_ID, "relu": _lib.DV_ACT_RELU, "gelu": _lib.DV_ACT_GELU
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """``torch.cuda.current_stream().cuda_stream`` without the Stream object (0.3 instead of 4 us a launch)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+def _device_stream(device: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if device.index is None else device.index)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -74,7 +79,7 @@ _retired_workspaces: list = []
 def _grown(cache: dict, device: torch.device, nbytes: int, floor: int) -> torch.Tensor:
     # one buffer per (device, stream): ops enqueued on different streams (the modules' side stream)
     # may run at the same time and must not share partial sums
-    key = (device.type, device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.type, device.index, _device_stream(device))
     ws = cache.get(key)
     if ws is None or ws.numel() < nbytes:
         if ws is not None:
@@ -135,7 +140,7 @@ _topk_workspaces: dict = {}
 
 def _topk_workspace(device: torch.device) -> torch.Tensor:
     """Histogram scratch per device and stream.  Top-k calls that share it must not overlap."""
-    key = (device.type, device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.type, device.index, _device_stream(device))
     ws = _topk_workspaces.get(key)
     if ws is None:
         ws = torch.empty(lib.dv_topk_workspace_bytes(65536) // 4, dtype=torch.int32, device=device)
