@@ -1,4 +1,4 @@
-// Products of a portion's rows (2..64 per tile) with a bf16 weight on the matrix cores, with the epilogues of
+// Products of a portion's rows (16..256 per tile) with a bf16 weight on the matrix cores, with the epilogues of
 // linear_rows.hpp.  The weight's bytes bound the product, not its operations.
 //
 // A tile is MB rows of W by NB activation rows.  Both operands go from memory straight into a ring of ST LDS slots (no

@@ -57,20 +57,40 @@ struct StreamPlan {
   int splits;        // of K
 };
 
-// Tiles are as narrow as the rows allow; the taller one of 64 columns where it makes one round of workgroups of what would
-// be one and a half (22016 x 4096: 41 against 47 us with 47 rows, but 27.5 against 24.5 us at 4096 x 11008).  K is split until there are about as many
-// workgroups as compute units (4096 x 11008 with 47 rows: 1, 2, 4, 8 splits take 52, 32, 24.5, 27 us); the narrow tiles'
-// workgroups are small, so they go on to two per unit.  A split has at least 256 columns.
+// Up to 64 rows: tiles are as narrow as the rows allow; the taller one of 64 columns where it makes one round of
+// workgroups of what would be one and a half (22016 x 4096: 41 against 47 us with 47 rows, but 27.5 against 24.5 us at
+// 4096 x 11008).  K is split until there are about as many workgroups as compute units (4096 x 11008 with 47 rows: 1, 2, 4,
+// 8 splits take 52, 32, 24.5, 27 us); the narrowest tiles' workgroups are small, so they go on to two per unit.
+// More rows: 128 rows of W, so that the activations are fetched less often (5120 x 20480 with 96 rows: 53 us, 60 with 64
+// rows of W), where that leaves 32 tiles and K is long enough to split; 192 where they fill the chip better (20480 x 5120
+// with 96 rows: 107 tiles in 2 splits take 53 us, 160 tiles of 128 rows 59).
+// A split has at least 256 columns.
 StreamPlan plan_stream(int n, int M, int K) {
+  constexpr int kUnits = 256;
   StreamPlan p;
-  p.nb = n <= 16 ? 16 : n <= 32 ? 32 : 64;
-  p.mb = p.nb == 16 ? 32 : p.nb == 64 && M >= 16384 ? 96 : 64;
-  p.rows = (M + p.mb - 1) / p.mb;
-  p.cols = (n + p.nb - 1) / p.nb;
-  const int64_t tiles = (int64_t)p.rows * p.cols;
-  int64_t s = p.nb == 16 ? (tiles >= 256 ? 1 : tiles >= 128 ? 4 : 8) : 288 / tiles;
-  if (s > K / 256) s = K / 256;
-  p.splits = (int)(s < 1 ? 1 : s > 8 ? 8 : s);
+  p.nb = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : n <= 128 ? 128 : n <= 192 ? 192 : n <= 256 ? 256 : 64;
+  auto lay = [&](int mb) {
+    p.mb = mb;
+    p.rows = (M + mb - 1) / mb;
+    p.cols = (n + p.nb - 1) / p.nb;
+    const int64_t tiles = (int64_t)p.rows * p.cols;
+    int64_t s = p.nb == 16 ? (tiles >= kUnits ? 1 : tiles >= kUnits / 2 ? 4 : 8) : (p.nb <= 64 ? 288 : kUnits) / tiles;
+    if (s > K / 256) s = K / 256;
+    p.splits = (int)(s < 1 ? 1 : s > 8 ? 8 : s);
+    return (int64_t)p.splits * tiles;
+  };
+  if (p.nb <= 64) {
+    lay(p.nb == 16 ? 32 : p.nb == 64 && M >= 16384 ? 96 : 64);
+  } else if (M < 32 * 128 || K < 2048) {
+    lay(64);
+  } else {
+    const bool tall = p.nb < 256 && K >= 4096;
+    const int64_t groups = lay(128);
+    if (tall && groups <= kUnits) {
+      const int64_t more = lay(192);
+      if (more > kUnits || more * 10 <= groups * 11) lay(128);
+    }
+  }
   return p;
 }
 
@@ -90,8 +110,16 @@ template <int AFTER>
 int linear_stream(const StreamPlan& p, const TileArgs& a, void* workspace, hipStream_t s) {
   if (p.nb == 16) return linear_stream_tiles<AFTER, 32, 16, 128, 4, 2, 1, true>(p, a, workspace, s);
   if (p.nb == 32) return linear_stream_tiles<AFTER, 64, 32, 64, 4, 4, 1, false>(p, a, workspace, s);
-  if (p.mb == 96) return linear_stream_tiles<AFTER, 96, 64, 64, 4, 2, 2, false>(p, a, workspace, s);
-  return linear_stream_tiles<AFTER, 64, 64, 64, 4, 2, 2, false>(p, a, workspace, s);
+  if (p.nb == 64 && p.mb == 96) return linear_stream_tiles<AFTER, 96, 64, 64, 4, 2, 2, false>(p, a, workspace, s);
+  if (p.nb == 64) return linear_stream_tiles<AFTER, 64, 64, 64, 4, 2, 2, false>(p, a, workspace, s);
+  if (p.nb == 128 && p.mb == 64) return linear_stream_tiles<AFTER, 64, 128, 64, 3, 2, 4, false>(p, a, workspace, s);
+  if (p.nb == 128 && p.mb == 128) return linear_stream_tiles<AFTER, 128, 128, 64, 4, 2, 4, false>(p, a, workspace, s);
+  if (p.nb == 128) return linear_stream_tiles<AFTER, 192, 128, 64, 3, 2, 4, false>(p, a, workspace, s);
+  if (p.nb == 192 && p.mb == 64) return linear_stream_tiles<AFTER, 64, 192, 64, 4, 2, 4, false>(p, a, workspace, s);
+  if (p.nb == 192 && p.mb == 128) return linear_stream_tiles<AFTER, 128, 192, 64, 3, 2, 4, false>(p, a, workspace, s);
+  if (p.nb == 192) return linear_stream_tiles<AFTER, 192, 192, 64, 3, 2, 4, false>(p, a, workspace, s);
+  if (p.mb == 64) return linear_stream_tiles<AFTER, 64, 256, 64, 3, 2, 4, false>(p, a, workspace, s);
+  return linear_stream_tiles<AFTER, 128, 256, 64, 3, 2, 4, false>(p, a, workspace, s);
 }
 
 // ---- one row ---------------------------------------------------------------

@@ -2,9 +2,9 @@
 
 Weights and activations are bf16 or fp32 (one type per model); the residual stream, norms, scores and recurrent state
 are fp32.  All ops enqueue on ``torch.cuda.current_stream()`` and refuse CPU tensors.  Products: one row goes to the
-row kernel, up to ``TILE_MAX_ROWS`` bf16 rows to the matrix-core kernel, both with the operation that follows in the
-same launch; longer portions (and several fp32 rows) take the library GEMM and a separate elementwise launch, as the
-dense products of long prompts do elsewhere in this package.
+row kernel, up to ``TILE_MAX_ROWS`` bf16 rows to the matrix-core kernel that streams the weight, both with the operation
+that follows in the same launch; longer portions (and several fp32 rows) take the library GEMM and a separate elementwise
+launch, as the dense products of long prompts do elsewhere in this package.
 """
 from __future__ import annotations
 
@@ -18,7 +18,13 @@ import torch.nn.functional as F
 from . import _lib_mixers as L
 from ._lib_mixers import check, lib
 
-TILE_MAX_ROWS = 64
+# The streaming kernel against the library GEMM without the launch that follows it, us: 4096 x 11008 with 96 / 192 / 256
+# rows 28 / 35 / 40 against 50 / 81 / 52, 22016 x 4096 52 / 58 / 65 against 47 / 61 / 64 (and 5 to 9 for the gated unit that
+# follows), 4096 x 4096 16 / 19 / 22 against 22 / 33 / 23.  The library is ahead for small weights from 192 rows on (2048 x
+# 2048 with 256 rows: 11.4 against 9.7) and beyond 256 rows, where the operations bound the product.
+TILE_MAX_ROWS = 256
+TILE_ALL_ROWS = 192          # up to here whatever the weight's size
+TILE_WEIGHT = 1 << 23        # elements from which the rows may be more
 
 _DTYPES = {torch.bfloat16: L.BF16, torch.float32: L.F32}
 _ref = ctypes.byref
@@ -90,8 +96,13 @@ def residual(y: Optional[torch.Tensor], stream: ResidualStream, post, pre, add_s
     return h
 
 
-def _tiles(x: torch.Tensor) -> bool:
-    return x.dtype == torch.bfloat16 and x.shape[0] <= TILE_MAX_ROWS
+def _tiles(x: torch.Tensor, W: torch.Tensor) -> bool:
+    """Whether the streaming kernel takes the product.  From 65 rows on the library takes what it would refuse."""
+    n = x.shape[0]
+    if x.dtype != torch.bfloat16 or n <= 64:
+        return x.dtype == torch.bfloat16
+    fits = all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, W)) and x.shape[1] % 8 == 0 and W.shape[0] % 2 == 0
+    return fits and (n <= TILE_ALL_ROWS or (n <= TILE_MAX_ROWS and W.numel() >= TILE_WEIGHT))
 
 
 def _product_ok(x, W):
@@ -173,7 +184,7 @@ def linear(x, W: torch.Tensor, bias: Optional[torch.Tensor] = None, f32: bool = 
         _row_launch(code, before, L.OUT_F32 if f32 else L.OUT_T, a)
         return out
     code = _product_ok(x, W)
-    if _tiles(x) or (f32 and code == L.BF16):
+    if _tiles(x, W) or (f32 and code == L.BF16):
         out = torch.empty(n, M, dtype=out_t, device=x.device)
         a = _tile_args(x, W)
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
@@ -192,7 +203,7 @@ def gated_unit(x, W: torch.Tensor, act: int, limit: float = 0.0) -> torch.Tensor
         _row_launch(code, before, L.OUT_GLU, a)
         return y
     code = _product_ok(x, W)
-    if _tiles(x):
+    if _tiles(x, W):
         a = _tile_args(x, W)
         a.out, a.ldo, a.act, a.limit = y.data_ptr(), M // 2, act, limit
         _tile_launch(L.OUT_GLU, a, x.device)
@@ -215,7 +226,7 @@ def linear_residual(x: torch.Tensor, W: torch.Tensor, stream: ResidualStream, po
     code = _product_ok(x, W)
     n = x.shape[0]
     assert stream.x.shape == (n, W.shape[0])
-    if n != 1 and not _tiles(x):
+    if n != 1 and not _tiles(x, W):
         return residual(F.linear(x, W), stream, post, pre, add_start)
     h = None if pre is None else stream.new_h()
     if n == 1:

@@ -25,6 +25,10 @@ BF16 = torch.bfloat16
     (64, 4104, 132),      # eight splits
     (47, 264, 16388),     # the taller tile, the last one of four rows
     (64, 72, 16384 + 96 * 3),
+    (65, 264, 70), (128, 2056, 4100), (96, 4104, 12296),      # 128 columns: 64, 128 and 192 rows of W
+    (129, 1032, 4100), (192, 2048, 5122), (140, 4096, 18436),  # 192 columns
+    (193, 8, 1 << 20), (256, 2056, 4100), (256, 1544, 5442),   # 256 columns: 64 and 128 rows
+    (256, 264, 72), (257, 520, 72),                            # the library (fp32 results: tiles of 64 columns)
 ])
 def test_edges(n, K, M):
     from dejavu_amd import mixer_ops as ops
@@ -46,6 +50,15 @@ def test_edges(n, K, M):
     want = host(x0) + f_post(prod)
     close(stream.x, want, OP_LIMIT[BF16], "residual")
     close(h, f_pre(want), OP_LIMIT[BF16], "next norm")
+
+
+def test_unaligned_operands():
+    """What the streaming kernel refuses is still multiplied where several kernels could."""
+    from dejavu_amd import mixer_ops as ops
+
+    g = torch.Generator().manual_seed(3)
+    x, W = torch.randn(70, 65, generator=g).to(BF16).cuda()[:, 1:], torch.randn(48, 64, generator=g).to(BF16).cuda()
+    close(ops.linear(x, W), host(x) @ host(W).T, OP_LIMIT[BF16], "rows that start at odd places")
 
 
 def test_odd_places_of_the_result():
