@@ -12,6 +12,7 @@
 #include "mix/hyper.hpp"
 #include "mix/linear_rows.hpp"
 #include "mix/linear_stream.hpp"
+#include "mix/linear_wide.hpp"
 #include "mix/short_conv.hpp"
 #include "mix/ssd.hpp"
 #include "mix/stream.hpp"
@@ -51,6 +52,15 @@ int launch_lds(dim3 grid, dim3 block, size_t lds, hipStream_t s, A... args) {
 }
 
 // ---- a portion's rows while the weight is the stream ------------------------
+int tile_args_ok(int after, const dvTileArgs* a) {
+  if (!a || !a->x || !a->W || a->n < 1 || a->M < 1 || a->K < 8) return DV_ERR_INVALID_ARG;
+  if (a->K % 8 || a->ldw % 8 || a->ldx % 8 || !al16(a->W) || !al16(a->x)) return DV_ERR_ALIGNMENT;
+  if (after != DV_OUT_RESIDUAL && !a->out) return DV_ERR_INVALID_ARG;
+  if (after == DV_OUT_GLU && a->M % 2) return DV_ERR_INVALID_ARG;
+  if (after == DV_OUT_RESIDUAL && (!a->res.x || !a->res.post.w || (a->res.h && !a->res.pre.w))) return DV_ERR_INVALID_ARG;
+  return DV_OK;
+}
+
 struct StreamPlan {
   int mb, nb;        // tile: rows of W, activation rows
   int rows, cols;    // tiles
@@ -497,11 +507,9 @@ size_t dv_mix_linear_tiles_workspace_bytes(int n, int M, int K) {
 }
 
 int dv_mix_linear_tiles_ws(int after, const dvTileArgs* a, void* workspace, size_t workspace_bytes, void* stream) {
-  if (!a || !a->x || !a->W || a->n < 1 || a->M < 1 || a->K < 8) return DV_ERR_INVALID_ARG;
-  if (a->K % 8 || a->ldw % 8 || a->ldx % 8 || !al16(a->W) || !al16(a->x) || !al16(workspace)) return DV_ERR_ALIGNMENT;
-  if (after != DV_OUT_RESIDUAL && !a->out) return DV_ERR_INVALID_ARG;
-  if (after == DV_OUT_GLU && a->M % 2) return DV_ERR_INVALID_ARG;
-  if (after == DV_OUT_RESIDUAL && (!a->res.x || !a->res.post.w || (a->res.h && !a->res.pre.w))) return DV_ERR_INVALID_ARG;
+  const int rc = tile_args_ok(after, a);
+  if (rc != DV_OK) return rc;
+  if (!al16(workspace)) return DV_ERR_ALIGNMENT;
   StreamPlan p = plan_stream(a->n, a->M, a->K);
   if (p.cols > 65535) return DV_ERR_UNSUPPORTED;
   const size_t need = dv_mix_linear_tiles_workspace_bytes(a->n, a->M, a->K);
@@ -514,6 +522,19 @@ int dv_mix_linear_tiles_ws(int after, const dvTileArgs* a, void* workspace, size
     case DV_OUT_RESIDUAL: return linear_stream<DV_OUT_RESIDUAL>(p, *a, workspace, st(stream));
     default: return DV_ERR_UNSUPPORTED;
   }
+}
+
+int dv_mix_linear_wide(int after, const dvTileArgs* a, void* stream) {
+  const int rc = tile_args_ok(after, a);
+  if (rc != DV_OK) return rc;
+  const int64_t rows = ((int64_t)a->M + kWideTile - 1) / kWideTile, cols = ((int64_t)a->n + kWideTile - 1) / kWideTile;
+  if (rows * cols > 0x7fffffff) return DV_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)(rows * cols)), threads(512);
+  if (after == DV_OUT_T)
+    return launch_lds<linear_wide_kernel<DV_OUT_T>>(grid, threads, kWideLds, st(stream), *a, (int)rows, (int)cols);
+  if (after == DV_OUT_GLU)
+    return launch_lds<linear_wide_kernel<DV_OUT_GLU>>(grid, threads, kWideLds, st(stream), *a, (int)rows, (int)cols);
+  return DV_ERR_UNSUPPORTED;
 }
 
 int dv_mix_linear_tiles(int after, const dvTileArgs* a, void* stream) {

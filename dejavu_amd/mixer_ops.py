@@ -96,13 +96,33 @@ def residual(y: Optional[torch.Tensor], stream: ResidualStream, post, pre, add_s
     return h
 
 
+# Where the 256 x 256 tiles of the wide kernel make two rounds of the chip's compute units or more and the chunks are many, it is
+# ahead of the library GEMM with the gated unit's launch (22016 x 4096 with 1500 / 1700 / 2048 / 3000 / 4096 rows: 290 / 304 /
+# 324 / 499 / 631 against 313 / 346 / 422 / 507 / 689 us; with 1280 rows, 430 tiles, 215 against 194), and for plain
+# products up to three rounds (18560 x 4096 with 1700 / 1999 / 3000 rows: 228 / 295 / 401 against 252 / 338 / 362;
+# 11264 x 2048 with 3000: 158 against 122).
+WIDE_TILE, WIDE_MIN_TILES, WIDE_MAX_PLAIN_TILES, WIDE_MIN_COLUMNS = 256, 500, 768, 4096
+
+
+def _aligned(x: torch.Tensor, W: torch.Tensor) -> bool:
+    return all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, W)) and x.shape[1] % 8 == 0 and W.shape[0] % 2 == 0
+
+
+def _wide(x: torch.Tensor, W: torch.Tensor, plain: bool) -> bool:
+    """Whether the wide kernel takes the product."""
+    M, K = W.shape
+    if x.dtype != torch.bfloat16 or K < WIDE_MIN_COLUMNS:
+        return False
+    tiles = -(-M // WIDE_TILE) * -(-x.shape[0] // WIDE_TILE)
+    return tiles >= WIDE_MIN_TILES and (not plain or tiles <= WIDE_MAX_PLAIN_TILES) and _aligned(x, W)
+
+
 def _tiles(x: torch.Tensor, W: torch.Tensor) -> bool:
     """Whether the streaming kernel takes the product.  From 65 rows on the library takes what it would refuse."""
     n = x.shape[0]
     if x.dtype != torch.bfloat16 or n <= 64:
         return x.dtype == torch.bfloat16
-    fits = all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, W)) and x.shape[1] % 8 == 0 and W.shape[0] % 2 == 0
-    return fits and (n <= TILE_ALL_ROWS or (n <= TILE_MAX_ROWS and W.numel() >= TILE_WEIGHT))
+    return (n <= TILE_ALL_ROWS or (n <= TILE_MAX_ROWS and W.numel() >= TILE_WEIGHT)) and _aligned(x, W)
 
 
 def _product_ok(x, W):
@@ -190,6 +210,12 @@ def linear(x, W: torch.Tensor, bias: Optional[torch.Tensor] = None, f32: bool = 
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
         _tile_launch(L.OUT_F32 if f32 else L.OUT_T, a, x.device)
         return out
+    if not f32 and _wide(x, W, True):
+        out = torch.empty(n, M, dtype=out_t, device=x.device)
+        a = _tile_args(x, W)
+        a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
+        check(lib.dv_mix_linear_wide(L.OUT_T, _ref(a), _stream()), "dv_mix_linear_wide")
+        return out
     return F.linear(x, W, bias)
 
 
@@ -207,6 +233,10 @@ def gated_unit(x, W: torch.Tensor, act: int, limit: float = 0.0) -> torch.Tensor
         a = _tile_args(x, W)
         a.out, a.ldo, a.act, a.limit = y.data_ptr(), M // 2, act, limit
         _tile_launch(L.OUT_GLU, a, x.device)
+    elif _wide(x, W, False):
+        a = _tile_args(x, W)
+        a.out, a.ldo, a.act, a.limit = y.data_ptr(), M // 2, act, limit
+        check(lib.dv_mix_linear_wide(L.OUT_GLU, _ref(a), _stream()), "dv_mix_linear_wide")
     else:
         gu = F.linear(x, W)
         check(lib.dv_mix_glu(code, _ptr(gu), y.numel(), act, limit, _ptr(y), _stream()), "dv_mix_glu")

@@ -292,6 +292,8 @@ DV_API int dv_mix_linear_row(int dtype, int before, int after, const dvRowArgs* 
 DV_API int dv_mix_linear_tiles(int after, const dvTileArgs* args, void* stream);
 DV_API size_t dv_mix_linear_tiles_workspace_bytes(int n, int M, int K);
 DV_API int dv_mix_linear_tiles_ws(int after, const dvTileArgs* args, void* workspace, size_t workspace_bytes, void* stream);
+/* The same product for many rows (DV_OUT_T and DV_OUT_GLU). */
+DV_API int dv_mix_linear_wide(int after, const dvTileArgs* args, void* stream);
 DV_API int dv_mix_short_conv(int dtype, int out_f32, const dvConvArgs* args, void* stream);
 DV_API int dv_mix_conv_state(int dtype, const void* in, int64_t ldi, int n, int channels, int taps, float* state,
                              void* stream);

@@ -52,6 +52,45 @@ def test_edges(n, K, M):
     close(h, f_pre(want), OP_LIMIT[BF16], "next norm")
 
 
+@pytest.mark.parametrize("n,K,M", [
+    (1, 8, 4), (256, 64, 256), (257, 72, 260), (300, 128, 514), (511, 200, 30),  # edges of tiles and chunks
+    (700, 1032, 2564),                                                          # 33 tiles: blocks of eight and a last one
+])
+def test_wide_tiles(n, K, M):
+    from dejavu_amd import _lib_mixers as L
+    from dejavu_amd import mixer_ops as ops
+
+    g = torch.Generator().manual_seed(n + M)
+    x = torch.randn(n, K + 8, generator=g).to(BF16).cuda()[:, :K]
+    W = (torch.randn(M, K, generator=g) * K ** -0.5).to(BF16).cuda()
+    bias = torch.randn(M, generator=g).to(BF16).cuda()
+    prod = host(x) @ host(W).T
+    for after, want in ((L.OUT_T, prod + host(bias)), (L.OUT_GLU, np.maximum(prod[:, 0::2], 0) * prod[:, 1::2])):
+        out = torch.empty(n, want.shape[1], dtype=BF16, device="cuda")
+        a = ops._tile_args(x, W)
+        a.out, a.ldo, a.act = out.data_ptr(), out.shape[1], L.GLU_RELU
+        a.bias = bias.data_ptr() if after == L.OUT_T else None
+        ops.check(ops.lib.dv_mix_linear_wide(after, ops._ref(a), ops._stream()), "dv_mix_linear_wide")
+        close(out, want, OP_LIMIT[BF16], f"{n}x{K}x{M}, after {after}")
+
+
+def test_wide_products_through_the_ops():
+    """A product on each side of the rule: 496 tiles go to the library, 512 to the wide kernel, both with the same result."""
+    from dejavu_amd import mixer_ops as ops
+
+    g = torch.Generator(device="cuda").manual_seed(1)
+    W = (torch.randn(31 * 256, 4096, generator=g, device="cuda") / 64).to(BF16)
+    x = torch.randn(4096 + 8, 4096, generator=g, device="cuda").to(BF16)
+    assert not ops._wide(x[:4096], W, True) and ops._wide(x, W, True) and not ops._wide(x[:, :2048], W[:, :2048], True)
+    for rows in (4096, 4096 + 8):
+        want = x[:rows].float() @ W.float().t()
+        got = ops.linear(x[:rows], W).float()
+        assert (got - want).norm() / want.norm() < 3e-3  # one rounding to bf16
+        unit = want[:, 0::2].clamp(min=0) * want[:, 1::2]
+        got = ops.relu_glu(x[:rows], W).float()
+        assert (got - unit).norm() / unit.norm() < 1e-2
+
+
 def test_unaligned_operands():
     """What the streaming kernel refuses is still multiplied where several kernels could."""
     from dejavu_amd import mixer_ops as ops
