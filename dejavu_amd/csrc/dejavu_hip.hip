@@ -12,8 +12,9 @@
 #include "common.hpp"
 #include "gemm_cols16.hpp"
 #include "gemm_mfma.hpp"
-#include "gemm_tiled.hpp"
 #include "gemm_big.hpp"
+#include "gemm_ring.hpp"
+#include "gemm_tiled.hpp"
 #include "gemv_cols.hpp"
 #include "gemv_rows.hpp"
 #include "layer_fused.hpp"
@@ -465,13 +466,6 @@ TiledPlan plan_tiled(int B, int N, int M) {
   return p;
 }
 
-bool big_applies(int B, int N);
-size_t tiled_workspace_bytes(int B, int N, int M) {
-  if (big_applies(B, N)) return 0;
-  const TiledPlan p = plan_tiled(B, N, M);
-  return p.nsplit > 1 ? (size_t)p.nsplit * B * M * sizeof(float) : 0;
-}
-
 template <int BT, int WT, int KC, int WAVES>
 int launch_tiled(const TiledPlan& p, const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const half_t* bias,
                  const void* idx, int idx_bytes, int B, int N, int Z, int M, half_t* Y, int64_t ldy, int relu,
@@ -486,12 +480,54 @@ int launch_tiled(const TiledPlan& p, const half_t* X, int64_t ldx, const half_t*
   return DV_OK;
 }
 
-// Many rows of X (two or more 128-row blocks): the product is bound by the matrix cores and by what
+// ---- products that share X (gemm_ring.hpp) ------------------------------------------
+struct RingLaunch {
+  template <auto KERNEL, typename... A>
+  int operator()(dim3 grid, dim3 threads, size_t lds, hipStream_t s, const A&... args) const {
+    static LdsGrant grant;
+    if (int rc = grant.ensure(reinterpret_cast<const void*>(KERNEL), lds); rc != DV_OK) return rc;
+    hipLaunchKernelGGL(KERNEL, grid, threads, lds, s, args...);
+    return launch_status();
+  }
+};
+
+// Splits need scratch: fewer, where the caller's does not hold them all, is an error as it always was.
+int ring_scratch(const RingPlan& p, const void* workspace, size_t workspace_bytes) {
+  if (p.splits > 1 && (workspace == nullptr || !aligned16(workspace) || workspace_bytes < p.workspace_bytes()))
+    return DV_ERR_WORKSPACE;
+  return DV_OK;
+}
+
+// Which kernel takes a product of B rows.  From 65 rows on the ring (12288 x 4096 with 100 / 190 / 256 rows: 31 / 38 / 46 us
+// against 39 / 59 / 57; QKV of 24 heads of 9216 with 96 / 160 / 240 rows 46 / 56 / 68 against 53 / 90 / 124; 32 heads of
+// 12288 with 320 and 480 rows 191 and 195 against 208 and 214 with gemm_big.hpp; 5120 x 20480 with 384 rows 134 against 245),
+// but not plain products of more than 512 rows, or of 16384 rows of W and more than 256, which gemm_big.hpp takes (20480 x
+// 5120 with 384 rows: 136 against 166).  Fewer rows are bound by the stream alone, and there
+// gemm_tiled.hpp, whose loads cover 512 bytes of a row, is ahead for large weights (12288 x 12288 with 16 / 64 rows: 58 / 68
+// against 71 / 89 us), the ring for small ones (4096 x 4096 with 50 rows 13 against 18; 4096 gathered rows of 12288 with 64
+// rows 27 against 31, with 32 rows 26 against 25; QKV of 16 heads of 5120 with 24 rows 19 against 23).
+enum class Shared { kRing, kTiled, kBig };
+Shared shared_kernel(int B, int N, int M, bool qkv) {
+  const int64_t weight = (int64_t)M * N;
+  if (!qkv && (B > 512 || (B > 256 && M > 16384))) return N % (kBgKC * kBgRing) == 0 ? Shared::kBig : Shared::kTiled;
+  if (B > 64) return Shared::kRing;
+  const int64_t most = B > 32 ? 52000000 : (qkv ? (B > 16 ? 32000000 : 0) : 20000000);
+  return weight <= most ? Shared::kRing : Shared::kTiled;
+}
+
+size_t tiled_workspace_bytes(int B, int N, int M, bool qkv = false) {
+  const Shared kind = shared_kernel(B, N, M, qkv);
+  if (kind == Shared::kBig) return 0;
+  if (kind == Shared::kRing) return plan_ring(B, M, N).workspace_bytes();
+  const TiledPlan p = plan_tiled(B, N, M);
+  return p.nsplit > 1 ? (size_t)p.nsplit * B * M * sizeof(float) : 0;
+}
+
+// Many rows of X: the product is bound by the matrix cores and by what
 // the L2 delivers, and gemm_big_mfma_kernel (weights straight into MFMA operands, 64 * WT weight rows
 // per workgroup) is the faster kernel -- measured at 12288 x 12288 against gemm_tiled_mfma_kernel:
-// 256 rows 172 against 259 us, 512 rows 225 against 278 us, 2048 rows 793 against 797 us.  Same bits.
+// 512 rows 225 against 278 us, 2048 rows 793 against 797 us.  Same bits.
 // WT: the tile height that fills the device best; on a tie the larger (fewer L2 reads per flop).
-bool big_applies(int B, int N) { return B >= 200 && N % (kBgKC * kBgRing) == 0; }
 int big_pick_wt(int B, int M, int max_wt) {
   const int cus = compute_units();
   const int xblocks = (B + kBgXRows - 1) / kBgXRows;
@@ -507,28 +543,23 @@ int big_pick_wt(int B, int M, int max_wt) {
   }
   return best_wt;
 }
-template <int WT, bool QKV>
+template <int WT>
 int launch_big(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const half_t* bias, const void* idx,
-               int idx_bytes, int B, int N, int Z, int M, half_t* Y, int64_t ldy, int act, const QkvScatter& qs,
-               hipStream_t s) {
-  auto kern = gemm_big_mfma_kernel<WT, QKV>;
+               int idx_bytes, int B, int N, int Z, int M, half_t* Y, int64_t ldy, int act, hipStream_t s) {
+  auto kern = gemm_big_mfma_kernel<WT>;
   static LdsGrant grant;
   if (int rc = grant.ensure(reinterpret_cast<const void*>(kern), big_lds_bytes()); rc != DV_OK) return rc;
   const dim3 grid((B + kBgXRows - 1) / kBgXRows, (M + 64 * WT - 1) / (64 * WT));
   hipLaunchKernelGGL(kern, grid, dim3(256), big_lds_bytes(), s, X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y,
-                     ldy, act, qs);
+                     ldy, act);
   return launch_status();
 }
-template <bool QKV>
 int gemm_big(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const half_t* bias, const void* idx,
-             int idx_bytes, int B, int N, int Z, int M, half_t* Y, int64_t ldy, int act, const QkvScatter& qs,
-             hipStream_t s) {
-  // (the scatter epilogue of the QKV form leaves no registers for the tallest tile)
-  constexpr int kMaxWt = QKV ? 3 : 4;
-  switch (big_pick_wt(B, M, kMaxWt)) {
-    case 2: return launch_big<2, QKV>(X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, act, qs, s);
-    case 3: return launch_big<3, QKV>(X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, act, qs, s);
-    default: return launch_big<(QKV ? 3 : 4), QKV>(X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, act, qs, s);
+             int idx_bytes, int B, int N, int Z, int M, half_t* Y, int64_t ldy, int act, hipStream_t s) {
+  switch (big_pick_wt(B, M, 4)) {
+    case 2: return launch_big<2>(X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, act, s);
+    case 3: return launch_big<3>(X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, act, s);
+    default: return launch_big<4>(X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, act, s);
   }
 }
 
@@ -536,12 +567,16 @@ int gemm_big(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const h
 int gemm_tiled_qkv(const half_t* X, int64_t ldx, const half_t* W, const half_t* bias, int B, int d, half_t* Y,
                    const QkvScatter& qs, void* workspace, size_t workspace_bytes, hipStream_t s) {
   const int M = 3 * qs.Hk * qs.hd, Z = 3 * qs.H * qs.hd;
-  if (big_applies(B, d))
-    return gemm_big<true>(X, ldx, W, (int64_t)d, bias, nullptr, 4, B, d, Z, M, Y, (int64_t)Z, 0, qs, s);
+  if (shared_kernel(B, d, M, true) == Shared::kRing) {
+    const RingPlan p = plan_ring(B, M, d);
+    if (int rc = ring_scratch(p, workspace, workspace_bytes); rc != DV_OK) return rc;
+    return gemm_ring(p, RingOperands<half_t>{X, ldx, W, (int64_t)d, B, M, d}, QkvRows{qs}, QkvOut{bias, Y, qs}, workspace, s,
+                     RingLaunch{});
+  }
   const TiledPlan p = plan_tiled(B, d, M);
   float* partial = nullptr;
   if (p.nsplit > 1) {
-    if (workspace == nullptr || !aligned16(workspace) || workspace_bytes < tiled_workspace_bytes(B, d, M))
+    if (workspace == nullptr || !aligned16(workspace) || workspace_bytes < tiled_workspace_bytes(B, d, M, true))
       return DV_ERR_WORKSPACE;
     partial = reinterpret_cast<float*>(workspace);
   }
@@ -579,8 +614,17 @@ int gemm_tiled_qkv(const half_t* X, int64_t ldx, const half_t* W, const half_t* 
 int gemm_tiled(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const half_t* bias, const void* idx,
                int idx_bytes, int B, int N, int Z, int M, int act, half_t* Y, int64_t ldy, void* workspace,
                size_t workspace_bytes, hipStream_t s) {
-  if (big_applies(B, N))
-    return gemm_big<false>(X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, act, QkvScatter{}, s);
+  const Shared kind = shared_kernel(B, N, M, false);
+  if (kind == Shared::kBig)
+    return gemm_big(X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, act, s);
+  if (kind == Shared::kRing) {
+    const RingPlan p = plan_ring(B, M, N);
+    if (int rc = ring_scratch(p, workspace, workspace_bytes); rc != DV_OK) return rc;
+    const RingOperands<half_t> a{X, ldx, W, ldw, B, M, N};
+    if (idx == nullptr) return gemm_ring(p, a, PlainRows{}, PlainOut{bias, act, Y, ldy, M}, workspace, s, RingLaunch{});
+    const GatheredRows rows{idx, idx_bytes, Z};
+    return gemm_ring(p, a, rows, GatheredOut{rows, bias, act, Y, ldy, M}, workspace, s, RingLaunch{});
+  }
   const TiledPlan p = plan_tiled(B, N, M);
   float* partial = nullptr;
   if (p.nsplit > 1) {
@@ -1278,7 +1322,7 @@ constexpr int kQkvTiledMinBatch = 9;
 
 size_t dv_qkv_proj_batch_workspace_bytes(int B, int d, int nnz, int hd) {
   if (B < kQkvTiledMinBatch || B > 32 || d <= 0 || nnz <= 0 || hd <= 0) return 0;
-  return tiled_workspace_bytes(B, d, 3 * nnz * hd);
+  return tiled_workspace_bytes(B, d, 3 * nnz * hd, true);
 }
 
 int dv_qkv_proj_batch_f16(const void* x, int64_t ldx, const void* W, const void* bias, const void* head_idx,
@@ -1696,7 +1740,7 @@ size_t dv_out_proj_sparse_t_ln_workspace_bytes(int B, int nnz, int hd, int N) {
 
 size_t dv_qkv_window_batch_workspace_bytes(int tokens, int nseq, int d, int nnz, int hd) {
   if (tokens < 1 || tokens > 16 || nseq < 1 || nseq > 32 || d <= 0 || nnz <= 0 || hd <= 0) return 0;
-  return tiled_workspace_bytes(tokens * nseq, d, 3 * nnz * hd);
+  return tiled_workspace_bytes(tokens * nseq, d, 3 * nnz * hd, true);
 }
 
 int dv_qkv_window_batch_f16(const void* x, int64_t ldx, const void* W, const void* bias, const void* head_idx,

@@ -1,6 +1,5 @@
-// Y[b, m] = act( sum_n X[b, n] * W[row(m), n] + bias[row(m)] ) for MANY rows of X (256 and more:
-// long prompts, the late positions of a batched back-fill window), where the product is bound by
-// the matrix cores and by LDS bandwidth rather than by the weight stream.
+// Y[b, m] = act( sum_n X[b, n] * W[row(m), n] + bias[row(m)] ) for MANY rows of X (more than 256:
+// long prompts), where the product is bound by the matrix cores and by LDS bandwidth rather than by the weight stream.
 //
 // gemm_tiled_mfma_kernel reads BOTH operands of every MFMA from LDS (the weights are staged through a
 // wavefront-private tile): 10 KiB of LDS reads per 16 MFMAs of a wavefront, more than the LDS delivers
@@ -20,7 +19,7 @@
 #pragma once
 #include "common.hpp"
 #include "gemm_mfma.hpp"
-#include "gemm_tiled.hpp"
+#include "gemm_out.hpp"
 
 namespace dv {
 
@@ -31,11 +30,11 @@ constexpr int kBgLd = kBgKC + 8;  // halfs per LDS row (bank spread)
 
 constexpr size_t big_lds_bytes() { return (size_t)2 * kBgXRows * kBgLd * sizeof(half_t); }
 
-template <int WT, bool QKV>
+template <int WT>
 __global__ __launch_bounds__(256, 1) void gemm_big_mfma_kernel(
     const half_t* __restrict__ X, int64_t ldx, const half_t* __restrict__ W, int64_t ldw,
     const half_t* __restrict__ bias, const void* __restrict__ idx, int idx_bytes, int B, int N, int Z, int M,
-    half_t* __restrict__ Y, int64_t ldy, int act, QkvScatter qs) {
+    half_t* __restrict__ Y, int64_t ldy, int act) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   half_t* xs = reinterpret_cast<half_t*>(smem_raw);  // [2][kBgXRows][kBgLd]
   constexpr int BT = kBgXRows / 16;
@@ -60,12 +59,8 @@ __global__ __launch_bounds__(256, 1) void gemm_big_mfma_kernel(
   int rid_mine = -1;  // weight row of output row m0 + lane (lanes < WROWS)
   if (lane < WROWS && m0 + lane < M) {
     const int m = m0 + lane;
-    if (QKV) {
-      rid_mine = qkv_row_of(qs, m);
-    } else {
-      const int64_t id = idx == nullptr ? (int64_t)m : load_index(idx, idx_bytes, m);
-      rid_mine = (id >= 0 && id < Z) ? (int)id : -1;
-    }
+    const int64_t id = idx == nullptr ? (int64_t)m : load_index(idx, idx_bytes, m);
+    rid_mine = (id >= 0 && id < Z) ? (int)id : -1;
   }
   // operand pointers: tile wt, row l16, k-group kg.  Rows out of range read row 0 (never stored).
   const half_t* wptr[WT];
@@ -162,11 +157,6 @@ __global__ __launch_bounds__(256, 1) void gemm_big_mfma_kernel(
   }
 
   // value v of a lane: output row m0 + wt * 16 + 4 * kg + v, X row b0 + bt * 16 + l16
-  QkvXRow xrow[QKV ? BT : 1];
-  if (QKV) {
-#pragma unroll
-    for (int bt = 0; bt < BT; ++bt) xrow[bt] = qkv_x_row(qs, b0 + bt * 16 + l16);
-  }
 #pragma unroll
   for (int wt = 0; wt < WT; ++wt) {
     const int mrow = m0 + wt * 16 + 4 * kg;
@@ -177,8 +167,6 @@ __global__ __launch_bounds__(256, 1) void gemm_big_mfma_kernel(
       rid[v] = __shfl(rid_mine, wt * 16 + 4 * kg + v, kWave);
       bv[v] = (bias != nullptr && rid[v] >= 0) ? (float)bias[rid[v]] : 0.f;
     }
-    QkvOutRows orow{};
-    if (QKV) orow = qkv_out_rows(qs, mrow, rid[0]);
 #pragma unroll
     for (int bt = 0; bt < BT; ++bt) {
       const int b = b0 + bt * 16 + l16;
@@ -188,11 +176,6 @@ __global__ __launch_bounds__(256, 1) void gemm_big_mfma_kernel(
       for (int v = 0; v < 4; ++v) {
         val[v] = rid[v] >= 0 ? acc[wt][bt][v] + bv[v] : 0.f;
         if (act) val[v] = act_f(val[v], act);
-      }
-      if (QKV) {
-        // the four values of a lane are four consecutive rows of one (q|k|v, head): hd % 4 == 0
-        qkv_store4(qs, Y, xrow[bt], orow, val);
-        continue;
       }
       half_t* dst = Y + (int64_t)b * ldy + mrow;
       if (mrow + 3 < M && (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(Y) & 7) == 0) {

@@ -1,0 +1,239 @@
+// Products of up to a few hundred rows with a weight on the matrix cores where the weight's bytes bound them, not the
+// operations: out(m, n) = sum_k W[rows(m), k] X[n, k], 16-bit operands, fp32 sums.
+//
+// A tile is MB rows of W by NB rows of X.  Both operands go from memory straight into a ring of ST LDS slots (no registers
+// on the way) ST - 1 chunks of KC columns ahead of their use: a wave's load covers 256 or 128 contiguous bytes of a row,
+// where loads in the matrix instruction's own layout cover 64 (a plain read of 22016 x 4096 in these pieces: 6.0, 5.2 and
+// 4.3 TB/s).  Where the tiles are fewer than the chip's workgroups, K is split over the grid and a second launch adds the
+// sums up; adding them up in the first one, by the workgroup that ends last, costs more (each hand-over between compute
+// dies 5 us, fences 40 us).
+//
+// 47 rows by 4096 x 4096 / 4096 x 11008 / 22016 x 4096: 12.5 / 24.5 / 41 us (loads in operand layout, 24 at a time: 24 / 47 /
+// 74); 16 rows 11 / 22 / 39 us (13 / 43 / 51).  Bound by the stream: 41 us are 4.4 TB/s beside a plain read's 6.
+#pragma once
+#include "common.hpp"
+
+namespace dv {
+
+typedef const __attribute__((address_space(1))) void* global_ptr_t;
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+typedef unsigned ring_word_t __attribute__((ext_vector_type(4)));  // eight elements
+
+// Waits until at most N of this wave's loads are still on their way.
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
+template <typename T>
+__device__ __forceinline__ float4_t ring_mfma(ring_word_t w, ring_word_t x, float4_t acc) {
+  typedef T vec_t __attribute__((ext_vector_type(8)));
+  const vec_t a = __builtin_bit_cast(vec_t, w), b = __builtin_bit_cast(vec_t, x);
+  if constexpr (__is_same(T, half_t)) return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+}
+
+template <typename T>
+struct RingOperands {
+  const T* X;
+  int64_t ldx;
+  const T* W;
+  int64_t ldw;
+  int n, M, K;  // K, ldx, ldw % 8 == 0, X and W on 16-byte boundaries
+};
+
+// Rows 0 .. M - 1 of the weight.
+struct PlainRows {
+  __device__ __forceinline__ int64_t operator()(int m) const { return m; }
+};
+
+struct RingPlan {
+  int mb, nb;        // tile: rows of W, rows of X
+  int rows, cols;    // tiles
+  int splits;        // of K
+  size_t workspace_bytes() const { return splits > 1 ? (size_t)splits * rows * cols * mb * nb * sizeof(float) : 0; }
+};
+
+// Up to 64 rows: tiles are as narrow as the rows allow; the taller one of 64 columns where it makes one round of
+// workgroups of what would be one and a half (22016 x 4096: 41 against 47 us with 47 rows, but 27.5 against 24.5 us at
+// 4096 x 11008).  K is split until there are about as many workgroups as compute units (4096 x 11008 with 47 rows: 1, 2, 4,
+// 8 splits take 52, 32, 24.5, 27 us); the narrowest tiles' workgroups are small, so they go on to two per unit.
+// More rows: 128 rows of W, so that X is fetched less often (5120 x 20480 with 96 rows: 53 us, 60 with 64 rows of W),
+// where that leaves 32 tiles and K is long enough to split; 192 where they fill the chip better (20480 x 5120 with 96 rows:
+// 107 tiles in 2 splits take 53 us, 160 tiles of 128 rows 59) or spare a round of it (36864 x 12288 with 128 rows: 192
+// tiles against 288).
+// A split has at least 256 columns.
+inline RingPlan plan_ring(int n, int M, int K) {
+  constexpr int kUnits = 256;
+  RingPlan p;
+  p.nb = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : n <= 128 ? 128 : n <= 192 ? 192 : 256;
+  auto lay = [&](int mb) {
+    p.mb = mb;
+    p.rows = (M + mb - 1) / mb;
+    p.cols = (n + p.nb - 1) / p.nb;
+    const int64_t tiles = (int64_t)p.rows * p.cols;
+    int64_t s = p.nb == 16 ? (tiles >= kUnits ? 1 : tiles >= kUnits / 2 ? 4 : 8) : (p.nb <= 64 ? 288 : kUnits) / tiles;
+    if (s > K / 256) s = K / 256;
+    p.splits = (int)(s < 1 ? 1 : s > 8 ? 8 : s);
+    return (int64_t)p.splits * tiles;
+  };
+  if (p.nb <= 64) {
+    lay(p.nb == 16 ? 32 : p.nb == 64 && M >= 16384 ? 96 : 64);
+  } else if (M < 32 * 128 || K < 2048) {
+    lay(64);
+  } else {
+    const bool tall = p.nb < 256 && K >= 4096;
+    const int64_t groups = lay(128);
+    if (tall) {
+      const int64_t more = lay(192), rounds = (groups + kUnits - 1) / kUnits, tall_rounds = (more + kUnits - 1) / kUnits;
+      const bool fuller = groups <= kUnits ? more <= kUnits && more * 10 > groups * 11 : tall_rounds * 192 < rounds * 128;
+      if (!fuller) lay(128);
+    }
+  }
+  return p;
+}
+
+// NT_W: the weight bypasses the caches (worth 10 % where the rows of X are few).
+// Out: called with (m, n, sums of rows m .. m + 3 and row n of X), m % 4 == 0, m < M, n < the operands' n.
+// Grid: (tiles of W, tiles of X, splits of K).  part: with several splits, the sums [split][tile][value][thread].
+template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, typename Rows, typename Out>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T> a, Rows rows, Out out, float4_t* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char slots[];
+  constexpr int WAVES = WM * WN, THREADS = WAVES * 64;
+  constexpr int CH = KC / 8;               // 16-byte pieces of a row's chunk
+  constexpr int RPL = 64 / CH;             // rows per load of a wave
+  constexpr int SWAP = (CH < 16 ? CH : 16) - 1;
+  constexpr int LI = (MB + NB) / RPL / WAVES;
+  constexpr int SLOT = (MB + NB) * KC * 2;
+  constexpr int RT = MB / WM / 16, NT = NB / WN / 16, KS = KC / 32;
+  static_assert((MB + NB) % (RPL * WAVES) == 0 && MB % RPL == 0, "loads do not tile");
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave % WM, wn = wave / WM, l16 = lane & 15, g = lane >> 4;
+  const int m0 = blockIdx.x * MB, n0 = blockIdx.y * NB;
+  const int nch = (a.K + KC - 1) / KC;
+  const int c0 = nch * blockIdx.z / gridDim.z, c1 = nch * (blockIdx.z + 1) / gridDim.z;
+
+  // A row's pieces lie in LDS at places exchanged by the row (place = piece ^ row), so that 16 rows' pieces are read
+  // from different banks; the lanes fetch them in that order.
+  const T* src[LI];
+  int piece[LI];
+#pragma unroll
+  for (int i = 0; i < LI; ++i) {
+    const int row = (wave * LI + i) * RPL + lane / CH;
+    piece[i] = (lane % CH) ^ (row & SWAP);
+    src[i] = row < MB ? a.W + rows(min(m0 + row, a.M - 1)) * a.ldw : a.X + (int64_t)min(n0 + row - MB, a.n - 1) * a.ldx;
+  }
+  const int pieces = a.K / 8;
+  auto load = [&](int c, int slot) {
+    // past the last piece: that one again (set to zero when it is used); past the last chunk: into a slot that is not read
+#pragma unroll
+    for (int i = 0; i < LI; ++i) {
+      const global_ptr_t from = (global_ptr_t)(src[i] + min(c * CH + piece[i], pieces - 1) * 8);
+      const lds_ptr_t to = (lds_ptr_t)(slots + slot * SLOT + (wave * LI + i) * 1024);
+      if (NT_W && (wave * LI + i) * RPL < MB) __builtin_amdgcn_global_load_lds(from, to, 16, 0, 2 /* read once */);
+      else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < ST - 1; ++d) load(c0 + d, d);
+
+  float4_t acc[RT][NT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+  int slot = 0;
+  for (int c = c0; c < c1; ++c) {
+    wait_loads<LI*(ST - 2)>();
+    __builtin_amdgcn_s_barrier();  // everybody's part of the slot is there, and the slot before it is free
+    asm volatile("" ::: "memory");
+    load(c + ST - 1, slot == 0 ? ST - 1 : slot - 1);
+    const unsigned char* wb = slots + slot * SLOT + (wm * RT * 16 + l16) * KC * 2;
+    const unsigned char* xb = slots + slot * SLOT + (MB + wn * NT * 16 + l16) * KC * 2;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int at = ((ks * 4 + g) ^ (l16 & SWAP)) * 16;
+      ring_word_t w[RT], x[NT];
+#pragma unroll
+      for (int i = 0; i < RT; ++i) w[i] = *reinterpret_cast<const ring_word_t*>(wb + i * 16 * KC * 2 + at);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) x[j] = *reinterpret_cast<const ring_word_t*>(xb + j * 16 * KC * 2 + at);
+      if ((c + 1) * CH > pieces && c * CH + ks * 4 + g >= pieces) {  // past the end of the rows
+#pragma unroll
+        for (int i = 0; i < RT; ++i) w[i] = ring_word_t{0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < NT; ++j) x[j] = ring_word_t{0, 0, 0, 0};
+      }
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = ring_mfma<T>(w[i], x[j], acc[i][j]);
+    }
+    slot = slot == ST - 1 ? 0 : slot + 1;
+  }
+  if (gridDim.z > 1) {
+    float4_t* p = part + (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (MB * NB / 4) + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) p[(i * NT + j) * THREADS] = acc[i][j];
+  } else {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int m = m0 + (wm * RT + i) * 16 + g * 4, n = n0 + (wn * NT + j) * 16 + l16;
+        if (m < a.M && n < a.n) out(m, n, acc[i][j]);
+      }
+  }
+  wait_loads<0>();  // no load into LDS outlives the workgroup
+}
+
+// Adds the splits' sums up, in their order.  Grid: (tiles of W, tiles of X, values of a thread).
+template <int MB, int NB, int WM, int WN, typename Out>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_ring_sum_kernel(int n_rows, int M, Out out, const float4_t* __restrict__ part, int splits) {
+  constexpr int THREADS = WM * WN * 64, RT = MB / WM / 16, NT = NB / WN / 16;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave % WM, wn = wave / WM;
+  const int i = blockIdx.z / NT, j = blockIdx.z % NT;
+  const int m = blockIdx.x * MB + (wm * RT + i) * 16 + (lane >> 4) * 4, n = blockIdx.y * NB + (wn * NT + j) * 16 + (lane & 15);
+  if (n >= n_rows || m >= M) return;
+  const int64_t step = (int64_t)gridDim.y * gridDim.x * (MB * NB / 4);
+  const float4_t* p = part + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (MB * NB / 4) + blockIdx.z * THREADS + threadIdx.x;
+  float4_t v = p[0];
+  for (int s = 1; s < splits; ++s) v += p[s * step];
+  out(m, n, v);
+}
+
+// launch(kernel as a template argument, grid, threads, LDS bytes, arguments) is the library's own way to launch with more
+// than 48 KiB of LDS.
+template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, typename Rows, typename Out, typename Launch>
+int gemm_ring_tiles(const RingPlan& p, const RingOperands<T>& a, const Rows& rows, const Out& out, void* workspace, hipStream_t s,
+                    const Launch& launch) {
+  float4_t* part = reinterpret_cast<float4_t*>(workspace);
+  const dim3 threads(WM * WN * 64);
+  const int rc = launch.template operator()<gemm_ring_kernel<T, MB, NB, KC, ST, WM, WN, NT_W, Rows, Out>>(
+      dim3(p.rows, p.cols, p.splits), threads, (size_t)ST * (MB + NB) * KC * 2, s, a, rows, out, part);
+  if (rc != 0 || p.splits == 1) return rc;
+  constexpr int values = (MB / WM / 16) * (NB / WN / 16);
+  return launch.template operator()<gemm_ring_sum_kernel<MB, NB, WM, WN, Out>>(dim3(p.rows, p.cols, values), threads, 0, s, a.n, a.M, out,
+                                                                               (const float4_t*)part, p.splits);
+}
+
+template <typename T, typename Rows, typename Out, typename Launch>
+int gemm_ring(const RingPlan& p, const RingOperands<T>& a, const Rows& rows, const Out& out, void* workspace, hipStream_t s,
+              const Launch& launch) {
+#define DV_RING(MB, NB, KC, ST, WM, WN, NT_W) gemm_ring_tiles<T, MB, NB, KC, ST, WM, WN, NT_W>(p, a, rows, out, workspace, s, launch)
+  switch (p.nb) {
+    case 16: return DV_RING(32, 16, 128, 4, 2, 1, true);
+    case 32: return DV_RING(64, 32, 64, 4, 4, 1, false);
+    case 64: return p.mb == 96 ? DV_RING(96, 64, 64, 4, 2, 2, false) : DV_RING(64, 64, 64, 4, 2, 2, false);
+    case 128: return p.mb == 64 ? DV_RING(64, 128, 64, 3, 2, 4, false)
+                     : p.mb == 128 ? DV_RING(128, 128, 64, 4, 2, 4, false) : DV_RING(192, 128, 64, 3, 2, 4, false);
+    case 192: return p.mb == 64 ? DV_RING(64, 192, 64, 4, 2, 4, false)
+                     : p.mb == 128 ? DV_RING(128, 192, 64, 3, 2, 4, false) : DV_RING(192, 192, 64, 3, 2, 4, false);
+    default: return p.mb == 64 ? DV_RING(64, 256, 64, 3, 2, 4, false) : DV_RING(128, 256, 64, 3, 2, 4, false);
+  }
+#undef DV_RING
+}
+
+}  // namespace dv

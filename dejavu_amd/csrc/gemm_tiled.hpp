@@ -23,6 +23,7 @@
 #pragma once
 #include "common.hpp"
 #include "gemm_mfma.hpp"
+#include "gemm_out.hpp"
 
 namespace dv {
 
@@ -32,106 +33,6 @@ constexpr int kTgPad = 8;  // halfs of padding per LDS row (bank spread)
 template <int BT, int WT, int KC, int WAVES = kTgWaves>
 constexpr size_t tiled_lds_bytes() {
   return (size_t)(2 * 16 * BT + WAVES * 16 * WT) * (KC + kTgPad) * sizeof(half_t);
-}
-
-// QKV mode: the M = 3 * Hk * hd output rows are the q, k, v rows of the selected heads
-// (m = (t * Hk + i) * hd + j -> weight row (t * H + head_idx[i]) * hd + j).  The X rows are `tokens`
-// window tokens of `nseq` sequences each, row r = s * nseq + b (tokens == 1: one token per sequence).
-// live[i * live_stride + s * live_tstride] < 0 skips (head i, token s); a head with no live token, or out
-// of range, is skipped altogether.  The result of token y_token goes to column `weight row` of
-// Y (nseq, 3, H, hd); the K / V rows of every live (head, token) are appended to the per-sequence caches
-// k_cache (nseq, H, hd/8, S, 8), v_cache (nseq, H, S, hd) at position
-// positions[per_sample ? b : 0] + pos_add + s.
-struct QkvScatter {
-  const int* head_idx;
-  const int* live;
-  int live_stride, Hk, H, hd;
-  half_t* k_cache;
-  half_t* v_cache;
-  const int* positions;
-  int per_sample, pos_add, S;
-  int nseq, tokens, live_tstride, y_token;
-};
-
-__device__ __forceinline__ int qkv_row_of(const QkvScatter& q, int m) {
-  const int t = m / (q.Hk * q.hd);
-  const int rem = m - t * q.Hk * q.hd;
-  const int i = rem / q.hd, j = rem - i * q.hd;
-  const int h = q.head_idx[i];
-  if (h < 0 || h >= q.H || t > 2) return -1;
-  if (q.live != nullptr) {
-    bool any = false;
-    for (int s = 0; s < q.tokens; ++s)
-      any |= q.live[(int64_t)i * q.live_stride + (int64_t)s * q.live_tstride] >= 0;
-    if (!any) return -1;
-  }
-  return (t * q.H + h) * q.hd + j;
-}
-
-// stores four finished values: consecutive output rows m .. m + 3 of X row r (m % 4 == 0, so they belong to
-// one head and one 8-pack of the key cache; weight rows rid .. rid + 3): one 8-byte store to Y for the token
-// that is wanted there and, for K / V rows, one to the cache
-__device__ __forceinline__ void qkv_store4(const QkvScatter& q, half_t* __restrict__ Y, int r, int m, int rid,
-                                           const float (&val)[4]) {
-  const int s = q.tokens > 1 ? r / q.nseq : 0;
-  const int b = r - s * q.nseq;
-  if (q.live != nullptr && q.tokens > 1) {
-    const int i = (m % (q.Hk * q.hd)) / q.hd;
-    if (q.live[(int64_t)i * q.live_stride + (int64_t)s * q.live_tstride] < 0) return;
-  }
-  const half4_t o = {(half_t)val[0], (half_t)val[1], (half_t)val[2], (half_t)val[3]};
-  if (s == q.y_token) *reinterpret_cast<half4_t*>(Y + (int64_t)b * 3 * q.H * q.hd + rid) = o;
-  if (q.k_cache == nullptr) return;
-  const int t = rid / (q.H * q.hd);
-  if (t == 0) return;
-  const int rem = rid - t * q.H * q.hd;
-  const int h = rem / q.hd, j = rem - h * q.hd;
-  const int dst = (q.positions ? q.positions[q.per_sample ? b : 0] : 0) + q.pos_add + s;
-  if (dst < 0 || dst >= q.S) return;
-  half_t* p = t == 1 ? q.k_cache + ((((int64_t)b * q.H + h) * (q.hd / 8) + j / 8) * q.S + dst) * 8 + (j & 7)
-                     : q.v_cache + (((int64_t)b * q.H + h) * q.S + dst) * q.hd + j;
-  *reinterpret_cast<half4_t*>(p) = o;
-}
-
-// qkv_store4 in two halves, for kernels whose lanes keep many (X row, output row) pairs: what depends
-// on the X row alone and what depends on the output rows alone is worked out once each.
-struct QkvXRow {  // X row r
-  int s, b, dst;  // window token, sequence, cache position (-1: not cached)
-};
-struct QkvOutRows {  // output rows m .. m + 3, weight rows rid .. rid + 3 (one head)
-  int i, t, rid;
-  int64_t head_off;  // ((h) * (hd / 8) + j / 8) * S * 8 + (j & 7) for K, h * S * hd + j for V, without the sequence
-};
-__device__ __forceinline__ QkvXRow qkv_x_row(const QkvScatter& q, int r) {
-  QkvXRow x;
-  x.s = q.tokens > 1 ? r / q.nseq : 0;
-  x.b = r - x.s * q.nseq;
-  const int dst = (q.positions ? q.positions[q.per_sample ? x.b : 0] : 0) + q.pos_add + x.s;
-  x.dst = (dst >= 0 && dst < q.S) ? dst : -1;
-  return x;
-}
-__device__ __forceinline__ QkvOutRows qkv_out_rows(const QkvScatter& q, int m, int rid) {
-  QkvOutRows o;
-  o.i = (m % (q.Hk * q.hd)) / q.hd;
-  o.rid = rid;
-  o.t = rid >= 0 ? rid / (q.H * q.hd) : 0;
-  const int rem = rid - o.t * q.H * q.hd;
-  const int h = rem / q.hd, j = rem - h * q.hd;
-  o.head_off = o.t == 1 ? ((int64_t)h * (q.hd / 8) + j / 8) * q.S * 8 + (j & 7) : (int64_t)h * q.S * q.hd + j;
-  return o;
-}
-__device__ __forceinline__ void qkv_store4(const QkvScatter& q, half_t* __restrict__ Y, const QkvXRow& x,
-                                           const QkvOutRows& o, const float (&val)[4]) {
-  if (o.rid < 0) return;
-  if (q.live != nullptr && q.tokens > 1 &&
-      q.live[(int64_t)o.i * q.live_stride + (int64_t)x.s * q.live_tstride] < 0)
-    return;
-  const half4_t v = {(half_t)val[0], (half_t)val[1], (half_t)val[2], (half_t)val[3]};
-  if (x.s == q.y_token) *reinterpret_cast<half4_t*>(Y + (int64_t)x.b * 3 * q.H * q.hd + o.rid) = v;
-  if (q.k_cache == nullptr || o.t == 0 || x.dst < 0) return;
-  half_t* p = o.t == 1 ? q.k_cache + (int64_t)x.b * q.H * q.hd * q.S + o.head_off + (int64_t)x.dst * 8
-                       : q.v_cache + (int64_t)x.b * q.H * q.S * q.hd + o.head_off + (int64_t)x.dst * q.hd;
-  *reinterpret_cast<half4_t*>(p) = v;
 }
 
 template <int BT, int WT, int KC, bool QKV = false, int WAVES = kTgWaves>

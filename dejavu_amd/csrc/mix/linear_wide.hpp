@@ -41,7 +41,7 @@ __global__ __launch_bounds__(512, 2) void linear_wide_kernel(TileArgs a, int row
   const bf16_t* X = reinterpret_cast<const bf16_t*>(a.x);
   const int nch = (a.K + KC - 1) / KC, pieces = a.K / 8;
 
-  // loads and places in LDS as in linear_stream_kernel
+  // loads and places in LDS as in gemm_ring_kernel
   const bf16_t* src[LI];
   int piece[LI];
 #pragma unroll
@@ -120,8 +120,10 @@ __global__ __launch_bounds__(512, 2) void linear_wide_kernel(TileArgs a, int row
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
-      tile_out<AFTER>(a, m0 + (wm * RT + i) * 16 + g * 4, n0 + (wn * NT + j) * 16 + l16, acc[i][j]);
+    for (int j = 0; j < NT; ++j) {
+      const int m = m0 + (wm * RT + i) * 16 + g * 4, n = n0 + (wn * NT + j) * 16 + l16;
+      if (m < a.M && n < a.n) tile_out<AFTER>(a, m, n, acc[i][j]);
+    }
 }
 
 }  // namespace dv

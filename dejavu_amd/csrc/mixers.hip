@@ -61,75 +61,17 @@ int tile_args_ok(int after, const dvTileArgs* a) {
   return DV_OK;
 }
 
-struct StreamPlan {
-  int mb, nb;        // tile: rows of W, activation rows
-  int rows, cols;    // tiles
-  int splits;        // of K
+struct MixLaunch {
+  template <auto KERNEL, typename... A>
+  int operator()(dim3 grid, dim3 threads, size_t lds, hipStream_t s, const A&... args) const {
+    return launch_lds<KERNEL>(grid, threads, lds, s, args...);
+  }
 };
 
-// Up to 64 rows: tiles are as narrow as the rows allow; the taller one of 64 columns where it makes one round of
-// workgroups of what would be one and a half (22016 x 4096: 41 against 47 us with 47 rows, but 27.5 against 24.5 us at
-// 4096 x 11008).  K is split until there are about as many workgroups as compute units (4096 x 11008 with 47 rows: 1, 2, 4,
-// 8 splits take 52, 32, 24.5, 27 us); the narrowest tiles' workgroups are small, so they go on to two per unit.
-// More rows: 128 rows of W, so that the activations are fetched less often (5120 x 20480 with 96 rows: 53 us, 60 with 64
-// rows of W), where that leaves 32 tiles and K is long enough to split; 192 where they fill the chip better (20480 x 5120
-// with 96 rows: 107 tiles in 2 splits take 53 us, 160 tiles of 128 rows 59).
-// A split has at least 256 columns.
-StreamPlan plan_stream(int n, int M, int K) {
-  constexpr int kUnits = 256;
-  StreamPlan p;
-  p.nb = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : n <= 128 ? 128 : n <= 192 ? 192 : n <= 256 ? 256 : 64;
-  auto lay = [&](int mb) {
-    p.mb = mb;
-    p.rows = (M + mb - 1) / mb;
-    p.cols = (n + p.nb - 1) / p.nb;
-    const int64_t tiles = (int64_t)p.rows * p.cols;
-    int64_t s = p.nb == 16 ? (tiles >= kUnits ? 1 : tiles >= kUnits / 2 ? 4 : 8) : (p.nb <= 64 ? 288 : kUnits) / tiles;
-    if (s > K / 256) s = K / 256;
-    p.splits = (int)(s < 1 ? 1 : s > 8 ? 8 : s);
-    return (int64_t)p.splits * tiles;
-  };
-  if (p.nb <= 64) {
-    lay(p.nb == 16 ? 32 : p.nb == 64 && M >= 16384 ? 96 : 64);
-  } else if (M < 32 * 128 || K < 2048) {
-    lay(64);
-  } else {
-    const bool tall = p.nb < 256 && K >= 4096;
-    const int64_t groups = lay(128);
-    if (tall && groups <= kUnits) {
-      const int64_t more = lay(192);
-      if (more > kUnits || more * 10 <= groups * 11) lay(128);
-    }
-  }
-  return p;
-}
-
-template <int AFTER, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W>
-int linear_stream_tiles(const StreamPlan& p, const TileArgs& a, void* workspace, hipStream_t s) {
-  float4_t* part = reinterpret_cast<float4_t*>(workspace);
-  const dim3 threads(WM * WN * 64);
-  const int rc = launch_lds<linear_stream_kernel<AFTER, MB, NB, KC, ST, WM, WN, NT_W>>(
-      dim3(p.rows, p.cols, p.splits), threads, (size_t)ST * (MB + NB) * KC * 2, s, a, part);
-  if (rc != DV_OK || p.splits == 1) return rc;
-  constexpr int values = (MB / WM / 16) * (NB / WN / 16);
-  hipLaunchKernelGGL((linear_stream_sum_kernel<AFTER, MB, NB, WM, WN>), dim3(p.rows, p.cols, values), threads, 0, s, a, part, p.splits);
-  return launched();
-}
-
 template <int AFTER>
-int linear_stream(const StreamPlan& p, const TileArgs& a, void* workspace, hipStream_t s) {
-  if (p.nb == 16) return linear_stream_tiles<AFTER, 32, 16, 128, 4, 2, 1, true>(p, a, workspace, s);
-  if (p.nb == 32) return linear_stream_tiles<AFTER, 64, 32, 64, 4, 4, 1, false>(p, a, workspace, s);
-  if (p.nb == 64 && p.mb == 96) return linear_stream_tiles<AFTER, 96, 64, 64, 4, 2, 2, false>(p, a, workspace, s);
-  if (p.nb == 64) return linear_stream_tiles<AFTER, 64, 64, 64, 4, 2, 2, false>(p, a, workspace, s);
-  if (p.nb == 128 && p.mb == 64) return linear_stream_tiles<AFTER, 64, 128, 64, 3, 2, 4, false>(p, a, workspace, s);
-  if (p.nb == 128 && p.mb == 128) return linear_stream_tiles<AFTER, 128, 128, 64, 4, 2, 4, false>(p, a, workspace, s);
-  if (p.nb == 128) return linear_stream_tiles<AFTER, 192, 128, 64, 3, 2, 4, false>(p, a, workspace, s);
-  if (p.nb == 192 && p.mb == 64) return linear_stream_tiles<AFTER, 64, 192, 64, 4, 2, 4, false>(p, a, workspace, s);
-  if (p.nb == 192 && p.mb == 128) return linear_stream_tiles<AFTER, 128, 192, 64, 3, 2, 4, false>(p, a, workspace, s);
-  if (p.nb == 192) return linear_stream_tiles<AFTER, 192, 192, 64, 3, 2, 4, false>(p, a, workspace, s);
-  if (p.mb == 64) return linear_stream_tiles<AFTER, 64, 256, 64, 3, 2, 4, false>(p, a, workspace, s);
-  return linear_stream_tiles<AFTER, 128, 256, 64, 3, 2, 4, false>(p, a, workspace, s);
+int linear_stream(const RingPlan& p, const TileArgs& a, void* workspace, hipStream_t s) {
+  const RingOperands<bf16_t> o{reinterpret_cast<const bf16_t*>(a.x), a.ldx, reinterpret_cast<const bf16_t*>(a.W), a.ldw, a.n, a.M, a.K};
+  return gemm_ring(p, o, PlainRows{}, MixOut<AFTER>{a}, workspace, s, MixLaunch{});
 }
 
 // ---- one row ---------------------------------------------------------------
@@ -502,19 +444,17 @@ int dv_mix_linear_row(int dtype, int before, int after, const dvRowArgs* a, void
 
 size_t dv_mix_linear_tiles_workspace_bytes(int n, int M, int K) {
   if (n < 1 || M < 1 || K < 8) return 0;
-  const StreamPlan p = plan_stream(n, M, K);
-  return p.splits > 1 ? (size_t)p.splits * p.rows * p.cols * p.mb * p.nb * sizeof(float) : 0;
+  return plan_ring(n, M, K).workspace_bytes();
 }
 
 int dv_mix_linear_tiles_ws(int after, const dvTileArgs* a, void* workspace, size_t workspace_bytes, void* stream) {
   const int rc = tile_args_ok(after, a);
   if (rc != DV_OK) return rc;
   if (!al16(workspace)) return DV_ERR_ALIGNMENT;
-  StreamPlan p = plan_stream(a->n, a->M, a->K);
+  RingPlan p = plan_ring(a->n, a->M, a->K);
   if (p.cols > 65535) return DV_ERR_UNSUPPORTED;
-  const size_t need = dv_mix_linear_tiles_workspace_bytes(a->n, a->M, a->K);
   if (!workspace) p.splits = 1;
-  else if (workspace_bytes < need) return DV_ERR_WORKSPACE;
+  else if (workspace_bytes < p.workspace_bytes()) return DV_ERR_WORKSPACE;
   switch (after) {
     case DV_OUT_F32: return linear_stream<DV_OUT_F32>(p, *a, workspace, st(stream));
     case DV_OUT_T: return linear_stream<DV_OUT_T>(p, *a, workspace, st(stream));

@@ -43,11 +43,13 @@ SIDE_STREAM_MIN_BATCH = 2
 # Prompt phase on this package's own kernels (dense products: dv_dense_linear_f16; causal attention
 # + cache fill: dv_prefill_attention_f16).  False: PyTorch's library GEMM and attention.
 USE_HIP_PROMPT = True
-# The dense products of a prompt are plain GEMMs.  Up to this many rows of X the package's X-shared
-# kernel is at least as fast as the library (it is bound by the weight stream: 85 against 96 us for
-# 128 rows x 12288 x 12288); beyond it the product is compute-bound and the library's GEMM is taken
-# (164 against 250 us at 512 rows, 515 against 763 us at 2048 rows on the same operands).
+# The dense products of a prompt are plain GEMMs.  Up to this many rows of X the package's kernel is at least as fast as
+# the library (it is bound by the weight stream: 5120 x 5120 with 128 / 190 rows 22 / 26 against 32 / 29 us, 15360 x 5120
+# with 190 rows 53 against 51 and a launch for the activation); beyond it the product is compute-bound and the library's
+# GEMM is taken -- but where the weight's rows are longer than they are many (fc2) it leaves most of the chip idle up to
+# HIP_PROMPT_LONG_MAX_ROWS rows (5120 x 20480 with 256 / 384 / 512 rows: 221 / 149 / 195 us, this package's kernel 84 / 134 / 135).
 HIP_PROMPT_MAX_ROWS = 192
+HIP_PROMPT_LONG_MAX_ROWS = 512
 # The package's causal-attention kernel (one wavefront per 16 queries, K / V straight from memory, cache fill
 # in the same launch) wins for short prompts (40 heads x 128: 29 us at 128 tokens against 36 us for the
 # library's attention plus the permuted cache copies) and loses from about 200 tokens on (512 tokens: 167
@@ -264,7 +266,8 @@ def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") ->
     on_hip = x.is_cuda and x.dtype == torch.float16 and linear.weight.dtype == torch.float16 and x.shape[-1] % 8 == 0
     if on_hip and x.dim() == 3 and x.shape[1] == 1 and x.shape[0] <= 64:
         return ops.dense_decode_linear(x, linear.weight, linear.bias, activation)
-    if on_hip and USE_HIP_PROMPT and x.numel() // x.shape[-1] <= HIP_PROMPT_MAX_ROWS:
+    most = HIP_PROMPT_LONG_MAX_ROWS if linear.in_features > linear.out_features else HIP_PROMPT_MAX_ROWS
+    if on_hip and USE_HIP_PROMPT and x.numel() // x.shape[-1] <= most:
         return ops.dense_linear(x, linear.weight, linear.bias, activation)
     y = linear(x)
     if activation == "relu":

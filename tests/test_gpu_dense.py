@@ -49,6 +49,46 @@ def test_dense_linear_matches_fp32_reference(rows, N, M, act):
     assert torch.equal(y, y2), "two runs differ (the split reduction must be deterministic)"
 
 
+# Both sides of the rules that choose a kernel and a tile (rows 64 | 65, 128 | 129, 192 | 193, 256 | 257, 512 | 513; weights of
+# 20 and 52 million elements; fewer than 32 tiles of 128 rows; rows of W too short to split), last tiles of one to four rows.
+@pytest.mark.parametrize("rows,N,M,act", [(9, 264, 70, "gelu"), (30, 4096, 4884, "id"), (20, 4096, 4100, "relu"),
+                                          (50, 12288, 4097, "id"), (65, 264, 70, "relu"), (128, 2056, 4099, "id"),
+                                          (100, 4104, 12290, "gelu_approx"), (129, 1032, 4101, "squared_relu"),
+                                          (192, 2048, 5121, "id"), (140, 4096, 18433, "id"), (193, 8, 33, "relu"),
+                                          (256, 2056, 4098, "relu"), (257, 520, 71, "id"), (512, 2056, 130, "relu"),
+                                          (513, 520, 70, "id"), (300, 256, 16390, "id")])
+def test_dense_linear_at_the_edges_of_its_rules(rows, N, M, act):
+    from dejavu_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(rows + M)
+    x = torch.randn(rows, N + 8, generator=g, device="cuda").half()[:, 8:]
+    W = (torch.randn(M, N, generator=g, device="cuda") * N ** -0.5).half()
+    b = torch.randn(M, generator=g, device="cuda").half()
+    print(f"case dense linear rows={rows} N={N} M={M} {act}", flush=True)
+    y = ops.dense_linear(x, W, b, act)
+    want = x.float() @ W.float().t() + b.float()
+    F = torch.nn.functional
+    want = {"id": want, "relu": want.relu(), "gelu": F.gelu(want), "gelu_approx": F.gelu(want, approximate="tanh"),
+            "squared_relu": want.relu() ** 2}[act]
+    assert_close(y.cpu().numpy(), want.cpu().numpy(), "dense linear", max_abs_tol=4e-2)  # half an ulp at 64: 0.031
+
+
+@pytest.mark.parametrize("rows", [40, 64])
+def test_gathered_rows_out_of_range(rows):
+    """An index outside the weight gives act(0), whichever kernel runs."""
+    from dejavu_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x, W = torch.randn(rows, 520, generator=g, device="cuda").half(), torch.randn(90, 520, generator=g, device="cuda").half()
+    b = torch.randn(90, generator=g, device="cuda").half()
+    idx = torch.tensor([3, -1, 89, 90, 0, 7, 1 << 40], device="cuda")
+    ok = (idx >= 0) & (idx < 90)
+    want = torch.zeros(rows, idx.numel(), device="cuda")
+    want[:, ok] = (x.float() @ W[idx[ok]].float().t() + b[idx[ok]].float()).relu()
+    got = ops.gather_gemv(x, W, idx, b, activation="relu")
+    assert_close(got.float().cpu().numpy(), want.cpu().numpy(), "gathered rows", max_abs_tol=8e-2)  # half an ulp at 128
+
+
 def test_dense_linear_three_dimensional_input():
     from dejavu_amd import ops
 
