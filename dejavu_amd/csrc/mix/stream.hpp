@@ -175,8 +175,11 @@ __global__ __launch_bounds__(256) void gated_head_norm_kernel(const float* __res
   }
 }
 
-// First index of the largest of `vocab` fp32 logits, and the bookkeeping of a generation loop (one workgroup):
-// token <- argmax, sequences[out_index++] <- token, position++, seq_pos++, scores[score_index++] <- logits.
+// First index of the largest of `vocab` fp32 logits (NaN ranks highest), and the bookkeeping of a generation loop (one
+// workgroup): token <- argmax, sequences[out_index++] <- token, position++, seq_pos++, scores[score_index++] <- logits.
+// Bound by the latency of its loads: eight of 16 bytes per thread are on their way at once, and the row of scores is stored
+// from registers (32768 logits: 11 us; one load at a time 17).  More workgroups would need a second launch or a
+// hand-over between compute dies, 5 us.
 __global__ __launch_bounds__(1024) void greedy_advance_f32_kernel(
     const float* __restrict__ logits, int vocab, int64_t* __restrict__ token, int64_t* __restrict__ position,
     int* __restrict__ seq_pos, int64_t* __restrict__ sequences, int64_t* __restrict__ out_index,
@@ -188,20 +191,39 @@ __global__ __launch_bounds__(1024) void greedy_advance_f32_kernel(
   int at = 0x7fffffff;
   const int64_t srow = scores ? *score_index : 0;
   const bool keep = scores && srow >= 0 && srow < score_rows;
-  for (int i = threadIdx.x; i < vocab; i += blockDim.x) {
-    const float v = logits[i];
-    if (v > best || at == 0x7fffffff) {
-      best = v;
-      at = i;
-    }
-    if (keep) scores[srow * score_ld + i] = v;
-  }
+  float* row = keep ? scores + srow * score_ld : nullptr;
   auto merge = [&](float ov, int oi) {
-    if (ov > best || (ov == best && oi < at)) {
+    const bool above = ov > best || (ov != ov && best == best);
+    if (above || ((ov == best || (ov != ov && best != best)) && oi < at)) {
       best = ov;
       at = oi;
     }
   };
+  constexpr int U = 8;
+  const bool wide_in = (reinterpret_cast<uintptr_t>(logits) & 15) == 0, wide_out = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
+  const int quads = wide_in ? vocab / 4 : 0;
+  for (int q0 = threadIdx.x; q0 < quads; q0 += U * 1024) {
+    float4_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = reinterpret_cast<const float4_t*>(logits)[min(q0 + u * 1024, quads - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = q0 + u * 1024;
+      if (q >= quads) break;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) merge(v[u][e], 4 * q + e);
+      if (row && wide_out) reinterpret_cast<float4_t*>(row)[q] = v[u];
+      else if (row) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) row[4 * q + e] = v[u][e];
+      }
+    }
+  }
+  for (int i = quads * 4 + threadIdx.x; i < vocab; i += 1024) {
+    const float v = logits[i];
+    merge(v, i);
+    if (row) row[i] = v;
+  }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     const float ov = __shfl_xor(best, off, kWave);

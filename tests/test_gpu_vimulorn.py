@@ -419,3 +419,31 @@ def test_trace_run_program(tmp_path, dtype):
     close(read(3), lb[[1]], limit, "other sequence")
     close(read(4), lb[[24, 5]], limit, "its rest, places in the order asked for")
     assert not (out / "2.f32").exists()
+
+
+@pytest.mark.parametrize("vocab", [3, 4100, 32768, 40003])
+def test_greedy_advance_of_fp32_logits(vocab):
+    """First index of the largest logit (NaN on top), the bookkeeping and the row of scores, from rows that start on a
+    16-byte boundary and rows that do not."""
+    from dejavu_amd import mixer_ops as ops
+
+    g = torch.Generator().manual_seed(vocab)
+    rows = {"random": torch.randn(vocab, generator=g), "ties": torch.randint(0, 3, (vocab,), generator=g).float(),
+            "lowest": torch.full((vocab,), -float("inf"))}
+    rows["nan"] = rows["random"].clone()
+    rows["nan"][vocab // 2] = float("nan")
+    for shift in (0, 1):
+        for ld in (vocab, vocab + 1):
+            for name, row in rows.items():
+                logits = torch.cat([row[:shift], row]).cuda()[shift:]
+                token, position, out_index, score_index = (torch.full((1, 1), v, dtype=torch.long, device="cuda") for v in (0, 5, 2, 1))
+                seq_pos = torch.full((1,), 5, dtype=torch.int32, device="cuda")
+                sequences = torch.full((1, 6), -1, dtype=torch.long, device="cuda")
+                scores = torch.zeros(3, ld, device="cuda")[:, :vocab]
+                ops.greedy_advance(logits, token, position, seq_pos, sequences, out_index, scores, score_index)
+                want = int(torch.argmax(row))
+                if name == "ties":
+                    want = int((row == row.max()).nonzero()[0])
+                assert int(token) == want and sequences.tolist() == [[-1, -1, want, -1, -1, -1]], (name, shift, ld)
+                assert [int(t) for t in (position, seq_pos, out_index, score_index)] == [6, 6, 3, 2]
+                assert torch.equal(scores[1].view(torch.int32), logits.view(torch.int32)) and not scores[0].any() and not scores[2].any()
