@@ -5,6 +5,7 @@
 
 #include <atomic>
 
+#include "mix/attn_f32.hpp"
 #include "mix/attn_latent.hpp"
 #include "mix/attn_rows.hpp"
 #include "mix/attn_tiles.hpp"
@@ -205,6 +206,16 @@ int attn_args_ok(const AttnArgs* a) {
       !al16(a->v) || !al16(a->q))
     return DV_ERR_ALIGNMENT;
   if (a->vdim_s > 2048 || a->n > 65535 || (int64_t)a->H > 65535) return DV_ERR_UNSUPPORTED;
+  return DV_OK;
+}
+
+// A portion's queries against keys and values that lie in a row.
+int attn_portion_ok(const dvAttnArgs* a, int keys) {
+  const int rc = attn_args_ok(a);
+  if (rc != DV_OK) return rc;
+  if (!a->out || a->ring > 0 || a->fresh_k || a->norm_dim > 0 || a->pos_dev || keys < 1 ||
+      a->pos_host - a->base < 0 || a->pos_host - a->base + a->n > keys)
+    return DV_ERR_INVALID_ARG;
   return DV_OK;
 }
 
@@ -541,12 +552,26 @@ int dv_mix_attn_rows(int dtype, int q_f32, const dvAttnArgs* a, void* stream) {
   return launched();
 }
 
-int dv_mix_attn_tiles(const dvAttnArgs* a, int keys, void* stream) {
-  int rc = attn_args_ok(a);
+int dv_mix_attn_tiles_f32(const dvAttnArgs* a, int keys, void* stream) {
+  const int rc = attn_portion_ok(a, keys);
   if (rc != DV_OK) return rc;
-  if (!a->out || a->ring > 0 || a->fresh_k || a->norm_dim > 0 || a->pos_dev || keys < 1 ||
-      a->pos_host - a->base < 0 || a->pos_host - a->base + a->n > keys)
-    return DV_ERR_INVALID_ARG;
+  if (a->ldq % 4 || !al16(a->out)) return DV_ERR_ALIGNMENT;
+  const int64_t groups = ((int64_t)a->n + kF32Q - 1) / kF32Q * a->H;
+  if (a->dim_s > 128 || a->vdim_s > 128 || groups > 0x7fffffff) return DV_ERR_UNSUPPORTED;
+#define DV_ATT(DU, VT) \
+  return launch_lds<attn_f32_kernel<DU, VT>>(dim3((unsigned)groups), dim3(256), f32_lds(VT), st(stream), *a, keys)
+  if (a->dim_s <= 64) {
+    if (a->vdim_s <= 64) DV_ATT(8, 2);
+    DV_ATT(8, 4);
+  }
+  if (a->vdim_s <= 64) DV_ATT(16, 2);
+  DV_ATT(16, 4);
+#undef DV_ATT
+}
+
+int dv_mix_attn_tiles(const dvAttnArgs* a, int keys, void* stream) {
+  const int rc = attn_portion_ok(a, keys);
+  if (rc != DV_OK) return rc;
   if (a->ldq % 8) return DV_ERR_ALIGNMENT;
   const int dt = (a->dim_s + 15) / 16, vt = (a->vdim_s + 31) / 32;
 #define DV_TILES_V(DT)                                                        \

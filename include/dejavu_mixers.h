@@ -304,6 +304,8 @@ DV_API int dv_mix_ring_copy(int dtype, void* buf, int64_t ldb, void* ring, int c
 DV_API int dv_mix_attn_rows(int dtype, int q_f32, const dvAttnArgs* args, void* stream);
 /* bf16, a portion on the matrix cores; `keys` rows behind k and v (contiguous, ring = 0). */
 DV_API int dv_mix_attn_tiles(const dvAttnArgs* args, int keys, void* stream);
+/* The same in fp32. */
+DV_API int dv_mix_attn_tiles_f32(const dvAttnArgs* args, int keys, void* stream);
 /* Latent decode row: out [H][rank] = q[h] W_uk[h]; W [H][dim_s][rank]. */
 DV_API int dv_mix_latent_absorb(int dtype, const float* q, const void* W, int H, int dim_s, int rank, float* out,
                                 void* stream);

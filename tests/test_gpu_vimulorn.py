@@ -145,6 +145,41 @@ def test_portion_attention(T, H, G, dim, vdim, window, dtype):
         lo = hi
 
 
+# fp32 sums over at most 128 entries and T keys; the oracle works in fp64: OP_LIMIT[float32]
+@pytest.mark.parametrize("T,H,G,dim,vdim,window,chunk,undefined", [
+    (31, 2, 1, 8, 8, None, None, None), (32, 3, 3, 64, 64, 5, None, 30), (33, 2, 2, 72, 72, None, 7, 32),
+    (129, 4, 2, 128, 128, None, None, 100), (161, 2, 1, 128, 40, 33, None, 64), (290, 2, 1, 40, 128, None, 64, 130)])
+def test_fp32_portions_on_the_matrix_cores(T, H, G, dim, vdim, window, chunk, undefined, monkeypatch):
+    """Edges of the tiles of 32 queries and keys and of both head sizes, whole and after earlier keys; infinite values
+    reach the queries that see them, and no other."""
+    from dejavu_amd import mixer_ops as ops
+
+    monkeypatch.setattr(ops, "F32_TILE_ROWS", 1)
+    q, k, v = (host(dev(a)) for a in _attention_case(T, H, G, dim, vdim, seed=T, sharp=2.0))
+    gate, rel = (host(dev(np.random.default_rng(s).normal(size=(n, H)))) for s, n in ((1, T), (2, 20)))
+    back = np.arange(T)[:, None] - np.arange(T)[None]
+    seen = (back >= 0) & (back < (window or T)) & ((np.arange(T)[:, None] // (chunk or T)) == (np.arange(T)[None] // (chunk or T)))
+    bias = rel.T[:, np.clip(back, 0, 19)]
+    s = np.einsum("qhd,khd->hqk", q, np.repeat(k, H // G, 1)) * 0.2 + bias
+    e = np.where(seen, np.exp(np.where(seen, s, 0.0)), 0.0)
+    want = np.einsum("hqk,khd->qhd", e / e.sum(-1, keepdims=True), np.repeat(v, H // G, 1)) * V.sigmoid(gate)[:, :, None]
+    at = np.zeros(T, bool)
+    if undefined is not None:
+        v[undefined, 0, 3] = np.inf
+        at = seen[:, undefined]
+        assert at.any() and not at.all()
+    qt, kt, vt, gt = (dev(a.reshape(T, -1)) for a in (q, k, v, gate))
+    for lo in (0, 1, T // 2):
+        first = max(0, lo - window + 1) if window else lo // chunk * chunk if chunk else 0
+        got = host(ops.portion_attention(qt[lo:], kt[first:], vt[first:], H, G, 0.2, first, lo, gate=gt[lo:], window=window,
+                                         chunk=chunk, rel=dev(rel.T.copy()))).reshape(T - lo, H, vdim)
+        hit = np.zeros((T, H, vdim), bool)
+        hit[at, :H // G, 3] = True
+        assert np.isposinf(got[hit[lo:]]).all()
+        got[hit[lo:]] = want[lo:][hit[lo:]]
+        close(got.reshape(T - lo, -1), want[lo:].reshape(T - lo, -1), OP_LIMIT[torch.float32], f"from {lo}")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("distance,window", [(39, 40), (40, 40), (63, 64), (64, 64), (127, 128), (128, 128), (200, None), (0, 1)])
 def test_a_single_key_at_the_edge_of_a_window(distance, window, dtype):
