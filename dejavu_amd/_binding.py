@@ -7,6 +7,19 @@ import os
 import torch  # noqa: F401  (loads the HIP runtime that the libraries bind to)
 
 
+def results_only(*tensors) -> bool:
+    """Whether a kernel may stand in for a library call that also knows gradients, functional transforms, tracers,
+    autocast, tensor subclasses and other devices: plain tensors of the current device, and none of these asked for."""
+    here = torch.cuda.current_device() if torch.cuda.is_initialized() else -1
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (not t.is_cuda or t.device.index != here or (grad and t.requires_grad) or
+                              type(t) not in (torch.Tensor, torch.nn.Parameter)):
+            return False
+    return (torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None and
+            not torch.is_autocast_enabled() and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+
+
 class DejavuHipError(RuntimeError):
     """An entry point of a kernel library returned a non-zero status."""
 

@@ -16,6 +16,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib_mixers as L
+from ._binding import results_only
 from ._lib_mixers import check, lib
 
 # The streaming kernel against the library GEMM without the launch that follows it, us: 4096 x 11008 with 96 / 192 / 256
@@ -108,21 +109,21 @@ def _aligned(x: torch.Tensor, W: torch.Tensor) -> bool:
     return all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, W)) and x.shape[1] % 8 == 0 and W.shape[0] % 2 == 0
 
 
-def _wide(x: torch.Tensor, W: torch.Tensor, plain: bool) -> bool:
+def _wide(x: torch.Tensor, W: torch.Tensor, plain: bool, bias=None) -> bool:
     """Whether the wide kernel takes the product."""
     M, K = W.shape
     if x.dtype != torch.bfloat16 or K < WIDE_MIN_COLUMNS:
         return False
     tiles = -(-M // WIDE_TILE) * -(-x.shape[0] // WIDE_TILE)
-    return tiles >= WIDE_MIN_TILES and (not plain or tiles <= WIDE_MAX_PLAIN_TILES) and _aligned(x, W)
+    return tiles >= WIDE_MIN_TILES and (not plain or tiles <= WIDE_MAX_PLAIN_TILES) and results_only(x, W, bias) and _aligned(x, W)
 
 
-def _tiles(x: torch.Tensor, W: torch.Tensor) -> bool:
+def _tiles(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
     """Whether the streaming kernel takes the product.  From 65 rows on the library takes what it would refuse."""
     n = x.shape[0]
     if x.dtype != torch.bfloat16 or n <= 64:
         return x.dtype == torch.bfloat16
-    return (n <= TILE_ALL_ROWS or (n <= TILE_MAX_ROWS and W.numel() >= TILE_WEIGHT)) and _aligned(x, W)
+    return (n <= TILE_ALL_ROWS or (n <= TILE_MAX_ROWS and W.numel() >= TILE_WEIGHT)) and results_only(x, W, bias) and _aligned(x, W)
 
 
 def _product_ok(x, W):
@@ -204,13 +205,13 @@ def linear(x, W: torch.Tensor, bias: Optional[torch.Tensor] = None, f32: bool = 
         _row_launch(code, before, L.OUT_F32 if f32 else L.OUT_T, a)
         return out
     code = _product_ok(x, W)
-    if _tiles(x, W) or (f32 and code == L.BF16):
+    if _tiles(x, W, bias) or (f32 and code == L.BF16):
         out = torch.empty(n, M, dtype=out_t, device=x.device)
         a = _tile_args(x, W)
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
         _tile_launch(L.OUT_F32 if f32 else L.OUT_T, a, x.device)
         return out
-    if not f32 and _wide(x, W, True):
+    if not f32 and _wide(x, W, True, bias):
         out = torch.empty(n, M, dtype=out_t, device=x.device)
         a = _tile_args(x, W)
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)

@@ -23,6 +23,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops
+from ._binding import results_only
 from ._lib import check, lib
 from .inference import InferenceParams  # noqa: F401  (part of this module's interface)
 
@@ -266,8 +267,11 @@ def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") ->
     on_hip = x.is_cuda and x.dtype == torch.float16 and linear.weight.dtype == torch.float16 and x.shape[-1] % 8 == 0
     if on_hip and x.dim() == 3 and x.shape[1] == 1 and x.shape[0] <= 64:
         return ops.dense_decode_linear(x, linear.weight, linear.bias, activation)
-    most = HIP_PROMPT_LONG_MAX_ROWS if linear.in_features > linear.out_features else HIP_PROMPT_MAX_ROWS
-    if on_hip and USE_HIP_PROMPT and x.numel() // x.shape[-1] <= most:
+    rows = x.numel() // x.shape[-1] if on_hip and USE_HIP_PROMPT else HIP_PROMPT_LONG_MAX_ROWS + 1
+    if rows <= HIP_PROMPT_MAX_ROWS or (
+            rows <= HIP_PROMPT_LONG_MAX_ROWS and linear.in_features > linear.out_features and
+            type(linear) is nn.Linear and not linear._forward_hooks and not linear._forward_pre_hooks and
+            results_only(x, linear.weight, linear.bias)):
         return ops.dense_linear(x, linear.weight, linear.bias, activation)
     y = linear(x)
     if activation == "relu":
