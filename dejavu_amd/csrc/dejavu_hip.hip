@@ -1373,16 +1373,16 @@ int dv_prefill_attention_f16(const void* qkv, int B, int T, int H, int hd, float
   if (!aligned16(qkv) || (k_cache && (!aligned16(k_cache) || !aligned16(v_cache)))) return DV_ERR_ALIGNMENT;
   if (T == 0) return DV_OK;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid((T + kPfWaves * 16 - 1) / (kPfWaves * 16), H, B);
-  if (hd == 128)
-    hipLaunchKernelGGL(prefill_attn_kernel<128>, grid, dim3(kPfWaves * 64), 0, s, reinterpret_cast<const half_t*>(qkv),
-                       T, H, scale, reinterpret_cast<half_t*>(ctx), reinterpret_cast<half_t*>(k_cache),
-                       reinterpret_cast<half_t*>(v_cache), pos0, S);
-  else
-    hipLaunchKernelGGL(prefill_attn_kernel<64>, grid, dim3(kPfWaves * 64), 0, s, reinterpret_cast<const half_t*>(qkv),
-                       T, H, scale, reinterpret_cast<half_t*>(ctx), reinterpret_cast<half_t*>(k_cache),
-                       reinterpret_cast<half_t*>(v_cache), pos0, S);
-  return launch_status();
+  const int64_t groups = ((int64_t)T + kPfQueries - 1) / kPfQueries * H;
+  if (groups > 0x7fffffff) return DV_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)groups, B);
+#define DV_PF(HD)                                                                                              \
+  RingLaunch{}.operator()<prefill_attn_kernel<HD>>(                                                            \
+      grid, dim3(kPfWaves * 64), pf_lds(HD), s, reinterpret_cast<const half_t*>(qkv), T, H, scale,             \
+      reinterpret_cast<half_t*>(ctx), (int)aligned16(ctx), reinterpret_cast<half_t*>(k_cache),                 \
+      reinterpret_cast<half_t*>(v_cache), pos0, S)
+  return hd == 128 ? DV_PF(128) : DV_PF(64);
+#undef DV_PF
 }
 
 int dv_kv_cache_copy_sparse_f16(const void* k, const void* v, int64_t ld_src, int nsrc,

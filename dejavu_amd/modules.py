@@ -51,10 +51,10 @@ USE_HIP_PROMPT = True
 # HIP_PROMPT_LONG_MAX_ROWS rows (5120 x 20480 with 256 / 384 / 512 rows: 221 / 149 / 195 us, this package's kernel 84 / 134 / 135).
 HIP_PROMPT_MAX_ROWS = 192
 HIP_PROMPT_LONG_MAX_ROWS = 512
-# The package's causal-attention kernel (one wavefront per 16 queries, K / V straight from memory, cache fill
-# in the same launch) wins for short prompts (40 heads x 128: 29 us at 128 tokens against 36 us for the
-# library's attention plus the permuted cache copies) and loses from about 200 tokens on (512 tokens: 167
-# against 53 us; 2048: 1461 against 216 us): longer prompts take the library's attention and the copies.
+# The package's causal-attention kernel (cache fill in the same launch) is ahead of the library's attention with the
+# permuted cache copies at all lengths (40 heads of 128 and 128 / 1024 tokens: 7.5 / 47 us against 25 / 100; 32 heads and
+# 777 / 2000 / 4000 tokens: 30 / 110 / 385 against 75 / 310 / 566).  Prompts of more than so many tokens leave gradients,
+# functional transforms and the like to the library.
 HIP_PROMPT_ATTN_MAX_TOKENS = 192
 
 _side_streams: dict = {}
@@ -359,7 +359,7 @@ class _MHABase(nn.Module):
         if inference_params is None or inference_params.sequence_len_offset == 0:
             causal = self.causal if inference_params is None else True
             if USE_HIP_PROMPT and qkv.is_cuda and qkv.dtype == torch.float16 and qkv.shape[-1] in (64, 128) \
-                    and (causal or s == 1) and s <= HIP_PROMPT_ATTN_MAX_TOKENS:
+                    and (causal or s == 1) and (s <= HIP_PROMPT_ATTN_MAX_TOKENS or results_only(qkv)):
                 # causal attention and the cache fill in one launch (no permuted copy of K / V)
                 kc = vc = None
                 if inference_params is not None:
@@ -368,7 +368,9 @@ class _MHABase(nn.Module):
                                                   qkv.dtype, qkv.device)
                     b0 = inference_params.batch_size_offset
                     kc, vc = k_cache[b0:b0 + B], v_cache[b0:b0 + B]
-                return ops.prefill_attention(qkv.contiguous(), kc, vc, 0, scale)
+                if s <= HIP_PROMPT_ATTN_MAX_TOKENS or kc is None or (  # the copies fill a caller's own caches of any stride
+                        kc.is_contiguous() and vc.is_contiguous() and results_only(kc, vc)):
+                    return ops.prefill_attention(qkv.contiguous(), kc, vc, 0, scale)
             if inference_params is not None:
                 assert self.layer_idx is not None, "Generation requires layer_idx in the constructor"
                 _update_kv_cache(qkv[:, :, 1:], inference_params, self.layer_idx)

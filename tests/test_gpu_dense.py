@@ -174,3 +174,42 @@ def test_prompt_runs_on_the_hip_kernels_and_matches_the_library_path(T):
         for got, ref, o in zip(caches[0][l], caches[1][l], state["caches"][l]):
             assert_close(got, o.astype(np.float32), f"layer {l} cache vs oracle")
             assert_close(got, ref, f"layer {l} cache, hip vs library path")
+
+
+# the weights of a row are fp16 values of 2^-12 relative rounding at most, as the result: 5e-4 of values below 5
+@pytest.mark.parametrize("B,T,H,hd", [(1, 31, 2, 64), (2, 32, 3, 128), (1, 33, 2, 128), (1, 129, 8, 64), (1, 257, 2, 128)])
+def test_prefill_attention_at_the_edges_of_its_blocks(B, T, H, hd):
+    """Prompts that end a block of 32 queries or keys, or begin one; a context that is not on 16 bytes; the results do
+    not depend on later tokens."""
+    from dejavu_amd._lib import check, lib
+
+    g = torch.Generator(device="cuda").manual_seed(T)
+    qkv = (torch.randn(B, T, 3, H, hd, generator=g, device="cuda") * 2).half()
+    print(f"case prefill attention B={B} T={T} H={H} hd={hd}", flush=True)
+    q, k, v = (t.transpose(1, 2).cpu().double() for t in qkv.unbind(2))
+    s = (q @ k.transpose(2, 3) * hd ** -0.5).masked_fill(torch.ones(T, T).triu(1).bool(), -1e300)
+    want = (s.softmax(-1) @ v).transpose(1, 2).reshape(B, T, H * hd)
+    got = {}
+    for offset, rows in ((0, T), (1, T), (0, T - 1)):
+        room = torch.zeros(B * rows * H * hd + 8, dtype=torch.float16, device="cuda")
+        part = qkv[:, :rows].contiguous()
+        ctx = room[offset:offset + B * rows * H * hd]
+        check(lib.dv_prefill_attention_f16(part.data_ptr(), B, rows, H, hd, hd ** -0.5, ctx.data_ptr(), None, None, 0, 0,
+                                           torch.cuda.current_stream().cuda_stream), "dv_prefill_attention_f16")
+        assert not room[:offset].any() and not room[offset + ctx.numel():].any()
+        got[offset, rows] = ctx.view(B, rows, H * hd).cpu()
+    torch.testing.assert_close(got[0, T].double(), want, rtol=1e-3, atol=5e-3)
+    assert torch.equal(got[1, T], got[0, T]) and torch.equal(got[0, T - 1], got[0, T][:, :T - 1])
+
+
+def test_gradients_of_a_long_prompts_attention():
+    from dejavu_amd.modules import HIP_PROMPT_ATTN_MAX_TOKENS, ParallelMHADejavu
+
+    T = HIP_PROMPT_ATTN_MAX_TOKENS + 8
+    mha = ParallelMHADejavu(128, 2, causal=True, device="cuda", dtype=torch.float16)
+    qkv = torch.randn(1, T, 3, 2, 64, device="cuda").half().requires_grad_()
+    ctx = mha._dense_context(qkv, None)
+    ctx.sum().backward()
+    assert qkv.grad.abs().sum() > 0
+    with torch.no_grad():
+        torch.testing.assert_close(mha._dense_context(qkv, None), ctx.detach(), rtol=2e-3, atol=5e-3)
