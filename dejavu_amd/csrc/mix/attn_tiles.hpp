@@ -5,7 +5,11 @@
 // A workgroup takes 128 queries of one head, a wave 32 of them.  Scores are computed transposed (keys x queries),
 // so a lane holds the scores of ONE query: the softmax is lane-local but for one exchange between the half waves,
 // and the weights are already in the operand layout of the second product when its keys are taken in the order
-// the accumulator has them (key permutation 0-3, 8-11 | 4-7, 12-15 inside 16).
+// the accumulator has them (key permutation 0-3, 8-11 | 4-7, 12-15 inside 16).  Values stay in LDS as they are in memory and
+// are read transposed; pairing keys by hand took eight 4-byte stores for each 16-byte one, and with the sums rescaled for
+// every tile, not only where a maximum has grown, 32 heads of 128 and 2048 tokens took 98 us instead of 89, 4096 tokens 331
+// instead of 304 (two heads a compute unit: the last queries' 32 tiles, one after the other, are the time at 2048).
+// Two buffers with one barrier a tile were slower (96).  Bound by the chain of a tile: LDS reads, two products, the softmax.
 #pragma once
 #include "attn_rows.hpp"
 
@@ -16,9 +20,11 @@ constexpr int kTileQ = 128, kTileK = 64;
 // DT: query/key tiles of 16, VT: value tiles of 32.  Grid: H * ceil(n / 128), head fastest, last queries first.
 template <int DT, int VT>
 __global__ __launch_bounds__(256) void attn_tiles_kernel(AttnArgs a, int keys /* rows behind k and v */) {
-  constexpr int DL = DT * 16 + 8, VL = kTileK + 4;  // LDS row lengths
+  typedef short tr_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) tr_t* tr_ptr_t;
+  constexpr int DL = DT * 16 + 8, VL = VT * 32;  // LDS row lengths
   __shared__ __attribute__((aligned(16))) bf16_t ks[kTileK * DL];
-  __shared__ __attribute__((aligned(16))) bf16_t vs[VT * 32 * VL];
+  __shared__ __attribute__((aligned(16))) bf16_t vs[kTileK * VL];
   __shared__ float rs[kTileQ + kTileK];  // biases of a tile: entry i is the distance off + q0 - k0 - (kTileK - 1) + i
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
   const int head = blockIdx.x % a.H, g = head / (a.H / a.G);
@@ -55,8 +61,10 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(AttnArgs a, int keys /*
   const int last = bhi;
 
   constexpr int KV = (kTileK * DT * 2 + 255) / 256;       // 16-byte loads of K per thread
-  constexpr int VV = (kTileK / 2 * VT * 4 + 255) / 256;   // pairs of 16-byte loads of V per thread
-  uint4_t kr[KV], vr[VV][2];
+  constexpr int VV = kTileK * VT * 4 / 256;               // and of V
+  // 16-byte piece p of row r of V: the rows of a transposed read are on different banks
+  auto piece = [](int r, int p) { return p ^ ((VT == 1 ? 0 : VT == 2 ? (r >> 1) & 1 : r & 3) << 2); };
+  uint4_t kr[KV], vr[VV];
   auto fetch = [&](int k0) {
     if (rel) rr = rel[min(max(off + q0 - k0 - (kTileK - 1) + tid, 0), a.rel_len - 1)] * kLog2e;
     // past the last key the weights are zero; past the last channel the queries are, or nothing is stored
@@ -67,9 +75,8 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(AttnArgs a, int keys /*
     }
 #pragma unroll
     for (int i = 0; i < VV; ++i) {
-      const int at = i * 256 + tid, r = at % (kTileK / 2) * 2, d = min(at / (kTileK / 2) * 8, a.vdim_s - 8);
-      vr[i][0] = *reinterpret_cast<const uint4_t*>(V + (int64_t)min(k0 + r, keys - 1) * a.ldv + d);
-      vr[i][1] = *reinterpret_cast<const uint4_t*>(V + (int64_t)min(k0 + r + 1, keys - 1) * a.ldv + d);
+      const int at = i * 256 + tid, r = at / (VT * 4), d = min(at % (VT * 4) * 8, a.vdim_s - 8);
+      vr[i] = *reinterpret_cast<const uint4_t*>(V + (int64_t)min(k0 + r, keys - 1) * a.ldv + d);
     }
   };
   auto put = [&]() {
@@ -81,15 +88,8 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(AttnArgs a, int keys /*
     }
 #pragma unroll
     for (int i = 0; i < VV; ++i) {
-      const int at = i * 256 + tid, r = at % (kTileK / 2) * 2, d = at / (kTileK / 2) * 8;
-      if (d < VT * 32) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {  // two keys of a value channel side by side
-          const unsigned x = vr[i][0][e], y = vr[i][1][e];
-          *reinterpret_cast<unsigned*>(&vs[(d + 2 * e) * VL + r]) = (x & 0xffffu) | (y << 16);
-          *reinterpret_cast<unsigned*>(&vs[(d + 2 * e + 1) * VL + r]) = (x >> 16) | (y & 0xffff0000u);
-        }
-      }
+      const int at = i * 256 + tid, r = at / (VT * 4);
+      *reinterpret_cast<uint4_t*>(&vs[r * VL + piece(r, at % (VT * 4)) * 8]) = vr[i];
     }
   };
 
@@ -100,6 +100,7 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(AttnArgs a, int keys /*
     for (int i = 0; i < 16; ++i) o[t][i] = 0.f;
   float m = -1e30f, l = 0.f;  // l: this half wave's share
   const float sc = a.scale * kLog2e;
+  const int tr_row = 4 * hh + ((lane & 15) >> 2), tr_col = 16 * ((lane >> 4) & 1) + (lane & 3) * 4;
 
   fetch(first);
   for (int k0 = first; k0 <= last; k0 += kTileK) {
@@ -159,10 +160,12 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(AttnArgs a, int keys /*
         s[kt][i] = p;
         l += p;
       }
+    if (__any(c != 1.f)) {  // a new maximum somewhere: rare after the first tiles
 #pragma unroll
-    for (int t = 0; t < VT; ++t)
+      for (int t = 0; t < VT; ++t)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) o[t][i] *= c;
+        for (int i = 0; i < 16; ++i) o[t][i] *= c;
+    }
 #pragma unroll
     for (int ks4 = 0; ks4 < 4; ++ks4) {
       bf16x8_t pf;
@@ -170,14 +173,16 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(AttnArgs a, int keys /*
       for (int e = 0; e < 8; ++e) pf[e] = (bf16_t)s[ks4 >> 1][8 * (ks4 & 1) + e];
 #pragma unroll
       for (int t = 0; t < VT; ++t) {
-        const bf16_t* vp = &vs[(t * 32 + l32) * VL + ks4 * 16 + 4 * hh];
-        uint4_t w;
-        const uint2_t w0 = *reinterpret_cast<const uint2_t*>(vp), w1 = *reinterpret_cast<const uint2_t*>(vp + 8);
-        w[0] = w0[0];
-        w[1] = w0[1];
-        w[2] = w1[0];
-        w[3] = w1[1];
-        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, w), pf, o[t], 0, 0, 0);
+        union {
+          tr_t part[2];
+          bf16x8_t all;
+        } w;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int r = ks4 * 16 + u * 8 + tr_row, col = t * 32 + tr_col;
+          w.part[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)(&vs[r * VL + piece(r, col >> 3) * 8 + (col & 7)]));
+        }
+        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w.all, pf, o[t], 0, 0, 0);
       }
     }
   }
