@@ -99,10 +99,11 @@ def residual(y: Optional[torch.Tensor], stream: ResidualStream, post, pre, add_s
 
 # Where the 256 x 256 tiles of the wide kernel make two rounds of the chip's compute units or more and the chunks are many, it is
 # ahead of the library GEMM with the gated unit's launch (22016 x 4096 with 1500 / 1700 / 2048 / 3000 / 4096 rows: 290 / 304 /
-# 324 / 499 / 631 against 313 / 346 / 422 / 507 / 689 us; with 1280 rows, 430 tiles, 215 against 194), and for plain
+# 324 / 499 / 631 against 313 / 346 / 422 / 507 / 689 us; with 1280 rows, 430 tiles, 215 against 194) up to six rounds (6000
+# rows, 2064 tiles: 972 against 925; 12000: 1865 against 1722), and for plain
 # products up to three rounds (18560 x 4096 with 1700 / 1999 / 3000 rows: 228 / 295 / 401 against 252 / 338 / 362;
 # 11264 x 2048 with 3000: 158 against 122).
-WIDE_TILE, WIDE_MIN_TILES, WIDE_MAX_PLAIN_TILES, WIDE_MIN_COLUMNS = 256, 500, 768, 4096
+WIDE_TILE, WIDE_MIN_TILES, WIDE_MAX_TILES, WIDE_MAX_PLAIN_TILES, WIDE_MIN_COLUMNS = 256, 500, 1536, 768, 4096
 
 
 def _aligned(x: torch.Tensor, W: torch.Tensor) -> bool:
@@ -115,7 +116,7 @@ def _wide(x: torch.Tensor, W: torch.Tensor, plain: bool, bias=None) -> bool:
     if x.dtype != torch.bfloat16 or K < WIDE_MIN_COLUMNS:
         return False
     tiles = -(-M // WIDE_TILE) * -(-x.shape[0] // WIDE_TILE)
-    return tiles >= WIDE_MIN_TILES and (not plain or tiles <= WIDE_MAX_PLAIN_TILES) and results_only(x, W, bias) and _aligned(x, W)
+    return WIDE_MIN_TILES <= tiles <= (WIDE_MAX_PLAIN_TILES if plain else WIDE_MAX_TILES) and results_only(x, W, bias) and _aligned(x, W)
 
 
 def _tiles(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
