@@ -102,7 +102,9 @@ def residual(y: Optional[torch.Tensor], stream: ResidualStream, post, pre, add_s
 # 324 / 499 / 631 against 313 / 346 / 422 / 507 / 689 us; with 1280 rows, 430 tiles, 215 against 194) up to six rounds (6000
 # rows, 2064 tiles: 972 against 925; 12000: 1865 against 1722), and for plain
 # products up to three rounds (18560 x 4096 with 1700 / 1999 / 3000 rows: 228 / 295 / 401 against 252 / 338 / 362;
-# 11264 x 2048 with 3000: 158 against 122).
+# 11264 x 2048 with 3000: 158 against 122) and 2048 rows (products with 4096 rows of W and 8192 of x, 512 tiles: 463 against
+# 379 on average).
+WIDE_MAX_PLAIN_ROWS = 2048
 WIDE_TILE, WIDE_MIN_TILES, WIDE_MAX_TILES, WIDE_MAX_PLAIN_TILES, WIDE_MIN_COLUMNS = 256, 500, 1536, 768, 4096
 
 
@@ -113,7 +115,7 @@ def _aligned(x: torch.Tensor, W: torch.Tensor) -> bool:
 def _wide(x: torch.Tensor, W: torch.Tensor, plain: bool, bias=None) -> bool:
     """Whether the wide kernel takes the product."""
     M, K = W.shape
-    if x.dtype != torch.bfloat16 or K < WIDE_MIN_COLUMNS:
+    if x.dtype != torch.bfloat16 or K < WIDE_MIN_COLUMNS or (plain and x.shape[0] > WIDE_MAX_PLAIN_ROWS):
         return False
     tiles = -(-M // WIDE_TILE) * -(-x.shape[0] // WIDE_TILE)
     return WIDE_MIN_TILES <= tiles <= (WIDE_MAX_PLAIN_TILES if plain else WIDE_MAX_TILES) and results_only(x, W, bias) and _aligned(x, W)

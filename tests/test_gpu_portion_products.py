@@ -75,14 +75,15 @@ def test_wide_tiles(n, K, M):
 
 
 def test_wide_products_through_the_ops():
-    """A product on each side of the rule: 496 tiles go to the library, 512 to the wide kernel, both with the same result."""
+    """A product on each side of the rule: 497 tiles go to the library, 568 to the wide kernel, both with the same result."""
     from dejavu_amd import mixer_ops as ops
 
     g = torch.Generator(device="cuda").manual_seed(1)
-    W = (torch.randn(31 * 256, 4096, generator=g, device="cuda") / 64).to(BF16)
-    x = torch.randn(4096 + 8, 4096, generator=g, device="cuda").to(BF16)
-    assert not ops._wide(x[:4096], W, True) and ops._wide(x, W, True) and not ops._wide(x[:, :2048], W[:, :2048], True)
-    for rows in (4096, 4096 + 8):
+    W = (torch.randn(71 * 256, 4096, generator=g, device="cuda") / 64).to(BF16)
+    x = torch.randn(1792 + 8, 4096, generator=g, device="cuda").to(BF16)
+    assert not ops._wide(x[:1792], W, True) and ops._wide(x, W, True) and not ops._wide(x[:, :2048], W[:, :2048], True)
+    assert not ops._wide(x.repeat(2, 1), W[: 36 * 256], True)  # 540 tiles of 3600 rows
+    for rows in (1792, 1792 + 8):
         want = x[:rows].float() @ W.float().t()
         got = ops.linear(x[:rows], W).float()
         assert (got - want).norm() / want.norm() < 3e-3  # one rounding to bf16
