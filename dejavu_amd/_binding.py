@@ -5,6 +5,14 @@ import ctypes
 import os
 
 import torch  # noqa: F401  (loads the HIP runtime that the libraries bind to)
+from torch.utils._device import DeviceContext
+
+
+def _watched() -> bool:
+    """Whether a dispatch mode (make_fx, FlopCounterMode ..) or a function mode is active, which would see a library call and
+    not a kernel's.  A default device is a function mode too, but one for the functions that make tensors."""
+    return torch._C._len_torch_dispatch_stack() > 0 or any(
+        type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
 
 
 def results_only(*tensors) -> bool:
@@ -17,7 +25,8 @@ def results_only(*tensors) -> bool:
                               type(t) not in (torch.Tensor, torch.nn.Parameter)):
             return False
     return (torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None and
-            not torch.is_autocast_enabled() and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+            not torch.is_autocast_enabled() and not torch.jit.is_tracing() and not torch.compiler.is_compiling() and
+            not _watched())
 
 
 class DejavuHipError(RuntimeError):
