@@ -119,3 +119,20 @@ def test_odd_places_of_the_result():
         want = np.maximum(prod[:, 0::2], 0) * prod[:, 1::2] if after == L.OUT_GLU else prod
         close(got[:, :want.shape[1]], want, 1e-5 if dtype == torch.float32 else OP_LIMIT[BF16], f"after {after}, rows {ldo} apart")
         assert not got[:, want.shape[1]:].any(), "stored past the end of a row"
+
+
+@pytest.mark.parametrize("n,K,M", [
+    (2, 2048, 32768), (16, 4096, 11008), (47, 4096, 22016), (100, 4096, 32768),  # one split
+    (24, 12288, 8192), (250, 4096, 11008),                                       # two
+    (64, 4096, 4096), (100, 4096, 4096),                                         # four, and eight
+])
+def test_fp32_results_of_long_rows(n, K, M):
+    """Sums of at most a quarter of K: the error in 64 bits is 2.9e-9 sqrt(K) of the result (1.9e-7 with 4096 columns), with
+    sums of half of K 4.3e-9 and with one sum 6.1e-9.  The limit lies between, at 3.8e-9."""
+    from dejavu_amd import mixer_ops as ops
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(n, K, generator=g, device="cuda").to(BF16)
+    W = (torch.randn(M, K, generator=g, device="cuda") * K ** -0.5).to(BF16)
+    want = x.double() @ W.double().t()
+    assert (ops.linear(x, W, f32=True) - want).norm() / want.norm() < 3.8e-9 * K ** 0.5
