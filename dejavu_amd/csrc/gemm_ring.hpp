@@ -154,8 +154,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T>
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
     for (; c < stop; ++c) {
-      wait_loads<LI*(ST - 2)>();
-      __builtin_amdgcn_s_barrier();  // everybody's part of the slot is there, and the slot before it is free
+      // Everybody's part of the slot is there, and nobody still reads the slot before it, which is loaded next: the reads have
+      // to have returned, which the barrier itself does not wait for and the instructions that use them need not come before.
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(LI * (ST - 2)) : "memory");
+      __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       load(c + ST - 1, slot == 0 ? ST - 1 : slot - 1);
       const unsigned char* wb = slots + slot * SLOT + (wm * RT * 16 + l16) * KC * 2;
