@@ -558,14 +558,16 @@ int dv_mix_attn_tiles_f32(const dvAttnArgs* a, int keys, void* stream) {
   if (a->ldq % 4 || !al16(a->out)) return DV_ERR_ALIGNMENT;
   const int64_t groups = ((int64_t)a->n + kF32Q - 1) / kF32Q * a->H;
   if (a->dim_s > 128 || a->vdim_s > 128 || groups > 0x7fffffff) return DV_ERR_UNSUPPORTED;
-#define DV_ATT(DU, VT) \
-  return launch_lds<attn_f32_kernel<DU, VT>>(dim3((unsigned)groups), dim3(256), f32_lds(VT), st(stream), *a, keys)
-  if (a->dim_s <= 64) {
-    if (a->vdim_s <= 64) DV_ATT(8, 2);
-    DV_ATT(8, 4);
-  }
-  if (a->vdim_s <= 64) DV_ATT(16, 2);
-  DV_ATT(16, 4);
+#define DV_ATT(DU, WHOLE, VT) \
+  return launch_lds<attn_f32_kernel<DU, WHOLE, VT>>(dim3((unsigned)groups), dim3(256), f32_lds(VT), st(stream), *a, keys)
+#define DV_ATT_V(DU, WHOLE)               \
+  if (a->vdim_s <= 64) DV_ATT(DU, WHOLE, 2); \
+  DV_ATT(DU, WHOLE, 4)
+  if (a->dim_s == 64) { DV_ATT_V(8, true); }
+  if (a->dim_s < 64) { DV_ATT_V(8, false); }
+  if (a->dim_s == 128) { DV_ATT_V(16, true); }
+  DV_ATT_V(16, false);
+#undef DV_ATT_V
 #undef DV_ATT
 }
 
