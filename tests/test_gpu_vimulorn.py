@@ -182,21 +182,27 @@ def test_fp32_portions_on_the_matrix_cores(T, H, G, dim, vdim, window, chunk, un
 
 @pytest.mark.parametrize("dim,entry", [(8, 7), (40, 39), (64, 60), (72, 68), (96, 0), (120, 119), (128, 127)])
 def test_fp32_portions_with_an_infinite_key(dim, entry, monkeypatch):
-    """A score of minus infinity has weight zero, whatever lies behind the entries of a head in the kernel's registers."""
+    """A score of minus infinity has weight zero and one of infinity leaves its row undefined, as by the row kernel, whatever
+    lies behind the entries of a head in the registers."""
     from dejavu_amd import mixer_ops as ops
 
-    monkeypatch.setattr(ops, "F32_TILE_ROWS", 1)
     T, H = 70, 2
     q, k, v = (host(dev(a)) for a in _attention_case(T, H, H, dim, dim, seed=dim))
-    q[:, :, entry] = -np.abs(q[:, :, entry]) - 0.1
     k[33, 1, entry] = np.inf
     s = np.einsum("qhd,khd->hqk", q, np.where(np.isinf(k), 0.0, k)) * 0.2
     s = np.where(np.tri(T, dtype=bool)[None], s, -np.inf)
-    s[1, :, 33] = -np.inf
+    s[1, 33:, 33] = -np.inf
     e = np.exp(s - s.max(-1, keepdims=True))
     want = np.einsum("hqk,khd->qhd", e / e.sum(-1, keepdims=True), v)
-    got = ops.portion_attention(*(dev(a.reshape(T, -1)) for a in (q, k, v)), H, H, 0.2, 0, 0)
-    close(got, want.reshape(T, -1), OP_LIMIT[torch.float32], f"heads of {dim}, entry {entry}")
+    undefined = np.zeros((T, H), bool)
+    undefined[33:, 1] = q[33:, 1, entry] > 0
+    assert undefined.any() and not undefined[33:, 1].all()
+    for rows in (1, 1 << 30):  # the matrix cores, row by row
+        monkeypatch.setattr(ops, "F32_TILE_ROWS", rows)
+        got = host(ops.portion_attention(*(dev(a.reshape(T, -1)) for a in (q, k, v)), H, H, 0.2, 0, 0)).reshape(T, H, dim)
+        assert np.isnan(got[undefined]).all()
+        got[undefined] = want[undefined]
+        close(got.reshape(T, -1), want.reshape(T, -1), OP_LIMIT[torch.float32], f"heads of {dim}, entry {entry}, from {rows} rows")
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
