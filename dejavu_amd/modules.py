@@ -259,6 +259,17 @@ class ParallelFusedMLPDejavu(nn.Module):
         return out, mlp_logit
 
 
+def _long_product(linear, x: torch.Tensor) -> bool:
+    """Whether ``dense_linear`` is the faster one for more than ``HIP_PROMPT_MAX_ROWS`` rows and does what ``linear(x)`` would:
+    a layer that is nothing but its weight and bias, operands that the kernel takes where they are, only results asked for."""
+    W, b = linear.weight, linear.bias
+    return (type(linear) is nn.Linear and W.dim() == 2 and W.shape[1] > W.shape[0] and x.shape[-1] == W.shape[1] and
+            "forward" not in linear.__dict__ and not (linear._forward_hooks or linear._forward_pre_hooks) and
+            not (nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks) and
+            results_only(x, W, b) and W.stride(1) == 1 and W.stride(0) % 8 == 0 and W.data_ptr() % 16 == 0 and
+            x.data_ptr() % 16 == 0 and (b is None or (b.dtype == W.dtype and b.shape == W.shape[:1])))
+
+
 def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") -> torch.Tensor:
     """``activation(linear(x))``.  The rows of a decode step (x: (B, 1, d) with B <= 64, fp16, on the GPU)
     always go to this package's row kernels (vector ALUs for one or two rows, matrix cores above).  The
@@ -268,10 +279,7 @@ def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") ->
     if on_hip and x.dim() == 3 and x.shape[1] == 1 and x.shape[0] <= 64:
         return ops.dense_decode_linear(x, linear.weight, linear.bias, activation)
     rows = x.numel() // x.shape[-1] if on_hip and USE_HIP_PROMPT else HIP_PROMPT_LONG_MAX_ROWS + 1
-    if rows <= HIP_PROMPT_MAX_ROWS or (
-            rows <= HIP_PROMPT_LONG_MAX_ROWS and linear.in_features > linear.out_features and
-            type(linear) is nn.Linear and not linear._forward_hooks and not linear._forward_pre_hooks and
-            results_only(x, linear.weight, linear.bias)):
+    if rows <= HIP_PROMPT_MAX_ROWS or (rows <= HIP_PROMPT_LONG_MAX_ROWS and _long_product(linear, x)):
         return ops.dense_linear(x, linear.weight, linear.bias, activation)
     y = linear(x)
     if activation == "relu":

@@ -29,24 +29,71 @@ def test_gradients_and_transforms_of_portion_products(n, K, M):
     assert torch.equal(tangent, F.linear(x, W))
 
 
+@pytest.fixture(scope="module")
+def fc2():
+    """A weight whose products of 193..512 rows are this package's, and rows."""
+    layer = nn.Linear(8192, 2048, device="cuda", dtype=torch.float16).requires_grad_(False)
+    return layer, torch.randn(1, 512, 8192, device="cuda").half()
+
+
+def _is_ours(layer, x):
+    """The two results are fp16 values below 4 of the same sums: a unit of rounding at most between them."""
+    from dejavu_amd.modules import _long_product, decode_linear
+
+    y = decode_linear(layer, x)
+    torch.testing.assert_close(y, F.linear(x, layer.weight, layer.bias), rtol=2e-3, atol=2e-3)
+    return _long_product(layer, x)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows", [193, 512])
-def test_gradients_and_hooks_of_a_long_prompts_linear(rows):
+def test_gradients_and_hooks_of_a_long_prompts_linear(fc2, rows):
     from dejavu_amd.modules import decode_linear
 
-    layer = nn.Linear(256, 64, device="cuda", dtype=torch.float16)
-    x = torch.randn(1, rows, 256, device="cuda").half()
+    layer, x = nn.Linear(8192, 2048, device="cuda", dtype=torch.float16), fc2[1][:, :rows]
     decode_linear(layer, x).sum().backward()
-    assert torch.equal(layer.bias.grad, torch.full((64,), float(rows), device="cuda").half())
+    assert torch.equal(layer.bias.grad, torch.full((2048,), float(rows), device="cuda").half())
     seen = []
-    handle = layer.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    hook = lambda m, i, o: seen.append(o.shape)  # noqa: E731
     with torch.no_grad():
-        decode_linear(layer, x)
-        assert seen == [(1, rows, 64)]
-        handle.remove()
-        y = decode_linear(layer, x)
-    assert len(seen) == 1
-    torch.testing.assert_close(y, layer(x).detach(), rtol=2e-3, atol=2e-3)  # two results in fp16, below 2 in size
+        for register in (layer.register_forward_hook, nn.modules.module.register_module_forward_hook):
+            handle = register(hook)
+            try:
+                decode_linear(layer, x)
+            finally:
+                handle.remove()
+            assert seen.pop() == (1, rows, 2048)
+        assert _is_ours(layer, x) and not seen
+        layer.forward = lambda t: t[..., :1]  # as wrappers of a module replace it
+        assert decode_linear(layer, x).shape == (1, rows, 1)
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+def test_operands_of_a_long_prompts_linear_that_only_the_library_takes(fc2):
+    """Weights and rows off a 16-byte boundary or with odd strides, and layers that are no nn.Linear."""
+    from dejavu_amd.modules import decode_linear
+
+    layer, x = fc2
+    x = x[:, :200]
+    assert _is_ours(layer, x)
+    M, K = layer.weight.shape
+    moved = torch.empty(M * K + 1, device="cuda", dtype=torch.float16)[1:].view(M, K).copy_(layer.weight)
+    apart = torch.empty(M, K + 4, device="cuda", dtype=torch.float16)[:, :K].copy_(layer.weight)
+    for weight in (moved, apart, layer.weight.t().contiguous().t()):
+        other = nn.Linear(1, 1, device="cuda", dtype=torch.float16)
+        other.weight, other.bias = nn.Parameter(weight, requires_grad=False), layer.bias
+        assert not _is_ours(other, x)
+    assert not _is_ours(layer, torch.empty(x.numel() + 1, device="cuda", dtype=torch.float16)[1:].view(x.shape).copy_(x))
+    assert _is_ours(layer, torch.randn(1, 200, K + 8, device="cuda").half()[:, :, :K])
+
+    class Duck:
+        weight, bias = layer.weight, layer.bias
+
+        def __call__(self, t):
+            return t[..., :2]
+
+    assert torch.equal(decode_linear(Duck(), x), x[..., :2])
 
 
 def test_modes_that_watch_library_calls():
@@ -72,7 +119,7 @@ def test_modes_that_watch_library_calls():
 
 @pytest.mark.gpu
 @torch.no_grad()
-def test_traces_of_what_kernels_take_over():
+def test_traces_of_what_kernels_take_over(fc2):
     """Graphs recorded by make_fx compute with the inputs that they are given later."""
     from torch.fx.experimental.proxy_tensor import make_fx
 
@@ -80,11 +127,11 @@ def test_traces_of_what_kernels_take_over():
     from dejavu_amd.modules import HIP_PROMPT_ATTN_MAX_TOKENS, ParallelMHADejavu, decode_linear
 
     W = torch.randn(32, 64, device="cuda").bfloat16()
-    layer = nn.Linear(256, 64, device="cuda", dtype=torch.float16)
+    layer = fc2[0]
     mha = ParallelMHADejavu(128, 2, causal=True, device="cuda", dtype=torch.float16)
     T = HIP_PROMPT_ATTN_MAX_TOKENS + 8
     for f, shape, dtype in ((lambda t: mixer_ops.linear(t, W), (65, 64), torch.bfloat16),
-                            (lambda t: decode_linear(layer, t), (1, 200, 256), torch.float16),
+                            (lambda t: decode_linear(layer, t), (1, 200, 8192), torch.float16),
                             (lambda t: mha._dense_context(t, None), (1, T, 3, 2, 64), torch.float16)):
         traced = make_fx(f)(torch.randn(shape, device="cuda").to(dtype))
         x = torch.randn(shape, device="cuda").to(dtype)
