@@ -326,6 +326,13 @@ def _update_kv_cache(kv, inference_params, layer_idx):
     return kv
 
 
+def _kernel_takes(*tensors) -> bool:
+    """Whether the prompt attention takes these where they are: the copies fill a caller's own caches of any type, stride and
+    place, and the library's attention reads from anywhere."""
+    return results_only(*tensors) and all(
+        t is None or (t.dtype == torch.float16 and t.is_contiguous() and t.data_ptr() % 16 == 0) for t in tensors)
+
+
 class _MHABase(nn.Module):
     """Shared dense / prompt machinery of the two attention modules."""
 
@@ -376,9 +383,9 @@ class _MHABase(nn.Module):
                                                   qkv.dtype, qkv.device)
                     b0 = inference_params.batch_size_offset
                     kc, vc = k_cache[b0:b0 + B], v_cache[b0:b0 + B]
-                if s <= HIP_PROMPT_ATTN_MAX_TOKENS or kc is None or (  # the copies fill a caller's own caches of any stride
-                        kc.is_contiguous() and vc.is_contiguous() and results_only(kc, vc)):
-                    return ops.prefill_attention(qkv.contiguous(), kc, vc, 0, scale)
+                rows = qkv.contiguous()
+                if s <= HIP_PROMPT_ATTN_MAX_TOKENS or _kernel_takes(rows, kc, vc):
+                    return ops.prefill_attention(rows, kc, vc, 0, scale)
             if inference_params is not None:
                 assert self.layer_idx is not None, "Generation requires layer_idx in the constructor"
                 _update_kv_cache(qkv[:, :, 1:], inference_params, self.layer_idx)

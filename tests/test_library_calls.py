@@ -1,5 +1,7 @@
 """Products and attention that a kernel takes over from the library still do what only the library can: gradients,
 functional transforms, tracing, module hooks."""
+import math
+
 import pytest
 import torch
 from torch import nn
@@ -136,3 +138,37 @@ def test_traces_of_what_kernels_take_over(fc2):
         traced = make_fx(f)(torch.randn(shape, device="cuda").to(dtype))
         x = torch.randn(shape, device="cuda").to(dtype)
         torch.testing.assert_close(traced(x), f(x), rtol=2e-2, atol=2e-2)  # one rounding of each side: 2^-8 and less
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+def test_operands_of_a_long_prompts_attention_that_only_the_library_takes():
+    """Caches of a caller's own, of another type, stride or place, are filled as ever; so are those that the kernel fills."""
+    from dejavu_amd import modules, ops
+    from dejavu_amd.modules import HIP_PROMPT_ATTN_MAX_TOKENS, InferenceParams, ParallelMHADejavu
+
+    T, S, H, hd = HIP_PROMPT_ATTN_MAX_TOKENS + 8, HIP_PROMPT_ATTN_MAX_TOKENS + 16, 2, 64
+    mha = ParallelMHADejavu(H * hd, H, causal=True, layer_idx=0, device="cuda", dtype=torch.float16)
+    qkv = torch.randn(1, T, 3, H, hd, device="cuda").half()
+    odd = torch.empty(qkv.numel() + 1, device="cuda", dtype=torch.float16)[1:].view(qkv.shape).copy_(qkv)
+    want = mha._dense_context(qkv, None)
+    shapes = (1, H, hd // 8, S, 8), (1, H, S, hd)
+
+    def plain(shape, dtype=torch.float16):
+        return torch.zeros(shape, device="cuda", dtype=dtype)
+
+    made = {"plain": [plain(s) for s in shapes], "fp32": [plain(s, torch.float32) for s in shapes],
+            "moved": [plain(math.prod(s) + 1)[1:].view(s) for s in shapes],
+            "strided": [plain(s[:-1] + (s[-1] + 8,))[..., :s[-1]] for s in shapes]}
+    for name, (k_cache, v_cache) in made.items():
+        for x in (qkv, odd):
+            k_cache.zero_(), v_cache.zero_()
+            ip = InferenceParams(max_sequence_len=S, max_batch_size=1)
+            ip.key_value_memory_dict[0] = k_cache, v_cache
+            torch.testing.assert_close(mha._dense_context(x, ip), want, rtol=2e-3, atol=2e-3)
+            k = k_cache[:, :, :, :T].permute(0, 3, 1, 2, 4).reshape(1, T, H, hd)
+            assert torch.equal(k.half(), qkv[:, :, 1]) and torch.equal(v_cache[:, :, :T].transpose(1, 2).half(), qkv[:, :, 2])
+            assert not k_cache[:, :, :, T:].any() and not v_cache[:, :, T:].any()
+        assert modules._kernel_takes(qkv, k_cache, v_cache) == (name == "plain")
+    assert not modules._kernel_takes(odd)
+    torch.testing.assert_close(ops.prefill_attention(qkv), want, rtol=2e-3, atol=2e-3)
