@@ -47,14 +47,23 @@ USE_HIP_PROMPT = True
 # The dense products of a prompt are plain GEMMs.  Up to this many rows of X the package's kernel is at least as fast as
 # the library (it is bound by the weight stream: 5120 x 5120 with 128 / 190 rows 22 / 26 against 32 / 29 us, 15360 x 5120
 # with 190 rows 53 against 51 and a launch for the activation); beyond it the product is compute-bound and the library's
-# GEMM is taken -- but where the weight's rows are longer than they are many (fc2) it leaves most of the chip idle up to
-# HIP_PROMPT_LONG_MAX_ROWS rows (5120 x 20480 with 256 / 384 / 512 rows: 221 / 149 / 195 us, this package's kernel 84 / 134 / 135).
+# GEMM is taken.
 HIP_PROMPT_MAX_ROWS = 192
+# But where the weight's rows are four times as long as they are many (fc2), the library leaves much of the chip idle for some
+# hundred rows more: up to 256 from 2^23 elements on (us, this kernel against the library, 256 rows: 1024 x 8192 20.8 / 21.0, 2048 x
+# 8192 24 / 28, 5120 x 20480 79 / 225, 12288 x 49152 396 / 478; but 768 x 3072 12.7 / 9.2, 4096 x 5120 31 / 29), and up to 512 for
+# weights of 4096 to 7168 rows (4096 x 16384 with 300 / 384 / 512 rows 81 / 82 / 86 against 88 / 90 / 110, 5120 x 20480 127 / 123 / 131
+# against 129 / 151 / 193, 7168 x 28672 233 / 234 / 243 against 266 / 276 / 289; but 3072 x 12288 76 against 58 to 73, 9216 x 36864
+# 500 against 380 to 409).  Just above 256 rows the second tile of rows is nearly empty (5120 x 20480, 257 rows: 126 / 121).
 HIP_PROMPT_LONG_MAX_ROWS = 512
+HIP_PROMPT_LONG_ROWS = 256
+HIP_PROMPT_LONG_MORE_ROWS = 288
+HIP_PROMPT_LONG_WEIGHT = 1 << 23
+HIP_PROMPT_LONG_WEIGHT_ROWS = (4096, 7168)
 # The package's causal-attention kernel (cache fill in the same launch) is ahead of the library's attention with the
-# permuted cache copies at all lengths (40 heads of 128 and 128 / 1024 tokens: 7.5 / 47 us against 25 / 100; 32 heads and
-# 777 / 2000 / 4000 tokens: 30 / 110 / 385 against 75 / 310 / 566).  Prompts of more than so many tokens leave gradients,
-# functional transforms and the like to the library.
+# permuted cache copies (40 heads of 128 and 128 / 1024 tokens: 7.5 / 47 us against 25 / 100; 32 heads and
+# 777 / 2000 / 4000 tokens: 30 / 110 / 385 against 75 / 310 / 566; 16 sequences of 1024: 547 against 768).  Prompts of more than so
+# many tokens leave gradients, functional transforms and the like to the library.
 HIP_PROMPT_ATTN_MAX_TOKENS = 192
 
 _side_streams: dict = {}
@@ -259,11 +268,19 @@ class ParallelFusedMLPDejavu(nn.Module):
         return out, mlp_logit
 
 
+def _long_rule(rows: int, M: int, K: int) -> bool:
+    if K < 4 * M or M * K < HIP_PROMPT_LONG_WEIGHT:
+        return False
+    low, high = HIP_PROMPT_LONG_WEIGHT_ROWS
+    return rows <= HIP_PROMPT_LONG_ROWS or (low <= M <= high and HIP_PROMPT_LONG_MORE_ROWS <= rows <= HIP_PROMPT_LONG_MAX_ROWS)
+
+
 def _long_product(linear, x: torch.Tensor) -> bool:
     """Whether ``dense_linear`` is the faster one for more than ``HIP_PROMPT_MAX_ROWS`` rows and does what ``linear(x)`` would:
     a layer that is nothing but its weight and bias, operands that the kernel takes where they are, only results asked for."""
     W, b = linear.weight, linear.bias
-    return (type(linear) is nn.Linear and W.dim() == 2 and W.shape[1] > W.shape[0] and x.shape[-1] == W.shape[1] and
+    return (type(linear) is nn.Linear and W.dim() == 2 and _long_rule(x.numel() // x.shape[-1], *W.shape) and
+            x.shape[-1] == W.shape[1] and
             "forward" not in linear.__dict__ and not (linear._forward_hooks or linear._forward_pre_hooks) and
             not (nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks) and
             results_only(x, W, b) and W.stride(1) == 1 and W.stride(0) % 8 == 0 and W.data_ptr() % 16 == 0 and
@@ -273,8 +290,8 @@ def _long_product(linear, x: torch.Tensor) -> bool:
 def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") -> torch.Tensor:
     """``activation(linear(x))``.  The rows of a decode step (x: (B, 1, d) with B <= 64, fp16, on the GPU)
     always go to this package's row kernels (vector ALUs for one or two rows, matrix cores above).  The
-    rows of a prompt go to the X-shared matrix-core kernel while the product is bound by the weight
-    stream (``USE_HIP_PROMPT``, up to ``HIP_PROMPT_MAX_ROWS`` rows), else to the library GEMM."""
+    rows of a prompt go to the matrix-core kernels that stream the weight while it is the bound (``USE_HIP_PROMPT``, up
+    to ``HIP_PROMPT_MAX_ROWS`` rows, and more of them for long-rowed weights: ``_long_product``), else to the library GEMM."""
     on_hip = x.is_cuda and x.dtype == torch.float16 and linear.weight.dtype == torch.float16 and x.shape[-1] % 8 == 0
     if on_hip and x.dim() == 3 and x.shape[1] == 1 and x.shape[0] <= 64:
         return ops.dense_decode_linear(x, linear.weight, linear.bias, activation)

@@ -34,8 +34,8 @@ def test_gradients_and_transforms_of_portion_products(n, K, M):
 @pytest.fixture(scope="module")
 def fc2():
     """A weight whose products of 193..512 rows are this package's, and rows."""
-    layer = nn.Linear(8192, 2048, device="cuda", dtype=torch.float16).requires_grad_(False)
-    return layer, torch.randn(1, 512, 8192, device="cuda").half()
+    layer = nn.Linear(16384, 4096, device="cuda", dtype=torch.float16).requires_grad_(False)
+    return layer, torch.randn(1, 512, 16384, device="cuda").half()
 
 
 def _is_ours(layer, x):
@@ -52,9 +52,9 @@ def _is_ours(layer, x):
 def test_gradients_and_hooks_of_a_long_prompts_linear(fc2, rows):
     from dejavu_amd.modules import decode_linear
 
-    layer, x = nn.Linear(8192, 2048, device="cuda", dtype=torch.float16), fc2[1][:, :rows]
+    layer, x = nn.Linear(16384, 4096, device="cuda", dtype=torch.float16), fc2[1][:, :rows]
     decode_linear(layer, x).sum().backward()
-    assert torch.equal(layer.bias.grad, torch.full((2048,), float(rows), device="cuda").half())
+    assert torch.equal(layer.bias.grad, torch.full((4096,), float(rows), device="cuda").half())
     seen = []
     hook = lambda m, i, o: seen.append(o.shape)  # noqa: E731
     with torch.no_grad():
@@ -64,10 +64,21 @@ def test_gradients_and_hooks_of_a_long_prompts_linear(fc2, rows):
                 decode_linear(layer, x)
             finally:
                 handle.remove()
-            assert seen.pop() == (1, rows, 2048)
+            assert seen.pop() == (1, rows, 4096)
         assert _is_ours(layer, x) and not seen
         layer.forward = lambda t: t[..., :1]  # as wrappers of a module replace it
         assert decode_linear(layer, x).shape == (1, rows, 1)
+
+
+def test_rule_of_a_long_prompts_linear():
+    """Both sides of each line, in rows and in the weight's size and shape."""
+    from dejavu_amd.modules import _long_rule
+
+    for rows, M, K, ours in ((193, 4096, 16384, True), (256, 4096, 16384, True), (257, 4096, 16384, False), (287, 4096, 16384, False),
+                             (288, 4096, 16384, True), (512, 7168, 28672, True), (513, 4096, 16384, False), (200, 1024, 8192, True),
+                             (200, 1024, 8184, False), (200, 4096, 16376, False), (256, 12288, 49152, True), (300, 12288, 49152, False),
+                             (300, 2048, 8192, False), (256, 768, 3072, False)):
+        assert _long_rule(rows, M, K) == ours, (rows, M, K)
 
 
 @pytest.mark.gpu
@@ -133,7 +144,7 @@ def test_traces_of_what_kernels_take_over(fc2):
     mha = ParallelMHADejavu(128, 2, causal=True, device="cuda", dtype=torch.float16)
     T = HIP_PROMPT_ATTN_MAX_TOKENS + 8
     for f, shape, dtype in ((lambda t: mixer_ops.linear(t, W), (65, 64), torch.bfloat16),
-                            (lambda t: decode_linear(layer, t), (1, 200, 8192), torch.float16),
+                            (lambda t: decode_linear(layer, t), (1, 200, 16384), torch.float16),
                             (lambda t: mha._dense_context(t, None), (1, T, 3, 2, 64), torch.float16)):
         traced = make_fx(f)(torch.randn(shape, device="cuda").to(dtype))
         x = torch.randn(shape, device="cuda").to(dtype)
