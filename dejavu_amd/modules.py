@@ -65,6 +65,12 @@ HIP_PROMPT_LONG_WEIGHT_ROWS = (4096, 7168)
 # 777 / 2000 / 4000 tokens: 30 / 110 / 385 against 75 / 310 / 566; 16 sequences of 1024: 547 against 768).  Prompts of more than so
 # many tokens leave gradients, functional transforms and the like to the library.
 HIP_PROMPT_ATTN_MAX_TOKENS = 192
+# Each workgroup reads the keys and values before its 32 queries, so the L2 bounds long prompts and the library, whose tiles
+# are larger, overtakes: with 40 heads of 128 from 8192 tokens on (1759 against 1691 us; 6000 tokens 961 against 1155, 16 sequences of
+# 4096 and 32 heads 5875 against 6316), with 96 heads above 2048 (four sequences of 2048 1329 against 1404, of 4096 5184 against 4784).
+HIP_PROMPT_ATTN_LONGEST = 6144
+HIP_PROMPT_ATTN_WIDE = 5120            # heads * head_dim above which it is
+HIP_PROMPT_ATTN_WIDE_LONGEST = 2048
 
 _side_streams: dict = {}
 _side_pending = False  # work was enqueued on the side stream since the last join_side_stream()
@@ -343,6 +349,11 @@ def _update_kv_cache(kv, inference_params, layer_idx):
     return kv
 
 
+def _longest_prompt(width: int) -> int:
+    """The most tokens of a prompt whose attention, heads * head_dim wide, this package's kernel computes."""
+    return HIP_PROMPT_ATTN_LONGEST if width <= HIP_PROMPT_ATTN_WIDE else HIP_PROMPT_ATTN_WIDE_LONGEST
+
+
 def _kernel_takes(*tensors) -> bool:
     """Whether the prompt attention takes these where they are: the copies fill a caller's own caches of any type, stride and
     place, and the library's attention reads from anywhere."""
@@ -391,7 +402,8 @@ class _MHABase(nn.Module):
         if inference_params is None or inference_params.sequence_len_offset == 0:
             causal = self.causal if inference_params is None else True
             if USE_HIP_PROMPT and qkv.is_cuda and qkv.dtype == torch.float16 and qkv.shape[-1] in (64, 128) \
-                    and (causal or s == 1) and (s <= HIP_PROMPT_ATTN_MAX_TOKENS or results_only(qkv)):
+                    and (causal or s == 1) and (s <= HIP_PROMPT_ATTN_MAX_TOKENS or (
+                        s <= _longest_prompt(qkv.shape[3] * qkv.shape[4]) and results_only(qkv))):
                 # causal attention and the cache fill in one launch (no permuted copy of K / V)
                 kc = vc = None
                 if inference_params is not None:

@@ -183,3 +183,24 @@ def test_operands_of_a_long_prompts_attention_that_only_the_library_takes():
         assert modules._kernel_takes(qkv, k_cache, v_cache) == (name == "plain")
     assert not modules._kernel_takes(odd)
     torch.testing.assert_close(ops.prefill_attention(qkv), want, rtol=2e-3, atol=2e-3)
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+@pytest.mark.parametrize("T,H,hd,ours", [(6144, 1, 64, True), (6145, 1, 64, False), (2048, 41, 128, True), (2049, 41, 128, False),
+                                         (2049, 40, 128, True)])
+def test_longest_prompts_of_the_attention_kernel(T, H, hd, ours, monkeypatch):
+    """On both sides of the lines; the last queries against every key in 64 bits, fp16 weights and results (5e-4 below 5)."""
+    from dejavu_amd import ops
+    from dejavu_amd.modules import ParallelMHADejavu
+
+    called, kernel = [], ops.prefill_attention
+    monkeypatch.setattr(ops, "prefill_attention", lambda *a: [called.append(1), kernel(*a)][1])
+    mha = ParallelMHADejavu(H * hd, H, causal=True, device="cuda", dtype=torch.float16)
+    qkv = torch.randn(1, T, 3, H, hd, device="cuda").half()
+    got = mha._dense_context(qkv, None).view(T, H, hd)[-3:].double()
+    assert bool(called) == ours
+    q, k, v = (t[0].double().transpose(0, 1) for t in qkv.unbind(2))
+    s = (q[:, -3:] @ k.transpose(1, 2).contiguous()) * hd ** -0.5
+    s[:, 0, -2:], s[:, 1, -1:] = -math.inf, -math.inf
+    torch.testing.assert_close(got, (s.softmax(-1) @ v.contiguous()).transpose(0, 1), rtol=1e-3, atol=5e-3)
