@@ -1142,9 +1142,12 @@ size_t dv_gather_gemv_workspace_bytes(int B, int N, int M) {
 int dv_gather_gemv_ws_f16(const void* x, const void* W, int64_t ldw, const void* bias, const void* idx,
                           int idx_bytes, int B, int N, int Z, int M, int act, void* y, void* workspace,
                           size_t workspace_bytes, void* stream) {
-  if (B < kTiledMinBatch || B > 64 || M <= 0 || workspace == nullptr ||
-      workspace_bytes < dv_gather_gemv_workspace_bytes(B, N, M) || !aligned16(workspace))
-    return dv_gather_gemv_f16(x, W, ldw, bias, idx, idx_bytes, B, N, Z, M, act, y, stream);
+  const size_t needed = dv_gather_gemv_workspace_bytes(B, N, M);
+  // the ring kernel may need none (33..64 rows by 12288 x 4096: 31 us, gather_rows_mfma 72)
+  const bool shared = B >= kTiledMinBatch && B <= 64 && N > 0 && M > 0 &&
+                      (needed > 0 ? workspace != nullptr && workspace_bytes >= needed && aligned16(workspace)
+                                  : workspace != nullptr || shared_kernel(B, N, M, false) == Shared::kRing);
+  if (!shared) return dv_gather_gemv_f16(x, W, ldw, bias, idx, idx_bytes, B, N, Z, M, act, y, stream);
   if (!x || !W || N <= 0 || Z <= 0 || (idx && !idx_ok(idx_bytes)) || !y || (!idx && M > Z) ||
       act < DV_ACT_ID || act > DV_ACT_SQUARED_RELU)
     return DV_ERR_INVALID_ARG;

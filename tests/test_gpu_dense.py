@@ -89,6 +89,21 @@ def test_gathered_rows_out_of_range(rows):
     assert_close(got.float().cpu().numpy(), want.cpu().numpy(), "gathered rows", max_abs_tol=8e-2)  # half an ulp at 128
 
 
+@pytest.mark.parametrize("rows,N,M", [(33, 4096, 12288), (64, 4096, 10240), (48, 264, 16390)])
+def test_gathered_rows_that_need_no_workspace(rows, N, M):
+    """Weights with tiles enough for the chip are not split, and go to the same kernel as the dense product: the same bits."""
+    from dejavu_amd import ops
+    from dejavu_amd._lib import lib
+
+    assert lib.dv_gather_gemv_workspace_bytes(rows, N, M) == 0
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x, W = torch.randn(rows, N, generator=g, device="cuda").half(), (torch.randn(M, N, generator=g, device="cuda") * N ** -0.5).half()
+    want = ops.dense_linear(x, W)
+    assert torch.equal(ops.gather_gemv(x, W, None), want)
+    idx = torch.randperm(M, generator=g, device="cuda")
+    assert torch.equal(ops.gather_gemv(x, W, idx), want[:, idx])
+
+
 def test_dense_linear_three_dimensional_input():
     from dejavu_amd import ops
 
