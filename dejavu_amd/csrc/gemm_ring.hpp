@@ -61,12 +61,13 @@ struct RingPlan {
 // More rows: 128 rows of W, so that X is fetched less often (5120 x 20480 with 96 rows: 53 us, 60 with 64 rows of W),
 // where that leaves 32 tiles and K is long enough to split; 192 where they fill the chip better (20480 x 5120 with 96 rows:
 // 107 tiles in 2 splits take 53 us, 160 tiles of 128 rows 59) or spare a round of it (36864 x 12288 with 128 rows: 192
-// tiles against 288).
+// tiles against 288).  257 to 384 rows are two tiles of 192, not of 256 (320 rows: QKV of 24 heads of 9216 97 against 147 us, of
+// 32 heads of 12288 141 against 195).
 // A split has at least 256 columns.
 inline RingPlan plan_ring(int n, int M, int K) {
   constexpr int kUnits = 256;
   RingPlan p;
-  p.nb = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : n <= 128 ? 128 : n <= 192 ? 192 : 256;
+  p.nb = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : n <= 128 ? 128 : n <= 192 || (n > 256 && n <= 384) ? 192 : 256;
   auto lay = [&](int mb) {
     p.mb = mb;
     p.rows = (M + mb - 1) / mb;

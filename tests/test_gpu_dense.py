@@ -49,13 +49,14 @@ def test_dense_linear_matches_fp32_reference(rows, N, M, act):
     assert torch.equal(y, y2), "two runs differ (the split reduction must be deterministic)"
 
 
-# Both sides of the rules that choose a kernel and a tile (rows 64 | 65, 128 | 129, 192 | 193, 256 | 257, 512 | 513; weights of
+# Both sides of the rules that choose a kernel and a tile (rows 64 | 65, 128 | 129, 192 | 193, 256 | 257, 384 | 385, 512 | 513; weights of
 # 20 and 52 million elements; fewer than 32 tiles of 128 rows; rows of W too short to split), last tiles of one to four rows.
 @pytest.mark.parametrize("rows,N,M,act", [(9, 264, 70, "gelu"), (30, 4096, 4884, "id"), (20, 4096, 4100, "relu"),
                                           (50, 12288, 4097, "id"), (65, 264, 70, "relu"), (128, 2056, 4099, "id"),
                                           (100, 4104, 12290, "gelu_approx"), (129, 1032, 4101, "squared_relu"),
                                           (192, 2048, 5121, "id"), (140, 4096, 18433, "id"), (193, 8, 33, "relu"),
-                                          (256, 2056, 4098, "relu"), (257, 520, 71, "id"), (512, 2056, 130, "relu"),
+                                          (256, 2056, 4098, "relu"), (257, 520, 71, "id"), (384, 2056, 5442, "id"), (385, 2056, 130, "id"),
+                                          (512, 2056, 130, "relu"),
                                           (513, 520, 70, "id"), (300, 256, 16390, "id")])
 def test_dense_linear_at_the_edges_of_its_rules(rows, N, M, act):
     from dejavu_amd import ops
