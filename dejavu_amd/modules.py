@@ -51,15 +51,13 @@ USE_HIP_PROMPT = True
 HIP_PROMPT_MAX_ROWS = 192
 # But where the weight's rows are four times as long as they are many (fc2), the library leaves much of the chip idle for some
 # hundred rows more: up to 256 from 2^23 elements on (us, this kernel against the library, 256 rows: 1024 x 8192 20.8 / 21.0, 2048 x
-# 8192 24 / 28, 5120 x 20480 79 / 225, 12288 x 49152 396 / 478; but 768 x 3072 12.7 / 9.2, 4096 x 5120 31 / 29), and up to 512 for
-# weights of 4096 to 7168 rows (4096 x 16384 with 300 / 384 / 512 rows 81 / 82 / 86 against 88 / 90 / 110, 5120 x 20480 127 / 123 / 131
-# against 129 / 151 / 193, 7168 x 28672 233 / 234 / 243 against 266 / 276 / 289; but 3072 x 12288 76 against 58 to 73, 9216 x 36864
-# 500 against 380 to 409).  Just above 256 rows the second tile of rows is nearly empty (5120 x 20480, 257 rows: 126 / 121).
+# 8192 24 / 28, 5120 x 20480 79 / 225, 12288 x 49152 396 / 478; but 768 x 3072 12.7 / 9.2, 4096 x 5120 31 / 29), up to 384 from 4096
+# weight rows on (300 rows: 4096 x 16384 70 / 88, 5120 x 20480 103 / 129, 9216 x 36864 301 / 375; but 3072 x 12288 62 / 57) and up to
+# 512 to 8192 of them (4096 x 16384 86 / 108, 8192 x 32768 292 / 347; but 9216 x 36864 506 / 403).
 HIP_PROMPT_LONG_MAX_ROWS = 512
-HIP_PROMPT_LONG_ROWS = 256
-HIP_PROMPT_LONG_MORE_ROWS = 288
+HIP_PROMPT_LONG_ROWS = 256, 384
 HIP_PROMPT_LONG_WEIGHT = 1 << 23
-HIP_PROMPT_LONG_WEIGHT_ROWS = (4096, 7168)
+HIP_PROMPT_LONG_WEIGHT_ROWS = 4096, 8192
 # The package's causal-attention kernel (cache fill in the same launch) is ahead of the library's attention with the
 # permuted cache copies (40 heads of 128 and 128 / 1024 tokens: 7.5 / 47 us against 25 / 100; 32 heads and
 # 777 / 2000 / 4000 tokens: 30 / 110 / 385 against 75 / 310 / 566; 16 sequences of 1024: 547 against 768).  Prompts of more than so
@@ -277,8 +275,8 @@ class ParallelFusedMLPDejavu(nn.Module):
 def _long_rule(rows: int, M: int, K: int) -> bool:
     if K < 4 * M or M * K < HIP_PROMPT_LONG_WEIGHT:
         return False
-    low, high = HIP_PROMPT_LONG_WEIGHT_ROWS
-    return rows <= HIP_PROMPT_LONG_ROWS or (low <= M <= high and HIP_PROMPT_LONG_MORE_ROWS <= rows <= HIP_PROMPT_LONG_MAX_ROWS)
+    (few, more), (low, high) = HIP_PROMPT_LONG_ROWS, HIP_PROMPT_LONG_WEIGHT_ROWS
+    return rows <= few or (M >= low and (rows <= more or (rows <= HIP_PROMPT_LONG_MAX_ROWS and M <= high)))
 
 
 def _long_product(linear, x: torch.Tensor) -> bool:

@@ -74,10 +74,9 @@ def test_rule_of_a_long_prompts_linear():
     """Both sides of each line, in rows and in the weight's size and shape."""
     from dejavu_amd.modules import _long_rule
 
-    for rows, M, K, ours in ((193, 4096, 16384, True), (256, 4096, 16384, True), (257, 4096, 16384, False), (287, 4096, 16384, False),
-                             (288, 4096, 16384, True), (512, 7168, 28672, True), (513, 4096, 16384, False), (200, 1024, 8192, True),
-                             (200, 1024, 8184, False), (200, 4096, 16376, False), (256, 12288, 49152, True), (300, 12288, 49152, False),
-                             (300, 2048, 8192, False), (256, 768, 3072, False)):
+    for rows, M, K, ours in ((193, 4096, 16384, True), (256, 1024, 8192, True), (256, 1024, 8184, False), (256, 4096, 16376, False),
+                             (256, 768, 3072, False), (257, 4096, 16384, True), (257, 4088, 16384, False), (384, 12288, 49152, True),
+                             (385, 8192, 32768, True), (385, 8200, 32800, False), (512, 4096, 16384, True), (513, 4096, 16384, False)):
         assert _long_rule(rows, M, K) == ours, (rows, M, K)
 
 
