@@ -501,17 +501,23 @@ int ring_scratch(const RingPlan& p, const void* workspace, size_t workspace_byte
 // Which kernel takes a product of B rows.  From 65 rows on the ring (12288 x 4096 with 100 / 190 / 256 rows: 31 / 38 / 46 us
 // against 39 / 59 / 57; QKV of 24 heads of 9216 with 96 / 160 / 240 rows 46 / 56 / 68 against 53 / 90 / 124; 32 heads of
 // 12288 with 320 and 480 rows 191 and 195 against 208 and 214 with gemm_big.hpp; 5120 x 20480 with 384 rows 134 against 245),
-// but not plain products of more than 512 rows, or of 16384 rows of W and more than 256, which gemm_big.hpp takes (20480 x
-// 5120 with 384 rows: 136 against 166).  Fewer rows are bound by the stream alone, and there
-// gemm_tiled.hpp, whose loads cover 512 bytes of a row, is ahead for large weights (12288 x 12288 with 16 / 64 rows: 58 / 68
-// against 71 / 89 us), the ring for small ones (4096 x 4096 with 50 rows 13 against 18; 4096 gathered rows of 12288 with 64
-// rows 27 against 31, with 32 rows 26 against 25; QKV of 16 heads of 5120 with 24 rows 19 against 23).
+// but not plain products of more than 512 rows, or of more than 40960 rows of W and 256, which gemm_big.hpp takes where its
+// chunks divide N (50272 x 4096 with 300 / 400 rows: the ring 259 / 309, that 243 / 349; 36864 x 4096 199 / 237 against 195 / 242, 20480
+// x 5120 105 / 165 against 132 / 200), nor of up to 128 rows and more than 32768 of W, which are more than a round of tiles
+// (50272 x 4096 with 72 / 128 rows: 122 / 126 us, gemm_tiled.hpp 105 / 114).  Fewer rows are bound by the stream alone, and there
+// gemm_tiled.hpp, whose loads cover 512 bytes of a row, is ahead for large weights, the ring for small ones (us, the ring against
+// it: 33 to 64 rows 4096 x 4096 14 / 19, 5120 x 5120 18 / 21, 4096 x 8192 23 / 22, 12288 x 12288 89 / 68; up to 32 rows 2048 x 4096 9.5 / 10,
+// 4096 x 3072 13 / 12, QKV of 16 heads of 5120 26 / 23).  Of 33 to 64 rows it also takes 4096 to 7680 rows of a larger weight, which
+// make 64 to 120 tiles in whole rounds with two to four splits (7168 x 5120 21 / 24, 9216 x 4096 21 / 22, but 2560 x 10240 22 / 19,
+// 12288 x 3072 31 / 26).
 enum class Shared { kRing, kTiled, kBig };
 Shared shared_kernel(int B, int N, int M, bool qkv) {
   const int64_t weight = (int64_t)M * N;
-  if (!qkv && (B > 512 || (B > 256 && M > 16384))) return N % (kBgKC * kBgRing) == 0 ? Shared::kBig : Shared::kTiled;
+  if (!qkv && (B > 512 || (B > 256 && M > 40960)) && N % (kBgKC * kBgRing) == 0) return Shared::kBig;
+  if (!qkv && (B > 512 || (B > 64 && B <= 128 && M > 32768))) return Shared::kTiled;
   if (B > 64) return Shared::kRing;
-  const int64_t most = B > 32 ? 52000000 : (qkv ? (B > 16 ? 32000000 : 0) : 20000000);
+  const bool rounds = !qkv && B > 32 && M >= 4096 && M <= 7680;
+  const int64_t most = B > 32 ? (qkv ? 26000000 : rounds ? 52000000 : 21000000) : qkv ? 0 : 1 << 23;
   return weight <= most ? Shared::kRing : Shared::kTiled;
 }
 

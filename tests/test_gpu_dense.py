@@ -49,15 +49,20 @@ def test_dense_linear_matches_fp32_reference(rows, N, M, act):
     assert torch.equal(y, y2), "two runs differ (the split reduction must be deterministic)"
 
 
-# Both sides of the rules that choose a kernel and a tile (rows 64 | 65, 128 | 129, 192 | 193, 256 | 257, 384 | 385, 512 | 513; weights of
-# 20 and 52 million elements; fewer than 32 tiles of 128 rows; rows of W too short to split), last tiles of one to four rows.
+# Both sides of the rules that choose a kernel and a tile (rows 64 | 65, 128 | 129, 192 | 193, 256 | 257, 384 | 385, 512 | 513;
+# weights of 2^23, 21 and 52 million elements; 7680, 32768 and 40960 rows of W; fewer than 32 tiles of 128 rows; one round of
+# tiles of 64; rows of W too short to split), last tiles of one to four rows.
 @pytest.mark.parametrize("rows,N,M,act", [(9, 264, 70, "gelu"), (30, 4096, 4884, "id"), (20, 4096, 4100, "relu"),
                                           (50, 12288, 4097, "id"), (65, 264, 70, "relu"), (128, 2056, 4099, "id"),
                                           (100, 4104, 12290, "gelu_approx"), (129, 1032, 4101, "squared_relu"),
                                           (192, 2048, 5121, "id"), (140, 4096, 18433, "id"), (193, 8, 33, "relu"),
                                           (256, 2056, 4098, "relu"), (257, 520, 71, "id"), (384, 2056, 5442, "id"), (385, 2056, 130, "id"),
                                           (512, 2056, 130, "relu"),
-                                          (513, 520, 70, "id"), (300, 256, 16390, "id")])
+                                          (513, 520, 70, "id"), (300, 256, 16390, "id"),
+                                          (32, 2048, 4096, "id"), (32, 2048, 4104, "id"), (40, 5120, 4104, "relu"),
+                                          (64, 6656, 7680, "id"), (64, 6656, 7688, "id"), (64, 264, 32770, "id"),
+                                          (65, 264, 32768, "id"), (65, 264, 32770, "id"), (129, 264, 32770, "id"),
+                                          (300, 264, 40970, "id"), (300, 256, 40970, "relu")])
 def test_dense_linear_at_the_edges_of_its_rules(rows, N, M, act):
     from dejavu_amd import ops
 
@@ -90,7 +95,7 @@ def test_gathered_rows_out_of_range(rows):
     assert_close(got.float().cpu().numpy(), want.cpu().numpy(), "gathered rows", max_abs_tol=8e-2)  # half an ulp at 128
 
 
-@pytest.mark.parametrize("rows,N,M", [(33, 4096, 12288), (64, 4096, 10240), (48, 264, 16390)])
+@pytest.mark.parametrize("rows,N,M", [(33, 1024, 12288), (64, 2048, 10240), (48, 264, 16390)])
 def test_gathered_rows_that_need_no_workspace(rows, N, M):
     """Weights with tiles enough for the chip are not split, and go to the same kernel as the dense product: the same bits."""
     from dejavu_amd import ops
