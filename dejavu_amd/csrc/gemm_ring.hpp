@@ -59,7 +59,8 @@ struct RingPlan {
 // 4096 x 11008).  K is split until there are about as many workgroups as compute units (4096 x 11008 with 47 rows: 1, 2, 4,
 // 8 splits take 52, 32, 24.5, 27 us); the narrowest tiles' workgroups are small, so they go on to two per unit.
 // More rows: 128 rows of W, so that X is fetched less often (5120 x 20480 with 96 rows: 53 us, 60 with 64 rows of W),
-// where that leaves 32 tiles and K is long enough to split; 192 where they fill the chip better (20480 x 5120 with 96 rows:
+// where that leaves 32 tiles and K is long enough to split (but 64 where these make one round and K is short: 16384 x 4096 with
+// 72 / 128 rows 41.5 / 45 us, in two splits 47.5 / 48); 192 where they fill the chip better (20480 x 5120 with 96 rows:
 // 107 tiles in 2 splits take 53 us, 160 tiles of 128 rows 59) or spare a round of it (36864 x 12288 with 128 rows: 192
 // tiles against 288).  257 to 384 rows are two tiles of 192, not of 256 (320 rows: QKV of 24 heads of 9216 97 against 147 us, of
 // 32 heads of 12288 141 against 195).
@@ -80,7 +81,7 @@ inline RingPlan plan_ring(int n, int M, int K) {
   };
   if (p.nb <= 64) {
     lay(p.nb == 16 ? 32 : p.nb == 64 && M >= 16384 ? 96 : 64);
-  } else if (M < 32 * 128 || K < 2048) {
+  } else if (M < 32 * 128 || K < 2048 || (p.nb == 128 && K <= 4096 && M > 224 * 64 && M <= kUnits * 64)) {
     lay(64);
   } else {
     const bool tall = p.nb < 256 && K >= 4096;

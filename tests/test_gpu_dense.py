@@ -55,7 +55,8 @@ def test_dense_linear_matches_fp32_reference(rows, N, M, act):
 @pytest.mark.parametrize("rows,N,M,act", [(9, 264, 70, "gelu"), (30, 4096, 4884, "id"), (20, 4096, 4100, "relu"),
                                           (50, 12288, 4097, "id"), (65, 264, 70, "relu"), (128, 2056, 4099, "id"),
                                           (100, 4104, 12290, "gelu_approx"), (129, 1032, 4101, "squared_relu"),
-                                          (192, 2048, 5121, "id"), (140, 4096, 18433, "id"), (193, 8, 33, "relu"),
+                                          (192, 2048, 5121, "id"), (140, 4096, 18433, "id"),
+                                          (128, 2048, 14340, "id"), (100, 4096, 16383, "id"), (193, 8, 33, "relu"),
                                           (256, 2056, 4098, "relu"), (257, 520, 71, "id"), (384, 2056, 5442, "id"), (385, 2056, 130, "id"),
                                           (512, 2056, 130, "relu"),
                                           (513, 520, 70, "id"), (300, 256, 16390, "id"),
