@@ -10,6 +10,7 @@
 
 #include "attention.hpp"
 #include "common.hpp"
+#include "device.hpp"
 #include "gemm_cols16.hpp"
 #include "gemm_mfma.hpp"
 #include "gemm_big.hpp"
@@ -32,26 +33,6 @@ inline bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7
 inline bool idx_ok(int idx_bytes) { return idx_bytes == 4 || idx_bytes == 8; }
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? DV_OK : DV_ERR_LAUNCH; }
-
-constexpr int kMaxDevices = 64;
-
-int current_device() {
-  int dev = 0;
-  return (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices) ? dev : -1;
-}
-
-// Compute units of the current device (remembered per device).
-int compute_units() {
-  static std::atomic<int> cus[kMaxDevices];
-  const int dev = current_device();
-  if (dev < 0) return 256;
-  int v = cus[dev].load(std::memory_order_relaxed);
-  if (v == 0) {
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
-    cus[dev].store(v, std::memory_order_relaxed);
-  }
-  return v;
-}
 
 // Dynamic LDS above 48 KiB has to be granted per kernel and per device.  One object per kernel
 // (static storage: starts at zero) remembers the largest size granted on each device, so a steady
@@ -524,7 +505,7 @@ Shared shared_kernel(int B, int N, int M, bool qkv) {
 size_t tiled_workspace_bytes(int B, int N, int M, bool qkv = false) {
   const Shared kind = shared_kernel(B, N, M, qkv);
   if (kind == Shared::kBig) return 0;
-  if (kind == Shared::kRing) return plan_ring(B, M, N).workspace_bytes();
+  if (kind == Shared::kRing) return plan_ring(B, M, N, compute_units()).workspace_bytes();
   const TiledPlan p = plan_tiled(B, N, M);
   return p.nsplit > 1 ? (size_t)p.nsplit * B * M * sizeof(float) : 0;
 }
@@ -574,7 +555,7 @@ int gemm_tiled_qkv(const half_t* X, int64_t ldx, const half_t* W, const half_t* 
                    const QkvScatter& qs, void* workspace, size_t workspace_bytes, hipStream_t s) {
   const int M = 3 * qs.Hk * qs.hd, Z = 3 * qs.H * qs.hd;
   if (shared_kernel(B, d, M, true) == Shared::kRing) {
-    const RingPlan p = plan_ring(B, M, d);
+    const RingPlan p = plan_ring(B, M, d, compute_units());
     if (int rc = ring_scratch(p, workspace, workspace_bytes); rc != DV_OK) return rc;
     return gemm_ring(p, RingOperands<half_t>{X, ldx, W, (int64_t)d, B, M, d}, QkvRows{qs}, QkvOut{bias, Y, qs}, workspace, s,
                      RingLaunch{});
@@ -624,7 +605,7 @@ int gemm_tiled(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const
   if (kind == Shared::kBig)
     return gemm_big(X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, act, s);
   if (kind == Shared::kRing) {
-    const RingPlan p = plan_ring(B, M, N);
+    const RingPlan p = plan_ring(B, M, N, compute_units());
     if (int rc = ring_scratch(p, workspace, workspace_bytes); rc != DV_OK) return rc;
     const RingOperands<half_t> a{X, ldx, W, ldw, B, M, N};
     if (idx == nullptr) return gemm_ring(p, a, PlainRows{}, PlainOut{bias, act, Y, ldy, M}, workspace, s, RingLaunch{});

@@ -65,8 +65,8 @@ struct RingPlan {
 // tiles against 288).  257 to 384 rows are two tiles of 192, not of 256 (320 rows: QKV of 24 heads of 9216 97 against 147 us, of
 // 32 heads of 12288 141 against 195).
 // A split has at least 256 columns.
-inline RingPlan plan_ring(int n, int M, int K) {
-  constexpr int kUnits = 256;
+// The row counts 14336 and 16384 of these are what 224 and 256 of `units`, the device's compute units, take in a round.
+inline RingPlan plan_ring(int n, int M, int K, int units) {
   RingPlan p;
   p.nb = n <= 16 ? 16 : n <= 32 ? 32 : n <= 64 ? 64 : n <= 128 ? 128 : n <= 192 || (n > 256 && n <= 384) ? 192 : 256;
   auto lay = [&](int mb) {
@@ -74,21 +74,21 @@ inline RingPlan plan_ring(int n, int M, int K) {
     p.rows = (M + mb - 1) / mb;
     p.cols = (n + p.nb - 1) / p.nb;
     const int64_t tiles = (int64_t)p.rows * p.cols;
-    int64_t s = p.nb == 16 ? (tiles >= kUnits ? 1 : tiles >= kUnits / 2 ? 4 : 8) : (p.nb <= 64 ? 288 : kUnits) / tiles;
+    int64_t s = p.nb == 16 ? (tiles >= units ? 1 : tiles >= units / 2 ? 4 : 8) : (p.nb <= 64 ? units * 9 / 8 : units) / tiles;
     if (s > K / 256) s = K / 256;
     p.splits = (int)(s < 1 ? 1 : s > 8 ? 8 : s);
     return (int64_t)p.splits * tiles;
   };
   if (p.nb <= 64) {
-    lay(p.nb == 16 ? 32 : p.nb == 64 && M >= 16384 ? 96 : 64);
-  } else if (M < 32 * 128 || K < 2048 || (p.nb == 128 && K <= 4096 && M > 224 * 64 && M <= kUnits * 64)) {
+    lay(p.nb == 16 ? 32 : p.nb == 64 && M >= units * 64 ? 96 : 64);
+  } else if (M < 32 * 128 || K < 2048 || (p.nb == 128 && K <= 4096 && M > units * 56 && M <= units * 64)) {
     lay(64);
   } else {
     const bool tall = p.nb < 256 && K >= 4096;
     const int64_t groups = lay(128);
     if (tall) {
-      const int64_t more = lay(192), rounds = (groups + kUnits - 1) / kUnits, tall_rounds = (more + kUnits - 1) / kUnits;
-      const bool fuller = groups <= kUnits ? more <= kUnits && more * 10 > groups * 11 : tall_rounds * 192 < rounds * 128;
+      const int64_t more = lay(192), rounds = (groups + units - 1) / units, tall_rounds = (more + units - 1) / units;
+      const bool fuller = groups <= units ? more <= units && more * 10 > groups * 11 : tall_rounds * 192 < rounds * 128;
       if (!fuller) lay(128);
     }
   }

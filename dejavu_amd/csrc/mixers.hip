@@ -5,6 +5,7 @@
 
 #include <atomic>
 
+#include "device.hpp"
 #include "mix/attn_f32.hpp"
 #include "mix/attn_latent.hpp"
 #include "mix/attn_rows.hpp"
@@ -455,14 +456,14 @@ int dv_mix_linear_row(int dtype, int before, int after, const dvRowArgs* a, void
 
 size_t dv_mix_linear_tiles_workspace_bytes(int n, int M, int K) {
   if (n < 1 || M < 1 || K < 8) return 0;
-  return plan_ring(n, M, K).workspace_bytes();
+  return plan_ring(n, M, K, compute_units()).workspace_bytes();
 }
 
 int dv_mix_linear_tiles_ws(int after, const dvTileArgs* a, void* workspace, size_t workspace_bytes, void* stream) {
   const int rc = tile_args_ok(after, a);
   if (rc != DV_OK) return rc;
   if (!al16(workspace)) return DV_ERR_ALIGNMENT;
-  RingPlan p = plan_ring(a->n, a->M, a->K);
+  RingPlan p = plan_ring(a->n, a->M, a->K, compute_units());
   if (p.cols > 65535) return DV_ERR_UNSUPPORTED;
   if (!workspace) p.splits = 1;
   else if (workspace_bytes < p.workspace_bytes()) return DV_ERR_WORKSPACE;

@@ -186,12 +186,15 @@ def _tile_args(x, W) -> L.TileArgs:
                       K=W.shape[1])
 
 
-_tile_workspace_bytes = lru_cache(maxsize=4096)(lib.dv_mix_linear_tiles_workspace_bytes)  # a function of the sizes alone
+@lru_cache(maxsize=4096)
+def _tile_workspace_bytes(device: int, n: int, M: int, K: int) -> int:
+    """A function of the sizes and of the current device, whose compute units the splits are made for."""
+    return lib.dv_mix_linear_tiles_workspace_bytes(n, M, K)
 
 
 def _tile_launch(after, a, device) -> None:
     """The workspace is this call's own: calls on other streams have theirs, and a captured one is its graph's."""
-    nbytes = _tile_workspace_bytes(a.n, a.M, a.K)
+    nbytes = _tile_workspace_bytes(torch._C._cuda_getDevice(), a.n, a.M, a.K)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
     check(lib.dv_mix_linear_tiles_ws(after, _ref(a), _ptr(ws), nbytes, _stream()), "dv_mix_linear_tiles_ws")
 
