@@ -585,8 +585,7 @@ int gemm_tiled_qkv(const half_t* X, int64_t ldx, const half_t* W, const half_t* 
   } while (0)
   if (p.bt == 1) { if (p.wt == 2) DV_TQ(1, 2); else DV_TQ(1, 1); }
   else if (p.bt == 2) { if (p.wt == 2) DV_TQW(2, 2, 128, 8); else DV_TQ(2, 1); }
-  else if (p.bt == 4) DV_TQW(4, 2, 128, 8);
-  else DV_TQW(8, 2, 128, 8);
+  else DV_TQW(4, 2, 128, 8);  // (more than 64 rows go to the ring)
 #undef DV_TQW
 #undef DV_TQ
   if (p.nsplit > 1) {
