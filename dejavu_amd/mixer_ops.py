@@ -2,9 +2,10 @@
 
 Weights and activations are bf16 or fp32 (one type per model); the residual stream, norms, scores and recurrent state
 are fp32.  All ops enqueue on ``torch.cuda.current_stream()`` and refuse CPU tensors.  Products: one row goes to the
-row kernel, up to ``TILE_MAX_ROWS`` bf16 rows to the matrix-core kernel that streams the weight, both with the operation
-that follows in the same launch; longer portions (and several fp32 rows) take the library GEMM and a separate elementwise
-launch, as the dense products of long prompts do elsewhere in this package.
+row kernel, up to 64 bf16 rows, and up to ``TILE_MAX_ROWS`` where it is the faster one (``_tile_rule``), to the matrix-core
+kernel that streams the weight, some portions of more than a thousand rows to the one with wide tiles (``_wide_rule``), all
+with the operation that follows in the same launch; the other portions (and several fp32 rows) take the library GEMM and a
+separate elementwise launch, as the dense products of long prompts do elsewhere in this package.
 """
 from __future__ import annotations
 
@@ -19,13 +20,21 @@ from . import _lib_mixers as L
 from ._binding import results_only
 from ._lib_mixers import check, lib
 
-# The streaming kernel against the library GEMM without the launch that follows it, us: 4096 x 11008 with 96 / 192 / 256
-# rows 28 / 35 / 40 against 50 / 81 / 52, 22016 x 4096 52 / 58 / 65 against 47 / 61 / 64 (and 5 to 9 for the gated unit that
-# follows), 4096 x 4096 16 / 19 / 22 against 22 / 33 / 23.  The library is ahead for small weights from 192 rows on (2048 x
-# 2048 with 256 rows: 11.4 against 9.7) and beyond 256 rows, where the operations bound the product.
+# Beyond 64 rows the streaming kernel where it is ahead of the library GEMM and the launch that follows it, with weights that are
+# not in the caches (24 weights, 65 to 256 rows).  us, library / kernel:
+#   the gated unit up to 192 rows: 6144 x 4096 with 65 / 128 / 192 rows 1.25 / 1.32 / 1.45 times the library's speed, 11264 x 2048
+#   1.07 / 1.01 / 1.13, 12288 x 4096 1.17 / 1.14 / 1.18; but 22016 x 4096 0.88 / 0.89 / 1.00, 50000 x 2048 1.01 / 0.96 / 0.92: there the
+#   tiles make more than a round and the library's larger ones read x less often;
+#   norm and residual, or nothing, up to 192 rows: 4096 x 4096 with 96 / 192 rows 26 / 20 and 38 / 27, 4096 x 11008 54 / 33 and 86 / 40,
+#   2048 x 2048 14.6 / 11.5 and 16 / 14; but 4096 x 2048 with 130 rows 18 / 21, 5120 x 2048 with 96 17 / 19, plain 8192 x 2048 0.9 of it;
+#   beyond 192: the gated unit of 4096 x 4096 1.02, 12288 x 4096 1.00 to 1.20, 4096 x 2048 0.8; the others of 4096 x 11008
+#   52 / 44, 4096 x 8192 39 / 38, but 4096 x 4096 27 / 29, 4096 x 5632 30 / 33, 4096 x 2048 19 / 25.
 TILE_MAX_ROWS = 256
-TILE_ALL_ROWS = 192          # up to here whatever the weight's size
-TILE_WEIGHT = 1 << 23        # elements from which the rows may be more
+TILE_MORE_ROWS = 192               # beyond these the lines are narrower
+TILE_MAX_WEIGHT_ROWS = 12288
+TILE_MIN_COLUMNS = 4096            # or TILE_SMALL_WEIGHT elements at most
+TILE_SMALL_WEIGHT = 1 << 22
+TILE_MORE_COLUMNS = 8192
 
 _DTYPES = {torch.bfloat16: L.BF16, torch.float32: L.F32}
 _ref = ctypes.byref
@@ -97,36 +106,58 @@ def residual(y: Optional[torch.Tensor], stream: ResidualStream, post, pre, add_s
     return h
 
 
-# Where the 256 x 256 tiles of the wide kernel make two rounds of the chip's compute units or more and the chunks are many, it is
-# ahead of the library GEMM with the gated unit's launch (22016 x 4096 with 1500 / 1700 / 2048 / 3000 / 4096 rows: 290 / 304 /
-# 324 / 499 / 631 against 313 / 346 / 422 / 507 / 689 us; with 1280 rows, 430 tiles, 215 against 194) up to six rounds (6000
-# rows, 2064 tiles: 972 against 925; 12000: 1865 against 1722), and for plain
-# products up to three rounds (18560 x 4096 with 1700 / 1999 / 3000 rows: 228 / 295 / 401 against 252 / 338 / 362;
-# 11264 x 2048 with 3000: 158 against 122) and 2048 rows (products with 4096 rows of W and 8192 of x, 512 tiles: 463 against
-# 379 on average).
-WIDE_MAX_PLAIN_ROWS = 2048
-WIDE_TILE, WIDE_MIN_TILES, WIDE_MAX_TILES, WIDE_MAX_PLAIN_TILES, WIDE_MIN_COLUMNS = 256, 500, 1536, 768, 4096
+# The wide kernel and the library GEMM take about as long for a full round of 256 x 256 tiles (one on each of 256 compute units); the
+# library also has tiles 192 wide, and where they are the right ones it wins: 24576 x 4096 with 1435 rows 0.85 of its time, plain
+# 0.77; 21760 x 4096 with 1624 rows 0.82 and 0.75.  Where the wide tiles make three rounds, and those of 192 by 256 four either way, the
+# library's choice costs it more (gated unit / plain product, times its speed: 22016 x 4096 with 1603 / 1904 / 2048 rows 1.12 / 1.07,
+# 1.29 / 1.24, 1.33 / 1.27; 18560 x 4096 with 2000 1.20 / 1.15; 18944 x 5120 with 2000 1.26 / 1.16; 20480 x 4096 with 1918 1.27 / 1.20).
+# Outside of these lines it is the other way round as often as not: weights whose rows 192 divides (19200 x 4096 with 1939 rows
+# 0.89 / 0.82), taller ones (28672 x 4096 with 1365 rows 0.86 / 0.80), longer rows (22016 x 8192 with 1700 rows 1.04 / 0.98, 18560 x
+# 6144 with 1999 1.11 / 1.01), and more than 2048 rows of x, where the library ranges from 0.85 to 1.45 (17920 x 4096 with 2191 / 2520 rows 0.87 /
+# 1.41).
+WIDE_MAX_ROWS = 2048
+WIDE_COLUMNS = 4096, 5120
+WIDE_MAX_WEIGHT_ROWS = 22528
+WIDE_TILE, NARROW_TILE, WIDE_ROUND = 256, 192, 256
+WIDE_TILES = 2 * WIDE_ROUND + 1, 3 * WIDE_ROUND - 10  # (a third round that is all but full is the library's again)
+
+
+def _tiles_of(n: int, M: int, rows: int, weight_rows: int) -> int:
+    return -(-n // rows) * -(-M // weight_rows)
+
+
+def _wide_rule(n: int, M: int, K: int) -> bool:
+    if n > WIDE_MAX_ROWS or M > WIDE_MAX_WEIGHT_ROWS or M % NARROW_TILE == 0 or not WIDE_COLUMNS[0] <= K <= WIDE_COLUMNS[1]:
+        return False
+    narrow = min(_tiles_of(n, M, NARROW_TILE, WIDE_TILE), _tiles_of(n, M, WIDE_TILE, NARROW_TILE))
+    return WIDE_TILES[0] <= _tiles_of(n, M, WIDE_TILE, WIDE_TILE) <= WIDE_TILES[1] and narrow > 3 * WIDE_ROUND
+
+
+def _tile_rule(n: int, M: int, K: int, gated: bool) -> bool:
+    if n > TILE_MAX_ROWS or M > TILE_MAX_WEIGHT_ROWS:
+        return False
+    if n > TILE_MORE_ROWS:
+        return K >= (TILE_MIN_COLUMNS if gated else TILE_MORE_COLUMNS)
+    return gated or K >= TILE_MIN_COLUMNS or M * K <= TILE_SMALL_WEIGHT
 
 
 def _aligned(x: torch.Tensor, W: torch.Tensor) -> bool:
     return all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, W)) and x.shape[1] % 8 == 0 and W.shape[0] % 2 == 0
 
 
-def _wide(x: torch.Tensor, W: torch.Tensor, plain: bool, bias=None) -> bool:
+def _wide(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
     """Whether the wide kernel takes the product."""
-    M, K = W.shape
-    if x.dtype != torch.bfloat16 or K < WIDE_MIN_COLUMNS or (plain and x.shape[0] > WIDE_MAX_PLAIN_ROWS):
-        return False
-    tiles = -(-M // WIDE_TILE) * -(-x.shape[0] // WIDE_TILE)
-    return WIDE_MIN_TILES <= tiles <= (WIDE_MAX_PLAIN_TILES if plain else WIDE_MAX_TILES) and results_only(x, W, bias) and _aligned(x, W)
+    return x.dtype == torch.bfloat16 and _wide_rule(x.shape[0], *W.shape) and results_only(x, W, bias) and _aligned(x, W)
 
 
-def _tiles(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
-    """Whether the streaming kernel takes the product.  From 65 rows on the library takes what it would refuse."""
+def _tiles(x: torch.Tensor, W: torch.Tensor, bias=None, gated: bool = False, whole: bool = True) -> bool:
+    """Whether the streaming kernel takes the product.  From 65 rows on the library takes what it would refuse; whole: a
+    separate launch can follow the library (else what the streaming kernel can take is its own)."""
     n = x.shape[0]
     if x.dtype != torch.bfloat16 or n <= 64:
         return x.dtype == torch.bfloat16
-    return (n <= TILE_ALL_ROWS or (n <= TILE_MAX_ROWS and W.numel() >= TILE_WEIGHT)) and results_only(x, W, bias) and _aligned(x, W)
+    taken = _tile_rule(n, *W.shape, gated) if whole else n <= TILE_MAX_ROWS
+    return taken and results_only(x, W, bias) and _aligned(x, W)
 
 
 def _product_ok(x, W):
@@ -217,7 +248,7 @@ def linear(x, W: torch.Tensor, bias: Optional[torch.Tensor] = None, f32: bool = 
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
         _tile_launch(L.OUT_F32 if f32 else L.OUT_T, a, x.device)
         return out
-    if not f32 and _wide(x, W, True, bias):
+    if not f32 and _wide(x, W, bias):
         out = torch.empty(n, M, dtype=out_t, device=x.device)
         a = _tile_args(x, W)
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
@@ -236,11 +267,11 @@ def gated_unit(x, W: torch.Tensor, act: int, limit: float = 0.0) -> torch.Tensor
         _row_launch(code, before, L.OUT_GLU, a)
         return y
     code = _product_ok(x, W)
-    if _tiles(x, W):
+    if _tiles(x, W, gated=True, whole=y.numel() % 4 == 0):
         a = _tile_args(x, W)
         a.out, a.ldo, a.act, a.limit = y.data_ptr(), M // 2, act, limit
         _tile_launch(L.OUT_GLU, a, x.device)
-    elif _wide(x, W, False):
+    elif _wide(x, W):
         a = _tile_args(x, W)
         a.out, a.ldo, a.act, a.limit = y.data_ptr(), M // 2, act, limit
         check(lib.dv_mix_linear_wide(L.OUT_GLU, _ref(a), _stream()), "dv_mix_linear_wide")
@@ -263,7 +294,7 @@ def linear_residual(x: torch.Tensor, W: torch.Tensor, stream: ResidualStream, po
     code = _product_ok(x, W)
     n = x.shape[0]
     assert stream.x.shape == (n, W.shape[0])
-    if n != 1 and not _tiles(x, W):
+    if n != 1 and not _tiles(x, W, whole=W.shape[0] % 8 == 0):
         return residual(F.linear(x, W), stream, post, pre, add_start)
     h = None if pre is None else stream.new_h()
     if n == 1:

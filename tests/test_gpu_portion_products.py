@@ -75,21 +75,47 @@ def test_wide_tiles(n, K, M):
 
 
 def test_wide_products_through_the_ops():
-    """A product on each side of the rule: 497 tiles go to the library, 568 to the wide kernel, both with the same result."""
+    """A product on each side of the rule: 584 tiles of 1920 and 1922 rows, which ten and eleven tiles of 192 rows cover; the
+    first go to the library, the others to the wide kernel, both with the same result."""
     from dejavu_amd import mixer_ops as ops
 
     g = torch.Generator(device="cuda").manual_seed(1)
-    W = (torch.randn(71 * 256, 4096, generator=g, device="cuda") / 64).to(BF16)
-    x = torch.randn(1792 + 8, 4096, generator=g, device="cuda").to(BF16)
-    assert not ops._wide(x[:1792], W, True) and ops._wide(x, W, True) and not ops._wide(x[:, :2048], W[:, :2048], True)
-    assert not ops._wide(x.repeat(2, 1), W[: 36 * 256], True)  # 540 tiles of 3600 rows
-    for rows in (1792, 1792 + 8):
+    W = (torch.randn(18500, 4096, generator=g, device="cuda") / 64).to(BF16)
+    x = torch.randn(1922, 4096, generator=g, device="cuda").to(BF16)
+    assert not ops._wide(x[:1920], W) and ops._wide(x, W) and not ops._wide(x[:, :2048], W[:, :2048])
+    for rows in (1920, 1922):
         want = x[:rows].float() @ W.float().t()
         got = ops.linear(x[:rows], W).float()
         assert (got - want).norm() / want.norm() < 3e-3  # one rounding to bf16
         unit = want[:, 0::2].clamp(min=0) * want[:, 1::2]
         got = ops.relu_glu(x[:rows], W).float()
         assert (got - unit).norm() / unit.norm() < 1e-2
+
+
+@pytest.mark.parametrize("n,K,M,gated", [
+    (129, 4096, 68, False), (192, 2048, 2048, False), (193, 8192, 68, False), (256, 8200, 130, False),
+    (65, 520, 12288, True), (192, 2048, 6146, True), (193, 4096, 12288, True), (256, 4104, 66, True),
+    (65, 72, 12290, True), (130, 2048, 5122, False)])  # sizes that the launch behind the library's product refuses
+def test_streamed_products_through_the_ops(n, K, M, gated):
+    """The rows, columns and weights at which the rule ends, with each epilogue behind the tiles."""
+    from dejavu_amd import mixer_ops as ops
+
+    g = torch.Generator().manual_seed(n + M)
+    x = torch.randn(n, K, generator=g).to(BF16).cuda()
+    W = (torch.randn(M, K, generator=g) * K ** -0.5).to(BF16).cuda()
+    assert ops._tiles(x, W, gated=gated) or (n * M // 2 if gated else M) % 4
+    prod = host(x) @ host(W).T
+    if gated:
+        close(ops.relu_glu(x, W), np.maximum(prod[:, 0::2], 0) * prod[:, 1::2], OP_LIMIT[BF16], "gated unit")
+        return
+    close(ops.linear(x, W), prod, OP_LIMIT[BF16], "plain")
+    (post, f_post), (pre, f_pre) = _norm(M, 1), _norm(M, 2)
+    x0 = torch.randn(n, M, generator=g).cuda()
+    stream = ops.ResidualStream(x0.clone(), None, BF16)
+    h = ops.linear_residual(x, W, stream, post, pre)
+    want = host(x0) + f_post(prod)
+    close(stream.x, want, OP_LIMIT[BF16], "residual")
+    close(h, f_pre(want), OP_LIMIT[BF16], "next norm")
 
 
 def test_unaligned_operands():

@@ -10,13 +10,13 @@ F = torch.nn.functional
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,K,M", [(65, 64, 32), (192, 64, 32), (2048, 4096, 16128)])
+@pytest.mark.parametrize("n,K,M", [(65, 64, 32), (192, 64, 32), (2048, 4096, 22016)])
 def test_gradients_and_transforms_of_portion_products(n, K, M):
     from dejavu_amd import mixer_ops as ops
 
     g = torch.Generator(device="cuda").manual_seed(n)
     x, W = (torch.randn(s, generator=g, device="cuda").to(torch.bfloat16) for s in ((n, K), (M, K)))
-    assert ops._tiles(x, W) or ops._wide(x, W, True)
+    assert ops._tiles(x, W) or ops._wide(x, W)
     x.requires_grad_()
     ops.linear(x, W).sum().backward()
     got, x.grad = x.grad, None
@@ -26,9 +26,30 @@ def test_gradients_and_transforms_of_portion_products(n, K, M):
     bias = torch.zeros(M, dtype=torch.bfloat16, device="cuda", requires_grad=True)
     assert ops.linear(x, W, bias).requires_grad
     with torch.no_grad():
-        assert ops._tiles(x, W, bias) or ops._wide(x, W, True, bias)
+        assert ops._tiles(x, W, bias) or ops._wide(x, W, bias)
     tangent = torch.func.jvp(lambda t: ops.linear(t, W), (x,), (x,))[1]
     assert torch.equal(tangent, F.linear(x, W))
+
+
+def test_which_products_of_a_portion_are_taken_over():
+    """Sizes on both sides of the rules' lines; each was measured against the library with its weights out of the caches."""
+    from dejavu_amd.mixer_ops import _tile_rule, _wide_rule
+
+    for n, M, K in ((1603, 22016, 4096), (2048, 22016, 4096), (2000, 22016, 5120), (2000, 18560, 4096), (2000, 18944, 5120),
+                    (1918, 20480, 4096), (1862, 21760, 4096)):
+        assert _wide_rule(n, M, K), (n, M, K)                    # 1.07 to 1.33 times the library's speed
+    for n, M, K in ((1512, 22016, 4096), (1624, 21760, 4096), (1435, 24576, 4096), (1939, 19200, 4096), (1365, 28672, 4096),
+                    (2191, 17920, 4096), (1999, 16384, 4096), (1700, 22016, 8192), (12288, 4096, 4096), (8192, 4096, 4096),
+                    (6000, 22016, 4096)):
+        assert not _wide_rule(n, M, K), (n, M, K)                # 0.75 to 1.07 times
+    for n, M, K in ((65, 6144, 4096), (192, 11264, 2048), (192, 12288, 4096), (256, 8192, 4096)):
+        assert _tile_rule(n, M, K, True)
+    for n, M, K in ((65, 22016, 4096), (192, 50000, 2048), (256, 4096, 2048), (257, 4096, 8192)):
+        assert not _tile_rule(n, M, K, True)
+    for n, M, K in ((65, 2048, 2048), (96, 4096, 4096), (192, 4096, 11008), (256, 4096, 8192)):
+        assert _tile_rule(n, M, K, False)
+    for n, M, K in ((130, 4096, 2048), (96, 8192, 2048), (96, 14336, 4096), (208, 4096, 4096), (257, 4096, 8192)):
+        assert not _tile_rule(n, M, K, False)
 
 
 @pytest.fixture(scope="module")
