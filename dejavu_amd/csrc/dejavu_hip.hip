@@ -1365,12 +1365,15 @@ int dv_prefill_attention_f16(const void* qkv, int B, int T, int H, int hd, float
   const int64_t groups = ((int64_t)T + kPfQueries - 1) / kPfQueries * H;
   if (groups > 0x7fffffff) return DV_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)groups, B);
-#define DV_PF(HD)                                                                                              \
-  RingLaunch{}.operator()<prefill_attn_kernel<HD>>(                                                            \
-      grid, dim3(kPfWaves * 64), pf_lds(HD), s, reinterpret_cast<const half_t*>(qkv), T, H, scale,             \
+  // Two wavefronts from two workgroups a compute unit on; measured to 128 tokens, beyond which each has a block to take.
+  const bool two = T <= 128 && groups * B >= 2 * compute_units();
+#define DV_PF(HD, WAVES)                                                                                       \
+  RingLaunch{}.operator()<prefill_attn_kernel<HD, WAVES>>(                                                     \
+      grid, dim3(WAVES * 64), pf_lds(HD, WAVES), s, reinterpret_cast<const half_t*>(qkv), T, H, scale,         \
       reinterpret_cast<half_t*>(ctx), (int)aligned16(ctx), reinterpret_cast<half_t*>(k_cache),                 \
       reinterpret_cast<half_t*>(v_cache), pos0, S)
-  return hd == 128 ? DV_PF(128) : DV_PF(64);
+  if (hd == 128) return two ? DV_PF(128, 2) : DV_PF(128, 4);
+  return two ? DV_PF(64, 2) : DV_PF(64, 4);
 #undef DV_PF
 }
 

@@ -5,7 +5,7 @@
 //   k_cache[b, h, j / 8, pos0 + t, j % 8] = k[b, t, h, j];  v_cache[b, h, pos0 + t, j] = v[b, t, h, j]
 //
 // qkv is the output of the Wqkv product, (B, T, 3, H, hd) fp16.  A workgroup takes 32 queries of one
-// (b, h); its four wavefronts take every fourth block of 32 keys with an online softmax (fp32 scores,
+// (b, h); its four wavefronts (WAVES) take every fourth block of 32 keys with an online softmax (fp32 scores,
 // maximum and sum) and add up in LDS: 128 tokens of 40 heads are 160 workgroups with one block per
 // wavefront, where 64 queries and a wavefront for 16 of them were 80 with eight blocks in a row.
 //   S^T (32 keys x 32 queries) = K . Q^T   v_mfma_f32_32x32x16_f16, both operands straight from memory;
@@ -22,9 +22,11 @@
 // 40 heads of 128 and 128 tokens: 7.5 us (one wavefront for 16 queries and all their keys: 27); 32 heads
 // and 777 tokens 30 us (215, and 75 with the library's attention and the copies into the caches).  Short
 // prompts are bound by one block's chain of loads and exchanges, long ones by L2: each workgroup reads
-// the keys and values before its 32 queries, 160 MB at 777 tokens.
+// the keys and values before its 32 queries, 160 MB at 777 tokens.  Where short prompts make workgroups enough, two
+// wavefronts do: of four, some have no block at all, yet hold their registers and LDS (16 sequences of 16 / 33 / 128
+// tokens and 96 heads of 64: 9.4 / 17.4 / 38 us with four, 7.0 / 13.8 / 33 with two; of 128: 16 / 35 / 107 and 15 / 25 / 97).
 //
-// HD in {64, 128}.  Grid (H * ceil(T / 32), B), head fastest, 256 threads: the workgroups of a head run
+// HD in {64, 128}.  Grid (H * ceil(T / 32), B), head fastest, WAVES * 64 threads: the workgroups of a head run
 // on one die where the heads are a multiple of eight, the last queries (the most keys) first.
 #pragma once
 #include "common.hpp"
@@ -32,11 +34,10 @@
 
 namespace dv {
 
-constexpr int kPfWaves = 4;
 constexpr int kPfQueries = 32;
 constexpr int kPfKeys = 32;  // keys per step of a wavefront
 constexpr int pf_row(int hd) { return hd + 4; }  // floats of a query's sums
-constexpr size_t pf_lds(int hd) { return (size_t)kPfWaves * kPfQueries * pf_row(hd) * sizeof(float); }
+constexpr size_t pf_lds(int hd, int waves) { return (size_t)waves * kPfQueries * pf_row(hd) * sizeof(float); }
 
 // 16-byte piece p of row r of V in LDS: four rows of 32 columns are then on different banks.
 template <int HD>
@@ -44,8 +45,8 @@ __device__ __forceinline__ int pf_piece(int r, int p) {
   return p ^ ((HD == 128 ? r & 3 : (r >> 1) & 1) << 2);
 }
 
-template <int HD>
-__global__ __launch_bounds__(kPfWaves * 64, 2) void prefill_attn_kernel(
+template <int HD, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 2) void prefill_attn_kernel(
     const half_t* __restrict__ qkv, int T, int H, float scale, half_t* __restrict__ ctx, int ctx16 /* ctx on 16 bytes */,
     half_t* __restrict__ k_cache, half_t* __restrict__ v_cache, int pos0, int S) {
   typedef float acc_t __attribute__((ext_vector_type(16)));
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void prefill_attn_kernel(
   typedef __attribute__((address_space(3))) tr_t* tr_ptr_t;
   constexpr int DT = HD / 16, VT = HD / 32, P8 = HD / 8, ROW = pf_row(HD);
   extern __shared__ __attribute__((aligned(16))) float sums[];  // [wavefront][query][ROW]; V blocks before
-  __shared__ float s_m[kPfWaves][kPfQueries], s_l[kPfWaves][kPfQueries];
+  __shared__ float s_m[WAVES][kPfQueries], s_l[WAVES][kPfQueries];
   static_assert(kPfKeys * HD * sizeof(half_t) <= kPfQueries * ROW * sizeof(float), "a block of V fits into the sums");
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -93,8 +94,8 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void prefill_attn_kernel(
   if (k_cache != nullptr) {
     const int64_t bh = (int64_t)b * H + h;
 #pragma unroll
-    for (int i = 0; i < kPfQueries * P8 / 256; ++i) {
-      const int at = i * 256 + tid, j8 = at / kPfQueries, t = q0 + at % kPfQueries;
+    for (int i = 0; i < kPfQueries * P8 / (WAVES * 64); ++i) {
+      const int at = i * (WAVES * 64) + tid, j8 = at / kPfQueries, t = q0 + at % kPfQueries;
       const int vt = q0 + at / P8, vj = at % P8;
       if (t < T && pos0 + t < S)
         store8(k_cache + ((bh * P8 + j8) * S + pos0 + t) * 8, load8(Kb + (int64_t)t * tstride + j8 * 8));
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void prefill_attn_kernel(
   float m = -1e30f, l = 0.f;  // l: this half wavefront's share
   const float sc = scale * 1.44269504088896340736f;
   const int j = lane & 15, tr_row = 4 * hh + (j >> 2), tr_col = 16 * ((lane >> 4) & 1) + (j & 3) * 4;
-  for (; k0 <= last; k0 += kPfWaves * kPfKeys) {
+  for (; k0 <= last; k0 += WAVES * kPfKeys) {
     acc_t s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void prefill_attn_kernel(
       const int at = i * 64 + lane, r = at / P8;
       store8(vs + r * HD + pf_piece<HD>(r, at % P8) * 8, vr[i]);
     }
-    const int k1 = k0 + kPfWaves * kPfKeys;
+    const int k1 = k0 + WAVES * kPfKeys;
     if (k1 <= last) {
       fetch_k(k1);
       fetch_v(k1);
@@ -190,13 +191,13 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void prefill_attn_kernel(
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kPfQueries * P8 / 256; ++i) {
-    const int at = i * 256 + tid, qq = at / P8, d = at % P8 * 8;
+  for (int i = 0; i < kPfQueries * P8 / (WAVES * 64); ++i) {
+    const int at = i * (WAVES * 64) + tid, qq = at / P8, d = at % P8 * 8;
     float mm = s_m[0][qq], den = 0.f, v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 1; w < kPfWaves; ++w) mm = fmaxf(mm, s_m[w][qq]);
+    for (int w = 1; w < WAVES; ++w) mm = fmaxf(mm, s_m[w][qq]);
 #pragma unroll
-    for (int w = 0; w < kPfWaves; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       const float e = __builtin_amdgcn_exp2f(s_m[w][qq] - mm);
       const float* part = sums + ((int64_t)w * kPfQueries + qq) * ROW + d;
       den = __builtin_fmaf(s_l[w][qq], e, den);

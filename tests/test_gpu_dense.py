@@ -124,7 +124,8 @@ def test_dense_linear_three_dimensional_input():
 
 
 @pytest.mark.parametrize("B,T,H,hd", [(1, 1, 2, 64), (1, 7, 3, 64), (2, 37, 4, 128), (1, 64, 2, 128), (1, 128, 5, 128),
-                                      (1, 130, 2, 64), (3, 200, 2, 128)])
+                                      (1, 130, 2, 64), (3, 200, 2, 128),
+                                      (2, 37, 128, 64), (4, 100, 33, 64), (4, 128, 32, 128), (3, 1, 171, 128)])  # 512 workgroups: two wavefronts
 def test_prefill_attention_matches_oracle(B, T, H, hd):
     """Causal attention over the prompt against the oracle's prompt_attention, and the K / V rows in the
     packed caches bit for bit (they are copies); prompt lengths that are not multiples of 16 / 32 / 64."""
@@ -155,9 +156,9 @@ def test_prompt_runs_on_the_hip_kernels_and_matches_the_library_path(T):
     """The prompt phase of a small model through dv_dense_linear_f16 / dv_prefill_attention_f16
     (USE_HIP_PROMPT) against PyTorch's library GEMM and attention on the same weights, and against
     the oracle's model_prompt; the caches the two paths leave behind agree within fp16 rounding.
-    The 230-token prompt is past both switch-over lengths (HIP_PROMPT_MAX_ROWS,
-    HIP_PROMPT_ATTN_MAX_TOKENS): its products and attention are the library's, the cache layout and
-    everything after the prompt are the package's."""
+    The 230-token prompt is past both lengths (HIP_PROMPT_MAX_ROWS, HIP_PROMPT_ATTN_MAX_TOKENS) from which
+    on the library may be taken: its products are the library's, its attention and cache fill the kernel's
+    as long as only results are asked for."""
     import dejavu_amd.modules as M
     from dejavu_amd.gpt import GPTLMHeadModel, SparseGPTConfig
     from dejavu_amd.modules import InferenceParams
