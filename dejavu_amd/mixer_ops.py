@@ -21,20 +21,20 @@ from ._binding import results_only
 from ._lib_mixers import check, lib
 
 # Beyond 64 rows the streaming kernel where it is ahead of the library GEMM and the launch that follows it, with weights that are
-# not in the caches (24 weights, 65 to 256 rows).  us, library / kernel:
-#   the gated unit up to 192 rows: 6144 x 4096 with 65 / 128 / 192 rows 1.25 / 1.32 / 1.45 times the library's speed, 11264 x 2048
-#   1.07 / 1.01 / 1.13, 12288 x 4096 1.17 / 1.14 / 1.18; but 22016 x 4096 0.88 / 0.89 / 1.00, 50000 x 2048 1.01 / 0.96 / 0.92: there the
-#   tiles make more than a round and the library's larger ones read x less often;
-#   norm and residual, or nothing, up to 192 rows: 4096 x 4096 with 96 / 192 rows 26 / 20 and 38 / 27, 4096 x 11008 54 / 33 and 86 / 40,
-#   2048 x 2048 14.6 / 11.5 and 16 / 14; but 4096 x 2048 with 130 rows 18 / 21, 5120 x 2048 with 96 17 / 19, plain 8192 x 2048 0.9 of it;
-#   beyond 192: the gated unit of 4096 x 4096 1.02, 12288 x 4096 1.00 to 1.20, 4096 x 2048 0.8; the others of 4096 x 11008
-#   52 / 44, 4096 x 8192 39 / 38, but 4096 x 4096 27 / 29, 4096 x 5632 30 / 33, 4096 x 2048 19 / 25.
+# not in the caches (us, library / kernel, or times the library's speed; its call costs the host 5 to 15 us less):
+#   up to 192 rows weights of up to 12288 rows: the gated unit of 6144 x 4096 with 65 / 128 / 192 rows 1.25 / 1.32 / 1.45, of 11264 x 2048
+#   1.07 / 1.01 / 1.13; norm and residual of 4096 x 4096 with 96 / 192 rows 26 / 20 and 38 / 27, 4096 x 11008 54 / 33 and 86 / 40, 2048 x 2048
+#   14.6 / 11.5 and 16 / 14 (with 2048 columns also where it is behind, 4096 x 2048 with 130 rows 18 / 21: such models wait for the host).
+#   Of taller weights the tiles make more than a round, and the library's larger ones read x less often (22016 x 4096 with 65 / 128 /
+#   192 rows 0.88 / 0.89 / 1.00, plain 0.83 / 0.82 / 0.95; 50000 x 2048 0.9): it takes them, but gated units of 97 to 192 rows only: with fewer the
+#   calls are the time, with more it is not ahead inside a model (a prompt of vimulorn-4k with 65 / 100 / 128 / 200 / 256 tokens 1.60 /
+#   1.65 / 1.70 / 2.00 / 2.09 ms with the kernel, 1.77 / 1.62 / 1.64 / 2.02 / 2.13 with the library);
+#   beyond 192: 4096 x 11008 52 / 44, 4096 x 8192 39 / 38, 3072 x 4096 26 / 24, 2048 x 5632 24 / 21, gated 4096 x 4096 1.02 and 11264 x 2048
+#   1.06, 8192 x 4096 with 208 / 256 rows 0.94 / 1.29; but 2048 x 2048 with 256 rows 0.9 and 4096 x 2048 0.7.
 TILE_MAX_ROWS = 256
-TILE_MORE_ROWS = 192               # beyond these the lines are narrower
-TILE_MAX_WEIGHT_ROWS = 12288
-TILE_MIN_COLUMNS = 4096            # or TILE_SMALL_WEIGHT elements at most
-TILE_SMALL_WEIGHT = 1 << 22
-TILE_MORE_COLUMNS = 8192
+TILE_MAX_WEIGHT_ROWS, TILE_TALL_ROWS = 12288, 96
+TILE_ALL_ROWS = 192                # up to here whatever the weight's size
+TILE_WEIGHT, TILE_COLUMNS = 1 << 23, 4096   # elements from which the rows may be more; twice as many where the columns are fewer
 
 _DTYPES = {torch.bfloat16: L.BF16, torch.float32: L.F32}
 _ref = ctypes.byref
@@ -134,11 +134,11 @@ def _wide_rule(n: int, M: int, K: int) -> bool:
 
 
 def _tile_rule(n: int, M: int, K: int, gated: bool) -> bool:
-    if n > TILE_MAX_ROWS or M > TILE_MAX_WEIGHT_ROWS:
+    if n > TILE_MAX_ROWS:
         return False
-    if n > TILE_MORE_ROWS:
-        return K >= (TILE_MIN_COLUMNS if gated else TILE_MORE_COLUMNS)
-    return gated or K >= TILE_MIN_COLUMNS or M * K <= TILE_SMALL_WEIGHT
+    if M > TILE_MAX_WEIGHT_ROWS:
+        return gated and not TILE_TALL_ROWS < n <= TILE_ALL_ROWS
+    return n <= TILE_ALL_ROWS or M * K >= (TILE_WEIGHT if K >= TILE_COLUMNS else 2 * TILE_WEIGHT)
 
 
 def _aligned(x: torch.Tensor, W: torch.Tensor) -> bool:

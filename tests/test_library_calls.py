@@ -42,14 +42,11 @@ def test_which_products_of_a_portion_are_taken_over():
                     (2191, 17920, 4096), (1999, 16384, 4096), (1700, 22016, 8192), (12288, 4096, 4096), (8192, 4096, 4096),
                     (6000, 22016, 4096)):
         assert not _wide_rule(n, M, K), (n, M, K)                # 0.75 to 1.07 times
-    for n, M, K in ((65, 6144, 4096), (192, 11264, 2048), (192, 12288, 4096), (256, 8192, 4096)):
-        assert _tile_rule(n, M, K, True)
-    for n, M, K in ((65, 22016, 4096), (192, 50000, 2048), (256, 4096, 2048), (257, 4096, 8192)):
-        assert not _tile_rule(n, M, K, True)
-    for n, M, K in ((65, 2048, 2048), (96, 4096, 4096), (192, 4096, 11008), (256, 4096, 8192)):
-        assert _tile_rule(n, M, K, False)
-    for n, M, K in ((130, 4096, 2048), (96, 8192, 2048), (96, 14336, 4096), (208, 4096, 4096), (257, 4096, 8192)):
-        assert not _tile_rule(n, M, K, False)
+    for n, M, K in ((65, 2048, 2048), (192, 4096, 11008), (192, 12288, 4096), (256, 11264, 2048), (256, 2048, 4096), (256, 4096, 8192)):
+        assert _tile_rule(n, M, K, True) and _tile_rule(n, M, K, False)
+    for n, M, K in ((97, 22016, 4096), (192, 50000, 2048), (193, 4096, 2048), (256, 2048, 2048), (257, 4096, 8192)):
+        assert not _tile_rule(n, M, K, True) and not _tile_rule(n, M, K, False)
+    assert _tile_rule(96, 22016, 4096, True) and _tile_rule(193, 22016, 4096, True) and not _tile_rule(65, 22016, 4096, False)
 
 
 @pytest.fixture(scope="module")
