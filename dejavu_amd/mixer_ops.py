@@ -26,13 +26,13 @@ from ._lib_mixers import check, lib
 #   1.07 / 1.01 / 1.13; norm and residual of 4096 x 4096 with 96 / 192 rows 26 / 20 and 38 / 27, 4096 x 11008 54 / 33 and 86 / 40, 2048 x 2048
 #   14.6 / 11.5 and 16 / 14 (with 2048 columns also where it is behind, 4096 x 2048 with 130 rows 18 / 21: such models wait for the host).
 #   Of taller weights the tiles make more than a round, and the library's larger ones read x less often (22016 x 4096 with 65 / 128 /
-#   192 rows 0.88 / 0.89 / 1.00, plain 0.83 / 0.82 / 0.95; 50000 x 2048 0.9): it takes them, but gated units of 97 to 192 rows only: with fewer the
-#   calls are the time, with more it is not ahead inside a model (a prompt of vimulorn-4k with 65 / 100 / 128 / 200 / 256 tokens 1.60 /
-#   1.65 / 1.70 / 2.00 / 2.09 ms with the kernel, 1.77 / 1.62 / 1.64 / 2.02 / 2.13 with the library);
+#   192 rows 0.88 / 0.89 / 1.00, plain 0.83 / 0.82 / 0.95; 50000 x 2048 0.9): it takes them, but gated units of 129 to 192 rows only: with fewer the
+#   calls are the time, with more it is not ahead inside a model (a prompt of vimulorn-4k by itself with 65 / 100 / 128 / 160 tokens 1.71 /
+#   1.77 / 1.83 / 2.04 ms with the kernel, 1.86 / 1.89 / 1.87 / 1.98 with the library; among others 200 / 256 tokens 2.00 / 2.09 and 2.02 / 2.13);
 #   beyond 192: 4096 x 11008 52 / 44, 4096 x 8192 39 / 38, 3072 x 4096 26 / 24, 2048 x 5632 24 / 21, gated 4096 x 4096 1.02 and 11264 x 2048
 #   1.06, 8192 x 4096 with 208 / 256 rows 0.94 / 1.29; but 2048 x 2048 with 256 rows 0.9 and 4096 x 2048 0.7.
 TILE_MAX_ROWS = 256
-TILE_MAX_WEIGHT_ROWS, TILE_TALL_ROWS = 12288, 96
+TILE_MAX_WEIGHT_ROWS, TILE_TALL_ROWS = 12288, 128
 TILE_ALL_ROWS = 192                # up to here whatever the weight's size
 TILE_WEIGHT, TILE_COLUMNS = 1 << 23, 4096   # elements from which the rows may be more; twice as many where the columns are fewer
 

@@ -94,9 +94,9 @@ def test_wide_products_through_the_ops():
 
 @pytest.mark.parametrize("n,K,M,gated", [
     (129, 4096, 68, False), (192, 2048, 2048, False), (193, 4096, 2048, False), (256, 8200, 1026, False), (241, 4096, 4104, False),
-    (200, 2048, 8192, False), (65, 520, 12288, True), (96, 264, 12296, True), (193, 4096, 12288, True), (256, 4104, 2050, True),
+    (200, 2048, 8192, False), (65, 520, 12288, True), (128, 264, 12296, True), (193, 4096, 12288, True), (256, 4104, 2050, True),
     (193, 2048, 8192, True),
-    (97, 72, 12290, True), (210, 2048, 5122, False)])  # sizes that the launch behind the library's product refuses
+    (131, 72, 12290, True), (210, 2048, 5122, False)])  # sizes that the launch behind the library's product refuses
 def test_streamed_products_through_the_ops(n, K, M, gated):
     """The rows, columns and weights at which the rule ends, with each epilogue behind the tiles."""
     from dejavu_amd import mixer_ops as ops

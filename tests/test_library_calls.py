@@ -44,9 +44,9 @@ def test_which_products_of_a_portion_are_taken_over():
         assert not _wide_rule(n, M, K), (n, M, K)                # 0.75 to 1.07 times
     for n, M, K in ((65, 2048, 2048), (192, 4096, 11008), (192, 12288, 4096), (256, 11264, 2048), (256, 2048, 4096), (256, 4096, 8192)):
         assert _tile_rule(n, M, K, True) and _tile_rule(n, M, K, False)
-    for n, M, K in ((97, 22016, 4096), (192, 50000, 2048), (193, 4096, 2048), (256, 2048, 2048), (257, 4096, 8192)):
+    for n, M, K in ((129, 22016, 4096), (192, 50000, 2048), (193, 4096, 2048), (256, 2048, 2048), (257, 4096, 8192)):
         assert not _tile_rule(n, M, K, True) and not _tile_rule(n, M, K, False)
-    assert _tile_rule(96, 22016, 4096, True) and _tile_rule(193, 22016, 4096, True) and not _tile_rule(65, 22016, 4096, False)
+    assert _tile_rule(128, 22016, 4096, True) and _tile_rule(193, 22016, 4096, True) and not _tile_rule(65, 22016, 4096, False)
 
 
 @pytest.fixture(scope="module")
