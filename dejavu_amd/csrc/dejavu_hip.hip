@@ -510,7 +510,8 @@ size_t tiled_workspace_bytes(int B, int N, int M, bool qkv = false) {
   return p.nsplit > 1 ? (size_t)p.nsplit * B * M * sizeof(float) : 0;
 }
 
-// Many rows of X: the product is bound by the matrix cores and by what
+// Many rows of X (callers of dv_dense_linear_f16 itself: the modules' products have 192 rows at most, up to 512 where the
+// weight's rows are long): the product is bound by the matrix cores and by what
 // the L2 delivers, and gemm_big_mfma_kernel (weights straight into MFMA operands, 64 * WT weight rows
 // per workgroup) is the faster kernel -- measured at 12288 x 12288 against gemm_tiled_mfma_kernel:
 // 512 rows 225 against 278 us, 2048 rows 793 against 797 us.  Same bits.

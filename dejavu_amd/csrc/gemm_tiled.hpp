@@ -1,6 +1,8 @@
 // Y[b, m] = act( sum_n X[b, n] * W[row(m), n] + bias[row(m)] ) for a block of X rows that is
-// SHARED through LDS by the whole workgroup, on the matrix cores: batched fc1 (17..64 rows),
-// batched predictor products and the dense products of the prompt phase (128 rows per block).
+// SHARED through LDS by the whole workgroup, on the matrix cores: batched fc1 (17..64 rows) and QKV, batched
+// predictor products, and dense products where gemm_ring.hpp and gemm_big.hpp are not the faster ones: up to 64 rows of
+// large weights, 65..128 rows of more than 32768 weight rows, more than 512 rows whose columns gemm_big.hpp's chunks do not
+// divide (128 rows per block).
 //
 // gather_rows_mfma_kernel gives every workgroup 16 weight rows and lets each wavefront fetch its
 // own X operands, so X travels from L2 once per 16-row tile: B/16 times the weight bytes.  Here a

@@ -12,8 +12,9 @@
 // of 128) and 1.67e-7 (after another 500) beside 1.32e-7 and 1.88e-7.  The empty asm statements keep the compiler from
 // running all short sums side by side, which the registers don't hold (45 us instead of 37).
 //
-// 500 tokens, 16 heads of 128: 37 us; the row kernel, which reads a key for one query at a time, 180.  Bound by the matrix
-// instructions (64 cycles each) of the last queries' tiles and the additions between them.
+// 500 tokens, 16 heads of 128: 37 us; the row kernel, which reads a key for one query at a time, 180.  Bound by the
+// chain of the last queries' tiles: 33 of its 80 thousand cycles are matrix instructions (64 each), the rest loads and the additions
+// between them.
 #pragma once
 #include "attn_rows.hpp"
 
