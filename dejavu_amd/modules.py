@@ -411,7 +411,7 @@ class _MHABase(nn.Module):
                     b0 = inference_params.batch_size_offset
                     kc, vc = k_cache[b0:b0 + B], v_cache[b0:b0 + B]
                 rows = qkv.contiguous()
-                if s <= HIP_PROMPT_ATTN_MAX_TOKENS or _kernel_takes(rows, kc, vc):
+                if s <= HIP_PROMPT_ATTN_MAX_TOKENS or (_kernel_takes(rows, kc, vc) and (kc is None or kc.shape[3] == vc.shape[2])):
                     return ops.prefill_attention(rows, kc, vc, 0, scale)
             if inference_params is not None:
                 assert self.layer_idx is not None, "Generation requires layer_idx in the constructor"

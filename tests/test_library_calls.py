@@ -171,7 +171,7 @@ def test_traces_of_what_kernels_take_over(fc2):
 @pytest.mark.gpu
 @torch.no_grad()
 def test_operands_of_a_long_prompts_attention_that_only_the_library_takes():
-    """Caches of a caller's own, of another type, stride or place, are filled as ever; so are those that the kernel fills."""
+    """Caches of a caller's own, of another type, stride, place or length, are filled as ever; so are those that the kernel fills."""
     from dejavu_amd import modules, ops
     from dejavu_amd.modules import HIP_PROMPT_ATTN_MAX_TOKENS, InferenceParams, ParallelMHADejavu
 
@@ -187,7 +187,8 @@ def test_operands_of_a_long_prompts_attention_that_only_the_library_takes():
 
     made = {"plain": [plain(s) for s in shapes], "fp32": [plain(s, torch.float32) for s in shapes],
             "moved": [plain(math.prod(s) + 1)[1:].view(s) for s in shapes],
-            "strided": [plain(s[:-1] + (s[-1] + 8,))[..., :s[-1]] for s in shapes]}
+            "strided": [plain(s[:-1] + (s[-1] + 8,))[..., :s[-1]] for s in shapes],
+            "longer": [plain((1, H, hd // 8, S + 8, 8)), plain(shapes[1])]}
     for name, (k_cache, v_cache) in made.items():
         for x in (qkv, odd):
             k_cache.zero_(), v_cache.zero_()
@@ -197,7 +198,7 @@ def test_operands_of_a_long_prompts_attention_that_only_the_library_takes():
             k = k_cache[:, :, :, :T].permute(0, 3, 1, 2, 4).reshape(1, T, H, hd)
             assert torch.equal(k.half(), qkv[:, :, 1]) and torch.equal(v_cache[:, :, :T].transpose(1, 2).half(), qkv[:, :, 2])
             assert not k_cache[:, :, :, T:].any() and not v_cache[:, :, T:].any()
-        assert modules._kernel_takes(qkv, k_cache, v_cache) == (name == "plain")
+        assert modules._kernel_takes(qkv, k_cache, v_cache) == (name in ("plain", "longer"))
     assert not modules._kernel_takes(odd)
     torch.testing.assert_close(ops.prefill_attention(qkv), want, rtol=2e-3, atol=2e-3)
 
