@@ -8,8 +8,8 @@
 // sums up; adding them up in the first one, by the workgroup that ends last, costs more (each hand-over between compute
 // dies 5 us, fences 40 us).
 //
-// 47 rows by 4096 x 4096 / 4096 x 11008 / 22016 x 4096: 12.5 / 24.5 / 41 us (loads in operand layout, 24 at a time: 24 / 47 /
-// 74); 16 rows 11 / 22 / 39 us (13 / 43 / 51).  Bound by the stream: 41 us are 4.4 TB/s beside a plain read's 6.
+// 47 rows by 4096 x 4096 / 4096 x 11008 / 22016 x 4096: 11.1 / 22 / 33.5 us (loads in operand layout, 24 at a time: 24 / 47 /
+// 74); 16 rows 10.8 / 20 / 31.8 us (13 / 43 / 51).  Bound by the stream: 33.5 us are 5.4 TB/s beside a plain read's 6.
 #pragma once
 #include "common.hpp"
 
@@ -54,10 +54,14 @@ struct RingPlan {
   size_t workspace_bytes() const { return splits > 1 ? (size_t)splits * rows * cols * mb * nb * sizeof(float) : 0; }
 };
 
-// Up to 64 rows: tiles are as narrow as the rows allow; the taller one of 64 columns where it makes one round of
-// workgroups of what would be one and a half (22016 x 4096: 41 against 47 us with 47 rows, but 27.5 against 24.5 us at
-// 4096 x 11008).  K is split until there are about as many workgroups as compute units (4096 x 11008 with 47 rows: 1, 2, 4,
-// 8 splits take 52, 32, 24.5, 27 us); the narrowest tiles' workgroups are small, so they go on to two per unit.
+// Up to 64 rows: tiles are as narrow as the rows allow and of 64 weight rows for small weights.  Beyond, taller ones fetch X less
+// often and split K into a round of workgroups with less left over (us, 64 weight rows a tile against 128, 47 rows: 6144 x 4096 17.4 /
+// 14.3, 8512 x 4096 25 / 18.7, 12288 x 4096 25 / 22.2, but 4096 x 4096 11.1 / 12.1 and 6400 x 2048 12.0 / 12.6; 30 rows: 8512 x 4096 21 / 17.5,
+// 22016 x 4096 39 / 31.8, 11264 x 2048 15.6 / 12.7); of 33 to 64 rows with more than a round of 64, 96 (22016 x 4096: 33.5 us, 128
+// weight rows 34.2, 64 51), but 128 where these still make one round (32768 x 4096: 57 / 43.7).
+// K is split until there are about as many workgroups as compute units (4096 x 11008 with 47 rows: 1, 2, 4, 8 splits of 64
+// weight rows take 52, 32, 24.5, 27 us; 8512 x 4096 3 and 4 splits of 128, 201 and 268 workgroups, 18.7 and 26); the narrowest tiles'
+// workgroups are small, so they go on to two per unit.
 // More rows: 128 rows of W, so that X is fetched less often (5120 x 20480 with 96 rows: 53 us, 60 with 64 rows of W),
 // where that leaves 32 tiles and K is long enough to split (but 64 where these make one round and K is short: 16384 x 4096 with
 // 72 / 128 rows 41.5 / 45 us, in two splits 47.5 / 48); 192 where they fill the chip better (20480 x 5120 with 96 rows:
@@ -74,13 +78,16 @@ inline RingPlan plan_ring(int n, int M, int K, int units) {
     p.rows = (M + mb - 1) / mb;
     p.cols = (n + p.nb - 1) / p.nb;
     const int64_t tiles = (int64_t)p.rows * p.cols;
-    int64_t s = p.nb == 16 ? (tiles >= units ? 1 : tiles >= units / 2 ? 4 : 8) : (p.nb <= 64 ? units * 9 / 8 : units) / tiles;
+    int64_t s = p.nb == 16 ? (tiles >= units ? 1 : tiles >= units / 2 ? 4 : 8) : (p.nb <= 64 && mb == 64 ? units * 9 / 8 : units) / tiles;
     if (s > K / 256) s = K / 256;
     p.splits = (int)(s < 1 ? 1 : s > 8 ? 8 : s);
     return (int64_t)p.splits * tiles;
   };
   if (p.nb <= 64) {
-    lay(p.nb == 16 ? 32 : p.nb == 64 && M >= units * 64 ? 96 : 64);
+    const bool taller = M >= units * 24 && K >= (p.nb == 32 ? 2048 : 4096);
+    if (p.nb == 16) lay(32);
+    else if (p.nb == 64 && M >= units * 64) lay((M + 95) / 96 > units && (M + 127) / 128 <= units ? 128 : 96);
+    else lay(taller && (p.nb == 32 || M <= units * 60) ? 128 : 64);  // (33 to 64 rows: not where 64 make a round)
   } else if (M < 32 * 128 || K < 2048 || (p.nb == 128 && K <= 4096 && M > units * 56 && M <= units * 64)) {
     lay(64);
   } else {
@@ -113,7 +120,20 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T>
   const int wm = wave % WM, wn = wave / WM, l16 = lane & 15, g = lane >> 4;
   const int m0 = blockIdx.x * MB, n0 = blockIdx.y * NB;
   const int nch = (a.K + KC - 1) / KC;
-  const int c0 = nch * blockIdx.z / gridDim.z, c1 = nch * (blockIdx.z + 1) / gridDim.z;
+  const int c0 = nch * blockIdx.z / gridDim.z, len = nch * (blockIdx.z + 1) / gridDim.z - c0;
+  // Up to 128 rows of X and with other than 64 weight rows a tile the columns are taken in parts, and workgroups begin with
+  // different ones and go round: all of them at the same column, of rows that are a power of two apart, wait for the same few
+  // channels of the memory.  The parts' sums are added in the columns' order (two: in any) wherever the workgroup began, so a
+  // row's result does not depend on its place.  (A different chunk for each instead: the same time, other bits.)
+  // us without and with: 47 rows by 22016 x 4096 37.7, 32.2; 22016 x 6144 60.0, 47.1; 16 rows by 22016 x 4096 37.3, 31.8; 100 rows by
+  // 16384 x 4096 40.2, 35.7, 12288 x 4096 31.8, 29.0; 128 rows by 15360 x 5120 46.5, 44.1, four parts 44.3; 5120 x 20480 55.1, 55.7, four
+  // parts 65.  But tiles of 64 weight rows (12288 x 4096, 47 rows) 25.2, 30.1, and more rows of X the same time either way.
+  constexpr int PARTS = NB > 128 || MB == 64 ? 1 : NB == 128 ? 2 : 4, CHAINS = 4 / PARTS;  // sums of a part
+  const int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);  // (these go round the eight dies)
+  const int begin = PARTS == 4 ? id / 8 % 4 : PARTS == 2 ? id / 16 % 2 : 0;
+  const int part_len = (len + PARTS - 1) / PARTS, chain_len = ((PARTS == 1 ? nch : part_len) + CHAINS - 1) / CHAINS;
+  const int first = begin * part_len < len ? begin * part_len : 0;
+  auto chunk = [&](int i) { return c0 + (i + first < len ? i + first : i + first - len); };
 
   // A row's pieces lie in LDS at places exchanged by the row (place = piece ^ row), so that 16 rows' pieces are read
   // from different banks; the lanes fetch them in that order.
@@ -126,7 +146,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T>
     src[i] = row < MB ? a.W + rows(min(m0 + row, a.M - 1)) * a.ldw : a.X + (int64_t)min(n0 + row - MB, a.n - 1) * a.ldx;
   }
   const int pieces = a.K / 8;
-  auto load = [&](int c, int slot) {
+  auto load = [&](int at, int slot) {
+    const int c = chunk(at);
     // past the last piece: that one again (set to zero when it is used); past the last chunk: into a slot that is not read
 #pragma unroll
     for (int i = 0; i < LI; ++i) {
@@ -137,41 +158,44 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T>
     }
   };
 #pragma unroll
-  for (int d = 0; d < ST - 1; ++d) load(c0 + d, d);
+  for (int d = 0; d < ST - 1; ++d) load(d, d);
 
   // The instruction adds its products one after the other, so no sum has more than a quarter of K: one over all of 4096
   // columns is 3.95e-7 from its value in 64 bits, four are 1.9e-7.  (A sum for each step of a chunk instead, side by side:
   // 0.3 us more for the smallest products, whose time is that of fetching the instructions.)
-  const int quarter = (nch + 3) / 4;
-  float4_t acc[RT][NT], total[RT][NT];
+  float4_t acc[RT][NT], sums[PARTS][RT][NT];
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
+  for (auto& sum : sums)
 #pragma unroll
-    for (int j = 0; j < NT; ++j) total[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) sum[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
   int slot = 0;
-  for (int c = c0, stop; c < c1;) {
-    stop = min(c + quarter, c1);
+  for (int at = 0, step = 0; PARTS == 1 ? at < len : step < 4; ++step) {
+    const int in_part = min(part_len, len - (begin + step / CHAINS) % PARTS * part_len) - step % CHAINS * chain_len;
+    const int stop = PARTS == 1 ? min(at + chain_len, len) : at + max(min(chain_len, in_part), 0);
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-    for (; c < stop; ++c) {
+    for (; at < stop; ++at) {
+      const int c = chunk(at);
       // Everybody's part of the slot is there, and nobody still reads the slot before it, which is loaded next: the reads have
       // to have returned, which the barrier itself does not wait for and the instructions that use them need not come before.
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(LI * (ST - 2)) : "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      load(c + ST - 1, slot == 0 ? ST - 1 : slot - 1);
+      load(at + ST - 1, slot == 0 ? ST - 1 : slot - 1);
       const unsigned char* wb = slots + slot * SLOT + (wm * RT * 16 + l16) * KC * 2;
       const unsigned char* xb = slots + slot * SLOT + (MB + wn * NT * 16 + l16) * KC * 2;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        const int at = ((ks * 4 + g) ^ (l16 & SWAP)) * 16;
+        const int place = ((ks * 4 + g) ^ (l16 & SWAP)) * 16;
         ring_word_t w[RT], x[NT];
 #pragma unroll
-        for (int i = 0; i < RT; ++i) w[i] = *reinterpret_cast<const ring_word_t*>(wb + i * 16 * KC * 2 + at);
+        for (int i = 0; i < RT; ++i) w[i] = *reinterpret_cast<const ring_word_t*>(wb + i * 16 * KC * 2 + place);
 #pragma unroll
-        for (int j = 0; j < NT; ++j) x[j] = *reinterpret_cast<const ring_word_t*>(xb + j * 16 * KC * 2 + at);
+        for (int j = 0; j < NT; ++j) x[j] = *reinterpret_cast<const ring_word_t*>(xb + j * 16 * KC * 2 + place);
         if ((c + 1) * CH > pieces && c * CH + ks * 4 + g >= pieces) {  // past the end of the rows
 #pragma unroll
           for (int i = 0; i < RT; ++i) w[i] = ring_word_t{0, 0, 0, 0};
@@ -184,25 +208,55 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T>
           for (int j = 0; j < NT; ++j) acc[i][j] = ring_mfma<T>(w[i], x[j], acc[i][j]);
       }
       slot = slot == ST - 1 ? 0 : slot + 1;
+      if constexpr (RT * NT == 1) {
+        // The instruction's sums are there eight states after it.  The compiler has been seen to read the first of them two
+        // after it behind this loop, and a copy of this kernel in which that was one got the sum without its last products.
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_nop 7\n\ts_nop 1" ::: "memory");
+      }
     }
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
-      for (int j = 0; j < NT; ++j) total[i][j] += acc[i][j];
+      for (int j = 0; j < NT; ++j) {
+        if (PARTS > 1 && step % CHAINS == 0) {
+#pragma unroll
+          for (int k = 1; k < PARTS; ++k) sums[k - 1][i][j] = sums[k][i][j];
+          sums[PARTS - 1][i][j] = acc[i][j];
+        } else {
+          sums[PARTS - 1][i][j] += acc[i][j];
+        }
+      }
   }
+  if constexpr (PARTS == 4) {
+    for (int r = begin; r > 0; --r)  // the columns' order
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const float4_t last = sums[3][i][j];
+          sums[3][i][j] = sums[2][i][j], sums[2][i][j] = sums[1][i][j], sums[1][i][j] = sums[0][i][j], sums[0][i][j] = last;
+        }
+  }
+#pragma unroll
+  for (int k = 1; k < PARTS; ++k)
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) sums[0][i][j] += sums[k][i][j];
   if (gridDim.z > 1) {
     float4_t* p = part + (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (MB * NB / 4) + threadIdx.x;
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
-      for (int j = 0; j < NT; ++j) p[(i * NT + j) * THREADS] = total[i][j];
+      for (int j = 0; j < NT; ++j) p[(i * NT + j) * THREADS] = sums[0][i][j];
   } else {
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         const int m = m0 + (wm * RT + i) * 16 + g * 4, n = n0 + (wn * NT + j) * 16 + l16;
-        if (m < a.M && n < a.n) out(m, n, total[i][j]);
+        if (m < a.M && n < a.n) out(m, n, sums[0][i][j]);
       }
   }
   wait_loads<0>();  // no load into LDS outlives the workgroup
@@ -244,10 +298,11 @@ int gemm_ring(const RingPlan& p, const RingOperands<T>& a, const Rows& rows, con
 #define DV_RING(MB, NB, KC, ST, WM, WN, NT_W) gemm_ring_tiles<T, MB, NB, KC, ST, WM, WN, NT_W>(p, a, rows, out, workspace, s, launch)
   switch (p.nb) {
     case 16: return DV_RING(32, 16, 128, 4, 2, 1, true);
-    case 32: return DV_RING(64, 32, 64, 4, 4, 1, false);
-    case 64: return p.mb == 96 ? DV_RING(96, 64, 64, 4, 2, 2, false) : DV_RING(64, 64, 64, 4, 2, 2, false);
-    case 128: return p.mb == 64 ? DV_RING(64, 128, 64, 3, 2, 4, false)
-                     : p.mb == 128 ? DV_RING(128, 128, 64, 4, 2, 4, false) : DV_RING(192, 128, 64, 3, 2, 4, false);
+    case 32: return p.mb == 128 ? DV_RING(128, 32, 64, 4, 4, 1, true) : DV_RING(64, 32, 64, 4, 4, 1, true);
+    case 64: return p.mb == 128 ? DV_RING(128, 64, 64, 4, 4, 2, true)
+                    : p.mb == 96 ? DV_RING(96, 64, 64, 4, 2, 2, true) : DV_RING(64, 64, 64, 4, 2, 2, true);
+    case 128: return p.mb == 64 ? DV_RING(64, 128, 64, 3, 2, 4, true)
+                     : p.mb == 128 ? DV_RING(128, 128, 64, 4, 2, 4, true) : DV_RING(192, 128, 64, 3, 2, 4, true);
     case 192: return p.mb == 64 ? DV_RING(64, 192, 64, 4, 2, 4, false)
                      : p.mb == 128 ? DV_RING(128, 192, 64, 3, 2, 4, false) : DV_RING(192, 192, 64, 3, 2, 4, false);
     default: return p.mb == 64 ? DV_RING(64, 256, 64, 3, 2, 4, false) : DV_RING(128, 256, 64, 3, 2, 4, false);

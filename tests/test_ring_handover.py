@@ -46,3 +46,22 @@ def test_reads_have_returned_before_a_slot_is_loaded_again(tmp_path):
             before.append(line)
         waits = " ".join(line for line in before if line.startswith("s_waitcnt"))
         assert re.search(r"lgkmcnt\(0\)", waits) and re.search(r"vmcnt\(\d+\)", waits), before
+
+
+def test_sums_of_the_narrowest_tile_are_waited_for(tmp_path):
+    """One matrix instruction a step leaves nothing between the last of them and the reads of its sums: the wait stands in the
+    kernel, in front of the branch that leaves the loop."""
+    try:
+        hipcc = hipcc_path()
+    except RuntimeError as e:
+        pytest.skip(str(e))
+    src, out = tmp_path / "ring.hip", tmp_path / "ring.s"
+    src.write_text("\n".join(SOURCE.splitlines()[:-2]))
+    flags = [f for f in HIPCC_FLAGS if f not in ("-shared", "-fPIC")]
+    subprocess.run([hipcc, *flags, "-w", "-S", "--cuda-device-only", "-I", CSRC, "-I", os.path.join(CSRC, "..", "..", "include"),
+                    str(src), "-o", str(out)], check=True)
+    lines = [line.split(";")[0].strip() for line in out.read_text().splitlines()]
+    lines = lines[next(i for i, line in enumerate(lines) if re.match(r"_ZN2dv16gemm_ring.*Li32ELi16E.*:$", line)):]
+    last = max(i for i, line in enumerate(lines) if line.startswith("v_mfma"))
+    behind = lines[last + 1:next(i for i in range(last + 1, len(lines)) if lines[i].startswith(("s_cbranch", "s_branch")))]
+    assert "s_nop 7" in behind, behind
