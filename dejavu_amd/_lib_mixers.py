@@ -91,6 +91,7 @@ SIGNATURES = {
     "dv_mix_attn_tiles": (_i, [_P(AttnArgs), _i, _p]),
     "dv_mix_attn_tiles_f32": (_i, [_P(AttnArgs), _i, _p]),
     "dv_mix_latent_absorb": (_i, [_i, _p, _p, _i, _i, _i, _p, _p]),
+    "dv_mix_latent_one": (_i, [_P(AttnArgs), _i, _p, _i, _p, _i, _p, _p]),
     "dv_mix_latent_attn": (_i, [_i, _P(AttnArgs), _p, _i, _p, _p]),
     "dv_mix_delta_gates": (_i, [_i, _p, _l, _p, _l, _p, _p, _i, _i, _i, _p, _p, _p]),
     "dv_mix_delta_scan": (_i, [_P(DeltaArgs), _p]),

@@ -8,6 +8,7 @@
 #include "device.hpp"
 #include "mix/attn_f32.hpp"
 #include "mix/attn_latent.hpp"
+#include "mix/attn_one.hpp"
 #include "mix/attn_rows.hpp"
 #include "mix/attn_tiles.hpp"
 #include "mix/delta_rule.hpp"
@@ -153,6 +154,31 @@ int attn_rows_any(const AttnArgs& a, hipStream_t s) {
   if (rep >= 3) return attn_rows_rh<T, TQ, 4>(a, s);
   if (rep == 2) return attn_rows_rh<T, TQ, 2>(a, s);
   return attn_rows_rh<T, TQ, 1>(a, s);
+}
+
+// One bf16 row whose keys (a ring of them, at most) one launch takes: attn_one.hpp.
+bool attn_one_takes(const AttnArgs& a) {
+  return a.n == 1 && a.splits == 1 && a.dim_s <= 128 && a.vdim_s <= 128 && al16(a.fresh_k) && al16(a.fresh_v) && al16(a.other_v) &&
+         al16(a.q_w) && al16(a.k_w);
+}
+int attn_one(const AttnArgs& a, hipStream_t s) {
+  int most = a.ring > 0 ? a.ring : 512;
+  if (a.window > 0 && a.window < most) most = a.window;
+  if (a.chunk > 0 && a.chunk < most) most = a.chunk;
+  const dim3 grid(a.H), threads(kOneThreads);
+  if (most <= 64) hipLaunchKernelGGL((attn_one_kernel<1>), grid, threads, 0, s, a);
+  else if (most <= 128) hipLaunchKernelGGL((attn_one_kernel<2>), grid, threads, 0, s, a);
+  else hipLaunchKernelGGL((attn_one_kernel<4>), grid, threads, 0, s, a);
+  return launched();
+}
+template <int LPK>
+int latent_one(const AttnArgs& a, int keys, const bf16_t* Wk, int dim_s, const bf16_t* Wv, int vrows, bf16_t* out, hipStream_t s) {
+  constexpr int G = kOneThreads / LPK;
+  const dim3 grid(a.H), threads(kOneThreads);
+  if (keys <= 4 * G) hipLaunchKernelGGL((latent_one_kernel<LPK, 4>), grid, threads, 0, s, a, Wk, dim_s, Wv, vrows, out);
+  else if (LPK == 64 || keys <= 8 * G) hipLaunchKernelGGL((latent_one_kernel<LPK, 8>), grid, threads, 0, s, a, Wk, dim_s, Wv, vrows, out);
+  else hipLaunchKernelGGL((latent_one_kernel<LPK, LPK == 64 ? 8 : 12>), grid, threads, 0, s, a, Wk, dim_s, Wv, vrows, out);
+  return launched();
 }
 
 // ---- delta rule --------------------------------------------------------------
@@ -543,6 +569,7 @@ int dv_mix_attn_rows(int dtype, int q_f32, const dvAttnArgs* a, void* stream) {
   if (rc != DV_OK) return rc;
   if (!a->out) return DV_ERR_INVALID_ARG;
   if (dtype == DV_F32) rc = attn_rows_any<float, float>(*a, st(stream));
+  else if (q_f32 && attn_one_takes(*a)) rc = attn_one(*a, st(stream));
   else if (q_f32) rc = attn_rows_any<bf16_t, float>(*a, st(stream));
   else rc = attn_rows_any<bf16_t, bf16_t>(*a, st(stream));
   if (rc != DV_OK || a->splits == 1) return rc;
@@ -625,6 +652,20 @@ int dv_mix_latent_attn(int dtype, const dvAttnArgs* a, const void* W, int vrows,
   else
     hipLaunchKernelGGL((latent_out_kernel<float>), grid, dim3(256), lds, st(stream), *a, (const float*)W, vrows, (float*)out);
   return launched();
+}
+
+int dv_mix_latent_one(const dvAttnArgs* a, int keys, const void* Wk, int dim_s, const void* Wv, int vrows, void* out, void* stream) {
+  if (!Wk || !Wv || !out || dim_s < 1 || vrows < 1 || keys < 1 || !a || a->n != 1 || a->G != 1 || a->splits != 1 || a->k != a->v ||
+      a->dim_s != a->vdim_s || a->window > 0 || a->chunk > 0 || a->ring > 0 || a->base != 0 || a->fresh_k || a->norm_dim > 0 || a->rel ||
+      (!a->pos_dev && (a->pos_host < 0 || a->pos_host >= keys)))
+    return DV_ERR_INVALID_ARG;
+  const int rc = attn_args_ok(a);
+  if (rc != DV_OK) return rc;
+  if (!al16(Wk) || !al16(Wv)) return DV_ERR_ALIGNMENT;
+  if (a->dim_s > 512) return DV_ERR_UNSUPPORTED;
+  const bf16_t *k = (const bf16_t*)Wk, *v = (const bf16_t*)Wv;
+  if (a->dim_s <= 256) return latent_one<32>(*a, keys, k, dim_s, v, vrows, (bf16_t*)out, st(stream));
+  return latent_one<64>(*a, keys, k, dim_s, v, vrows, (bf16_t*)out, st(stream));
 }
 
 int dv_mix_delta_gates(int dtype, const void* z, int64_t ldz, const void* b, int64_t ldb, const float* A_log,

@@ -521,6 +521,15 @@ def ring_copy(buf: torch.Tensor, ring: torch.Tensor, first: int, to_ring: bool) 
                                buf.shape[0], buf.shape[1], int(to_ring), _stream()), "dv_mix_ring_copy")
 
 
+# Up to so many keys that a decode row can ever see, one launch (a workgroup per head) takes it all in bf16; beyond, splits
+# and a merge.  us, split against one: 16 heads on 4 key heads of 128 + 128, 81 / 256 / 366 / 512 / 768 keys 10.9 / 11.0 / 10.9 / 11.2 /
+# 11.2 against 6.4 / 7.7 / 10.2 / 10.6 / 13.0 (32 heads on 8, 366 and 512 keys: 10.7 and 11.1, 10.7 and 11.3); latent attention of 16 heads
+# and rank 256, 81 / 366 / 512 keys 12.3 / 13.1 / 13.1 against 6.1 / 9.3 / 12.9, of 32 heads and rank 512 17.4 / 19.2 / 19.6 against
+# 10.2 / 16.7 / 20.0.
+ONE_LAUNCH_KEYS = 384
+ONE_LAUNCH_LATENTS = 400
+
+
 def decode_splits(keys: int) -> int:
     """Workgroups that share the keys of a decode row.  ``keys`` is the most there can be: the value may not depend
     on the position, which captured steps only know on the device."""
@@ -602,7 +611,8 @@ def ring_attention_row(row, k_ring, v_ring, heads, kv_heads, dim, scale, eps, po
     a.out, a.norm_dim, a.eps = out.data_ptr(), dim, eps
     a.fresh_k = row.data_ptr() + 4 * heads * dim_s
     a.fresh_v = row.data_ptr() + 4 * (heads + kv_heads) * dim_s
-    a.splits = decode_splits(cap)
+    if k_ring.dtype != torch.bfloat16 or dim_s > 128 or vdim_s > 128 or min(cap, window or cap, chunk or cap) > ONE_LAUNCH_KEYS:
+        a.splits = decode_splits(cap)
     part = None
     if a.splits > 1:
         part = torch.empty(heads * a.splits * (vdim_s + 2), dtype=torch.float32, device=row.device)
@@ -621,6 +631,13 @@ def latent_attention_row(q, k_up, v_up, cache, heads, scale, gate, pos_dev, pos)
     _f32(q)
     rank, dim_s, vdim_s = cache.shape[1], k_up.shape[0] // heads, v_up.shape[0] // heads
     code = _code(cache)
+    out = torch.empty(1, heads * vdim_s, dtype=cache.dtype, device=q.device)
+    if cache.dtype == torch.bfloat16 and rank <= 512 and cache.shape[0] <= ONE_LAUNCH_LATENTS:
+        a = _attn_args(q, cache, cache, 1, heads, 1, rank, rank, scale, None, None, None, 0, 0, pos_dev, pos)
+        a.gate, a.ldg, a.out = gate.data_ptr(), heads, out.data_ptr()
+        check(lib.dv_mix_latent_one(_ref(a), cache.shape[0], _ptr(k_up), dim_s, _ptr(v_up), vdim_s, _ptr(out), _stream()),
+              "dv_mix_latent_one")
+        return out
     ql = torch.empty(heads, rank, dtype=torch.float32, device=q.device)
     check(lib.dv_mix_latent_absorb(code, _ptr(q), _ptr(k_up), heads, dim_s, rank, _ptr(ql), _stream()),
           "dv_mix_latent_absorb")
@@ -629,7 +646,6 @@ def latent_attention_row(q, k_up, v_up, cache, heads, scale, gate, pos_dev, pos)
     a.splits = max(2, min(128, (cache.shape[0] + 127) // 128))
     part = torch.empty(heads * a.splits * (rank + 2), dtype=torch.float32, device=q.device)
     a.part = part.data_ptr()
-    out = torch.empty(1, heads * vdim_s, dtype=cache.dtype, device=q.device)
     check(lib.dv_mix_latent_attn(code, _ref(a), _ptr(v_up), vdim_s, _ptr(out), _stream()), "dv_mix_latent_attn")
     return out
 

@@ -312,6 +312,10 @@ DV_API int dv_mix_latent_absorb(int dtype, const float* q, const void* W, int H,
 /* Latent decode row: attention over the cache (args: G = 1, k == v, dim_s = vdim_s = rank, at least two splits with
  * `part`, q and gate fp32), gated, times W_uv [H][vrows][rank]; out [H][vrows]. */
 DV_API int dv_mix_latent_attn(int dtype, const dvAttnArgs* args, const void* W, int vrows, void* out, void* stream);
+/* Latent decode row in bf16, in one launch: W_uk [H][dim_s][rank], attention over the cache of at most `keys` rows, W_uv
+ * [H][vrows][rank] (args: q fp32 [H][dim_s], G = 1, k == v, dim_s = vdim_s = rank <= 512, one split, gate fp32; `out` as below). */
+DV_API int dv_mix_latent_one(const dvAttnArgs* args, int keys, const void* Wk, int dim_s, const void* Wv, int vrows, void* out,
+                             void* stream);
 DV_API int dv_mix_delta_gates(int dtype, const void* z, int64_t ldz, const void* b, int64_t ldb, const float* A_log,
                               const float* dt_bias, int n, int heads, int dim_s, float* g, float* beta, void* stream);
 DV_API int dv_mix_delta_scan(const dvDeltaArgs* args, void* stream);
