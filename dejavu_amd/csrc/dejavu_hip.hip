@@ -1021,6 +1021,10 @@ int dv_topk_f16(const void* logits, int B, int n, int k, void* idx_out, int idx_
     return DV_ERR_WORKSPACE;
   unsigned* ws = reinterpret_cast<unsigned*>(workspace);
   const int blocks = (n + kTopkItemsPerBlock - 1) / kTopkItemsPerBlock;
+  if (B == 1 && n <= kTopkOneMax) {
+    hipLaunchKernelGGL(topk_one_kernel, dim3(1), dim3(1024), 0, s, lg, n, k, idx_out, idx_bytes);
+    return launch_status();
+  }
   if (B > 1 && B <= 64) {
     // one pass reduces the batch to a row of column-wise maxima and takes that row's coarse histogram;
     // the selection then reads the row

@@ -336,7 +336,7 @@ __global__ __launch_bounds__(256 * kTopkBatchGroups) void topk_batch_hist_kernel
   if (q == 0) ws[blockIdx.x * kTopkBins + t] = s_coarse[t];
 }
 
-// Inclusive prefix sum over the 256 threads of a workgroup (s_w: 4 words of LDS).
+// Inclusive prefix sum over the threads of a workgroup (s_w: a word of LDS per wavefront).
 __device__ __forceinline__ unsigned block256_inclusive_scan(unsigned v, unsigned* s_w) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -351,8 +351,8 @@ __device__ __forceinline__ unsigned block256_inclusive_scan(unsigned v, unsigned
   return v;
 }
 
-// In a 256-bin histogram given in DESCENDING bin order over the threads (thread t owns bin
-// 255 - t, count c): the bin in which the k-th largest element lies and the number of elements
+// In a 256-bin histogram given in DESCENDING bin order over the threads (thread t < 256 owns bin
+// 255 - t, count c; others pass 0): the bin in which the k-th largest element lies and the number of elements
 // in higher bins.  All threads return the same pair.
 __device__ __forceinline__ void topk_crossing_bin(unsigned c, unsigned k, unsigned* s_w, unsigned* s_pair,
                                                   unsigned& bin, unsigned& above) {
@@ -487,6 +487,75 @@ __global__ __launch_bounds__(256) void topk_emit_kernel(const half_t* __restrict
                                                         const unsigned* __restrict__ ws,
                                                         void* __restrict__ idx_out, int idx_bytes) {
   topk_emit_body(logits, B, n, k, ws, idx_out, idx_bytes, blockIdx.x, gridDim.x);
+}
+
+// One row of up to 8192 logits by one workgroup, in one launch: a thread keeps eight keys in registers, two histograms of 256
+// bins in LDS (upper, then lower bytes inside the bin where the k-th key lies) give the threshold, prefix sums the places.
+// Same result as above.  Requires n % 8 == 0 and 1 <= k <= n.
+// Bound by its chain of barriers.  us in a row of launches, the three launches against this one: 1536 of 512 9.8 / 6.5, 3072 of 1024
+// 10.6 / 6.8, 8192 of 2048 11.0 / 8.2 (equal values 13.7 / 8.3); with sixteen keys a thread 16384 took 11.5 / 13.2.
+constexpr int kTopkOneMax = 8192;
+__global__ __launch_bounds__(1024) void topk_one_kernel(const half_t* __restrict__ logits, int n, int k, void* __restrict__ idx_out,
+                                                        int idx_bytes) {
+  __shared__ unsigned s_hist[kTopkBins], s_w[16], s_pair[2], s_count[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const half8_t x = load8(logits + min(t * 8, n - 8));
+  const bool in = t * 8 < n;
+  if (t < kTopkBins) s_hist[t] = 0u;
+  __syncthreads();
+  // equal bins in all the lanes that take part are one addition
+  auto count = [&](unsigned bin) {
+    if (__all(bin == (unsigned)__builtin_amdgcn_readfirstlane((int)bin))) {
+      const unsigned long long who = __ballot(1);
+      if (lane == __builtin_ctzll(who)) atomicAdd(&s_hist[bin], (unsigned)__popcll(who));
+    } else {
+      atomicAdd(&s_hist[bin], 1u);
+    }
+  };
+  if (in) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) count(topk_key(x[e]) >> 8);
+  }
+  __syncthreads();
+  unsigned coarse, above, fine, above_fine;
+  topk_crossing_bin(t < kTopkBins ? s_hist[255 - t] : 0u, (unsigned)k, s_w, s_pair, coarse, above);
+  if (t < kTopkBins) s_hist[t] = 0u;
+  __syncthreads();
+  if (in) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (topk_key(x[e]) >> 8 == coarse) count(topk_key(x[e]) & 255u);
+  }
+  __syncthreads();
+  topk_crossing_bin(t < kTopkBins ? s_hist[255 - t] : 0u, (unsigned)k - above, s_w, s_pair, fine, above_fine);
+  const unsigned T = coarse * 256u + fine, need = (unsigned)k - above - above_fine;  // ties to take, lowest index first
+  // larger keys in the lower half of a word, equal ones in the upper
+  unsigned own = 0u;
+  if (in) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) own += topk_key(x[e]) > T ? 1u : topk_key(x[e]) == T ? 0x10000u : 0u;
+  }
+  unsigned before = own;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const unsigned o = __shfl_up(before, off, kWave);
+    if (lane >= off) before += o;
+  }
+  if (lane == kWave - 1) s_count[wave] = before;
+  before -= own;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 15; ++w) before += w < wave ? s_count[w] : 0u;
+  unsigned rank = before >> 16, pos = (before & 0xffffu) + (rank < need ? rank : need);
+  if (!in) return;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const unsigned key = topk_key(x[e]);
+    if (key > T || (key == T && rank++ < need)) {
+      if (idx_bytes == 8) reinterpret_cast<int64_t*>(idx_out)[pos++] = t * 8 + e;
+      else reinterpret_cast<int32_t*>(idx_out)[pos++] = t * 8 + e;
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------

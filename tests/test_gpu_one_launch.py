@@ -81,3 +81,20 @@ def test_latent_row(rank, vdim, cap, pos):
         lat = attend(ql, cd[:pos + 1], cd[:pos + 1], 2.0) / (1.0 + np.exp(-gate[h].item()))
         want[h] = vd[h * vdim:(h + 1) * vdim] @ lat
     close(got, want)
+
+
+@pytest.mark.parametrize("n", [1032, 2048, 8184, 8192, 8200])
+def test_top_k_of_one_row(n):
+    """Both sides of the line up to which one workgroup selects: ties, few values, all kinds of k."""
+    from dejavu_amd import ops
+    from oracle import dejavu_oracle as O
+
+    rng = np.random.default_rng(n)
+    mixed = np.round(rng.normal(size=n) * 2).astype(np.float16)
+    mixed[[0, n // 2, n - 1]] = np.inf, np.nan, -np.inf
+    for x in (rng.normal(size=n).astype(np.float16), mixed, np.full(n, -1.5, dtype=np.float16)):
+        for k in (1, n // 3, n - 1, n):
+            want = O.topk_lower_index(x, k)
+            for dtype in (torch.int32, torch.int64):
+                got = ops.topk_indices(torch.from_numpy(x).cuda(), k, dtype=dtype)
+                assert np.array_equal(got.cpu().numpy().astype(np.int64), want)
