@@ -59,9 +59,10 @@ class DynamicTanh(nn.Module):
 
     def struct(self):
         """The kernels' argument; alpha is read back once per loaded value."""
-        stamp = (self.weight.data_ptr(), self.bias.data_ptr(), self.alpha.data_ptr(), self.alpha._version)
+        weight, bias, alpha = self.weight, self.bias, self.alpha
+        stamp = (weight.data_ptr(), bias.data_ptr(), alpha.data_ptr(), alpha._version)
         if self._stamp != stamp:
-            self._struct = ops.L.DynTanh(w=self.weight.data_ptr(), b=self.bias.data_ptr(), alpha=float(self.alpha.item()))
+            self._struct = ops.L.DynTanh(w=stamp[0], b=stamp[1], alpha=float(alpha.item()))
             self._stamp = stamp
         return self._struct
 

@@ -134,7 +134,8 @@ def _transposed_copy(module, attr: str, weight: torch.Tensor) -> torch.Tensor:
             cur.shape != (weight.shape[1], weight.shape[0]):
         cur = weight.t().contiguous()
         setattr(module, attr, cur)
-    setattr(module, attr + "_stamp", stamp)
+    if getattr(module, attr + "_stamp", None) != stamp:
+        setattr(module, attr + "_stamp", stamp)
     return cur
 
 
@@ -224,8 +225,6 @@ class ParallelFusedMLPDejavu(nn.Module):
         layer's MLP, only when decoding one token.  defer_join: when the predictor runs on the side
         stream, the current stream does not wait for it: mlp_logit is then only good for work
         enqueued on the side stream (the next layer's top-k is) or after ``join_side_stream()``."""
-        self._streams()
-        curr_stream = torch.cuda.current_stream()
         do_token_generation = x.size(1) == 1
         # The predictor only needs `residual`, so it streams its weights on the side
         # stream while fc1 / fc2 run (the reference starts it after the MLP, to
@@ -238,8 +237,10 @@ class ParallelFusedMLPDejavu(nn.Module):
         mlp_logit = None
         side = do_token_generation and side_stream_enabled(x.shape[0])
         if side:
+            self._streams()
+            curr_stream = torch.cuda.current_stream()
             curr_stream.record_event(self.event_mlp)
-        if idx != None:
+        if idx is not None:
             assert x.size(1) == 1
             h = ops.gather_gemv(x.squeeze(1), self.fc1.weight, idx, self.fc1.bias, activation=self.activation)
         else:
@@ -251,7 +252,7 @@ class ParallelFusedMLPDejavu(nn.Module):
                 self.sp_stream.wait_event(self.event_mlp)
                 mlp_logit = self.sp(residual)
                 self.sp_stream.record_event(self.event_mlp_sp)
-        if idx != None:
+        if idx is not None:
             out = ops.gather_transposed_gemv(h, self.transposed_fc2(), idx, self.fc2.bias, defer_reduce=defer_reduce)
             if not isinstance(out, ops.PendingRows):
                 out = out.unsqueeze(1)
@@ -674,7 +675,7 @@ class ParallelMHASparseAttMlp(_MHABase):
         if x.size(1) != 1:  # prompt: remember where the decode window starts
             self._set_cache_offset(x.size(1), x.device)
             self.reset_window()
-        sparse = inference_params is not None and inference_params.sequence_len_offset > 0 and head_idx != None
+        sparse = inference_params is not None and inference_params.sequence_len_offset > 0 and head_idx is not None
         self._side_fork(x.shape[0])
         side_done = None
         joined_early = False
