@@ -83,6 +83,8 @@ SIGNATURES = {
     "dv_mix_linear_tiles": (_i, [_i, _P(TileArgs), _p]),
     "dv_mix_linear_tiles_workspace_bytes": (ctypes.c_size_t, [_i, _i, _i]),
     "dv_mix_linear_tiles_ws": (_i, [_i, _P(TileArgs), _p, ctypes.c_size_t, _p]),
+    "dv_mix_linear_split_workspace_bytes": (ctypes.c_size_t, [_i, _i, _i]),
+    "dv_mix_linear_split": (_i, [_p, _l, _p, _l, _p, _i, _i, _i, _p, _l, _p, ctypes.c_size_t, _p]),
     "dv_mix_linear_wide": (_i, [_i, _P(TileArgs), _p]),
     "dv_mix_short_conv": (_i, [_i, _i, _P(ConvArgs), _p]),
     "dv_mix_conv_state": (_i, [_i, _p, _l, _i, _i, _i, _p, _p]),

@@ -166,6 +166,33 @@ def _product_ok(x, W):
     return _code(W)
 
 
+# fp32 products by parts in fp16 (linear_split.hpp), where they are ahead of the library's fp32 GEMM (times its speed): 11264 x 2048 with 200 /
+# 400 / 500 / 2000 rows 1.25 / 1.49 / 1.73 / 1.90, 2048 x 5632 with 260 / 500 / 1000 1.07 / 1.29 / 1.54, 4368 x 2048 with 300 / 512 1.03 / 1.73, 22016 x 4096 with
+# 200 / 1000 1.32 / 1.99; but its three launches take 20 us whatever the work (500 rows by 2048 x 2048 1.01, 300 by 3072 x 2048 0.86, 260
+# by 4368 x 2048 0.83, 200 by 2048 x 5632 0.88), and few rows leave much of a tile empty (150 by 11264 x 2048 0.91).
+SPLIT_MIN_ROWS, SPLIT_COLUMNS = 161, 512
+SPLIT_WORK = 2_400_000_000  # rows * weight
+
+
+def _split_product(x: torch.Tensor, W: torch.Tensor, bias=None) -> Optional[torch.Tensor]:
+    """``F.linear`` of fp32 rows by the kernel that multiplies fp16 parts; None where the library takes them."""
+    (n, K), M = x.shape, W.shape[0]
+    if (x.dtype != torch.float32 or n < SPLIT_MIN_ROWS or K < SPLIT_COLUMNS or n * M * K < SPLIT_WORK or M % 4 or K % 4 or not results_only(x, W, bias) or
+            any(t.stride(0) % 4 or t.data_ptr() % 16 for t in (x, W)) or (bias is not None and bias.data_ptr() % 16)):
+        return None
+    out = torch.empty(n, M, dtype=torch.float32, device=x.device)
+    nbytes = lib.dv_mix_linear_split_workspace_bytes(n, M, K)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    check(lib.dv_mix_linear_split(_ptr(x), x.stride(0), _ptr(W), W.stride(0), _ptr(bias), n, M, K, _ptr(out), M, _ptr(ws), nbytes,
+                                  _stream()), "dv_mix_linear_split")
+    return out
+
+
+def _library_or_split(x: torch.Tensor, W: torch.Tensor, bias=None) -> torch.Tensor:
+    y = _split_product(x, W, bias)
+    return F.linear(x, W, bias) if y is None else y
+
+
 class RmsRow:
     """One fp32 row that still has to be RMS-normed and weighted; the products that read it do that themselves."""
 
@@ -254,7 +281,7 @@ def linear(x, W: torch.Tensor, bias: Optional[torch.Tensor] = None, f32: bool = 
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
         check(lib.dv_mix_linear_wide(L.OUT_T, _ref(a), _stream()), "dv_mix_linear_wide")
         return out
-    return F.linear(x, W, bias)
+    return _library_or_split(x, W, bias)
 
 
 def gated_unit(x, W: torch.Tensor, act: int, limit: float = 0.0) -> torch.Tensor:
@@ -276,7 +303,7 @@ def gated_unit(x, W: torch.Tensor, act: int, limit: float = 0.0) -> torch.Tensor
         a.out, a.ldo, a.act, a.limit = y.data_ptr(), M // 2, act, limit
         check(lib.dv_mix_linear_wide(L.OUT_GLU, _ref(a), _stream()), "dv_mix_linear_wide")
     else:
-        gu = F.linear(x, W)
+        gu = _library_or_split(x, W)
         check(lib.dv_mix_glu(code, _ptr(gu), y.numel(), act, limit, _ptr(y), _stream()), "dv_mix_glu")
     return y
 
@@ -295,7 +322,7 @@ def linear_residual(x: torch.Tensor, W: torch.Tensor, stream: ResidualStream, po
     n = x.shape[0]
     assert stream.x.shape == (n, W.shape[0])
     if n != 1 and not _tiles(x, W, whole=W.shape[0] % 8 == 0):
-        return residual(F.linear(x, W), stream, post, pre, add_start)
+        return residual(_library_or_split(x, W), stream, post, pre, add_start)
     h = None if pre is None else stream.new_h()
     if n == 1:
         a = _row_args(x, W)
