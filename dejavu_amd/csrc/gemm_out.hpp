@@ -65,6 +65,7 @@ __device__ __forceinline__ void qkv_store4(const QkvScatter& q, half_t* __restri
 }
 
 struct QkvRows {  // (a head out of range reads row 0 and is not stored)
+  static constexpr bool kPastCaches = false;
   QkvScatter q;
   __device__ __forceinline__ int64_t operator()(int m) const {
     const int t = m / (q.Hk * q.hd), rem = m - t * q.Hk * q.hd, i = rem / q.hd, h = q.head_idx[i];
@@ -118,6 +119,7 @@ struct PlainOut {
 };
 
 struct GatheredRows {
+  static constexpr bool kPastCaches = true;
   const void* idx;
   int idx_bytes, Z;
   __device__ __forceinline__ int64_t operator()(int m) const {  // an index out of range reads row 0; its result is act(0)

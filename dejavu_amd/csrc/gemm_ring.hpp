@@ -44,6 +44,7 @@ struct RingOperands {
 
 // Rows 0 .. M - 1 of the weight.
 struct PlainRows {
+  static constexpr bool kPastCaches = true;
   __device__ __forceinline__ int64_t operator()(int m) const { return m; }
 };
 
@@ -102,10 +103,13 @@ inline RingPlan plan_ring(int n, int M, int K, int units) {
   return p;
 }
 
-// NT_W: the weight bypasses the caches (worth 10 % where the rows of X are few).
+// NT_W: the weight bypasses the caches: worth 10 % where the rows of X are few and the weight comes from memory (128 rows by
+// 20480 x 5120 and its like, of a prompt's layer: 235 us the layer, 223), but a small weight (17 rows by 1024 x 5120: 7.2, 7.7
+// us) and the chosen heads' rows of a block (192 rows a tile, 128 of X, 9216 columns: 39.2, 40.7) stay in the last cache from
+// one call to the next.  These rows also gain nothing by beginning at different columns (kPastCaches of the rows).
 // Out: called with (m, n, sums of rows m .. m + 3 and row n of X), m % 4 == 0, m < M, n < the operands' n.
 // Grid: (tiles of W, tiles of X, splits of K).  part: with several splits, the sums [split][tile][value][thread].
-template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, typename Rows, typename Out>
+template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, bool ROUND, typename Rows, typename Out>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T> a, Rows rows, Out out, float4_t* __restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) unsigned char slots[];
   constexpr int WAVES = WM * WN, THREADS = WAVES * 64;
@@ -121,14 +125,15 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T>
   const int m0 = blockIdx.x * MB, n0 = blockIdx.y * NB;
   const int nch = (a.K + KC - 1) / KC;
   const int c0 = nch * blockIdx.z / gridDim.z, len = nch * (blockIdx.z + 1) / gridDim.z - c0;
-  // Up to 128 rows of X and with other than 64 weight rows a tile the columns are taken in parts, and workgroups begin with
-  // different ones and go round: all of them at the same column, of rows that are a power of two apart, wait for the same few
-  // channels of the memory.  The parts' sums are added in the columns' order (two: in any) wherever the workgroup began, so a
-  // row's result does not depend on its place.  (A different chunk for each instead: the same time, other bits.)
+  // ROUND: the columns are taken in parts, and workgroups begin with different ones and go round: all of them at the same
+  // column, of rows that are a power of two apart, wait for the same few channels of the memory.  The parts' sums are added in
+  // the columns' order (two: in any) wherever the workgroup began, so a row's result does not depend on its place.  (A different
+  // chunk for each instead: the same time, other bits.)
   // us without and with: 47 rows by 22016 x 4096 37.7, 32.2; 22016 x 6144 60.0, 47.1; 16 rows by 22016 x 4096 37.3, 31.8; 100 rows by
-  // 16384 x 4096 40.2, 35.7, 12288 x 4096 31.8, 29.0; 128 rows by 15360 x 5120 46.5, 44.1, four parts 44.3; 5120 x 20480 55.1, 55.7, four
-  // parts 65.  But tiles of 64 weight rows (12288 x 4096, 47 rows) 25.2, 30.1, and more rows of X the same time either way.
-  constexpr int PARTS = NB > 128 || MB == 64 ? 1 : NB == 128 ? 2 : 4, CHAINS = 4 / PARTS;  // sums of a part
+  // 16384 x 4096 40.2, 35.7, 12288 x 4096 31.8, 29.0; 128 rows by 15360 x 5120 46.5, 44.1, four parts 44.3; 5120 x 20480 55.1, 55.7,
+  // four parts 65.  But tiles of 64 weight rows (12288 x 4096, 47 rows) 25.2, 30.1, more rows of X the same time either way, and a
+  // split of a few chunks (16 rows by 1024 x 4096 in eight) 5.4, 5.7.
+  constexpr int PARTS = !ROUND ? 1 : NB == 128 ? 2 : 4, CHAINS = 4 / PARTS;  // sums of a part
   const int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);  // (these go round the eight dies)
   const int begin = PARTS == 4 ? id / 8 % 4 : PARTS == 2 ? id / 16 % 2 : 0;
   const int part_len = (len + PARTS - 1) / PARTS, chain_len = ((PARTS == 1 ? nch : part_len) + CHAINS - 1) / CHAINS;
@@ -279,12 +284,12 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_sum_kernel(int n_rows,
 
 // launch(kernel as a template argument, grid, threads, LDS bytes, arguments) is the library's own way to launch with more
 // than 48 KiB of LDS.
-template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, typename Rows, typename Out, typename Launch>
+template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, bool ROUND, typename Rows, typename Out, typename Launch>
 int gemm_ring_tiles(const RingPlan& p, const RingOperands<T>& a, const Rows& rows, const Out& out, void* workspace, hipStream_t s,
                     const Launch& launch) {
   float4_t* part = reinterpret_cast<float4_t*>(workspace);
   const dim3 threads(WM * WN * 64);
-  const int rc = launch.template operator()<gemm_ring_kernel<T, MB, NB, KC, ST, WM, WN, NT_W, Rows, Out>>(
+  const int rc = launch.template operator()<gemm_ring_kernel<T, MB, NB, KC, ST, WM, WN, NT_W, ROUND, Rows, Out>>(
       dim3(p.rows, p.cols, p.splits), threads, (size_t)ST * (MB + NB) * KC * 2, s, a, rows, out, part);
   if (rc != 0 || p.splits == 1) return rc;
   constexpr int values = (MB / WM / 16) * (NB / WN / 16);
@@ -295,17 +300,18 @@ int gemm_ring_tiles(const RingPlan& p, const RingOperands<T>& a, const Rows& row
 template <typename T, typename Rows, typename Out, typename Launch>
 int gemm_ring(const RingPlan& p, const RingOperands<T>& a, const Rows& rows, const Out& out, void* workspace, hipStream_t s,
               const Launch& launch) {
-#define DV_RING(MB, NB, KC, ST, WM, WN, NT_W) gemm_ring_tiles<T, MB, NB, KC, ST, WM, WN, NT_W>(p, a, rows, out, workspace, s, launch)
+  constexpr bool kPast = Rows::kPastCaches;
+#define DV_RING(MB, NB, KC, ST, WM, WN, NT_W, ROUND) gemm_ring_tiles<T, MB, NB, KC, ST, WM, WN, NT_W, ROUND>(p, a, rows, out, workspace, s, launch)
   switch (p.nb) {
-    case 16: return DV_RING(32, 16, 128, 4, 2, 1, true);
-    case 32: return p.mb == 128 ? DV_RING(128, 32, 64, 4, 4, 1, true) : DV_RING(64, 32, 64, 4, 4, 1, true);
-    case 64: return p.mb == 128 ? DV_RING(128, 64, 64, 4, 4, 2, true)
-                    : p.mb == 96 ? DV_RING(96, 64, 64, 4, 2, 2, true) : DV_RING(64, 64, 64, 4, 2, 2, true);
-    case 128: return p.mb == 64 ? DV_RING(64, 128, 64, 3, 2, 4, true)
-                     : p.mb == 128 ? DV_RING(128, 128, 64, 4, 2, 4, true) : DV_RING(192, 128, 64, 3, 2, 4, true);
-    case 192: return p.mb == 64 ? DV_RING(64, 192, 64, 4, 2, 4, false)
-                     : p.mb == 128 ? DV_RING(128, 192, 64, 3, 2, 4, false) : DV_RING(192, 192, 64, 3, 2, 4, false);
-    default: return p.mb == 64 ? DV_RING(64, 256, 64, 3, 2, 4, false) : DV_RING(128, 256, 64, 3, 2, 4, false);
+    case 16: return p.splits == 8 ? DV_RING(32, 16, 128, 4, 2, 1, true, false) : DV_RING(32, 16, 128, 4, 2, 1, true, true);
+    case 32: return p.mb == 128 ? DV_RING(128, 32, 64, 4, 4, 1, kPast, true) : DV_RING(64, 32, 64, 4, 4, 1, false, false);
+    case 64: return p.mb == 128 ? DV_RING(128, 64, 64, 4, 4, 2, kPast, true)
+                    : p.mb == 96 ? DV_RING(96, 64, 64, 4, 2, 2, kPast, true) : DV_RING(64, 64, 64, 4, 2, 2, false, false);
+    case 128: return p.mb == 64 ? DV_RING(64, 128, 64, 3, 2, 4, false, false)
+                     : p.mb == 128 ? DV_RING(128, 128, 64, 4, 2, 4, kPast, kPast) : DV_RING(192, 128, 64, 3, 2, 4, kPast, kPast);
+    case 192: return p.mb == 64 ? DV_RING(64, 192, 64, 4, 2, 4, false, false)
+                     : p.mb == 128 ? DV_RING(128, 192, 64, 3, 2, 4, false, false) : DV_RING(192, 192, 64, 3, 2, 4, false, false);
+    default: return p.mb == 64 ? DV_RING(64, 256, 64, 3, 2, 4, false, false) : DV_RING(128, 256, 64, 3, 2, 4, false, false);
   }
 #undef DV_RING
 }
