@@ -109,7 +109,8 @@ inline RingPlan plan_ring(int n, int M, int K, int units) {
 // one call to the next.  These rows also gain nothing by beginning at different columns (kPastCaches of the rows).
 // Out: called with (m, n, sums of rows m .. m + 3 and row n of X), m % 4 == 0, m < M, n < the operands' n.
 // Grid: (tiles of W, tiles of X, splits of K).  part: with several splits, the sums [split][tile][value][thread].
-template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, bool ROUND, typename Rows, typename Out>
+template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, typename Rows, typename Out,
+          bool ROUND = MB != 64 && NB <= 128>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T> a, Rows rows, Out out, float4_t* __restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) unsigned char slots[];
   constexpr int WAVES = WM * WN, THREADS = WAVES * 64;
@@ -289,7 +290,7 @@ int gemm_ring_tiles(const RingPlan& p, const RingOperands<T>& a, const Rows& row
                     const Launch& launch) {
   float4_t* part = reinterpret_cast<float4_t*>(workspace);
   const dim3 threads(WM * WN * 64);
-  const int rc = launch.template operator()<gemm_ring_kernel<T, MB, NB, KC, ST, WM, WN, NT_W, ROUND, Rows, Out>>(
+  const int rc = launch.template operator()<gemm_ring_kernel<T, MB, NB, KC, ST, WM, WN, NT_W, Rows, Out, ROUND>>(
       dim3(p.rows, p.cols, p.splits), threads, (size_t)ST * (MB + NB) * KC * 2, s, a, rows, out, part);
   if (rc != 0 || p.splits == 1) return rc;
   constexpr int values = (MB / WM / 16) * (NB / WN / 16);
