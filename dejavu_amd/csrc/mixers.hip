@@ -78,14 +78,18 @@ int linear_stream(const RingPlan& p, const TileArgs& a, void* workspace, hipStre
   return gemm_ring(p, o, PlainRows{}, MixOut<AFTER>{a}, workspace, s, MixLaunch{});
 }
 
-// ---- fp32 rows on the fp16 instructions ----
-template <int NB>
-int linear_split(const SplitPlan& p, const SplitOperands& a, const SplitOut& out, float4_t* part, hipStream_t s) {
+// ---- fp32 rows on the bf16 instructions ----
+int linear_split(const SplitPlan& p, const SplitOperands& a, const SplitOut& out, float4_t* sums, hipStream_t s) {
+  const int64_t blocks = ((int64_t)a.n + kSplitPartRows - 1) / kSplitPartRows * p.chunks;
+  if (blocks > 0x7fffffff || p.tiles() > 0x7fffffff) return DV_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
+  int rc = launched();
+  if (rc != DV_OK) return rc;
   const dim3 threads(kSplitThreads);
-  const int rc = launch_lds<linear_split_kernel<NB, SplitOut>>(dim3(p.rows, p.cols, p.splits), threads, split_lds(NB), s, a, out, part);
+  rc = launch_lds<linear_split_kernel<SplitOut>>(dim3((unsigned)p.tiles(), p.splits), threads, kSplitLds, s, a, p.rows, out, sums);
   if (rc != DV_OK || p.splits == 1) return rc;
-  return launch_lds<linear_split_sum_kernel<NB, SplitOut>>(dim3(p.rows, p.cols, NB / 16), threads, 0, s, a.n, a.M, out, (const float4_t*)part,
-                                                           p.splits);
+  return launch_lds<linear_split_sum_kernel<SplitOut>>(dim3((unsigned)p.tiles(), kSplitCols / 8), threads, 0, s, a.n, a.M, p.rows, out,
+                                                       (const float4_t*)sums, p.splits);
 }
 
 // ---- one row ---------------------------------------------------------------
@@ -515,7 +519,7 @@ int dv_mix_linear_tiles_ws(int after, const dvTileArgs* a, void* workspace, size
 
 size_t dv_mix_linear_split_workspace_bytes(int n, int M, int K) {
   if (n < 1 || M < 1 || K < 4) return 0;
-  return plan_split(n, M, K, compute_units()).workspace_bytes(n, M);
+  return plan_split(n, M, K, compute_units()).workspace_bytes(n);
 }
 
 int dv_mix_linear_split(const float* x, int64_t ldx, const float* W, int64_t ldw, const float* bias, int n, int M, int K, float* out,
@@ -523,19 +527,10 @@ int dv_mix_linear_split(const float* x, int64_t ldx, const float* W, int64_t ldw
   if (!x || !W || !out || n < 1 || M < 1 || K < 4) return DV_ERR_INVALID_ARG;
   if (M % 4 || K % 4 || ldx % 4 || ldw % 4 || ldo % 4 || !al16(x) || !al16(W) || !al16(bias) || !al16(out)) return DV_ERR_ALIGNMENT;
   const SplitPlan p = plan_split(n, M, K, compute_units());
-  if (p.cols > 65535 || (int64_t)n + M > 0x7ffffff0) return DV_ERR_UNSUPPORTED;
-  if (!workspace || workspace_bytes < p.workspace_bytes(n, M)) return DV_ERR_WORKSPACE;
+  if (!workspace || workspace_bytes < p.workspace_bytes(n)) return DV_ERR_WORKSPACE;
   if (!al16(workspace)) return DV_ERR_ALIGNMENT;
-  unsigned char* ws = (unsigned char*)workspace;
-  int* exps = (int*)(ws + p.parts_bytes(n));
-  const SplitOperands a{x, ldx, W, ldw, (half_t*)ws, exps, exps + n, n, M, K, p.KP};
-  hipLaunchKernelGGL(split_rows_kernel, dim3(blocks_of((int64_t)n + M, 4)), dim3(256), 0, st(stream), a);
-  const int rc = launched();
-  if (rc != DV_OK) return rc;
-  float4_t* sums = (float4_t*)(ws + p.sums_offset(n, M));
-  const SplitOut o{out, ldo, bias};
-  if (p.nb == 128) return linear_split<128>(p, a, o, sums, st(stream));
-  return linear_split<256>(p, a, o, sums, st(stream));
+  const SplitOperands a{x, ldx, W, ldw, (bf16_t*)workspace, n, M, K};
+  return linear_split(p, a, SplitOut{out, ldo, bias}, (float4_t*)((unsigned char*)workspace + p.parts_bytes(n)), st(stream));
 }
 
 int dv_mix_linear_wide(int after, const dvTileArgs* a, void* stream) {

@@ -166,22 +166,46 @@ def _product_ok(x, W):
     return _code(W)
 
 
-# fp32 products by parts in fp16 (linear_split.hpp), where they are ahead of the library's fp32 GEMM (times its speed): 11264 x 2048 with 200 /
-# 400 / 500 / 2000 rows 1.25 / 1.49 / 1.73 / 1.90, 2048 x 5632 with 260 / 500 / 1000 1.07 / 1.29 / 1.54, 4368 x 2048 with 300 / 512 1.03 / 1.73, 22016 x 4096 with
-# 200 / 1000 1.32 / 1.99; but its three launches take 20 us whatever the work (500 rows by 2048 x 2048 1.01, 300 by 3072 x 2048 0.86, 260
-# by 4368 x 2048 0.83, 200 by 2048 x 5632 0.88), and few rows leave much of a tile empty (150 by 11264 x 2048 0.91).
+# fp32 products by parts in bf16 (linear_split.hpp), which are as exact as fp32 products for values of any range, where what the launches take
+# (``_split_us``: a round of tiles 2.2 us a chunk of columns, splits of K 4 us and 0.05 for each tile, all launches 8) is less than the
+# library's fp32 GEMM does at 118 TFLOP/s; it ranges from 85 to 140.  Times the library's speed: 11264 x 2048 with 256 / 400 / 500 /
+# 1000 / 2000 rows 1.03 / 1.10 / 1.27 / 1.25 / 1.31, 2048 x 5632 with 400 / 500 / 1000 1.14 / 1.07 / 1.13, 4368 x 2048 with 384 / 512 1.03 /
+# 1.46, 22016 x 4096 with 200 / 500 / 1000 / 2048 1.15 / 1.23 / 1.42 / 1.25, 500 by 3072 x 2048 1.11, 300 by 8192 x 4096 1.11, 200 by 4096 x
+# 11008 1.21, 4000 by 4096 x 512 1.24.  Left to the library: too little for the launches (500 by 2048 x 2048 0.91, 256 by 2048 x 5632 0.77, 260
+# by 4368 x 2048 0.81, 400 0.95, 2000 by 1024 x 1024 0.84), tiles that are half empty (161 by 11264 x 2048 0.91, 161 by 22016 x 4096
+# 0.99; but 300 by 11264 x 2048 1.14).  On the line: 300 by 22016 x 4096 0.98, 300 by 4096 x 4096 1.00, 2000 by 2048 x 768 0.96.
 SPLIT_MIN_ROWS, SPLIT_COLUMNS = 161, 512
-SPLIT_WORK = 2_400_000_000  # rows * weight
+SPLIT_RATE = 59_000_000        # products a us (118 TFLOP/s) that the tiles have to reach
+SPLIT_VALUES = 1 << 27         # of x, whose parts take 6 bytes each: beyond, the library, which needs no memory for them
+SPLIT_TILE, SPLIT_CHUNK, SPLIT_ROUND = (256, 128), 32, 256
+
+
+@lru_cache(maxsize=4096)
+def _split_us(n: int, M: int, K: int) -> float:
+    """What the launches take, as estimated for the choice of the splits of K."""
+    tiles, chunks = _tiles_of(n, M, SPLIT_TILE[1], SPLIT_TILE[0]), -(-K // SPLIT_CHUNK)
+    return 8 + min(2.2 * -(-tiles * s // SPLIT_ROUND) * -(-chunks // s) + (4 + 0.05 * s * tiles if s > 1 else 0)
+                   for s in range(1, max(1, min(8, K // 256)) + 1))
+
+
+def _split_rule(n: int, M: int, K: int) -> bool:
+    return n >= SPLIT_MIN_ROWS and K >= SPLIT_COLUMNS and n * K <= SPLIT_VALUES and n * M * K >= SPLIT_RATE * _split_us(n, M, K)
+
+
+@lru_cache(maxsize=4096)
+def _split_workspace_bytes(device: int, n: int, M: int, K: int) -> int:
+    """As ``_tile_workspace_bytes``."""
+    return lib.dv_mix_linear_split_workspace_bytes(n, M, K)
 
 
 def _split_product(x: torch.Tensor, W: torch.Tensor, bias=None) -> Optional[torch.Tensor]:
-    """``F.linear`` of fp32 rows by the kernel that multiplies fp16 parts; None where the library takes them."""
+    """``F.linear`` of fp32 rows by the kernel that multiplies parts in bf16; None where the library takes them."""
     (n, K), M = x.shape, W.shape[0]
-    if (x.dtype != torch.float32 or n < SPLIT_MIN_ROWS or K < SPLIT_COLUMNS or n * M * K < SPLIT_WORK or M % 4 or K % 4 or not results_only(x, W, bias) or
+    if (x.dtype != torch.float32 or not _split_rule(n, M, K) or M % 4 or K % 4 or not results_only(x, W, bias) or
             any(t.stride(0) % 4 or t.data_ptr() % 16 for t in (x, W)) or (bias is not None and bias.data_ptr() % 16)):
         return None
     out = torch.empty(n, M, dtype=torch.float32, device=x.device)
-    nbytes = lib.dv_mix_linear_split_workspace_bytes(n, M, K)
+    nbytes = _split_workspace_bytes(torch._C._cuda_getDevice(), n, M, K)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     check(lib.dv_mix_linear_split(_ptr(x), x.stride(0), _ptr(W), W.stride(0), _ptr(bias), n, M, K, _ptr(out), M, _ptr(ws), nbytes,
                                   _stream()), "dv_mix_linear_split")
