@@ -573,10 +573,12 @@ def ring_copy(buf: torch.Tensor, ring: torch.Tensor, first: int, to_ring: bool) 
 
 
 # Up to so many keys that a decode row can ever see, one launch (a workgroup per head) takes it all in bf16; beyond, splits
-# and a merge.  us, split against one: 16 heads on 4 key heads of 128 + 128, 81 / 256 / 366 / 512 / 768 keys 10.9 / 11.0 / 10.9 / 11.2 /
-# 11.2 against 6.4 / 7.7 / 10.2 / 10.6 / 13.0 (32 heads on 8, 366 and 512 keys: 10.7 and 11.1, 10.7 and 11.3); latent attention of 16 heads
-# and rank 256, 81 / 366 / 512 keys 12.3 / 13.1 / 13.1 against 6.1 / 9.3 / 12.9, of 32 heads and rank 512 17.4 / 19.2 / 19.6 against
-# 10.2 / 16.7 / 20.0.
+# and a merge.  us, split / one, all of the keys seen: 16 heads on 4 key heads of 128 + 128, 81 / 256 / 320 / 384 / 400 / 448 / 512 / 768 keys 10.9 /
+# 6.4, 11.0 / 7.7, 11.0 / 10.1, 11.1 / 10.2, 10.6 / 10.2, 11.0 / 10.4, 11.1 / 10.5, 11.2 / 13.0; 32 heads on 8, 320 to 512 keys 11.1 / 10.3, 11.1 / 10.9,
+# 10.8 / 10.9, 11.1 / 11.0, 11.0 / 11.2; 64 heads on 8, 384 keys 14.9 / 11.0; 32 heads with keys of their own are behind from 300 on when
+# all keys are seen (9.3 / 10.3, at 384 10.3 / 10.9) and ahead with five eighths of them (8.6 / 7.6, 8.4 / 7.9).  Latent attention of 16
+# heads and rank 256, 81 / 256 / 384 / 400 / 448 / 512 keys 12.3 / 6.1, 12.9 / 7.8, 13.0 / 9.4, 13.0 / 12.5, 13.1 / 12.6, 13.0 / 12.8, of 32 heads and rank
+# 512, 256 to 512 keys 18.9 / 13.9, 19.3 / 17.0, 19.4 / 19.2, 19.4 / 19.6, 19.4 / 20.0.
 ONE_LAUNCH_KEYS = 384
 ONE_LAUNCH_LATENTS = 400
 
