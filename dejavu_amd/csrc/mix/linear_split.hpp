@@ -1,13 +1,15 @@
 // fp32 products of many rows on the bf16 matrix instructions: out(m, n) = sum_k W[m, k] x[n, k].
 //
 // A value is the sum of three bf16 parts, rounded one after the other (the published bf16x3 splitting: Henry, Tang and Heinecke,
-// 2019), which hold all of its 24 bits.  Products of parts are exact in the instruction's fp32 sums; the six largest are taken, what
-// is left out is below 2^-25 of a product.  Products of one size have sums of their own, in which the second and third parts stand
-// 2^8 and 2^16 times as large: so the smallest values' parts are no zeros, and no sum overflows where that of the values'
-// magnitudes would not.  What is lost is relative to each value and not to its row, so rows of any range are as exact as others (two fp16
-// parts with an exponent for a row, three quarters of this time, lose what lies far below the row's largest value: with one column 2^24 times
-// as large as the others and the weight's as much smaller a row was 2e-5 from 64 bits, with 2^40 0.9).  Infinities and NaN are in the first
-// parts, whose sums are the result where they are not finite; other results do not see them.
+// 2019), which hold all of its 24 bits (2^-8 and 2^-17 of it at most, the others).  Products of parts are exact in the instruction's
+// fp32 sums; the six largest are taken, what is left out is 2^-24 of a product at most and 2^-27.5 in the root mean square.  Products of
+// one size have sums of their own, in which the second and third parts stand 2^8 and 2^16 times as large: so the smallest values'
+// parts are no zeros, and no sum overflows where that of the values' magnitudes would not.  What is lost is relative to each value and
+// not to its row, so rows of any range are as exact as others (two fp16 parts with an exponent for a row, three quarters of this time, lose
+// what lies far below the row's largest value: with one column 2^24 times as large as the others and the weight's as much smaller a row was
+// 2e-5 from 64 bits, with 2^40 0.9).  Infinities and NaN are in the first parts, whose sums are the result where they are not finite;
+// other results do not see them.  At the very end of the range: a weight below 2^-126 loses its last bit, and values below 2^-133
+// are zeros to an infinity.
 //
 // The parts of x are made beforehand (split_rows_kernel); those of W in registers, by the one wave that uses them.
 // Six bf16 products at 2.5 PFLOP/s are 2.6 times the fp32 instructions' 157 TFLOP/s.  500 rows by 11264 x 2048: 155 us, the library's fp32
