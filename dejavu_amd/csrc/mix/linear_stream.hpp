@@ -1,8 +1,8 @@
-// The epilogues of linear_rows.hpp behind the tiles of gemm_ring.hpp and linear_wide.hpp.
+// The epilogues of linear_rows.hpp behind the tiles of gemm_ring.hpp and gemm_wide.hpp.
 #pragma once
 #include <type_traits>
 
-#include "../gemm_ring.hpp"
+#include "../gemm_wide.hpp"
 #include "elem.hpp"
 #include "stream.hpp"
 
@@ -52,6 +52,28 @@ template <int AFTER>
 struct MixOut {
   TileArgs a;
   __device__ __forceinline__ void operator()(int m, int n, const float4_t& v) const { tile_out<AFTER>(a, m, n, v); }
+};
+
+// What gemm_wide.hpp stores: the results of rows m .. m + 3 of W (DV_OUT_T or DV_OUT_GLU).
+template <int AFTER>
+struct WideOut {
+  static constexpr int kOuts = AFTER == DV_OUT_GLU ? 2 : 4;
+  typedef bf16_t vec_t __attribute__((ext_vector_type(kOuts)));
+  TileArgs a;
+  __device__ __forceinline__ bf16_t* base() const { return reinterpret_cast<bf16_t*>(a.out); }
+  __device__ __forceinline__ int64_t ld() const { return a.ldo; }
+  __device__ __forceinline__ int columns() const { return AFTER == DV_OUT_GLU ? a.M / 2 : a.M; }
+  __device__ __forceinline__ vec_t make(int m, float4_t v) const {
+    if constexpr (AFTER == DV_OUT_GLU) {
+      return vec_t{(bf16_t)glu_f(v[0], v[1], a.act, a.limit), (bf16_t)glu_f(v[2], v[3], a.act, a.limit)};
+    } else {
+      if (a.bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += to_f(reinterpret_cast<const bf16_t*>(a.bias)[min(m + e, a.M - 1)]);
+      }
+      return vec_t{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+    }
+  }
 };
 
 }  // namespace dv

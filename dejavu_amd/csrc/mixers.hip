@@ -16,7 +16,6 @@
 #include "mix/linear_rows.hpp"
 #include "mix/linear_split.hpp"
 #include "mix/linear_stream.hpp"
-#include "mix/linear_wide.hpp"
 #include "mix/short_conv.hpp"
 #include "mix/ssd.hpp"
 #include "mix/stream.hpp"
@@ -32,11 +31,12 @@ inline bool dtype_ok(int d) { return d == DV_BF16 || d == DV_F32; }
 inline unsigned blocks_of(int64_t work, int64_t per) { return (unsigned)((work + per - 1) / per); }
 
 // Dynamic LDS above 48 KiB is granted per kernel and device.
+// (a kernel may have a little of its own beside it)
 template <auto KERNEL>
-int grant(size_t bytes) {
+int grant(size_t bytes, size_t most = 158 * 1024) {
   static std::atomic<size_t> granted[64];
   if (bytes <= 48 * 1024) return DV_OK;
-  if (bytes > 158 * 1024) return DV_ERR_UNSUPPORTED;
+  if (bytes > most) return DV_ERR_UNSUPPORTED;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return DV_ERR_UNSUPPORTED;
   if (bytes <= granted[dev].load(std::memory_order_relaxed)) return DV_OK;
@@ -71,6 +71,23 @@ struct MixLaunch {
     return launch_lds<KERNEL>(grid, threads, lds, s, args...);
   }
 };
+
+struct WideLaunch {  // has no LDS but the dynamic one, which is all there is
+  template <auto KERNEL, typename... A>
+  int operator()(dim3 grid, dim3 threads, size_t lds, hipStream_t s, const A&... args) const {
+    const int rc = grant<KERNEL>(lds, kWideLds);
+    if (rc != DV_OK) return rc;
+    hipLaunchKernelGGL(KERNEL, grid, threads, lds, s, args...);
+    return launched();
+  }
+};
+
+template <int AFTER>
+int linear_wide(const TileArgs& a, hipStream_t s) {
+  const int nb = plan_wide(a.n, a.M, compute_units());
+  const RingOperands<bf16_t> o{reinterpret_cast<const bf16_t*>(a.x), a.ldx, reinterpret_cast<const bf16_t*>(a.W), a.ldw, a.n, a.M, a.K};
+  return gemm_wide(nb, o, WideOut<AFTER>{a}, s, WideLaunch{});
+}
 
 template <int AFTER>
 int linear_stream(const RingPlan& p, const TileArgs& a, void* workspace, hipStream_t s) {
@@ -536,13 +553,10 @@ int dv_mix_linear_split(const float* x, int64_t ldx, const float* W, int64_t ldw
 int dv_mix_linear_wide(int after, const dvTileArgs* a, void* stream) {
   const int rc = tile_args_ok(after, a);
   if (rc != DV_OK) return rc;
-  const int64_t rows = ((int64_t)a->M + kWideTile - 1) / kWideTile, cols = ((int64_t)a->n + kWideTile - 1) / kWideTile;
-  if (rows * cols > 0x7fffffff) return DV_ERR_UNSUPPORTED;
-  const dim3 grid((unsigned)(rows * cols)), threads(512);
-  if (after == DV_OUT_T)
-    return launch_lds<linear_wide_kernel<DV_OUT_T>>(grid, threads, kWideLds, st(stream), *a, (int)rows, (int)cols);
-  if (after == DV_OUT_GLU)
-    return launch_lds<linear_wide_kernel<DV_OUT_GLU>>(grid, threads, kWideLds, st(stream), *a, (int)rows, (int)cols);
+  const int64_t tiles = ((int64_t)a->M + kWideRows - 1) / kWideRows * (((int64_t)a->n + 127) / 128);
+  if (tiles > 0x7fffffff || a->ldw >= kWideMaxStride || a->ldx >= kWideMaxStride) return DV_ERR_UNSUPPORTED;
+  if (after == DV_OUT_T) return linear_wide<DV_OUT_T>(*a, st(stream));
+  if (after == DV_OUT_GLU) return linear_wide<DV_OUT_GLU>(*a, st(stream));
   return DV_ERR_UNSUPPORTED;
 }
 

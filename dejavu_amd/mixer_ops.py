@@ -3,7 +3,7 @@
 Weights and activations are bf16 or fp32 (one type per model); the residual stream, norms, scores and recurrent state
 are fp32.  All ops enqueue on ``torch.cuda.current_stream()`` and refuse CPU tensors.  Products: one row goes to the
 row kernel, up to 64 bf16 rows, and up to ``TILE_MAX_ROWS`` where it is the faster one (``_tile_rule``), to the matrix-core
-kernel that streams the weight, some portions of more than a thousand rows to the one with wide tiles (``_wide_rule``), all
+kernel that streams the weight, longer portions where they fill it to the one with wide tiles (``_wide_rule``, ``_fill_rule``), all
 with the operation that follows in the same launch; the other portions (and several fp32 rows) take the library GEMM and a
 separate elementwise launch, as the dense products of long prompts do elsewhere in this package.
 """
@@ -106,16 +106,14 @@ def residual(y: Optional[torch.Tensor], stream: ResidualStream, post, pre, add_s
     return h
 
 
-# The wide kernel and the library GEMM take about as long for a full round of 256 x 256 tiles (one on each of 256 compute units); the
-# library also has tiles 192 wide, and where they are the right ones it wins: 24576 x 4096 with 1435 rows 0.85 of its time, plain
-# 0.77; 21760 x 4096 with 1624 rows 0.82 and 0.75.  Where the wide tiles make three rounds, and those of 192 by 256 four either way, the
-# library's choice costs it more (gated unit / plain product, times its speed: 22016 x 4096 with 1603 / 1904 / 2048 rows 1.12 / 1.07,
-# 1.29 / 1.24, 1.33 / 1.27; 18560 x 4096 with 2000 1.20 / 1.15; 18944 x 5120 with 2000 1.26 / 1.16; 20480 x 4096 with 1918 1.27 / 1.20).
-# Outside of these lines it is the other way round as often as not: weights whose rows 192 divides (19200 x 4096 with 1939 rows
-# 0.89 / 0.82), taller ones (28672 x 4096 with 1365 rows 0.86 / 0.80), longer rows (22016 x 8192 with 1700 rows 1.04 / 0.98, 18560 x
-# 6144 with 1999 1.11 / 1.01), and more than 2048 rows of x, where the library ranges from 0.85 to 1.45 (17920 x 4096 with 2191 / 2520 rows 0.87 /
-# 1.41).
+# Tiles of 256 weight rows (gemm_wide.hpp) against the library GEMM, weights out of the caches (the library's time over the
+# kernel's).  The library also has tiles 192 wide; where the kernel's make three rounds of the compute units, and those of 192 by 256 four
+# either way, its choice costs it most: 22016 x 4096 with 1700 / 1999 / 2048 rows 1.24 / 1.40 / 1.42, 18560 x 4096 1.22 / 1.38 / 1.29.  Outside of
+# these lines a plain product of 4096 columns and more is ahead as often as it is behind (22016 x 4096 with 640 / 777 / 1000 / 1200 / 1435 rows 1.00 / 1.03 / 0.97 /
+# 0.93 / 1.31, 12288 x 4096 with 257 / 777 / 1200 / 1435 / 1999 rows 0.91 / 1.03 / 0.95 / 1.12 / 0.95, 8192 x 4096 0.73 / 1.08 / 1.05 / 1.04 / 0.93, 4096 x 11008 with 777 / 2048
+# rows 0.70 / 0.99).
 WIDE_MAX_ROWS = 2048
+WIDE_MAX_STRIDE = 1 << 25             # elements (the kernel counts 64 rows' bytes in 32 bits)
 WIDE_COLUMNS = 4096, 5120
 WIDE_MAX_WEIGHT_ROWS = 22528
 WIDE_TILE, NARROW_TILE, WIDE_ROUND = 256, 192, 256
@@ -133,6 +131,23 @@ def _wide_rule(n: int, M: int, K: int) -> bool:
     return WIDE_TILES[0] <= _tiles_of(n, M, WIDE_TILE, WIDE_TILE) <= WIDE_TILES[1] and narrow > 3 * WIDE_ROUND
 
 
+# Where the library's product is followed by a launch of its own for the gated unit, and for few columns, the kernel is ahead as
+# soon as its tiles fill the chip (at least so many tiles of 128 rows by 256 weight rows, by columns): gated units of 22016 x 4096 with 400 / 777 /
+# 1200 / 1435 / 1700 rows 1.03 / 1.04 / 0.98 / 1.37 / 1.29, 18560 x 4096 1.08 / 1.04 / 1.29 / 1.10 / 1.29, 12288 x 4096 with 640 / 777 / 1435 / 1999 rows 1.08 / 1.10 / 1.18 / 0.99,
+# 8192 x 4096 with 777 / 1200 / 1999 1.16 / 1.09 / 0.99, but with 512 0.85; 11264 x 2048 with 400 / 640 / 1000 / 1700 / 1999 1.15 / 1.18 / 1.22 / 1.29 / 1.08, with 300 0.97;
+# 6144 x 2048 with 777 / 1000 1.03 / 1.14, with 640 0.92.  Plain: 11264 x 2048 with 400 / 640 / 1000 / 1700 / 1999 1.10 / 0.99 / 1.12 / 1.22 / 1.00, 9216 x 2048 with 777 / 1000 /
+# 1700 / 1999 1.06 / 1.21 / 0.95 / 1.19, 4368 x 2048 with 1200 / 1700 / 2048 1.13 / 1.19 / 1.24, with 777 0.89.
+WIDE_FEW_COLUMNS, WIDE_GATED_COLUMNS = 2048, 8192
+WIDE_FILL_GATED, WIDE_FILL_FEW_GATED, WIDE_FILL_FEW = 200, 144, 176
+
+
+def _fill_rule(n: int, M: int, K: int, gated: bool) -> bool:
+    if not TILE_MAX_ROWS < n <= WIDE_MAX_ROWS or not 1024 <= K <= WIDE_GATED_COLUMNS or (K > WIDE_FEW_COLUMNS and not gated):
+        return False
+    fill = (WIDE_FILL_FEW_GATED if gated else WIDE_FILL_FEW) if K <= WIDE_FEW_COLUMNS else WIDE_FILL_GATED
+    return _tiles_of(n, M, 128, WIDE_TILE) >= fill
+
+
 def _tile_rule(n: int, M: int, K: int, gated: bool) -> bool:
     if n > TILE_MAX_ROWS:
         return False
@@ -145,9 +160,19 @@ def _aligned(x: torch.Tensor, W: torch.Tensor) -> bool:
     return all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, W)) and x.shape[1] % 8 == 0 and W.shape[0] % 2 == 0
 
 
+def _wide_fits(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
+    return (x.dtype == torch.bfloat16 and results_only(x, W, bias) and _aligned(x, W) and
+            max(x.stride(0), W.stride(0)) < WIDE_MAX_STRIDE)
+
+
 def _wide(x: torch.Tensor, W: torch.Tensor, bias=None) -> bool:
-    """Whether the wide kernel takes the product."""
-    return x.dtype == torch.bfloat16 and _wide_rule(x.shape[0], *W.shape) and results_only(x, W, bias) and _aligned(x, W)
+    """Whether the wide kernel takes the product whatever follows it."""
+    return _wide_rule(x.shape[0], *W.shape) and _wide_fits(x, W, bias)
+
+
+def _fills(x: torch.Tensor, W: torch.Tensor, bias=None, gated: bool = False) -> bool:
+    """Whether the wide kernel takes it for what follows, or for its few columns."""
+    return _fill_rule(x.shape[0], *W.shape, gated) and _wide_fits(x, W, bias)
 
 
 def _tiles(x: torch.Tensor, W: torch.Tensor, bias=None, gated: bool = False, whole: bool = True) -> bool:
@@ -299,7 +324,7 @@ def linear(x, W: torch.Tensor, bias: Optional[torch.Tensor] = None, f32: bool = 
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
         _tile_launch(L.OUT_F32 if f32 else L.OUT_T, a, x.device)
         return out
-    if not f32 and _wide(x, W, bias):
+    if not f32 and (_wide(x, W, bias) or _fills(x, W, bias)):
         out = torch.empty(n, M, dtype=out_t, device=x.device)
         a = _tile_args(x, W)
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
@@ -322,7 +347,7 @@ def gated_unit(x, W: torch.Tensor, act: int, limit: float = 0.0) -> torch.Tensor
         a = _tile_args(x, W)
         a.out, a.ldo, a.act, a.limit = y.data_ptr(), M // 2, act, limit
         _tile_launch(L.OUT_GLU, a, x.device)
-    elif _wide(x, W):
+    elif _wide(x, W) or _fills(x, W, gated=True):
         a = _tile_args(x, W)
         a.out, a.ldo, a.act, a.limit = y.data_ptr(), M // 2, act, limit
         check(lib.dv_mix_linear_wide(L.OUT_GLU, _ref(a), _stream()), "dv_mix_linear_wide")

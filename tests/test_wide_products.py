@@ -1,0 +1,155 @@
+"""gemm_wide.hpp: every width of its tiles at sizes where they end, the rule that sends products to it, and what the matrix
+instructions written in assembly rely on, seen in the assembly that the compiler makes of every form."""
+import os
+import re
+import subprocess
+
+import pytest
+import torch
+
+from dejavu_amd.build import CSRC, HIPCC_FLAGS, hipcc_path
+from test_ring_handover import registers, states_before_use
+
+# (rows, weight rows) whose tiles are 128 / 160 / 192 / 224 / 256 rows wide on 256 compute units
+SIZES = [(257, 1030), (300, 22016), (380, 32700), (777, 16380), (500, 22010)]
+WIDTHS = [128, 160, 192, 224, 256]
+SOURCE = """
+#include <stdio.h>
+#include "gemm_wide.hpp"
+template <typename T>
+struct Store {
+  T* y;
+  static constexpr int kOuts = 4;
+  typedef T vec_t __attribute__((ext_vector_type(4)));
+  __device__ T* base() const { return y; }
+  __device__ int64_t ld() const { return 4096; }
+  __device__ int columns() const { return 4090; }
+  __device__ vec_t make(int m, const dv::float4_t& v) const { return vec_t{(T)v[0], (T)v[1], (T)v[2], (T)v[3]}; }
+};
+struct Launch {
+  template <auto KERNEL, typename... A>
+  int operator()(dim3 grid, dim3 threads, size_t lds, hipStream_t s, A... args) const {
+    hipLaunchKernelGGL(KERNEL, grid, threads, lds, s, args...);
+    return 0;
+  }
+};
+int all(int nb, const dv::RingOperands<dv::half_t>& a, const dv::RingOperands<__bf16>& b) {
+  return dv::gemm_wide(nb, a, Store<dv::half_t>{}, nullptr, Launch{}) + dv::gemm_wide(nb, b, Store<__bf16>{}, nullptr, Launch{});
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    try:
+        hipcc = hipcc_path()
+    except RuntimeError as e:
+        pytest.skip(str(e))
+    where = tmp_path_factory.mktemp("wide")
+    src, out = where / "wide.hip", where / "wide.s"
+    src.write_text(SOURCE)
+    flags = [f for f in HIPCC_FLAGS if f not in ("-shared", "-fPIC")]
+    subprocess.run([hipcc, *flags, "-w", "-S", "--cuda-device-only", "-I", CSRC, "-I", os.path.join(CSRC, "..", "..", "include"),
+                    str(src), "-o", str(out)], check=True)
+    found, name = {}, None
+    for line in out.read_text().splitlines():
+        line = line.split(";")[0].strip()
+        if re.match(r"_ZN2dv16gemm_wide_kernel.*:$", line):
+            name = line[:-1]
+            found[name] = []
+        elif line.startswith(".Lfunc_end"):
+            name = None
+        elif name and line and (not line.startswith(".") or line.endswith(":")):
+            found[name].append(re.sub(r"\s+", " ", line))
+    assert len(found) == 2 * len(WIDTHS)
+    return found
+
+
+def test_matrix_instructions_in_assembly(kernels):
+    """Nothing in the hardware waits for their sums (8 states) or for operands that a vector instruction has just written (2), and
+    the compiler does not see what they are."""
+    for name, lines in kernels.items():
+        assert not any(line.startswith("scratch_") for line in lines), name
+        matrix = [i for i, line in enumerate(lines) if line.startswith("v_mfma")]
+        assert len(matrix) >= 2 * 2 * 8 * 4, name
+        uses = [states_before_use(lines, i) for i in matrix]
+        uses = [u for u in uses if u is not None]
+        assert uses and min(uses) >= 8, (name, sorted(uses)[:4])
+        for i in matrix:
+            operands = set().union(*map(registers, lines[i].split(None, 1)[1].split(", ")))
+            states = 0
+            for line in reversed(lines[:i]):
+                op = line.split()[0]
+                if states >= 2 or op.endswith(":"):
+                    break
+                if op.startswith("v_") and not op.startswith("v_mfma"):
+                    assert not registers(line.split(None, 1)[1].split(",")[0]) & operands, (name, line, lines[i])
+                states += int(line.split()[1]) + 1 if op == "s_nop" else 1
+
+
+def test_loop_keeps_its_sums_in_place(kernels):
+    """The loop over the chunks: one barrier, behind everybody's reads and the next chunk's loads, and no copies of sums."""
+    for name, lines in kernels.items():
+        width = int(re.search(r"Li(\d+)E", name)[1])
+        starts = [i for i, line in enumerate(lines) if line.endswith(":")] + [len(lines)]
+        blocks = [lines[a:b] for a, b in zip(starts, starts[1:])]
+        loop = [b for b in blocks if sum(line.startswith("v_mfma") for line in b) == width // 2 and any(line.startswith("buffer_load") for line in b)]
+        assert len(loop) == 1, name
+        assert not any(line.startswith("v_accvgpr") for line in loop[0]), name
+        at = [i for i, line in enumerate(loop[0]) if line.startswith("s_barrier")]
+        assert len(at) == 1 and re.search(r"vmcnt\(8\) lgkmcnt\(0\)", loop[0][at[0] - 1]), (name, loop[0][at[0] - 1])
+
+
+def test_which_products_the_wide_kernel_takes():
+    """Gated units and few columns on both sides of the lines; each was measured with its weights out of the caches."""
+    from dejavu_amd.mixer_ops import _fill_rule
+
+    for n, M, K in ((400, 22016, 4096), (2048, 22016, 4096), (1999, 18560, 4096), (640, 12288, 4096), (777, 8192, 4096)):
+        assert _fill_rule(n, M, K, True) and not _fill_rule(n, M, K, False), (n, M, K)
+    for n, M, K in ((400, 11264, 2048), (2048, 11264, 2048), (1000, 9216, 2048), (1200, 6144, 2048), (1999, 4368, 2048)):
+        assert _fill_rule(n, M, K, True) and _fill_rule(n, M, K, False), (n, M, K)
+    for n, M, K in ((256, 22016, 4096), (512, 8192, 4096), (1200, 4096, 4096), (300, 11264, 2048), (640, 6144, 2048), (2049, 22016, 4096),
+                    (1000, 22016, 16384)):
+        assert not _fill_rule(n, M, K, True) and not _fill_rule(n, M, K, False), (n, M, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [64, 136, 584])  # one chunk; two and a piece; nine and a piece
+@pytest.mark.parametrize("n,M", SIZES)
+def test_widths_of_the_tiles(n, M, K):
+    """Against fp32 sums; rows of the results on and off 16-byte boundaries, and nothing beside them written."""
+    from dejavu_amd import _lib_mixers as L
+    from dejavu_amd import mixer_ops as ops
+
+    g = torch.Generator(device="cuda").manual_seed(n + K)
+    x = torch.randn(n, K + 16, generator=g, device="cuda").to(torch.bfloat16)[:, 8:8 + K]
+    W = (torch.randn(M, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    bias = torch.randn(M, generator=g, device="cuda").to(torch.bfloat16)
+    prod = x.double() @ W.double().t()
+    for after, want in ((L.OUT_T, prod + bias.double()), (L.OUT_GLU, prod[:, 0::2].clamp(min=0) * prod[:, 1::2])):
+        for pad in (8 - want.shape[1] % 8, 3):
+            out = torch.full((n, want.shape[1] + pad), 77.0, dtype=torch.bfloat16, device="cuda")
+            a = ops._tile_args(x, W)
+            a.out, a.ldo, a.act = out.data_ptr(), out.shape[1], L.GLU_RELU
+            a.bias = bias.data_ptr() if after == L.OUT_T else None
+            ops.check(ops.lib.dv_mix_linear_wide(after, ops._ref(a), ops._stream()), "dv_mix_linear_wide")
+            assert (out[:, want.shape[1]:] == 77.0).all()
+            got = out[:, :want.shape[1]].double()
+            # one rounding to bf16, 2 ** -9 at most, and fp32 sums of values of unit size
+            assert ((got - want).abs() <= want.abs() * 2.0 ** -8 + 1e-5 * K ** 0.5).all(), (after, pad)
+
+
+@pytest.mark.gpu
+def test_gated_units_through_the_ops():
+    """A product on each side of the rule's line (144 tiles), both with the same result."""
+    from dejavu_amd import mixer_ops as ops
+
+    g = torch.Generator(device="cuda").manual_seed(1)
+    W = (torch.randn(9200, 2048, generator=g, device="cuda") / 45).to(torch.bfloat16)
+    x = torch.randn(385, 2048, generator=g, device="cuda").to(torch.bfloat16)
+    assert ops._fills(x, W, gated=True) and not ops._fills(x[:384], W, gated=True) and not ops._wide(x, W)
+    for rows in (384, 385):
+        want = x[:rows].float() @ W.float().t()
+        unit = want[:, 0::2].clamp(min=0) * want[:, 1::2]
+        got = ops.relu_glu(x[:rows], W).float()
+        assert (got - unit).norm() / unit.norm() < 1e-2
