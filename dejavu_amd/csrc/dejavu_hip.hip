@@ -22,6 +22,7 @@
 #include "norm.hpp"
 #include "prefill.hpp"
 #include "qkv_mfma.hpp"
+#include "qkv_window.hpp"
 #include "topk.hpp"
 
 using namespace dv;
@@ -551,10 +552,26 @@ int gemm_big(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const h
   }
 }
 
+// Windows of more than 64 rows take the rows that are live (qkv_window.hpp); up to there the weights' stream is the time whatever the rows.
+bool window_live(int tokens, int rows) { return tokens > 1 && rows > 64; }
+
 // QKV of the selected heads for B rows (see QkvScatter): M = 3 * Hk * hd output rows
 int gemm_tiled_qkv(const half_t* X, int64_t ldx, const half_t* W, const half_t* bias, int B, int d, half_t* Y,
                    const QkvScatter& qs, void* workspace, size_t workspace_bytes, hipStream_t s) {
   const int M = 3 * qs.Hk * qs.hd, Z = 3 * qs.H * qs.hd;
+  if (window_live(qs.tokens, B)) {
+    const WindowPlan p = plan_window(B, M, d, compute_units());
+    if (p.splits > 1 && (workspace == nullptr || !aligned16(workspace) || workspace_bytes < p.workspace_bytes())) return DV_ERR_WORKSPACE;
+    const RingOperands<half_t> a{X, ldx, W, (int64_t)d, B, M, d};
+    float4_t* part = reinterpret_cast<float4_t*>(workspace);
+    const dim3 threads(512);
+    const RingLaunch launch;
+    const int rc = launch.template operator()<qkv_window_live_kernel>(dim3(p.rows, p.chunks, p.splits), threads, kWindowLds, s, a, QkvRows{qs},
+                                                                      QkvOut{bias, Y, qs}, part);
+    if (rc != DV_OK || p.splits == 1) return rc;
+    return launch.template operator()<qkv_window_sum_kernel>(dim3(p.rows, p.chunks, kWindowRows * kWindowCols / 4 / 512), threads, 0, s,
+                                                             QkvRows{qs}, QkvOut{bias, Y, qs}, M, (const float4_t*)part, p.splits);
+  }
   if (shared_kernel(B, d, M, true) == Shared::kRing) {
     const RingPlan p = plan_ring(B, M, d, compute_units());
     if (int rc = ring_scratch(p, workspace, workspace_bytes); rc != DV_OK) return rc;
@@ -1737,6 +1754,7 @@ size_t dv_out_proj_sparse_t_ln_workspace_bytes(int B, int nnz, int hd, int N) {
 
 size_t dv_qkv_window_batch_workspace_bytes(int tokens, int nseq, int d, int nnz, int hd) {
   if (tokens < 1 || tokens > 16 || nseq < 1 || nseq > 32 || d <= 0 || nnz <= 0 || hd <= 0) return 0;
+  if (window_live(tokens, tokens * nseq)) return plan_window(tokens * nseq, 3 * nnz * hd, d, compute_units()).workspace_bytes();
   return tiled_workspace_bytes(tokens * nseq, d, 3 * nnz * hd, true);
 }
 

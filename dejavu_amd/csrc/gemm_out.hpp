@@ -66,6 +66,7 @@ __device__ __forceinline__ void qkv_store4(const QkvScatter& q, half_t* __restri
 
 struct QkvRows {  // (a head out of range reads row 0 and is not stored)
   static constexpr bool kPastCaches = false;
+  static constexpr int kMostCols = 64;  // (qkv_window.hpp takes more)
   QkvScatter q;
   __device__ __forceinline__ int64_t operator()(int m) const {
     const int t = m / (q.Hk * q.hd), rem = m - t * q.Hk * q.hd, i = rem / q.hd, h = q.head_idx[i];
@@ -120,6 +121,7 @@ struct PlainOut {
 
 struct GatheredRows {
   static constexpr bool kPastCaches = true;
+  static constexpr int kMostCols = 64;
   const void* idx;
   int idx_bytes, Z;
   __device__ __forceinline__ int64_t operator()(int m) const {  // an index out of range reads row 0; its result is act(0)

@@ -45,6 +45,7 @@ struct RingOperands {
 // Rows 0 .. M - 1 of the weight.
 struct PlainRows {
   static constexpr bool kPastCaches = true;
+  static constexpr int kMostCols = 256;  // the widest tile that is launched for them
   __device__ __forceinline__ int64_t operator()(int m) const { return m; }
 };
 
@@ -107,12 +108,12 @@ inline RingPlan plan_ring(int n, int M, int K, int units) {
 // 20480 x 5120 and its like, of a prompt's layer: 235 us the layer, 223), but a small weight (17 rows by 1024 x 5120: 7.2, 7.7
 // us) and the chosen heads' rows of a block (192 rows a tile, 128 of X, 9216 columns: 39.2, 40.7) stay in the last cache from
 // one call to the next.  These rows also gain nothing by beginning at different columns (kPastCaches of the rows).
-// Out: called with (m, n, sums of rows m .. m + 3 and row n of X), m % 4 == 0, m < M, n < the operands' n.
-// Grid: (tiles of W, tiles of X, splits of K).  part: with several splits, the sums [split][tile][value][thread].
-template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, typename Rows, typename Out,
-          bool ROUND = MB != 64 && NB <= 128>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T> a, Rows rows, Out out, float4_t* __restrict__ part) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char slots[];
+// One tile: rows of W from m0 on, columns n0 .. of the n that `cols` makes rows of X of.  Splits of K: blockIdx.z of gridDim.z.
+// Out: called with (m, row of X, sums of rows m .. m + 3), m % 4 == 0, m < M.
+// part: with several splits, this tile's sums [value][thread] of this split.
+template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, bool ROUND, typename Rows, typename Cols, typename Out>
+__device__ __forceinline__ void ring_tile(const RingOperands<T>& a, const Rows& rows, const Cols& cols, const Out& out, int m0, int n0, int n_cols,
+                                          float4_t* __restrict__ part, unsigned char* slots) {
   constexpr int WAVES = WM * WN, THREADS = WAVES * 64;
   constexpr int CH = KC / 8;               // 16-byte pieces of a row's chunk
   constexpr int RPL = 64 / CH;             // rows per load of a wave
@@ -123,7 +124,6 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T>
   static_assert((MB + NB) % (RPL * WAVES) == 0 && MB % RPL == 0, "loads do not tile");
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave % WM, wn = wave / WM, l16 = lane & 15, g = lane >> 4;
-  const int m0 = blockIdx.x * MB, n0 = blockIdx.y * NB;
   const int nch = (a.K + KC - 1) / KC;
   const int c0 = nch * blockIdx.z / gridDim.z, len = nch * (blockIdx.z + 1) / gridDim.z - c0;
   // ROUND: the columns are taken in parts, and workgroups begin with different ones and go round: all of them at the same
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T>
   for (int i = 0; i < LI; ++i) {
     const int row = (wave * LI + i) * RPL + lane / CH;
     piece[i] = (lane % CH) ^ (row & SWAP);
-    src[i] = row < MB ? a.W + rows(min(m0 + row, a.M - 1)) * a.ldw : a.X + (int64_t)min(n0 + row - MB, a.n - 1) * a.ldx;
+    src[i] = row < MB ? a.W + rows(min(m0 + row, a.M - 1)) * a.ldw : a.X + (int64_t)cols(min(n0 + row - MB, n_cols - 1)) * a.ldx;
   }
   const int pieces = a.K / 8;
   auto load = [&](int at, int slot) {
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T>
 #pragma unroll
       for (int j = 0; j < NT; ++j) sums[0][i][j] += sums[k][i][j];
   if (gridDim.z > 1) {
-    float4_t* p = part + (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (MB * NB / 4) + threadIdx.x;
+    float4_t* p = part + threadIdx.x;
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
@@ -262,10 +262,24 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T>
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         const int m = m0 + (wm * RT + i) * 16 + g * 4, n = n0 + (wn * NT + j) * 16 + l16;
-        if (m < a.M && n < a.n) out(m, n, sums[0][i][j]);
+        if (m < a.M && n < n_cols) out(m, cols(n), sums[0][i][j]);
       }
   }
   wait_loads<0>();  // no load into LDS outlives the workgroup
+}
+
+struct PlainCols {
+  __device__ __forceinline__ int operator()(int n) const { return n; }
+};
+
+// Grid: (tiles of W, tiles of X, splits of K).  part: with several splits, the sums [split][tile][value][thread].
+template <typename T, int MB, int NB, int KC, int ST, int WM, int WN, bool NT_W, typename Rows, typename Out,
+          bool ROUND = MB != 64 && NB <= 128>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_ring_kernel(RingOperands<T> a, Rows rows, Out out, float4_t* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char slots[];
+  ring_tile<T, MB, NB, KC, ST, WM, WN, NT_W, ROUND>(
+      a, rows, PlainCols{}, out, blockIdx.x * MB, blockIdx.y * NB, a.n,
+      part + (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (MB * NB / 4), slots);
 }
 
 // Adds the splits' sums up, in their order.  Grid: (tiles of W, tiles of X, values of a thread).
@@ -308,12 +322,15 @@ int gemm_ring(const RingPlan& p, const RingOperands<T>& a, const Rows& rows, con
     case 32: return p.mb == 128 ? DV_RING(128, 32, 64, 4, 4, 1, kPast, true) : DV_RING(64, 32, 64, 4, 4, 1, false, false);
     case 64: return p.mb == 128 ? DV_RING(128, 64, 64, 4, 4, 2, kPast, true)
                     : p.mb == 96 ? DV_RING(96, 64, 64, 4, 2, 2, kPast, true) : DV_RING(64, 64, 64, 4, 2, 2, false, false);
+  }
+  if constexpr (Rows::kMostCols > 64) switch (p.nb) {
     case 128: return p.mb == 64 ? DV_RING(64, 128, 64, 3, 2, 4, false, false)
                      : p.mb == 128 ? DV_RING(128, 128, 64, 4, 2, 4, kPast, kPast) : DV_RING(192, 128, 64, 3, 2, 4, kPast, kPast);
     case 192: return p.mb == 64 ? DV_RING(64, 192, 64, 4, 2, 4, false, false)
                      : p.mb == 128 ? DV_RING(128, 192, 64, 3, 2, 4, false, false) : DV_RING(192, 192, 64, 3, 2, 4, false, false);
     default: return p.mb == 64 ? DV_RING(64, 256, 64, 3, 2, 4, false, false) : DV_RING(128, 256, 64, 3, 2, 4, false, false);
   }
+  return -2;  // DV_ERR_UNSUPPORTED
 #undef DV_RING
 }
 
