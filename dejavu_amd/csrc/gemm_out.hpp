@@ -2,6 +2,7 @@
 // the q, k, v rows of selected heads with their scatter into the caches.
 #pragma once
 #include "common.hpp"
+#include "gemm_wide.hpp"
 
 namespace dv {
 
@@ -116,6 +117,32 @@ struct PlainOut {
 #pragma unroll
     for (int e = 0; e < 4; ++e) val[e] = v[e] + (bias != nullptr ? (float)bias[m + e < M ? m + e : M - 1] : 0.f);
     store_rows4(Y, ldy, M, m, n, val, act);
+  }
+};
+
+// The same as gemm_wide.hpp stores it, for the activations that are cheap enough to stand there once for every sum.
+template <int ACT>
+struct WidePlainOut {
+  static constexpr int kOuts = 4;
+  static_assert(ACT == 0 || ACT == 1 || ACT == 4, "identity, ReLU, squared ReLU");
+  const half_t* bias;
+  half_t* Y;
+  int64_t ldy;
+  int M;
+  __device__ __forceinline__ half_t* base() const { return Y; }
+  __device__ __forceinline__ int64_t ld() const { return ldy; }
+  __device__ __forceinline__ int columns() const { return M; }
+  struct Row : WideBias<half_t> {};
+  __device__ __forceinline__ Row row(int m) const {
+    Row r;
+    r.load(bias, M, m);
+    return r;
+  }
+  __device__ __forceinline__ half4_t make(const Row& r, const float4_t& v) const {
+    half4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (half_t)act_f(v[e] + (float)r.v[e], ACT);
+    return o;
   }
 };
 

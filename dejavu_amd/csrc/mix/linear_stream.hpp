@@ -63,16 +63,17 @@ struct WideOut {
   __device__ __forceinline__ bf16_t* base() const { return reinterpret_cast<bf16_t*>(a.out); }
   __device__ __forceinline__ int64_t ld() const { return a.ldo; }
   __device__ __forceinline__ int columns() const { return AFTER == DV_OUT_GLU ? a.M / 2 : a.M; }
-  __device__ __forceinline__ vec_t make(int m, float4_t v) const {
-    if constexpr (AFTER == DV_OUT_GLU) {
+  struct Row : WideBias<bf16_t> {};
+  __device__ __forceinline__ Row row(int m) const {
+    Row r;
+    r.load(AFTER == DV_OUT_GLU ? nullptr : reinterpret_cast<const bf16_t*>(a.bias), a.M, m);
+    return r;
+  }
+  __device__ __forceinline__ vec_t make(const Row& r, const float4_t& v) const {
+    if constexpr (AFTER == DV_OUT_GLU)
       return vec_t{(bf16_t)glu_f(v[0], v[1], a.act, a.limit), (bf16_t)glu_f(v[2], v[3], a.act, a.limit)};
-    } else {
-      if (a.bias) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += to_f(reinterpret_cast<const bf16_t*>(a.bias)[min(m + e, a.M - 1)]);
-      }
-      return vec_t{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
-    }
+    else
+      return vec_t{(bf16_t)(v[0] + to_f(r.v[0])), (bf16_t)(v[1] + to_f(r.v[1])), (bf16_t)(v[2] + to_f(r.v[2])), (bf16_t)(v[3] + to_f(r.v[3]))};
   }
 };
 

@@ -58,6 +58,15 @@ HIP_PROMPT_LONG_MAX_ROWS = 512
 HIP_PROMPT_LONG_ROWS = 256, 384
 HIP_PROMPT_LONG_WEIGHT = 1 << 23
 HIP_PROMPT_LONG_WEIGHT_ROWS = 4096, 8192
+# From 257 rows on the kernel of wide tiles (gemm_wide.hpp) takes fc1 with its activation, for which the library needs a launch more, where its tiles
+# of 128 rows by 256 weight rows are so many (below 4096 columns / from there on; the library's time over the kernel's: 8192 x 2048 with 400 / 600 /
+# 777 / 1200 / 2000 rows 1.07 / 1.18 / 1.36 / 1.28 / 1.11, 16384 x 4096 1.16 / 1.14 / 1.16 / 1.10 / 1.00, 20480 x 5120 with 400 / 600 / 777 / 1000 / 1435 / 2000 rows 1.02 / 1.27 /
+# 1.06 / 0.91 / 1.08 / 1.41; with 257 rows 0.98 to 1.01), and fc2 whose rows are the longest (5120 x 20480 with 777 / 1000 / 1200 / 1700 / 2000 rows 1.04 / 1.06 /
+# 1.17 / 1.66 / 0.96, 9216 x 36864 0.98 / 1.02 / 1.49 with 777 / 1200 / 2000, but 4096 x 16384 with 1200 0.90).
+HIP_PROMPT_WIDE_ROWS = 257, 2048
+HIP_PROMPT_WIDE_COLUMNS, HIP_PROMPT_WIDE_FILL = (2048, 4096), (128, 256)
+HIP_PROMPT_WIDE_LONG = 768, 20480      # rows, columns
+HIP_PROMPT_WIDE_STRIDE = 1 << 25
 # The package's causal-attention kernel (cache fill in the same launch) is ahead of the library's attention with the
 # permuted cache copies (40 heads of 128 and 128 / 1024 tokens: 7.5 / 47 us against 25 / 100; 32 heads and
 # 777 / 2000 / 4000 tokens: 30 / 110 / 385 against 75 / 310 / 566; 16 sequences of 1024: 547 against 768).  Prompts of more than so
@@ -280,29 +289,54 @@ def _long_rule(rows: int, M: int, K: int) -> bool:
     return rows <= few or (M >= low and (rows <= more or (rows <= HIP_PROMPT_LONG_MAX_ROWS and M <= high)))
 
 
-def _long_product(linear, x: torch.Tensor) -> bool:
-    """Whether ``dense_linear`` is the faster one for more than ``HIP_PROMPT_MAX_ROWS`` rows and does what ``linear(x)`` would:
-    a layer that is nothing but its weight and bias, operands that the kernel takes where they are, only results asked for."""
+def _wide_rule(rows: int, M: int, K: int, activation: str) -> bool:
+    if not HIP_PROMPT_WIDE_ROWS[0] <= rows <= HIP_PROMPT_WIDE_ROWS[1] or activation not in ("id", "relu", "squared_relu"):
+        return False
+    if activation == "id":
+        return K >= 4 * M and K >= HIP_PROMPT_WIDE_LONG[1] and rows >= HIP_PROMPT_WIDE_LONG[0]
+    few = K < HIP_PROMPT_WIDE_COLUMNS[1]
+    return K >= HIP_PROMPT_WIDE_COLUMNS[0] and -(-M // 256) * -(-rows // 128) >= HIP_PROMPT_WIDE_FILL[0 if few else 1]
+
+
+def _plain_layer(linear, x: torch.Tensor) -> bool:
+    """Whether a kernel does what ``linear(x)`` would: a layer that is nothing but its weight and bias, operands that the kernel
+    takes where they are, only results asked for."""
     W, b = linear.weight, linear.bias
-    return (type(linear) is nn.Linear and W.dim() == 2 and _long_rule(x.numel() // x.shape[-1], *W.shape) and
-            x.shape[-1] == W.shape[1] and
+    return (type(linear) is nn.Linear and W.dim() == 2 and x.shape[-1] == W.shape[1] and
             "forward" not in linear.__dict__ and not (linear._forward_hooks or linear._forward_pre_hooks) and
             not (nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks) and
             results_only(x, W, b) and W.stride(1) == 1 and W.stride(0) % 8 == 0 and W.data_ptr() % 16 == 0 and
             x.data_ptr() % 16 == 0 and (b is None or (b.dtype == W.dtype and b.shape == W.shape[:1])))
 
 
+def _long_product(linear, x: torch.Tensor) -> bool:
+    """Whether ``dense_linear`` is the faster one for more than ``HIP_PROMPT_MAX_ROWS`` rows and does what ``linear(x)`` would."""
+    W = linear.weight
+    return W.dim() == 2 and _long_rule(x.numel() // x.shape[-1], *W.shape) and _plain_layer(linear, x)
+
+
+def _wide_product(linear, x: torch.Tensor, activation: str) -> bool:
+    """The same of ``dense_linear_wide``."""
+    W, b = linear.weight, linear.bias
+    return (W.dim() == 2 and _wide_rule(x.numel() // x.shape[-1], *W.shape, activation) and x.is_contiguous() and
+            W.stride(0) < HIP_PROMPT_WIDE_STRIDE and (b is None or b.is_contiguous()) and _plain_layer(linear, x))
+
+
 def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") -> torch.Tensor:
     """``activation(linear(x))``.  The rows of a decode step (x: (B, 1, d) with B <= 64, fp16, on the GPU)
     always go to this package's row kernels (vector ALUs for one or two rows, matrix cores above).  The
     rows of a prompt go to the matrix-core kernels that stream the weight while it is the bound (``USE_HIP_PROMPT``, up
-    to ``HIP_PROMPT_MAX_ROWS`` rows, and more of them for long-rowed weights: ``_long_product``), else to the library GEMM."""
+    to ``HIP_PROMPT_MAX_ROWS`` rows, and more of them for long-rowed weights: ``_long_product``), with an activation or the longest
+    rows to the one with wide tiles (``_wide_product``), else to the library GEMM."""
     on_hip = x.is_cuda and x.dtype == torch.float16 and linear.weight.dtype == torch.float16 and x.shape[-1] % 8 == 0
     if on_hip and x.dim() == 3 and x.shape[1] == 1 and x.shape[0] <= 64:
         return ops.dense_decode_linear(x, linear.weight, linear.bias, activation)
-    rows = x.numel() // x.shape[-1] if on_hip and USE_HIP_PROMPT else HIP_PROMPT_LONG_MAX_ROWS + 1
-    if rows <= HIP_PROMPT_MAX_ROWS or (rows <= HIP_PROMPT_LONG_MAX_ROWS and _long_product(linear, x)):
-        return ops.dense_linear(x, linear.weight, linear.bias, activation)
+    if on_hip and USE_HIP_PROMPT:
+        rows = x.numel() // x.shape[-1]
+        if rows <= HIP_PROMPT_MAX_ROWS or (rows <= HIP_PROMPT_LONG_MAX_ROWS and _long_product(linear, x)):
+            return ops.dense_linear(x, linear.weight, linear.bias, activation)
+        if _wide_product(linear, x, activation):
+            return ops.dense_linear_wide(x, linear.weight, linear.bias, activation)
     y = linear(x)
     if activation == "relu":
         return F.relu(y)

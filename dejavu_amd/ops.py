@@ -270,6 +270,21 @@ def dense_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     return out.view(*lead, M) if out.is_contiguous() else out
 
 
+def dense_linear_wide(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                      activation: str = "id") -> torch.Tensor:
+    """``dense_linear`` on tiles of 256 weight rows, whatever the sizes; activation: id, relu or squared_relu.  x (..., N) whose rows
+    are contiguous and 16-byte aligned, as are those of weight (M, N); bias (M,) or None."""
+    _require_device(x, weight, bias)
+    M, N = weight.shape
+    x2 = x.reshape(-1, N)
+    assert x2.dtype == weight.dtype == torch.float16 and x2.stride(1) == 1 and weight.stride(1) == 1
+    assert bias is None or (bias.shape == (M,) and bias.dtype == x.dtype and bias.is_contiguous())
+    out = torch.empty(x2.shape[0], M, device=x.device, dtype=x.dtype)
+    check(lib.dv_dense_linear_wide_f16(_ptr(x2), x2.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), x2.shape[0], N, M,
+                                       _ACT[activation], _ptr(out), M, _stream()), "dv_dense_linear_wide_f16")
+    return out.view(*x.shape[:-1], M)
+
+
 def dense_decode_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                         activation: str = "id") -> torch.Tensor:
     """``activation(F.linear(x, weight, bias))`` for the few rows of a decode step (1..64), streamed

@@ -146,6 +146,13 @@ DV_API int dv_dense_linear_f16(const void* x, int64_t ldx, const void* W, int64_
                                size_t workspace_bytes, void* stream);
 
 /*
+ * The same product on tiles of 256 weight rows (long prompts, where the operations bound it); act: identity, ReLU or squared
+ * ReLU, others DV_ERR_UNSUPPORTED, as are row strides from 2^25 elements on.  No workspace.
+ */
+DV_API int dv_dense_linear_wide_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, int rows, int N,
+                                    int M, int act, void* y, int64_t ldy, void* stream);
+
+/*
  * y = x . W[idx] + bias.  Replaces gather_transposed_gemv,
  * Dejavu/src/ops/triton/gather_gemv.py:572-644 (deterministic: fixed-order
  * split over row groups instead of floating-point atomics).

@@ -24,7 +24,9 @@ struct Store {
   __device__ T* base() const { return y; }
   __device__ int64_t ld() const { return 4096; }
   __device__ int columns() const { return 4090; }
-  __device__ vec_t make(int m, const dv::float4_t& v) const { return vec_t{(T)v[0], (T)v[1], (T)v[2], (T)v[3]}; }
+  struct Row {};
+  __device__ Row row(int m) const { return {}; }
+  __device__ vec_t make(const Row&, const dv::float4_t& v) const { return vec_t{(T)v[0], (T)v[1], (T)v[2], (T)v[3]}; }
 };
 struct Launch {
   template <auto KERNEL, typename... A>
@@ -153,3 +155,57 @@ def test_gated_units_through_the_ops():
         unit = want[:, 0::2].clamp(min=0) * want[:, 1::2]
         got = ops.relu_glu(x[:rows], W).float()
         assert (got - unit).norm() / unit.norm() < 1e-2
+
+
+def test_which_products_of_a_prompt_the_wide_kernel_takes():
+    from dejavu_amd.modules import _wide_rule as rule
+
+    for rows, M, K in ((400, 8192, 2048), (777, 16384, 4096), (512, 20480, 5120), (2000, 16384, 4096)):
+        assert rule(rows, M, K, "relu") and rule(rows, M, K, "squared_relu") and not rule(rows, M, K, "id") and not rule(rows, M, K, "gelu")
+    for rows, M, K in ((256, 16384, 4096), (300, 16384, 4096), (257, 8192, 2048), (2049, 16384, 4096), (777, 3072, 768)):
+        assert not rule(rows, M, K, "relu"), (rows, M, K)
+    assert rule(777, 5120, 20480, "id") and not rule(767, 5120, 20480, "id") and not rule(1200, 4096, 16384, "id")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["id", "relu", "squared_relu"])
+@pytest.mark.parametrize("n,M,K", [(257, 1030, 136), (300, 1001, 72), (777, 520, 584)])
+def test_wide_products_in_fp16(n, M, K, act):
+    """Rows of results on and off 16-byte boundaries, the bias past the end of a tile."""
+    from dejavu_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(n, K, generator=g, device="cuda").half()
+    W = (torch.randn(M, K, generator=g, device="cuda") * K ** -0.5).half()
+    bias = torch.randn(M, generator=g, device="cuda").half()
+    for b in (bias, None):
+        want = x.double() @ W.double().t() + (0 if b is None else b.double())
+        want = {"id": lambda t: t, "relu": lambda t: t.clamp(min=0), "squared_relu": lambda t: t.clamp(min=0) ** 2}[act](want)
+        got = ops.dense_linear_wide(x, W, b, act).double()
+        # one rounding to fp16, 2 ** -11 at most, and fp32 sums of values of unit size
+        assert ((got - want).abs() <= want.abs() * 2.0 ** -10 + 1e-5 * K ** 0.5).all()
+
+
+@pytest.mark.gpu
+def test_long_prompts_through_the_layers():
+    """fc1 with its activation on both sides of the rule's line, and what only the library does."""
+    from dejavu_amd import modules
+
+    layer = torch.nn.Linear(2048, 8192, device="cuda", dtype=torch.float16)
+    x = torch.randn(1, 400, 2048, device="cuda").half()
+    with torch.no_grad():
+        for rows in (384, 385, 400):
+            assert modules._wide_product(layer, x[:, :rows], "relu") == (rows > 384)
+            want = torch.relu(layer(x[:, :rows]))
+            got = modules.decode_linear(layer, x[:, :rows], "relu")
+            assert got.shape == want.shape and (got - want).abs().max() <= 2.0 ** -9 * want.abs().max()
+        assert not modules._wide_product(layer, x[:, ::2].expand(1, 200, 2048), "relu")
+        seen = []
+        hook = layer.register_forward_hook(lambda *a: seen.append(1))
+        assert not modules._wide_product(layer, x, "relu")
+        modules.decode_linear(layer, x, "relu")
+        hook.remove()
+        assert seen == [1] and modules._wide_product(layer, x, "relu")
+    assert not modules._wide_product(layer, x, "relu")  # gradients
+    modules.decode_linear(layer, x, "relu").sum().backward()
+    assert layer.weight.grad is not None
