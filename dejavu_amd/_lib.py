@@ -123,6 +123,7 @@ SIGNATURES = {
                  _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr]),
     "dv_window_step_f16": (
         _c_int, [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr]),
+    "dv_window_reset": (_c_int, [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr]),
     "dv_kv_append_f16": (
         _c_int,
         [_c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int,

@@ -367,6 +367,13 @@ __global__ __launch_bounds__(256) void window_step_kernel(
   window_tracker_step(tracker, head_idx, nnz, H, counter, flush, batch_idx);
 }
 
+// A new window: every head has every token still to compute, and the window's place in the caches.
+__global__ __launch_bounds__(256) void window_reset_kernel(int* __restrict__ tracker, int slots, int* __restrict__ cache_offset, int value) {
+  const int o = blockIdx.x * 256 + threadIdx.x;
+  if (o < slots) tracker[o] = o & 15;
+  if (o == 0 && cache_offset != nullptr) *cache_offset = value;
+}
+
 // add + LayerNorm of `rows` rows (one workgroup each; a second copy of the normalised rows goes to
 // the window buffer's row of this step) and, in one more workgroup, the tracker step of the same
 // window position: add_layer_norm_kernel and window_step_kernel in one launch.

@@ -1469,6 +1469,13 @@ int dv_window_step_f16(const void* x, void* x_cache, int d, void* tracker, const
   return launch_status();
 }
 
+int dv_window_reset(void* tracker, int H, void* cache_offset, int value, void* stream) {
+  if (!tracker || H <= 0 || H > (1 << 26)) return DV_ERR_INVALID_ARG;
+  hipLaunchKernelGGL(window_reset_kernel, dim3((H * 16 + 255) / 256), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                     reinterpret_cast<int*>(tracker), H * 16, reinterpret_cast<int*>(cache_offset), value);
+  return launch_status();
+}
+
 int dv_kv_append_f16(const void* k, const void* v, int64_t ld_src, void* k_cache, void* v_cache,
                      const void* head_idx, int nheads, const void* lengths, int pos, int B, int H,
                      int hd, int S, void* stream) {

@@ -313,6 +313,12 @@ DV_API int dv_window_step_f16(const void* x, void* x_cache, int d, void* tracker
                               void* batch_idx, void* stream);
 
 /*
+ * A new back-fill window, as a prompt begins one: tracker (H, 16) int32 says that every head has all of its tokens to compute
+ * (ParallelTracker.reset, mha_dejavu.py:1124-1149), and cache_offset (int32[1], may be NULL) where it lies in the caches.
+ */
+DV_API int dv_window_reset(void* tracker, int H, void* cache_offset, int value, void* stream);
+
+/*
  * Writes the newest token's k, v at position pos (or lengths[b]) of the caches,
  * for all heads (head_idx NULL) or the listed ones.  This is the cache update
  * that ft_attention.single_query_attention performs internally (call sites

@@ -209,3 +209,16 @@ def test_long_prompts_through_the_layers():
     assert not modules._wide_product(layer, x, "relu")  # gradients
     modules.decode_linear(layer, x, "relu").sum().backward()
     assert layer.weight.grad is not None
+
+
+@pytest.mark.gpu
+def test_window_reset():
+    from dejavu_amd._lib import check, lib
+
+    for heads in (1, 17, 40):
+        tracker = torch.full((heads + 1, 16), -7, dtype=torch.int32, device="cuda")
+        place = torch.full((2,), -7, dtype=torch.int32, device="cuda")
+        check(lib.dv_window_reset(tracker.data_ptr(), heads, place.data_ptr(), 123, torch.cuda.current_stream().cuda_stream), "dv_window_reset")
+        assert torch.equal(tracker[:heads], torch.arange(16, device="cuda", dtype=torch.int32).repeat(heads, 1))
+        assert (tracker[heads] == -7).all() and place.tolist() == [123, -7]
+    assert lib.dv_window_reset(None, 4, None, 0, None) == -1
