@@ -40,7 +40,9 @@ TileArgs = _struct("TileArgs", ("x", _p), ("ldx", _l), ("W", _p), ("ldw", _l), (
 ConvGroup = _struct("ConvGroup", ("heads", _i), ("stride", _i), ("dim", _i), ("norm", _i), ("eps", _f), ("scale", _f),
                     ("out", _p), ("ld", _l))
 ConvArgs = _struct("ConvArgs", ("in_", _p), ("ldi", _l), ("n", _i), ("taps", _i), ("silu", _i), ("w", _p),
-                   ("b", _p), ("state", _p), ("g", ConvGroup * 3))
+                   ("b", _p), ("state", _p), ("g", ConvGroup * 3), ("next_state", _p))
+RmsRows = _struct("RmsRows", ("x", _p), ("dim", _i), ("padded", _i), ("w", _p), ("y", _p), ("ldy", _l))
+RingRows = _struct("RingRows", ("buf", _p), ("ldb", _l), ("ring", _p), ("ldr", _l), ("width", _i))
 HeadGroup = _struct("HeadGroup", ("heads", _i), ("stride", _i), ("dim", _i), ("w", _p), ("eps", _f), ("other", _p),
                     ("ldo", _l), ("lambda", _p), ("out", _p), ("ld", _l))
 HeadArgs = _struct("HeadArgs", ("in_", _p), ("ldi", _l), ("n", _i), ("g", HeadGroup * 3))
@@ -78,6 +80,7 @@ SIGNATURES = {
     "dv_mix_head_rows": (_i, [_i, _P(HeadArgs), _p]),
     "dv_mix_gated_group_norm": (_i, [_i, _p, _l, _p, _l, _l, _i, _i, _i, _p, _f, _p, _p]),
     "dv_mix_rms_rows": (_i, [_i, _p, _l, _l, _i, _i, _p, _f, _p, _l, _p]),
+    "dv_mix_rms_rows_two": (_i, [_i, _P(RmsRows), _P(RmsRows), _l, _l, _f, _p]),
     "dv_mix_gated_head_norm": (_i, [_i, _p, _p, _l, _l, _i, _i, _i, _p, _f, _p, _p]),
     "dv_mix_linear_row": (_i, [_i, _i, _i, _P(RowArgs), _p]),
     "dv_mix_linear_tiles": (_i, [_i, _P(TileArgs), _p]),
@@ -89,6 +92,7 @@ SIGNATURES = {
     "dv_mix_short_conv": (_i, [_i, _i, _P(ConvArgs), _p]),
     "dv_mix_conv_state": (_i, [_i, _p, _l, _i, _i, _i, _p, _p]),
     "dv_mix_ring_copy": (_i, [_i, _p, _l, _p, _i, _l, _i, _i, _i, _i, _p]),
+    "dv_mix_ring_copy_two": (_i, [_i, _P(RingRows), _P(RingRows), _i, _i, _i, _i, _p]),
     "dv_mix_attn_rows": (_i, [_i, _i, _P(AttnArgs), _p]),
     "dv_mix_attn_tiles": (_i, [_P(AttnArgs), _i, _p]),
     "dv_mix_attn_tiles_f32": (_i, [_P(AttnArgs), _i, _p]),

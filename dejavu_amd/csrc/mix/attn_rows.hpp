@@ -490,12 +490,24 @@ __global__ __launch_bounds__(256) void latent_out_kernel(AttnArgs a, const T* __
   }
 }
 
-// Copies rows of keys or values between a portion's buffer and a ring: dst row of token j is slot(j).
+// Copies rows of keys or values between a portion's buffers and their rings: dst row of token j is slot(j).
 //   to_ring : ring[(first + i) % cap] <- buf[at + i]       from ring: buf[at + i] <- ring[(first + i) % cap]
+// Grid: (.., keys and values).
 template <typename T>
-__global__ __launch_bounds__(256) void ring_copy_kernel(T* __restrict__ buf, int64_t ldb, T* __restrict__ ring, int cap,
-                                                        int64_t ldr, int first, int count, int width, int to_ring) {
-  const int vecs = width / 8;
+struct RingRows {
+  T* buf;
+  int64_t ldb;
+  T* ring;
+  int64_t ldr;
+  int width;
+};
+template <typename T>
+__global__ __launch_bounds__(256) void ring_copy_kernel(RingRows<T> k, RingRows<T> v, int cap, int first, int count, int to_ring) {
+  const RingRows<T>& rows = blockIdx.y == 0 ? k : v;
+  T* const __restrict__ buf = rows.buf;
+  T* const __restrict__ ring = rows.ring;
+  const int64_t ldb = rows.ldb, ldr = rows.ldr;
+  const int vecs = rows.width / 8;
   const int64_t total = (int64_t)count * vecs;
   for (int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x; at < total; at += (int64_t)gridDim.x * 256) {
     const int i = (int)(at / vecs), c = (int)(at % vecs) * 8;

@@ -75,6 +75,27 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvArgs a) {
       for (int e = 0; e < 8; ++e) u[j][e] = a.state[(int64_t)(ch + e) * (TAPS - 1) + TAPS - 1 + s];
     }
   }
+  // The state behind the last row: by the lanes that have read the one before the first (no other block reads it).
+  static_assert(kConvTokens >= TAPS - 1, "the first block alone reads the state");
+  if (TAPS > 1 && a.next_state && blockIdx.y == 0 && on) {
+    Pack8<T> last[TAPS];
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) last[j].load(in + (int64_t)max(a.n - (TAPS - 1) + j, 0) * a.ldi);
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) {
+      const int s = a.n - (TAPS - 1) + j;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float v = last[j].get(e);
+        if (s < 0) {
+#pragma unroll
+          for (int k = 1; k < TAPS - 1; ++k)
+            if (k == j + a.n) v = u[k][e];
+        }
+        a.next_state[(int64_t)(ch + e) * (TAPS - 1) + j] = v;
+      }
+    }
+  }
   TO* out = reinterpret_cast<TO*>(g.out) + (int64_t)h * g.stride + c;
 #pragma unroll
   for (int i = 0; i < kConvTokens; ++i) {
@@ -151,17 +172,17 @@ __global__ __launch_bounds__(256) void short_conv_any_kernel(ConvArgs a) {
   for (int c = lane; c < g.stride; c += 64) out[c] = from_f<TO>(value(c) * s);
 }
 
-// state <- the last taps - 1 inputs of (state, in[0..n)).  One thread per channel; in place: a slot is written
-// after every slot that is read later has a larger index.
+// next <- the last taps - 1 inputs of (state, in[0..n)).  One thread per channel; also in place: every slot that is read
+// after one was written has a larger index.
 template <typename T>
 __global__ __launch_bounds__(256) void conv_state_kernel(const T* __restrict__ in, int64_t ldi, int n, int channels,
-                                                         int taps, float* state) {
+                                                         int taps, const float* state, float* next) {
   const int ch = blockIdx.x * 256 + threadIdx.x;
   if (ch >= channels) return;
-  float* st = state + (int64_t)ch * (taps - 1);
+  const int64_t at = (int64_t)ch * (taps - 1);
   for (int j = 0; j < taps - 1; ++j) {
     const int s = n - (taps - 1) + j;
-    st[j] = s >= 0 ? to_f(in[(int64_t)s * ldi + ch]) : st[j + n];
+    next[at + j] = s >= 0 ? to_f(in[(int64_t)s * ldi + ch]) : state[at + j + n];
   }
 }
 

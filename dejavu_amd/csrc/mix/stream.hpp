@@ -92,12 +92,24 @@ __global__ __launch_bounds__(256) void glu_kernel(const T* __restrict__ gu, int6
 }
 
 // y = x / sqrt(mean(x^2) + eps) * w, the mean over the first `dim` entries (those up to `padded`, a multiple of 8, are
-// zero).  One wave per row, eight entries per lane at a time.
+// zero).  One wave per row, eight entries per lane at a time.  Grid: (rows / 4, kinds of rows: one or two).
 template <typename T>
-__global__ __launch_bounds__(256) void rms_rows_kernel(const T* __restrict__ x, int64_t ldx, int64_t rows, int dim,
-                                                       int padded, const float* __restrict__ w, float eps,
-                                                       T* __restrict__ y, int64_t ldy) {
+struct RmsRows {
+  const T* x;
+  int dim, padded;
+  const float* w;
+  T* y;
+  int64_t ldy;
+};
+template <typename T>
+__global__ __launch_bounds__(256) void rms_rows_kernel(RmsRows<T> first, RmsRows<T> second, int64_t ldx, int64_t rows, float eps) {
   constexpr int NP = 4;  // packets a lane keeps; longer rows read the rest twice
+  const RmsRows<T>& a = blockIdx.y == 0 ? first : second;
+  const T* const __restrict__ x = a.x;
+  const float* const __restrict__ w = a.w;
+  T* const __restrict__ y = a.y;
+  const int dim = a.dim, padded = a.padded;
+  const int64_t ldy = a.ldy;
   const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (r >= rows) return;
   const int lane = threadIdx.x & 63;

@@ -162,6 +162,13 @@ template <typename T, typename TO>
 int short_conv_types(const ConvArgs& a, int heads, int widest, hipStream_t s) {
   if (a.taps > 4 || widest > 512 || (a.n + kConvTokens - 1) / kConvTokens > 65535) {
     hipLaunchKernelGGL((short_conv_any_kernel<T, TO>), dim3(blocks_of((int64_t)a.n * heads, 4)), dim3(256), 0, s, a);
+    const int rc = launched();
+    if (rc != DV_OK || !a.next_state || a.taps == 1) return rc;
+    // behind it: its waves read the state in no order
+    int channels = 0;
+    for (const dvConvGroup& g : a.g) channels += g.heads * (g.heads > 0 ? g.stride : 0);
+    hipLaunchKernelGGL((conv_state_kernel<T>), dim3(blocks_of(channels, 256)), dim3(256), 0, s, (const T*)a.in, a.ldi, a.n, channels, a.taps,
+                       a.state, a.next_state);
     return launched();
   }
   if (widest <= 8) return short_conv_lanes<T, TO, 1>(a, heads, s);
@@ -464,13 +471,25 @@ int dv_mix_gated_group_norm(int dtype, const float* y, int64_t ldy, const void* 
 
 int dv_mix_rms_rows(int dtype, const void* x, int64_t ldx, int64_t rows, int dim, int padded, const float* w, float eps,
                     void* y, int64_t ldy, void* stream) {
-  if (!dtype_ok(dtype) || !x || !w || !y || rows < 1 || dim < 1 || padded < dim) return DV_ERR_INVALID_ARG;
-  if (padded % 8 || ldx % 8 || ldy % 8 || !al16(x) || !al16(y)) return DV_ERR_ALIGNMENT;
-  const dim3 grid(blocks_of(rows, 4));
-  if (dtype == DV_BF16)
-    hipLaunchKernelGGL((rms_rows_kernel<bf16_t>), grid, dim3(256), 0, st(stream), (const bf16_t*)x, ldx, rows, dim, padded, w, eps, (bf16_t*)y, ldy);
-  else
-    hipLaunchKernelGGL((rms_rows_kernel<float>), grid, dim3(256), 0, st(stream), (const float*)x, ldx, rows, dim, padded, w, eps, (float*)y, ldy);
+  const dvRmsRows a{x, dim, padded, w, y, ldy};
+  return dv_mix_rms_rows_two(dtype, &a, nullptr, ldx, rows, eps, stream);
+}
+
+int dv_mix_rms_rows_two(int dtype, const dvRmsRows* a, const dvRmsRows* b, int64_t ldx, int64_t rows, float eps, void* stream) {
+  if (!dtype_ok(dtype) || !a || rows < 1) return DV_ERR_INVALID_ARG;
+  for (const dvRmsRows* r : {a, b}) {
+    if (r == nullptr) continue;
+    if (!r->x || !r->w || !r->y || r->dim < 1 || r->padded < r->dim) return DV_ERR_INVALID_ARG;
+    if (r->padded % 8 || ldx % 8 || r->ldy % 8 || !al16(r->x) || !al16(r->y)) return DV_ERR_ALIGNMENT;
+  }
+  const dim3 grid(blocks_of(rows, 4), b ? 2 : 1);
+  auto launch = [&](auto type) {
+    using T = decltype(type);
+    auto rows_of = [](const dvRmsRows* r) { return RmsRows<T>{(const T*)r->x, r->dim, r->padded, r->w, (T*)r->y, r->ldy}; };
+    hipLaunchKernelGGL((rms_rows_kernel<T>), grid, dim3(256), 0, st(stream), rows_of(a), rows_of(b ? b : a), ldx, rows, eps);
+  };
+  if (dtype == DV_BF16) launch(bf16_t{});
+  else launch(float{});
   return launched();
 }
 
@@ -587,24 +606,38 @@ int dv_mix_conv_state(int dtype, const void* in, int64_t ldi, int n, int channel
   if (taps == 1) return DV_OK;
   const dim3 grid(blocks_of(channels, 256));
   if (dtype == DV_BF16)
-    hipLaunchKernelGGL((conv_state_kernel<bf16_t>), grid, dim3(256), 0, st(stream), (const bf16_t*)in, ldi, n, channels, taps, state);
+    hipLaunchKernelGGL((conv_state_kernel<bf16_t>), grid, dim3(256), 0, st(stream), (const bf16_t*)in, ldi, n, channels, taps, state, state);
   else
-    hipLaunchKernelGGL((conv_state_kernel<float>), grid, dim3(256), 0, st(stream), (const float*)in, ldi, n, channels, taps, state);
+    hipLaunchKernelGGL((conv_state_kernel<float>), grid, dim3(256), 0, st(stream), (const float*)in, ldi, n, channels, taps, state, state);
   return launched();
 }
 
 int dv_mix_ring_copy(int dtype, void* buf, int64_t ldb, void* ring, int cap, int64_t ldr, int first, int count, int width,
                      int to_ring, void* stream) {
-  if (!dtype_ok(dtype) || !buf || !ring || cap < 1 || first < 0 || count < 0 || count > cap || width < 8)
-    return DV_ERR_INVALID_ARG;
-  if (width % 8 || ldb % 8 || ldr % 8 || !al16(buf) || !al16(ring)) return DV_ERR_ALIGNMENT;
+  const dvRingRows a{buf, ldb, ring, ldr, width};
+  return dv_mix_ring_copy_two(dtype, &a, nullptr, cap, first, count, to_ring, stream);
+}
+
+int dv_mix_ring_copy_two(int dtype, const dvRingRows* a, const dvRingRows* b, int cap, int first, int count, int to_ring, void* stream) {
+  if (!dtype_ok(dtype) || !a || cap < 1 || first < 0 || count < 0 || count > cap) return DV_ERR_INVALID_ARG;
+  int widest = 0;
+  for (const dvRingRows* r : {a, b}) {
+    if (r == nullptr) continue;
+    if (!r->buf || !r->ring || r->width < 8) return DV_ERR_INVALID_ARG;
+    if (r->width % 8 || r->ldb % 8 || r->ldr % 8 || !al16(r->buf) || !al16(r->ring)) return DV_ERR_ALIGNMENT;
+    if (r->width > widest) widest = r->width;
+  }
   if (count == 0) return DV_OK;
-  unsigned grid = blocks_of((int64_t)count * (width / 8), 256);
+  unsigned grid = blocks_of((int64_t)count * (widest / 8), 256);
   if (grid > 4096) grid = 4096;
-  if (dtype == DV_BF16)
-    hipLaunchKernelGGL((ring_copy_kernel<bf16_t>), dim3(grid), dim3(256), 0, st(stream), (bf16_t*)buf, ldb, (bf16_t*)ring, cap, ldr, first, count, width, to_ring);
-  else
-    hipLaunchKernelGGL((ring_copy_kernel<float>), dim3(grid), dim3(256), 0, st(stream), (float*)buf, ldb, (float*)ring, cap, ldr, first, count, width, to_ring);
+  auto launch = [&](auto type) {
+    using T = decltype(type);
+    auto rows_of = [](const dvRingRows* r) { return RingRows<T>{(T*)r->buf, r->ldb, (T*)r->ring, r->ldr, r->width}; };
+    hipLaunchKernelGGL((ring_copy_kernel<T>), dim3(grid, b ? 2 : 1), dim3(256), 0, st(stream), rows_of(a), rows_of(b ? b : a), cap, first,
+                       count, to_ring);
+  };
+  if (dtype == DV_BF16) launch(bf16_t{});
+  else launch(float{});
   return launched();
 }
 

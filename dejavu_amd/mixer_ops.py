@@ -557,6 +557,17 @@ def rms_rows(x: torch.Tensor, weight: torch.Tensor, dim: int, eps: float, out: O
     return out
 
 
+def rms_rows_two(x: torch.Tensor, a, b, eps: float) -> None:
+    """``rms_rows`` of two stretches of the rows of x in one launch.  a, b: (first entry, weight, dim, out)."""
+    n, rows = x.shape[0], []
+    for at, weight, dim, out in (a, b):
+        assert out.dtype == x.dtype and x.stride(1) == out.stride(1) == 1 and out.shape == (n, weight.numel())
+        assert at + weight.numel() <= x.shape[1]
+        rows.append(L.RmsRows(x=x.data_ptr() + at * x.element_size(), dim=dim, padded=weight.numel(), w=weight.data_ptr(),
+                              y=out.data_ptr(), ldy=out.stride(0)))
+    check(lib.dv_mix_rms_rows_two(_code(x), _ref(rows[0]), _ref(rows[1]), x.stride(0), n, eps, _stream()), "dv_mix_rms_rows_two")
+
+
 def gated_head_norm(o: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, dim: int, eps: float):
     """o (n, heads, vdim_s) fp32, gate (n, heads * vdim_s) -> (n, heads * vdim_s)."""
     n, heads, vs = o.shape
@@ -570,12 +581,13 @@ NORM_NONE, NORM_RMS, NORM_UNIT = 0, 1, 2
 
 
 def short_conv(x: torch.Tensor, conv_w: torch.Tensor, state: torch.Tensor, groups, silu: bool,
-               conv_b: Optional[torch.Tensor] = None) -> None:
+               conv_b: Optional[torch.Tensor] = None, move: bool = False) -> None:
     """x (n, >= channels): the groups' channels one after the other.  groups: (heads, stride, dim, norm, eps, scale,
-    out) with out (n, heads * stride), all fp32 or all of x's type.  The state is read, not moved on."""
+    out) with out (n, heads * stride), all fp32 or all of x's type.  The state is read; with ``move`` it moves on by
+    the rows of x as well (``conv_state``)."""
     _f32(conv_w, conv_b)
     a = L.ConvArgs(in_=x.data_ptr(), ldi=x.stride(0), n=x.shape[0], taps=conv_w.shape[1], silu=int(silu),
-                   w=conv_w.data_ptr(), b=_ptr(conv_b), state=state.data_ptr())
+                   w=conv_w.data_ptr(), b=_ptr(conv_b), state=state.data_ptr(), next_state=state.data_ptr() if move else None)
     for i, (heads, stride, dim, norm, eps, scale, out) in enumerate(groups):
         assert out.shape == (x.shape[0], heads * stride) and out.stride(1) == 1
         a.g[i] = L.ConvGroup(heads=heads, stride=stride, dim=dim, norm=norm, eps=eps, scale=scale, out=out.data_ptr(),
@@ -588,6 +600,19 @@ def conv_state(x: torch.Tensor, channels: int, taps: int, state: torch.Tensor) -
     """Moves the state on by the n rows of x."""
     check(lib.dv_mix_conv_state(_code(x), _ptr(x), x.stride(0), x.shape[0], channels, taps, _ptr(state), _stream()),
           "dv_mix_conv_state")
+
+
+def _ring_rows(buf: torch.Tensor, ring: torch.Tensor) -> L.RingRows:
+    assert buf.dtype == ring.dtype and buf.shape[1] == ring.shape[1]
+    return L.RingRows(buf=buf.data_ptr(), ldb=buf.stride(0), ring=ring.data_ptr(), ldr=ring.stride(0), width=buf.shape[1])
+
+
+def ring_copy_two(bufs, rings, first: int, to_ring: bool) -> None:
+    """``ring_copy`` of two buffers of as many rows and two rings of as many in one launch."""
+    (a, b), (ra, rb) = bufs, rings
+    assert a.shape[0] == b.shape[0] and ra.shape[0] == rb.shape[0] and a.dtype == b.dtype
+    check(lib.dv_mix_ring_copy_two(_code(a), _ref(_ring_rows(a, ra)), _ref(_ring_rows(b, rb)), ra.shape[0], first, a.shape[0],
+                                   int(to_ring), _stream()), "dv_mix_ring_copy_two")
 
 
 def ring_copy(buf: torch.Tensor, ring: torch.Tensor, first: int, to_ring: bool) -> None:

@@ -152,8 +152,9 @@ class LatentAttention(nn.Module):
                                             step.pos_dev, step.pos)
         p = ops.linear(h, self.in_proj)
         end = step.pos + n
-        ops.rms_rows(p[:, qs:qs + ks], self.kv_norm, self.kv_rank, self.eps, out=cache[step.pos:end])
-        q = ops.linear(ops.rms_rows(p[:, :qs], self.q_norm, self.q_rank, self.eps), self.q_up)
+        q = torch.empty(n, qs, dtype=p.dtype, device=p.device)
+        ops.rms_rows_two(p, (0, self.q_norm, self.q_rank, q), (qs, self.kv_norm, self.kv_rank, cache[step.pos:end]), self.eps)
+        q = ops.linear(q, self.q_up)
         c = cache[:end]
         k, v = ops.linear(c, self.k_up), ops.linear(c, self.v_up)
         return ops.portion_attention(q, k, v, self.heads, self.heads, self.scale, 0, step.pos, gate=p[:, qs + ks:])
@@ -165,18 +166,18 @@ def _rings(tokens: int, k_width: int, v_width: int, like: torch.Tensor) -> dict:
     return {"k": new(k_width), "v": new(v_width)}
 
 
-def _behind_history(ring, first: int, hist: int, n: int):
-    """Rows for tokens first .. first + hist + n - 1, the first ``hist`` of them read from the ring."""
-    rows = torch.empty(hist + n, ring.shape[1], dtype=ring.dtype, device=ring.device)
+def _behind_history(rings, first: int, hist: int, n: int):
+    """Rows of keys and of values for tokens first .. first + hist + n - 1, the first ``hist`` of them read from the rings."""
+    rows = [torch.empty(hist + n, r.shape[1], dtype=r.dtype, device=r.device) for r in rings]
     if hist:
-        ops.ring_copy(rows[:hist], ring, first, to_ring=False)
+        ops.ring_copy_two([r[:hist] for r in rows], rings, first, to_ring=False)
     return rows
 
 
-def _keep_newest(ring, rows, n: int, end: int) -> None:
-    """The last of the n newest rows (tokens up to end - 1) go to the ring."""
-    keep = min(n, ring.shape[0])
-    ops.ring_copy(rows[rows.shape[0] - keep:], ring, end - keep, to_ring=True)
+def _keep_newest(rings, rows, n: int, end: int) -> None:
+    """The last of the n newest rows (tokens up to end - 1) go to the rings."""
+    keep = min(n, rings[0].shape[0])
+    ops.ring_copy_two([r[r.shape[0] - keep:] for r in rows], rings, end - keep, to_ring=True)
 
 
 class WindowAttention(nn.Module):
@@ -210,16 +211,14 @@ class WindowAttention(nn.Module):
         p = ops.linear(h, self.in_proj)
         hist = min(step.pos, self.window - 1)  # earlier tokens that this portion can still see
         q = torch.empty(n, H * ds, dtype=h.dtype, device=h.device)
-        k, v = (_behind_history(r, step.pos - hist, hist, n) for r in (kr, vr))
+        k, v = _behind_history((kr, vr), step.pos - hist, hist, n)
         ops.short_conv(p, self.conv, state["conv"],
                        [(H, ds, self.dim, ops.NORM_RMS, self.eps, 1.0, q),
                         (G, ds, self.dim, ops.NORM_RMS, self.eps, 1.0, k[hist:]),
-                        (G, vs, self.vdim, ops.NORM_NONE, 0.0, 1.0, v[hist:])], silu=False)
-        ops.conv_state(p, self.channels, self.taps, state["conv"])
+                        (G, vs, self.vdim, ops.NORM_NONE, 0.0, 1.0, v[hist:])], silu=False, move=True)
         o = ops.portion_attention(q, k, v, H, G, self.scale, step.pos - hist, step.pos, sink=self.sink,
                                   window=self.window)
-        for ring, rows in ((kr, k), (vr, v)):
-            _keep_newest(ring, rows, n, step.pos + n)
+        _keep_newest((kr, vr), (k, v), n, step.pos + n)
         return o
 
 
@@ -294,13 +293,12 @@ class ChunkAttention(nn.Module):
                                           mix_v=mix, gate=gate[0])
         hist = step.pos % self.chunk if self.chunk else step.pos  # earlier tokens that this portion can still see
         q = torch.empty(n, H * ds, dtype=h.dtype, device=h.device)
-        k, v = (_behind_history(r, step.pos - hist, hist, n) for r in (kr, vr))
+        k, v = _behind_history((kr, vr), step.pos - hist, hist, n)
         ops.head_rows(p, [(H, ds, self.dim, (self.q_norm, self.eps), q), (G, ds, self.dim, (self.k_norm, self.eps), k[hist:]),
                           (G, vs, self.vdim, mix, v[hist:])])
         o = ops.portion_attention(q, k, v, H, G, self.scale, step.pos - hist, step.pos, gate=gate, chunk=self.chunk,
                                   rel=self.rel)
-        for ring, rows in ((kr, k), (vr, v)):
-            _keep_newest(ring, rows, n, step.pos + n)
+        _keep_newest((kr, vr), (k, v), n, step.pos + n)
         return o
 
 
@@ -348,8 +346,7 @@ class Mamba2(nn.Module):
         xbc = ops.ssd_rows(n, self.channels, h.device)
         per = 8 if self.taps <= 4 else self.channels  # channels that the convolution kernel takes together
         ops.short_conv(p, self.conv, state["conv"], [(self.channels // per, per, per, ops.NORM_NONE, 0.0, 1.0, xbc)],
-                       silu=True, conv_b=self.conv_bias)
-        ops.conv_state(p, self.channels, self.taps, state["conv"])
+                       silu=True, conv_b=self.conv_bias, move=True)
         y = ops.ssd_scan(xbc, p[:, self.off_dt:self.off_dt + self.heads], *rule, self.inner_s)
         return ops.gated_group_norm(y, p[:, self.off_z:self.off_dt], self.norm, self.inner, self.norm_groups, self.eps)
 
@@ -398,8 +395,7 @@ class ChannelDelta(nn.Module):
         ops.short_conv(p, self.conv, state["conv"],
                        [(G, ds, self.dim, ops.NORM_UNIT, 0.0, self.dim ** -0.5, q),
                         (G, ds, self.dim, ops.NORM_UNIT, 0.0, 1.0, k),
-                        (H, vs, self.vdim, ops.NORM_NONE, 0.0, 1.0, v)], silu=True)
-        ops.conv_state(p, self.channels, self.taps, state["conv"])
+                        (H, vs, self.vdim, ops.NORM_NONE, 0.0, 1.0, v)], silu=True, move=True)
         z = ops.linear(p[:, off_a:off_g], self.decay_up)
         g, beta = ops.delta_gates(z, p[:, off_b:], self.A_log, self.dt_bias, H)
         o = ops.delta_scan(q, k, v, g, beta, state["S"], H, G)

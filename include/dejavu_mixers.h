@@ -136,7 +136,25 @@ typedef struct {
   const float* b;          /* [channels] or null */
   const float* state;      /* [channels][taps - 1] */
   dvConvGroup g[3];
+  float* next_state;       /* null, or where the state behind the last row goes (may be `state`) */
 } dvConvArgs;
+
+/* Rows that are RMS-normed: y = x / rms(x) * w; w has `padded` entries, the mean runs over `dim`. */
+typedef struct {
+  const void* x;
+  int dim, padded;
+  const float* w;
+  void* y;
+  int64_t ldy;
+} dvRmsRows;
+/* Rows of a portion's buffer and the ring that keeps them. */
+typedef struct {
+  void* buf;
+  int64_t ldb;
+  void* ring;
+  int64_t ldr;
+  int width;
+} dvRingRows;
 
 /* One group of heads of a projection's rows: RMS-normed per head with a weight, or mixed with other rows. */
 typedef struct {
@@ -284,6 +302,9 @@ DV_API int dv_mix_gated_group_norm(int dtype, const float* y, int64_t ldy, const
 /* y = x / rms(x) * w, row by row; w has `padded` entries, the mean runs over `dim`. */
 DV_API int dv_mix_rms_rows(int dtype, const void* x, int64_t ldx, int64_t rows, int dim, int padded, const float* w,
                            float eps, void* y, int64_t ldy, void* stream);
+/* One or two kinds of rows (b may be null) with one stride of x. */
+DV_API int dv_mix_rms_rows_two(int dtype, const dvRmsRows* a, const dvRmsRows* b, int64_t ldx, int64_t rows, float eps,
+                               void* stream);
 /* y = o / rms(o) * w * sigmoid(gate) per head; o fp32 [rows][heads][padded]. */
 DV_API int dv_mix_gated_head_norm(int dtype, const float* o, const void* gate, int64_t ldg, int64_t rows, int heads,
                                   int vdim, int padded, const float* w, float eps, void* y, void* stream);
@@ -305,6 +326,9 @@ DV_API int dv_mix_conv_state(int dtype, const void* in, int64_t ldi, int n, int 
 /* Rows of a portion's buffer <-> a ring of cap rows, token first .. first + count - 1 (count <= cap). */
 DV_API int dv_mix_ring_copy(int dtype, void* buf, int64_t ldb, void* ring, int cap, int64_t ldr, int first, int count,
                             int width, int to_ring, void* stream);
+/* One or two rings of as many rows (b may be null), keys and values. */
+DV_API int dv_mix_ring_copy_two(int dtype, const dvRingRows* a, const dvRingRows* b, int cap, int first, int count, int to_ring,
+                                void* stream);
 /* q_f32: the queries (and gate logits) are fp32 instead of `dtype`. */
 DV_API int dv_mix_attn_rows(int dtype, int q_f32, const dvAttnArgs* args, void* stream);
 /* bf16, a portion on the matrix cores; `keys` rows behind k and v (contiguous, ring = 0). */
