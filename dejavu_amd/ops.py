@@ -43,20 +43,21 @@ def _idx_bytes(idx: torch.Tensor) -> int:
     return 4 if idx.dtype == torch.int32 else 8
 
 
-def _expect(ok: bool, what: str) -> None:
-    """Precondition failures are ``AssertionError``s, as in the reference's wrappers."""
+def _expect(ok: bool, what) -> None:
+    """Precondition failures are ``AssertionError``s, as in the reference's wrappers.  what: the message, or what makes it: putting
+    one together costs more than half a microsecond, several of them a call as much as a launch."""
     if not ok:
-        raise AssertionError(what)
+        raise AssertionError(what if isinstance(what, str) else what())
 
 
 def _same_f16(name_a: str, a: torch.Tensor, name_b: str, b: Optional[torch.Tensor]) -> None:
     if b is not None:
-        _expect(a.dtype == b.dtype, f"{name_a} is {a.dtype} but {name_b} is {b.dtype}: they must agree")
-    _expect(a.dtype == torch.float16, f"{name_a} is {a.dtype}: the kernels are fp16 only")
+        _expect(a.dtype == b.dtype, lambda: f"{name_a} is {a.dtype} but {name_b} is {b.dtype}: they must agree")
+    _expect(a.dtype == torch.float16, lambda: f"{name_a} is {a.dtype}: the kernels are fp16 only")
 
 
 def _int32_vector(name: str, t: torch.Tensor, n: int) -> None:
-    _expect(t.dtype == torch.int32 and tuple(t.shape) == (n,), f"{name} must be an int32 vector of {n} entries, "
+    _expect(t.dtype == torch.int32 and tuple(t.shape) == (n,), lambda: f"{name} must be an int32 vector of {n} entries, "
             f"got {t.dtype} {tuple(t.shape)}")
 
 
@@ -128,9 +129,9 @@ def predictor_logits(x: torch.Tensor, fc0_weight: torch.Tensor, fc1_weight: torc
         nb = min(step, B - b0)
         nbytes = lib.dv_predictor_workspace_bytes(nb, d, r)
         ws = _workspace(x.device, nbytes) if nbytes else None
-        check(lib.dv_predictor_logits_ws_f16(_ptr(x[b0:]), _ptr(fc0_weight), fc0_weight.stride(0), _ptr(fc1_weight),
-                                             fc1_weight.stride(0), nb, d, r, n_out, _ptr(hidden[b0:]),
-                                             _ptr(logits[b0:]), _ptr(ws), 0 if ws is None else ws.numel(), _stream()),
+        check(lib.dv_predictor_logits_ws_f16(x.data_ptr() + 2 * b0 * d, _ptr(fc0_weight), fc0_weight.stride(0), _ptr(fc1_weight),
+                                             fc1_weight.stride(0), nb, d, r, n_out, hidden.data_ptr() + 2 * b0 * hidden.stride(0),
+                                             logits.data_ptr() + 2 * b0 * n_out, _ptr(ws), 0 if ws is None else ws.numel(), _stream()),
               "dv_predictor_logits_ws_f16")
     return logits
 
@@ -159,10 +160,8 @@ def topk_indices(logits: torch.Tensor, k: int, dtype: torch.dtype = torch.int64,
     _require_device(logits)
     assert logits.dtype == torch.float16
     lg = logits.contiguous()
-    if lg.dim() == 1:
-        lg = lg.unsqueeze(0)
-    assert lg.dim() == 2
-    B, n = lg.shape
+    assert lg.dim() in (1, 2)
+    B, n = (1, lg.shape[0]) if lg.dim() == 1 else lg.shape
     assert 0 <= k <= n, f"k={k} outside [0, {n}]"
     if out is None:
         out = torch.empty(k, device=lg.device, dtype=dtype)
@@ -210,16 +209,16 @@ def gather_gemv(x: torch.Tensor, weight: torch.Tensor, idx: Optional[torch.Tenso
     ``idx=None`` takes all Z rows in order (a dense product).  batch may go up to 64 (the
     reference's kernel stops at 4; from 3 rows on the product runs on the matrix cores).
     """
-    _expect(activation in ("id", "relu", "gelu", "gelu_approx", "squared_relu"), f"unknown activation {activation!r}")
+    _expect(activation in ("id", "relu", "gelu", "gelu_approx", "squared_relu"), lambda: f"unknown activation {activation!r}")
     _require_device(x, weight, idx, bias)
     _expect(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1],
-            f"x {tuple(x.shape)} and weight {tuple(weight.shape)} must share their last dimension")
+            lambda: f"x {tuple(x.shape)} and weight {tuple(weight.shape)} must share their last dimension")
     batch, N = x.shape
     Z = weight.shape[0]
-    _expect(1 <= batch <= 64, f"batch {batch} outside 1..64")
+    _expect(1 <= batch <= 64, lambda: f"batch {batch} outside 1..64")
     _same_f16("x", x, "weight", weight)
     if bias is not None:
-        _expect(tuple(bias.shape) == (Z,), f"bias {tuple(bias.shape)} does not match the {Z} weight rows")
+        _expect(tuple(bias.shape) == (Z,), lambda: f"bias {tuple(bias.shape)} does not match the {Z} weight rows")
         _same_f16("x", x, "bias", bias)
         bias = bias.contiguous()
     x = x.contiguous()
@@ -244,7 +243,7 @@ def dense_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     """``activation(F.linear(x, weight, bias))`` for any number of rows on the matrix cores: the dense
     products of the prompt phase.  x: (..., N) fp16 with a contiguous last dimension (rows may be
     strided after flattening); weight: (M, N); returns (..., M)."""
-    _expect(activation in _ACT, f"unknown activation {activation!r}")
+    _expect(activation in _ACT, lambda: f"unknown activation {activation!r}")
     _require_device(x, weight, bias, out)
     M, N = weight.shape
     assert x.shape[-1] == N and x.dtype == weight.dtype == torch.float16
@@ -348,13 +347,13 @@ def gather_transposed_gemv(x: torch.Tensor, weight: torch.Tensor, idx: torch.Ten
     """
     _require_device(x, weight, idx, bias)
     _expect(x.dim() == 2 and weight.dim() == 2 and idx.dim() == 1 and x.shape[1] == idx.shape[0],
-            f"x {tuple(x.shape)} needs one column per entry of idx {tuple(idx.shape)}")
+            lambda: f"x {tuple(x.shape)} needs one column per entry of idx {tuple(idx.shape)}")
     batch, M = x.shape
     Z, N = weight.shape
-    _expect(1 <= batch <= 64, f"batch {batch} outside 1..64")
+    _expect(1 <= batch <= 64, lambda: f"batch {batch} outside 1..64")
     _same_f16("x", x, "weight", weight)
     if bias is not None:
-        _expect(tuple(bias.shape) == (N,), f"bias {tuple(bias.shape)} does not match the {N} output columns")
+        _expect(tuple(bias.shape) == (N,), lambda: f"bias {tuple(bias.shape)} does not match the {N} output columns")
         _same_f16("x", x, "bias", bias)
         bias = bias.contiguous()
     x = x.contiguous()
@@ -410,21 +409,21 @@ def qkv_proj_sparse(x: torch.Tensor, weight: torch.Tensor, head_idx: torch.Tenso
     would do with ``seqlen_idx = batch_idx``.
     """
     _require_device(x, weight, head_idx, batch_idx, bias)
-    _expect(weight.dim() == 4 and weight.shape[0] == 3, f"weight {tuple(weight.shape)} is not (3, nheads, head_dim, hidden)")
+    _expect(weight.dim() == 4 and weight.shape[0] == 3, lambda: f"weight {tuple(weight.shape)} is not (3, nheads, head_dim, hidden)")
     _, nheads, head_dim, hidden_dim = weight.shape
-    _expect(head_dim in (32, 64, 128), f"head_dim {head_dim} not in 32 / 64 / 128")
-    _expect(hidden_dim % 128 == 0, f"hidden size {hidden_dim} is not a multiple of 128")
+    _expect(head_dim in (32, 64, 128), lambda: f"head_dim {head_dim} not in 32 / 64 / 128")
+    _expect(hidden_dim % 128 == 0, lambda: f"hidden size {hidden_dim} is not a multiple of 128")
     batch_size = x.shape[0]
     _expect(tuple(x.shape) == (batch_size, hidden_dim) and batch_size <= 16,
-            f"x {tuple(x.shape)} must be (rows <= 16, {hidden_dim})")
+            lambda: f"x {tuple(x.shape)} must be (rows <= 16, {hidden_dim})")
     n_active = head_idx.shape[0]
-    _expect(n_active <= nheads, f"{n_active} heads listed, the layer has {nheads}")
+    _expect(n_active <= nheads, lambda: f"{n_active} heads listed, the layer has {nheads}")
     _int32_vector("head_idx", head_idx, n_active)
     _expect(batch_idx.dtype == torch.int32 and tuple(batch_idx.shape) == (n_active, batch_size),
-            f"batch_idx must be int32 ({n_active}, {batch_size}), got {batch_idx.dtype} {tuple(batch_idx.shape)}")
+            lambda: f"batch_idx must be int32 ({n_active}, {batch_size}), got {batch_idx.dtype} {tuple(batch_idx.shape)}")
     _same_f16("x", x, "weight", weight)
     if bias is not None:
-        _expect(tuple(bias.shape) == (3, nheads, head_dim), f"bias {tuple(bias.shape)} is not (3, {nheads}, {head_dim})")
+        _expect(tuple(bias.shape) == (3, nheads, head_dim), lambda: f"bias {tuple(bias.shape)} is not (3, {nheads}, {head_dim})")
         _same_f16("x", x, "bias", bias)
         bias = bias.contiguous()
     x, weight, head_idx, batch_idx = x.contiguous(), weight.contiguous(), head_idx.contiguous(), batch_idx.contiguous()
@@ -522,21 +521,21 @@ def qkv_window_batch(x_window: torch.Tensor, weight: torch.Tensor, head_idx: tor
         heads that were not computed for it keep the content of ``out``
     """
     _require_device(x_window, weight, head_idx, batch_idx, bias, k_cache, v_cache, positions)
-    _expect(weight.dim() == 4 and weight.shape[0] == 3, f"weight {tuple(weight.shape)} is not (3, nheads, head_dim, hidden)")
+    _expect(weight.dim() == 4 and weight.shape[0] == 3, lambda: f"weight {tuple(weight.shape)} is not (3, nheads, head_dim, hidden)")
     _, nheads, head_dim, hidden_dim = weight.shape
     n_active = head_idx.shape[0]
     _int32_vector("head_idx", head_idx, n_active)
     _expect(batch_idx.dtype == torch.int32 and batch_idx.dim() == 2 and batch_idx.shape[0] == n_active
             and batch_idx.is_contiguous(), "batch_idx must be a contiguous int32 (nnz, tokens) matrix")
     tokens = batch_idx.shape[1]
-    _expect(1 <= tokens <= 16 and 1 <= nseq <= 32, f"{tokens} tokens x {nseq} sequences outside 16 x 32")
+    _expect(1 <= tokens <= 16 and 1 <= nseq <= 32, lambda: f"{tokens} tokens x {nseq} sequences outside 16 x 32")
     x2 = x_window.reshape(-1, hidden_dim)
     _expect(x2.shape[0] >= tokens * nseq and x2.is_contiguous(), "x_window must hold tokens * nseq contiguous rows")
     _same_f16("x_window", x2, "weight", weight)
     _expect(weight.is_contiguous() and head_idx.is_contiguous(), "weight and head_idx must be contiguous")
     if bias is not None:
         _expect(tuple(bias.shape) == (3, nheads, head_dim) and bias.is_contiguous() and bias.dtype == x2.dtype,
-                f"bias {tuple(bias.shape)} is not a contiguous fp16 (3, {nheads}, {head_dim}) tensor")
+                lambda: f"bias {tuple(bias.shape)} is not a contiguous fp16 (3, {nheads}, {head_dim}) tensor")
     if out is None:
         out = torch.empty(nseq, 3, nheads, head_dim, device=x2.device, dtype=x2.dtype)
     else:
@@ -576,16 +575,16 @@ def out_proj_sparse(x: torch.Tensor, weight: torch.Tensor, head_idx: torch.Tenso
     _require_device(x, weight, head_idx, bias)
     _expect(weight.dim() == 3 and x.dim() == 3, "x must be (batch, nheads, head_dim), weight (hidden, nheads, head_dim)")
     hidden_dim, nheads, head_dim = weight.shape
-    _expect(head_dim in (32, 64, 128), f"head_dim {head_dim} not in 32 / 64 / 128")
-    _expect(hidden_dim % 128 == 0, f"hidden size {hidden_dim} is not a multiple of 128")
+    _expect(head_dim in (32, 64, 128), lambda: f"head_dim {head_dim} not in 32 / 64 / 128")
+    _expect(hidden_dim % 128 == 0, lambda: f"hidden size {hidden_dim} is not a multiple of 128")
     batch = x.shape[0]
     _expect(tuple(x.shape) == (batch, nheads, head_dim) and batch <= 16,
-            f"x {tuple(x.shape)} must be (batch <= 16, {nheads}, {head_dim})")
+            lambda: f"x {tuple(x.shape)} must be (batch <= 16, {nheads}, {head_dim})")
     n_active = head_idx.shape[0]
     _int32_vector("head_idx", head_idx, n_active)
     _same_f16("x", x, "weight", weight)
     if bias is not None:
-        _expect(tuple(bias.shape) == (hidden_dim,), f"bias {tuple(bias.shape)} does not match hidden size {hidden_dim}")
+        _expect(tuple(bias.shape) == (hidden_dim,), lambda: f"bias {tuple(bias.shape)} does not match hidden size {hidden_dim}")
         _same_f16("x", x, "bias", bias)
         bias = bias.contiguous()
     x, weight, head_idx = x.contiguous(), weight.contiguous(), head_idx.contiguous()
@@ -669,14 +668,14 @@ def _cache_copy(k, v, k_cache, v_cache, head_idx, seqlen_idx, padding):
     _require_device(src, k_cache, v_cache, head_idx, seqlen_idx, padding)
     _expect(src.dim() == 3, "k / v must be (tokens, nheads, head_dim)")
     nnz_seqlen, nheads, head_dim = src.shape
-    _expect(head_dim in (32, 64, 128), f"head_dim {head_dim} not in 32 / 64 / 128")
-    _expect(nnz_seqlen <= 16, f"{nnz_seqlen} tokens: a back-fill window holds at most 16")
+    _expect(head_dim in (32, 64, 128), lambda: f"head_dim {head_dim} not in 32 / 64 / 128")
+    _expect(nnz_seqlen <= 16, lambda: f"{nnz_seqlen} tokens: a back-fill window holds at most 16")
     _expect(src.stride(2) == 1 and src.stride(1) == head_dim, "the heads of a k / v row must be contiguous")
     n_active = head_idx.shape[0]
-    _expect(n_active <= nheads, f"{n_active} heads listed, the layer has {nheads}")
+    _expect(n_active <= nheads, lambda: f"{n_active} heads listed, the layer has {nheads}")
     _int32_vector("head_idx", head_idx, n_active)
     _expect(seqlen_idx.dtype == torch.int32 and tuple(seqlen_idx.shape) == (n_active, nnz_seqlen),
-            f"seqlen_idx must be int32 ({n_active}, {nnz_seqlen}), got {seqlen_idx.dtype} {tuple(seqlen_idx.shape)}")
+            lambda: f"seqlen_idx must be int32 ({n_active}, {nnz_seqlen}), got {seqlen_idx.dtype} {tuple(seqlen_idx.shape)}")
     if padding is not None:
         _int32_vector("padding", padding, 1)
     head_idx, seqlen_idx = head_idx.contiguous(), seqlen_idx.contiguous()
@@ -685,12 +684,12 @@ def _cache_copy(k, v, k_cache, v_cache, head_idx, seqlen_idx, padding):
         _same_f16("k", k, "k_cache", k_cache)
         seqlen = k_cache.shape[3]
         _expect(tuple(k_cache.shape) == (1, nheads, head_dim // 8, seqlen, 8) and k_cache.is_contiguous(),
-                f"k_cache {tuple(k_cache.shape)} is not a contiguous (1, {nheads}, {head_dim // 8}, S, 8) tensor")
+                lambda: f"k_cache {tuple(k_cache.shape)} is not a contiguous (1, {nheads}, {head_dim // 8}, S, 8) tensor")
     if v_cache is not None:
         _same_f16("v", v, "v_cache", v_cache)
         seqlen = v_cache.shape[2]
         _expect(tuple(v_cache.shape) == (1, nheads, seqlen, head_dim) and v_cache.is_contiguous(),
-                f"v_cache {tuple(v_cache.shape)} is not a contiguous (1, {nheads}, S, {head_dim}) tensor")
+                lambda: f"v_cache {tuple(v_cache.shape)} is not a contiguous (1, {nheads}, S, {head_dim}) tensor")
     if k is not None and v is not None:
         _expect(k.stride(0) == v.stride(0), "k and v must have the same row stride")
     check(lib.dv_kv_cache_copy_sparse_f16(_ptr(k), _ptr(v), src.stride(0), nnz_seqlen, _ptr(k_cache), _ptr(v_cache),
@@ -940,14 +939,14 @@ def ln_qkv_proj_sparse(r: torch.Tensor, parts: torch.Tensor, ln_weight: torch.Te
     _require_device(r, parts, ln_weight, ln_bias, x_cache, weight, head_idx, batch_idx, bias)
     _, nheads, head_dim, hidden_dim = weight.shape
     nb = token + 1
-    _expect(head_dim in (64, 128), f"head_dim {head_dim} not 64 / 128")
+    _expect(head_dim in (64, 128), lambda: f"head_dim {head_dim} not 64 / 128")
     _expect(r.numel() == hidden_dim and r.dtype == torch.float16, "r must be one fp16 row")
     _expect(parts.dtype == torch.float32 and tuple(parts.shape) == ((hidden_dim + 63) // 64, 2), "parts from add_ln_parts")
     _expect(tuple(x_cache.shape) == (16, hidden_dim) and x_cache.is_contiguous(), "x_cache must be the (16, hidden) window buffer")
     n_active = head_idx.shape[0]
     _int32_vector("head_idx", head_idx, n_active)
     _expect(batch_idx.dtype == torch.int32 and tuple(batch_idx.shape) == (n_active, nb),
-            f"batch_idx must be int32 ({n_active}, {nb})")
+            lambda: f"batch_idx must be int32 ({n_active}, {nb})")
     if bias is not None:
         bias = bias.contiguous()
     r, weight, head_idx, batch_idx = r.contiguous(), weight.contiguous(), head_idx.contiguous(), batch_idx.contiguous()
