@@ -12,19 +12,21 @@
 // are zeros to an infinity.
 //
 // The parts of x are made beforehand (split_rows_kernel); those of W in registers, by the one wave that uses them.
-// Six bf16 products at 2.5 PFLOP/s are 2.6 times the fp32 instructions' 157 TFLOP/s.  500 rows by 11264 x 2048: 155 us, the library's fp32
-// GEMM 197 (two fp16 parts 123); 2048 by 22016 x 4096 2112 us, 2630.  From 64 bits 2.7e-7 and 4e-7, the library 8.1e-7 and 1.15e-6.
-// Bound by the matrix instructions and what stands between them: their units work in 57 % of the cycles (at 2.1 GHz) of the 176 compute
-// units that have a tile of the first; wave priorities, reads further ahead, a third slot, 128 x 256 tiles and chunks of 16 columns took as
-// long or longer.
+// Six bf16 products at 2.5 PFLOP/s are 2.6 times the fp32 instructions' 157 TFLOP/s.  From 64 bits 2.7e-7 (K = 2048) and 4e-7 (4096), the library
+// 8.1e-7 and 1.15e-6.  While W's parts of half a chunk are multiplied, the next half's are made, four instructions of that behind each
+// multiplication, and x is read a step ahead, also over the barrier, so that the matrix units wait neither for the splitting nor for LDS:
+// 500 rows by 11264 x 2048 180 -> 153 us (all of it: 171 -> 125 on another card; the library's fp32 GEMM 195), 2048 by 22016 x 4096 2124 -> 1773 (2580),
+// 500 by 2048 x 5632 75 -> 67, 300 by 11264 x 2048 135 -> 116.  (Split beside the multiplication, but with x read where it is used: 165 and 1960.)
+// Bound by power: the second was 5930 cycles a chunk at 1.89 GHz, 3072 of them the matrix units', and is 4500 at 1.74.  So the same work dealt
+// out evenly to all compute units, where the first's 176 tiles leave 80 of them idle, takes as long (155 us).
 #pragma once
 #include "../gemm_ring.hpp"
 #include "elem.hpp"
 
 namespace dv {
 
-// A workgroup's tile (rows of W, rows of x), columns of a chunk, LDS slots for chunks.  A wave has 32 rows of W and all of x.
-constexpr int kSplitRows = 256, kSplitCols = 128, kSplitChunk = 32, kSplitThreads = 512, kSplitSlots = 2;
+// A workgroup's tile (rows of W, rows of x), columns of a chunk.  A wave has 32 rows of W and all of x.
+constexpr int kSplitRows = 256, kSplitCols = 128, kSplitChunk = 32, kSplitThreads = 512;
 
 __device__ __forceinline__ unsigned bf16_pair(float a, float b) {
   typedef bf16_t pair_t __attribute__((ext_vector_type(2)));
@@ -101,46 +103,46 @@ inline SplitPlan plan_split(int n, int M, int K, int units) {
   }
   return p;
 }
-constexpr size_t kSplitLds = (size_t)kSplitSlots * (kSplitRows * kSplitChunk * sizeof(float) + 3 * kSplitCols * kSplitChunk * sizeof(bf16_t));
+constexpr int kSplitWSlots = 3, kSplitXSlots = 2;
+constexpr size_t kSplitLds = (size_t)kSplitWSlots * kSplitRows * kSplitChunk * sizeof(float) + (size_t)kSplitXSlots * 3 * kSplitCols * kSplitChunk * sizeof(bf16_t);
+constexpr int64_t kSplitMaxStride = 1 << 25;  // 32 rows' bytes are counted in 32 bits
+constexpr int kSplitMostRows = 1 << 24;       // and those of a chunk's parts
 
 // Grid: (tiles, those of W first; splits of K).  part: with several splits, the sums [split][tile][value][thread].
 template <typename Out>
 __global__ __launch_bounds__(kSplitThreads, 2) void linear_split_kernel(SplitOperands a, int row_tiles, Out out, float4_t* __restrict__ part) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the loads' resources have no type on the host)
   extern __shared__ __attribute__((aligned(16))) unsigned char slots[];
   constexpr int KC = kSplitChunk, MB = kSplitRows, NB = kSplitCols, NT = NB / 32, WAVES = kSplitThreads / 64;
-  constexpr int WBYTES = MB * KC * 4, PLANE = NB * KC * 2, SLOT = WBYTES + 3 * PLANE, PX = kSplitPieces, PW = KC / 4;
-  constexpr int LW = WBYTES / 1024 / WAVES, LX = 3 * PLANE / 1024 / WAVES;  // a wave's loads of a chunk, 1 KiB each
-  static_assert(MB == WAVES * 32 && (LW * WAVES + LX * WAVES) * 1024 == SLOT && KC == 32, "tile");
+  constexpr int WBYTES = MB * KC * 4, PLANE = NB * KC * 2, XBYTES = 3 * PLANE, PX = kSplitPieces, PW = KC / 4;
+  constexpr int LW = WBYTES / 1024 / WAVES, LX = XBYTES / 1024 / WAVES;  // a wave's loads of a chunk, 1 KiB each
+  static_assert(MB == WAVES * 32 && LW * 64 / PW == 32 && LX * WAVES * 1024 == XBYTES && KC == 32 && kSplitXSlots == 2 && NT == 4 && LW <= 4, "tile");
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l32 = lane & 31, half = lane >> 5;
   const int m0 = blockIdx.x % row_tiles * MB, n0 = blockIdx.x / row_tiles * NB;
   const int nch = a.chunks(), c0 = nch * blockIdx.y / gridDim.y, c1 = nch * (blockIdx.y + 1) / gridDim.y;
 
   // A load is eight rows of W (eight pieces of 16 bytes each) or sixteen of a part of x (four pieces).  Pieces are exchanged by the row,
-  // so that sixteen rows' are read from different banks.
-  const float* wsrc[LW];
-  const bf16_t* xsrc[LX];
-  int step[LW];
+  // so that sixteen rows' are read from different banks.  A wave loads the 32 rows of W that it multiplies.  What is loaded for rows past the
+  // end (nothing, or other rows' values) is in results that are not stored.
+  const int w_row = min(m0 + wave * 32, a.M - 1);
+  const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.W) + w_row * a.ldw, 0,
+                                                    (int)((unsigned)(min(32, a.M - w_row) - 1) * (unsigned)a.ldw * 4u + a.K * 4u), 0x00020000);
+  const unsigned w_at = (unsigned)(lane / PW) * (unsigned)a.ldw * 4u, w_step = (unsigned)(64 / PW) * (unsigned)a.ldw * 4u;
+  const int w_col = (lane % PW ^ lane / PW) * 4;
+  const unsigned x_at = lane / PX * (KC * 2) + (lane % PX ^ (lane / PX >> 2 & 3)) * 16;
+  auto load_w = [&](int c, int slot, int i) {  // (past the end of a row its last piece: set to zero when it is used)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_ptr_t)(slots + slot * WBYTES + (wave * LW + i) * 1024), 16,
+                                             w_at + (unsigned)min(c * KC + w_col, a.K - 4) * 4u + i * w_step, 0, 0, 0);
+  };
+  auto load_x = [&](int c, int slot) {
+    const auto xr = __builtin_amdgcn_make_buffer_rsrc(a.parts + (int64_t)c * 3 * a.n * KC, 0, (int)((unsigned)a.n * (3u * KC * 2u)), 0x00020000);
 #pragma unroll
-  for (int i = 0; i < LW; ++i) {
-    const int row = (wave * LW + i) * (64 / PW) + lane / PW;
-    step[i] = (lane % PW ^ (row & 7)) * 4;
-    wsrc[i] = a.W + (int64_t)min(m0 + row, a.M - 1) * a.ldw;
-  }
-#pragma unroll
-  for (int i = 0; i < LX; ++i) {
-    const int row = (wave * LX + i) * (64 / PX) + lane / PX, s = row / NB, r = row % NB;
-    xsrc[i] = a.parts + ((int64_t)s * a.n + min(n0 + r, a.n - 1)) * KC + (lane % PX ^ (r >> 2 & 3)) * 8;
-  }
-  const int64_t xstep = (int64_t)3 * a.n * KC;
-  auto load = [&](int c, int slot) {
-    unsigned char* to = slots + slot * SLOT;
-#pragma unroll
-    for (int i = 0; i < LW; ++i)  // (past the end of a row its last piece: set to zero when it is used)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(wsrc[i] + min(c * KC + step[i], a.K - 4)), (lds_ptr_t)(to + (wave * LW + i) * 1024), 16, 0, 0);
-#pragma unroll
-    for (int i = 0; i < LX; ++i)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(xsrc[i] + c * xstep), (lds_ptr_t)(to + WBYTES + (wave * LX + i) * 1024), 16, 0, 0);
+    for (int i = 0; i < LX; ++i) {
+      const int row = (wave * LX + i) * (64 / PX), s = row / NB;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr_t)(slots + kSplitWSlots * WBYTES + slot * XBYTES + (wave * LX + i) * 1024), 16,
+                                               x_at + ((unsigned)s * a.n + n0 + row % NB) * (KC * 2u), 0, 0, 0);
+    }
   };
   float16_t sum[3][NT];  // of products of 1, 2^-8 and 2^-16 of the values' size
 #pragma unroll
@@ -152,41 +154,87 @@ __global__ __launch_bounds__(kSplitThreads, 2) void linear_split_kernel(SplitOpe
   auto add = [](float16_t& acc, const uint4_t& w, const uint4_t& x) {
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), acc, 0, 0, 0);
   };
+  const unsigned char* wb = slots + (wave * 32 + l32) * KC * 4;
+  const unsigned char* xb = slots + kSplitWSlots * WBYTES + l32 * KC * 2;
+  // The eight values of W of a lane of half a chunk.  (Read as words: with reads as floats the compiler waits for all loads into LDS
+  // in front of them.)
+  auto read_w = [&](uint4_t (&raw)[2], int c, int slot, int ks) {
+    const int p = ks * 4 + half * 2;
 #pragma unroll
-  for (int d = 0; d < kSplitSlots - 1; ++d) load(min(c0 + d, nch - 1), d);
-  int slot = 0;
-  for (int c = c0; c < c1; ++c, slot = slot == kSplitSlots - 1 ? 0 : slot + 1) {
-    // everybody's part of the slot is there, and nobody reads the one before it any more, which is loaded next
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"((LW + LX) * (kSplitSlots - 2)) : "memory");
+    for (int i = 0; i < 2; ++i) raw[i] = *reinterpret_cast<const uint4_t*>(wb + slot * WBYTES + (((p + i) ^ (l32 & 7)) * 16));
+    if ((c + 1) * KC > a.K) {  // past the end of the rows
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (c * KC + p * 4 + i * 4 >= a.K) raw[i] = uint4_t{0, 0, 0, 0};
+    }
+  };
+  auto split = [](const uint4_t (&raw)[2], uint4_t (&w)[3], int i) {
+    unsigned p[3];
+    split_pair<true>(__uint_as_float(raw[i / 2][i % 2 * 2]), __uint_as_float(raw[i / 2][i % 2 * 2 + 1]), p);
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      asm volatile("" : "+v"(p[s]));  // made here, not where it is used
+      w[s][i] = p[s];
+    }
+  };
+  auto read_x = [&](uint4_t (&x)[3], int slot, int ks, int j) {
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+      x[s] = *reinterpret_cast<const uint4_t*>(xb + slot * XBYTES + s * PLANE + j * 32 * KC * 2 + (((ks * 2 + half) ^ (l32 >> 2 & 3)) * 16));
+  };
+  if (c0 < c1) {
+    const int last = nch - 1;  // (past it: that chunk again, into slots that are not read)
+    uint4_t raw[2], w[2][3], x[2][3];
+#pragma unroll
+    for (int i = 0; i < LW; ++i) load_w(c0, 0, i);
+    load_x(c0, 0);
+#pragma unroll
+    for (int i = 0; i < LW; ++i) load_w(min(c0 + 1, last), 1, i);
+    load_x(min(c0 + 1, last), 1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(LW + LX) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    load(min(c + kSplitSlots - 1, nch - 1), slot == 0 ? kSplitSlots - 1 : slot - 1);  // (past the end: into a slot that is not read)
-    const unsigned char* wb = slots + slot * SLOT + (wave * 32 + l32) * KC * 4;
-    const unsigned char* xb = slots + slot * SLOT + WBYTES + l32 * KC * 2;
+    read_w(raw, c0, 0, 0);
+    read_x(x[0], 0, 0, 0);
 #pragma unroll
-    for (int ks = 0; ks < KC / 16; ++ks) {
-      const int p = ks * 4 + half * 2;
-      // (read as words: with reads as floats the compiler waits for all loads into LDS in front of them)
-      uint4_t w0 = *reinterpret_cast<const uint4_t*>(wb + ((p ^ (l32 & 7)) * 16));
-      uint4_t w1 = *reinterpret_cast<const uint4_t*>(wb + (((p + 1) ^ (l32 & 7)) * 16));
-      if ((c + 1) * KC > a.K) {  // past the end of the rows
-        if (c * KC + p * 4 >= a.K) w0 = uint4_t{0, 0, 0, 0};
-        if (c * KC + p * 4 + 4 >= a.K) w1 = uint4_t{0, 0, 0, 0};
+    for (int i = 0; i < 4; ++i) split(raw, w[0], i);
+    int slot = 0, x_slot = 0;
+    for (int c = c0; c < c1; ++c) {
+      const int after = slot == kSplitWSlots - 1 ? 0 : slot + 1, free_slot = slot == 0 ? kSplitWSlots - 1 : slot - 1;
+      // Eight steps: 32 rows of x by half of the columns.  While one is multiplied, x of the next is read and a pair of W's values of the
+      // next half is taken apart.
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        const int ks = g / 4, j = g % 4;
+        if (g == 0) read_w(raw, c, slot, 1);
+        if (g == 4) {
+          asm volatile("s_waitcnt vmcnt(%0)" ::"i"(LW + LX) : "memory");  // the next chunk's W
+          read_w(raw, min(c + 1, last), after, 0);
+        }
+        if (g == 7) {  // everybody's part of the next chunk's x is there (what was loaded behind it is W), and nobody reads this one's any more
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(LW) : "memory");
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+          load_x(min(c + 2, last), x_slot);
+        }
+        if (g < LW) load_w(min(c + 2, last), free_slot, g);
+        read_x(x[(g + 1) & 1], x_slot ^ (g == 7), (g + 1) / 4 & 1, (g + 1) % 4);
+        const uint4_t(&v)[3] = x[g & 1];
+        add(sum[2][j], w[ks][2], v[0]);
+        add(sum[0][j], w[ks][0], v[0]);
+        add(sum[1][j], w[ks][1], v[0]);
+        add(sum[2][j], w[ks][1], v[1]);
+        add(sum[1][j], w[ks][0], v[1]);
+        add(sum[2][j], w[ks][0], v[2]);
+        split(raw, w[ks ^ 1], j);
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {  // four of the splitting's instructions behind each multiplication
+          __builtin_amdgcn_sched_group_barrier(8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(2, 4, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      uint4_t w[3], x[3];
-      split8<true>(__builtin_bit_cast(float4_t, w0), __builtin_bit_cast(float4_t, w1), w);
-#pragma unroll
-      for (int j = 0; j < NT; ++j) {
-#pragma unroll
-        for (int s = 0; s < 3; ++s)
-          x[s] = *reinterpret_cast<const uint4_t*>(xb + s * PLANE + j * 32 * KC * 2 + (((ks * 2 + half) ^ (l32 >> 2 & 3)) * 16));
-        add(sum[0][j], w[0], x[0]);
-        add(sum[1][j], w[1], x[0]);
-        add(sum[2][j], w[2], x[0]);
-        add(sum[1][j], w[0], x[1]);
-        add(sum[2][j], w[1], x[1]);
-        add(sum[2][j], w[0], x[2]);
-      }
+      slot = after, x_slot ^= 1;
     }
   }
   wait_loads<0>();  // no load into LDS outlives the workgroup
@@ -208,6 +256,7 @@ __global__ __launch_bounds__(kSplitThreads, 2) void linear_split_kernel(SplitOpe
         if (m < a.M && n < a.n) out(m, n, v);
       }
     }
+#endif
 }
 
 // Adds the splits' sums up, in their order.  Grid: (tiles, values of a thread).

@@ -562,6 +562,7 @@ int dv_mix_linear_split(const float* x, int64_t ldx, const float* W, int64_t ldw
                         int64_t ldo, void* workspace, size_t workspace_bytes, void* stream) {
   if (!x || !W || !out || n < 1 || M < 1 || K < 4) return DV_ERR_INVALID_ARG;
   if (M % 4 || K % 4 || ldx % 4 || ldw % 4 || ldo % 4 || !al16(x) || !al16(W) || !al16(bias) || !al16(out)) return DV_ERR_ALIGNMENT;
+  if (ldw >= kSplitMaxStride || K >= kSplitMaxStride || n >= kSplitMostRows) return DV_ERR_UNSUPPORTED;
   const SplitPlan p = plan_split(n, M, K, compute_units());
   if (!workspace || workspace_bytes < p.workspace_bytes(n)) return DV_ERR_WORKSPACE;
   if (!al16(workspace)) return DV_ERR_ALIGNMENT;

@@ -194,15 +194,16 @@ def _product_ok(x, W):
 # fp32 products by parts in bf16 (linear_split.hpp), which are as exact as fp32 products for values of any range, where what the launches take
 # (``_split_us``: a round of tiles 2.2 us a chunk of columns, splits of K 4 us and 0.05 for each tile, all launches 8) is less than the
 # library's fp32 GEMM does at 118 TFLOP/s; it ranges from 85 to 140.  Times the library's speed: 11264 x 2048 with 256 / 400 / 500 /
-# 1000 / 2000 rows 1.03 / 1.10 / 1.27 / 1.25 / 1.31, 2048 x 5632 with 400 / 500 / 1000 1.14 / 1.07 / 1.13, 4368 x 2048 with 384 / 512 1.03 /
-# 1.46, 22016 x 4096 with 200 / 500 / 1000 / 2048 1.15 / 1.23 / 1.42 / 1.25, 500 by 3072 x 2048 1.11, 300 by 8192 x 4096 1.11, 200 by 4096 x
-# 11008 1.21, 4000 by 4096 x 512 1.24.  Left to the library: too little for the launches (500 by 2048 x 2048 0.91, 256 by 2048 x 5632 0.77, 260
-# by 4368 x 2048 0.81, 400 0.95, 2000 by 1024 x 1024 0.84), tiles that are half empty (161 by 11264 x 2048 0.91, 161 by 22016 x 4096
-# 0.99; but 300 by 11264 x 2048 1.14).  On the line: 300 by 22016 x 4096 0.98, 300 by 4096 x 4096 1.00, 2000 by 2048 x 768 0.96.
+# 1000 / 2000 rows 1.30 / 1.28 / 1.56 / 1.41 / 1.50, 2048 x 5632 with 400 / 500 / 1000 1.18 / 1.15 / 1.22, 4368 x 2048 with 384 / 500 1.10 /
+# 1.58, 22016 x 4096 with 200 / 500 / 1000 / 2048 1.32 / 1.42 / 1.61 / 1.46, 500 by 3072 x 2048 1.18, 300 by 8192 x 4096 1.20, 200 by 4096 x
+# 11008 1.32, 4000 by 4096 x 512 1.31.  Left to the library: too little for the launches (500 by 2048 x 2048 0.91, 256 by 2048 x 5632 0.93, 200
+# by 4368 x 2048 0.89, 2000 by 1024 x 1024 0.87), and where its own speed, which jumps with the sizes, decides (161 by 11264 x 2048 1.13, 161 by
+# 22016 x 4096 1.08, 400 by 4368 x 2048 1.02).  On the line: 300 by 22016 x 4096 1.07, 300 by 4096 x 4096 1.07, 2000 by 2048 x 768 1.00.
 SPLIT_MIN_ROWS, SPLIT_COLUMNS = 161, 512
 SPLIT_RATE = 59_000_000        # products a us (118 TFLOP/s) that the tiles have to reach
 SPLIT_VALUES = 1 << 27         # of x, whose parts take 6 bytes each: beyond, the library, which needs no memory for them
 SPLIT_TILE, SPLIT_CHUNK, SPLIT_ROUND = (256, 128), 32, 256
+SPLIT_MAX_STRIDE = 1 << 25     # 32 rows' bytes are counted in 32 bits
 
 
 @lru_cache(maxsize=4096)
@@ -227,6 +228,7 @@ def _split_product(x: torch.Tensor, W: torch.Tensor, bias=None) -> Optional[torc
     """``F.linear`` of fp32 rows by the kernel that multiplies parts in bf16; None where the library takes them."""
     (n, K), M = x.shape, W.shape[0]
     if (x.dtype != torch.float32 or not _split_rule(n, M, K) or M % 4 or K % 4 or not results_only(x, W, bias) or
+            W.stride(0) >= SPLIT_MAX_STRIDE or
             any(t.stride(0) % 4 or t.data_ptr() % 16 for t in (x, W)) or (bias is not None and bias.data_ptr() % 16)):
         return None
     out = torch.empty(n, M, dtype=torch.float32, device=x.device)

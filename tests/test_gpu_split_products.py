@@ -140,3 +140,16 @@ def test_which_products_are_split(n, M, K, taken):
     from dejavu_amd import mixer_ops
 
     assert mixer_ops._split_rule(n, M, K) == taken
+
+
+@pytest.mark.parametrize("stride,taken", [(2 ** 25 - 4, True), (2 ** 25, False)])
+def test_rows_of_a_weight_that_are_far_apart(ops, stride, taken):
+    """32 rows' bytes are counted in 32 bits."""
+    x, W, _ = operands(8, 40, 68)
+    room = torch.empty(39 * stride + 68, device="cuda")
+    far = room.as_strided((40, 68), (stride, 1))
+    far.copy_(W)
+    got = ops._split_product(x, far)
+    assert (got is not None) == taken
+    if taken:
+        assert torch.equal(got, ops._split_product(x, W))
