@@ -54,46 +54,62 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvArgs a) {
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) w[j][e] = wv[(e * TAPS + j) >> 2][(e * TAPS + j) & 3];
   }
-  float bias[8];
+  typedef float part_t __attribute__((ext_vector_type(4), aligned(4)));
+  part_t bias[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  if (a.b) {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) bias[e] = a.b ? a.b[ch + e] : 0.f;
+    for (int i = 0; i < 2; ++i) bias[i] = *reinterpret_cast<const part_t*>(a.b + ch + i * 4);
+  }
   const int t0 = blockIdx.y * kConvTokens, t1 = min(a.n, t0 + kConvTokens);
   Pack8<T> next[kConvTokens];
 #pragma unroll
   for (int i = 0; i < kConvTokens; ++i) {
     next[i].load(in + (int64_t)min(t0 + i, t1 - 1) * a.ldi);
   }
-#pragma unroll
-  for (int j = 0; j < TAPS - 1; ++j) {  // the inputs before the block
-    const int s = t0 - (TAPS - 1) + j;
-    Pack8<T> v;
-    v.load(in + (int64_t)max(s, 0) * a.ldi);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) u[j][e] = v.get(e);
-    if (s < 0) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) u[j][e] = a.state[(int64_t)(ch + e) * (TAPS - 1) + TAPS - 1 + s];
-    }
-  }
-  // The state behind the last row: by the lanes that have read the one before the first (no other block reads it).
+  // The inputs before the block, which are the state of the first one; and the state behind the last row, by the lanes that have read the
+  // one before the first (no other block reads it).  All blocks are at work at once, so what the first does beside its rows lasts as long as the
+  // launch: a lane's state goes in pieces of 16 bytes (one value at a time 47 rows of 2048 channels took 13.6 us, now 10.1, 2048 rows of
+  // 1536 21.5, now 16.6).
   static_assert(kConvTokens >= TAPS - 1, "the first block alone reads the state");
-  if (TAPS > 1 && a.next_state && blockIdx.y == 0 && on) {
-    Pack8<T> last[TAPS];
-#pragma unroll
-    for (int j = 0; j < TAPS - 1; ++j) last[j].load(in + (int64_t)max(a.n - (TAPS - 1) + j, 0) * a.ldi);
+  if (blockIdx.y > 0) {
 #pragma unroll
     for (int j = 0; j < TAPS - 1; ++j) {
-      const int s = a.n - (TAPS - 1) + j;
+      Pack8<T> v;
+      v.load(in + (int64_t)(t0 - (TAPS - 1) + j) * a.ldi);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float v = last[j].get(e);
-        if (s < 0) {
+      for (int e = 0; e < 8; ++e) u[j][e] = v.get(e);
+    }
+  } else if constexpr (TAPS > 1) {
+    constexpr int PARTS = 2 * (TAPS - 1);
+    const float* from = a.state + (int64_t)ch * (TAPS - 1);
+    part_t st[PARTS];
+    Pack8<T> last[TAPS];
 #pragma unroll
-          for (int k = 1; k < TAPS - 1; ++k)
-            if (k == j + a.n) v = u[k][e];
+    for (int i = 0; i < PARTS; ++i) st[i] = *reinterpret_cast<const part_t*>(from + i * 4);
+    if (a.next_state) {
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j) last[j].load(in + (int64_t)max(a.n - (TAPS - 1) + j, 0) * a.ldi);
+    }
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) u[j][e] = st[(e * (TAPS - 1) + j) >> 2][(e * (TAPS - 1) + j) & 3];
+    if (a.next_state && on) {
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          float v = last[j].get(e);
+          if (a.n - (TAPS - 1) + j < 0) {
+#pragma unroll
+            for (int k = 1; k < TAPS - 1; ++k)
+              if (k == j + a.n) v = u[k][e];
+          }
+          st[(e * (TAPS - 1) + j) >> 2][(e * (TAPS - 1) + j) & 3] = v;
         }
-        a.next_state[(int64_t)(ch + e) * (TAPS - 1) + j] = v;
-      }
+      float* to = a.next_state + (int64_t)ch * (TAPS - 1);
+#pragma unroll
+      for (int i = 0; i < PARTS; ++i) *reinterpret_cast<part_t*>(to + i * 4) = st[i];
     }
   }
   TO* out = reinterpret_cast<TO*>(g.out) + (int64_t)h * g.stride + c;
@@ -103,7 +119,7 @@ __global__ __launch_bounds__(256) void short_conv_kernel(ConvArgs a) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       u[TAPS - 1][e] = next[i].get(e);
-      float v = bias[e];
+      float v = bias[e >> 2][e & 3];
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) v = __builtin_fmaf(w[j][e], u[j][e], v);
       y[e] = a.silu ? silu_f(v) : v;
