@@ -482,8 +482,8 @@ int ring_scratch(const RingPlan& p, const void* workspace, size_t workspace_byte
 }
 
 // Which kernel takes a product of B rows.  From 65 rows on the ring (12288 x 4096 with 100 / 190 / 256 rows: 31 / 38 / 46 us
-// against 39 / 59 / 57; QKV of 24 heads of 9216 with 96 / 160 / 240 rows 46 / 56 / 68 against 53 / 90 / 124; 32 heads of
-// 12288 with 320 and 480 rows 191 and 195 against 208 and 214 with gemm_big.hpp; 5120 x 20480 with 384 rows 134 against 245),
+// against 39 / 59 / 57; QKV of 24 heads of 9216 with 96 / 160 / 240 rows 46 / 56 / 68 against 53 / 90 / 124, of which a window's go
+// to qkv_window.hpp; 5120 x 20480 with 384 rows 134 against 245),
 // but not plain products of more than 512 rows, or of more than 40960 rows of W and 256, which gemm_big.hpp takes where its
 // chunks divide N (50272 x 4096 with 300 / 400 rows: the ring 259 / 309, that 243 / 349; 36864 x 4096 199 / 237 against 195 / 242, 20480
 // x 5120 105 / 165 against 132 / 200), nor of up to 128 rows and more than 32768 of W, which are more than a round of tiles
@@ -513,7 +513,7 @@ size_t tiled_workspace_bytes(int B, int N, int M, bool qkv = false) {
 }
 
 // Many rows of X (callers of dv_dense_linear_f16 itself: the modules' products have 192 rows at most, up to 512 where the
-// weight's rows are long): the product is bound by the matrix cores and by what
+// weight's rows are long, and ask for the wide tiles beyond) that the wide tiles do not take: the product is bound by the matrix cores and by what
 // the L2 delivers, and gemm_big_mfma_kernel (weights straight into MFMA operands, 64 * WT weight rows
 // per workgroup) is the faster kernel -- measured at 12288 x 12288 against gemm_tiled_mfma_kernel:
 // 512 rows 225 against 278 us, 2048 rows 793 against 797 us.  Same bits.
