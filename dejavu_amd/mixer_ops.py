@@ -137,12 +137,19 @@ def _wide_rule(n: int, M: int, K: int) -> bool:
 # 8192 x 4096 with 777 / 1200 / 1999 1.16 / 1.09 / 0.99, but with 512 0.85; 11264 x 2048 with 400 / 640 / 1000 / 1700 / 1999 1.15 / 1.18 / 1.22 / 1.29 / 1.08, with 300 0.97;
 # 6144 x 2048 with 777 / 1000 1.03 / 1.14, with 640 0.92.  Plain: 11264 x 2048 with 400 / 640 / 1000 / 1700 / 1999 1.10 / 0.99 / 1.12 / 1.22 / 1.00, 9216 x 2048 with 777 / 1000 /
 # 1700 / 1999 1.06 / 1.21 / 0.95 / 1.19, 4368 x 2048 with 1200 / 1700 / 2048 1.13 / 1.19 / 1.24, with 777 0.89.
+# Gated units of 2049 to 8192 rows: 22016 x 4096 with 2100 / 2560 / 3000 / 4096 / 6000 / 8192 rows 1.50 / 0.95 / 1.20 / 1.10 / 1.04 / 1.14, 18560 x 4096 1.00 / 1.24 /
+# 1.02 / 1.28 / 1.17 / 1.03, 12288 x 4096 1.07 / 0.94 / 1.09 / 0.99 / 1.27 / 0.98, 11264 x 2048 1.08 / 0.97 / 1.10 / 1.15 / 1.27 / 1.19, but 8192 x 4096 1.15 / 1.05 / 1.09 /
+# 0.98 / 0.99 / 0.96.
 WIDE_FEW_COLUMNS, WIDE_GATED_COLUMNS = 2048, 8192
+WIDE_LONG_GATED = 8192, 11264, 4096    # rows at most, weight rows at least, columns at most
 WIDE_FILL_GATED, WIDE_FILL_FEW_GATED, WIDE_FILL_FEW = 200, 144, 176
 
 
 def _fill_rule(n: int, M: int, K: int, gated: bool) -> bool:
-    if not TILE_MAX_ROWS < n <= WIDE_MAX_ROWS or not 1024 <= K <= WIDE_GATED_COLUMNS or (K > WIDE_FEW_COLUMNS and not gated):
+    if n <= TILE_MAX_ROWS or not 1024 <= K <= WIDE_GATED_COLUMNS or (K > WIDE_FEW_COLUMNS and not gated):
+        return False
+    most, rows, columns = WIDE_LONG_GATED
+    if n > (most if gated and M >= rows and K <= columns else WIDE_MAX_ROWS):
         return False
     fill = (WIDE_FILL_FEW_GATED if gated else WIDE_FILL_FEW) if K <= WIDE_FEW_COLUMNS else WIDE_FILL_GATED
     return _tiles_of(n, M, 128, WIDE_TILE) >= fill

@@ -62,8 +62,11 @@ HIP_PROMPT_LONG_WEIGHT_ROWS = 4096, 8192
 # of 128 rows by 256 weight rows are so many (below 4096 columns / from there on; the library's time over the kernel's: 8192 x 2048 with 400 / 600 /
 # 777 / 1200 / 2000 rows 1.07 / 1.18 / 1.36 / 1.28 / 1.11, 16384 x 4096 1.16 / 1.14 / 1.16 / 1.10 / 1.00, 20480 x 5120 with 400 / 600 / 777 / 1000 / 1435 / 2000 rows 1.02 / 1.27 /
 # 1.06 / 0.91 / 1.08 / 1.41; with 257 rows 0.98 to 1.01), and fc2 whose rows are the longest (5120 x 20480 with 777 / 1000 / 1200 / 1700 / 2000 rows 1.04 / 1.06 /
-# 1.17 / 1.66 / 0.96, 9216 x 36864 0.98 / 1.02 / 1.49 with 777 / 1200 / 2000, but 4096 x 16384 with 1200 0.90).
+# 1.17 / 1.66 / 0.96, 9216 x 36864 0.98 / 1.02 / 1.49 with 777 / 1200 / 2000, but 4096 x 16384 with 1200 0.90).  Of more than 2048 rows fc1 with up to 5120
+# columns (2100 / 2560 / 3000 / 4096 / 6000 / 8192 rows: 16384 x 4096 1.24 / 1.47 / 1.00 / 1.02 / 1.01 / 1.00, 20480 x 5120 1.01 / 1.16 / 1.06 / 1.04 / 1.04 / 1.01, 8192 x 2048
+# 1.36 / 1.19 / 1.19 / 1.07 / 1.05 / 1.04; but 36864 x 9216 1.02 / 0.90 / 0.94 / 0.93 / 0.95 / 0.93, and fc2 of 5120 x 20480 1.01 / 1.23 / 0.93 / 0.96 / 1.33 / 1.31).
 HIP_PROMPT_WIDE_ROWS = 257, 2048
+HIP_PROMPT_WIDE_LONGEST = 8192, 5120   # rows, columns
 HIP_PROMPT_WIDE_COLUMNS, HIP_PROMPT_WIDE_FILL = (2048, 4096), (128, 256)
 HIP_PROMPT_WIDE_LONG = 768, 20480      # rows, columns
 HIP_PROMPT_WIDE_STRIDE = 1 << 25
@@ -290,7 +293,10 @@ def _long_rule(rows: int, M: int, K: int) -> bool:
 
 
 def _wide_rule(rows: int, M: int, K: int, activation: str) -> bool:
-    if not HIP_PROMPT_WIDE_ROWS[0] <= rows <= HIP_PROMPT_WIDE_ROWS[1] or activation not in ("id", "relu", "squared_relu"):
+    if rows < HIP_PROMPT_WIDE_ROWS[0] or activation not in ("id", "relu", "squared_relu"):
+        return False
+    most, columns = HIP_PROMPT_WIDE_LONGEST
+    if rows > (most if activation != "id" and K <= columns else HIP_PROMPT_WIDE_ROWS[1]):
         return False
     if activation == "id":
         return K >= 4 * M and K >= HIP_PROMPT_WIDE_LONG[1] and rows >= HIP_PROMPT_WIDE_LONG[0]

@@ -106,12 +106,13 @@ def test_which_products_the_wide_kernel_takes():
     """Gated units and few columns on both sides of the lines; each was measured with its weights out of the caches."""
     from dejavu_amd.mixer_ops import _fill_rule
 
-    for n, M, K in ((400, 22016, 4096), (2048, 22016, 4096), (1999, 18560, 4096), (640, 12288, 4096), (777, 8192, 4096)):
+    for n, M, K in ((400, 22016, 4096), (2048, 22016, 4096), (1999, 18560, 4096), (640, 12288, 4096), (777, 8192, 4096),
+                    (2049, 22016, 4096), (8192, 11264, 4096)):
         assert _fill_rule(n, M, K, True) and not _fill_rule(n, M, K, False), (n, M, K)
     for n, M, K in ((400, 11264, 2048), (2048, 11264, 2048), (1000, 9216, 2048), (1200, 6144, 2048), (1999, 4368, 2048)):
         assert _fill_rule(n, M, K, True) and _fill_rule(n, M, K, False), (n, M, K)
-    for n, M, K in ((256, 22016, 4096), (512, 8192, 4096), (1200, 4096, 4096), (300, 11264, 2048), (640, 6144, 2048), (2049, 22016, 4096),
-                    (1000, 22016, 16384)):
+    for n, M, K in ((256, 22016, 4096), (512, 8192, 4096), (1200, 4096, 4096), (300, 11264, 2048), (640, 6144, 2048), (8193, 22016, 4096), (2049, 8192, 4096),
+                    (2049, 22016, 8192), (1000, 22016, 16384)):
         assert not _fill_rule(n, M, K, True) and not _fill_rule(n, M, K, False), (n, M, K)
 
 
@@ -150,7 +151,9 @@ def test_gated_units_through_the_ops():
     W = (torch.randn(9200, 2048, generator=g, device="cuda") / 45).to(torch.bfloat16)
     x = torch.randn(385, 2048, generator=g, device="cuda").to(torch.bfloat16)
     assert ops._fills(x, W, gated=True) and not ops._fills(x[:384], W, gated=True) and not ops._wide(x, W)
-    for rows in (384, 385):
+    W2, x2 = W.repeat(2, 1)[:11264], x.repeat(22, 1)[:8193]
+    assert ops._fills(x2[:8192], W2, gated=True) and not ops._fills(x2, W2, gated=True)
+    for x, W, rows in ((x, W, 384), (x, W, 385), (x2, W2, 2049), (x2, W2, 8192), (x2, W2, 8193)):
         want = x[:rows].float() @ W.float().t()
         unit = want[:, 0::2].clamp(min=0) * want[:, 1::2]
         got = ops.relu_glu(x[:rows], W).float()
@@ -160,9 +163,9 @@ def test_gated_units_through_the_ops():
 def test_which_products_of_a_prompt_the_wide_kernel_takes():
     from dejavu_amd.modules import _wide_rule as rule
 
-    for rows, M, K in ((400, 8192, 2048), (777, 16384, 4096), (512, 20480, 5120), (2000, 16384, 4096)):
+    for rows, M, K in ((400, 8192, 2048), (777, 16384, 4096), (512, 20480, 5120), (2000, 16384, 4096), (8192, 20480, 5120)):
         assert rule(rows, M, K, "relu") and rule(rows, M, K, "squared_relu") and not rule(rows, M, K, "id") and not rule(rows, M, K, "gelu")
-    for rows, M, K in ((256, 16384, 4096), (300, 16384, 4096), (257, 8192, 2048), (2049, 16384, 4096), (777, 3072, 768)):
+    for rows, M, K in ((256, 16384, 4096), (300, 16384, 4096), (257, 8192, 2048), (8193, 16384, 4096), (2049, 36864, 9216), (777, 3072, 768)):
         assert not rule(rows, M, K, "relu"), (rows, M, K)
     assert rule(777, 5120, 20480, "id") and not rule(767, 5120, 20480, "id") and not rule(1200, 4096, 16384, "id")
 
@@ -199,6 +202,11 @@ def test_long_prompts_through_the_layers():
             want = torch.relu(layer(x[:, :rows]))
             got = modules.decode_linear(layer, x[:, :rows], "relu")
             assert got.shape == want.shape and (got - want).abs().max() <= 2.0 ** -9 * want.abs().max()
+        long = x.repeat(1, 21, 1)[:, :8193]
+        for rows in (2049, 8192, 8193):
+            assert modules._wide_product(layer, long[:, :rows], "relu") == (rows < 8193)
+            want, got = torch.relu(layer(long[:, :rows])), modules.decode_linear(layer, long[:, :rows], "relu")
+            assert (got - want).abs().max() <= 2.0 ** -9 * want.abs().max()
         assert not modules._wide_product(layer, x[:, ::2].expand(1, 200, 2048), "relu")
         seen = []
         hook = layer.register_forward_hook(lambda *a: seen.append(1))
