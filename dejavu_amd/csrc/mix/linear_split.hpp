@@ -15,9 +15,9 @@
 // Six bf16 products at 2.5 PFLOP/s are 2.6 times the fp32 instructions' 157 TFLOP/s.  From 64 bits 2.7e-7 (K = 2048) and 4e-7 (4096), the library
 // 8.1e-7 and 1.15e-6.  While W's parts of half a chunk are multiplied, the next half's are made, four instructions of that behind each
 // multiplication, and x is read a step ahead, also over the barrier, so that the matrix units wait neither for the splitting nor for LDS:
-// 500 rows by 11264 x 2048 180 -> 153 us (all of it: 171 -> 125 on another card; the library's fp32 GEMM 195), 2048 by 22016 x 4096 2124 -> 1773 (2580),
+// 500 rows by 11264 x 2048 180 -> 153 us (inside a prompt 170 -> 127, where the library's fp32 GEMM takes 195 with its weight cold), 2048 by 22016 x 4096 2124 -> 1773 (2580),
 // 500 by 2048 x 5632 75 -> 67, 300 by 11264 x 2048 135 -> 116.  (Split beside the multiplication, but with x read where it is used: 165 and 1960.)
-// Bound by power: the second was 5930 cycles a chunk at 1.89 GHz, 3072 of them the matrix units', and is 4500 at 1.74.  So the same work dealt
+// Bound by power: the second was 5930 cycles a chunk at 1.89 GHz, 3072 of them the matrix units', and is 4080 at 1.64.  So the same work dealt
 // out evenly to all compute units, where the first's 176 tiles leave 80 of them idle, takes as long (155 us).
 #pragma once
 #include "../gemm_ring.hpp"
