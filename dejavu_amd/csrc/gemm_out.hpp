@@ -120,7 +120,8 @@ struct PlainOut {
   }
 };
 
-// The same as gemm_wide.hpp stores it, for the activations that are cheap enough to stand there once for every sum.
+// The same as gemm_wide.hpp stores it, for the activations that are cheap enough to stand there once for every sum.  It stands in
+// for the library's product with the activation behind it, so a sum that is no number stays one (act_f makes it zero).
 template <int ACT>
 struct WidePlainOut {
   static constexpr int kOuts = 4;
@@ -141,7 +142,11 @@ struct WidePlainOut {
   __device__ __forceinline__ half4_t make(const Row& r, const float4_t& v) const {
     half4_t o;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = (half_t)act_f(v[e] + (float)r.v[e], ACT);
+    for (int e = 0; e < 4; ++e) {
+      float s = v[e] + (float)r.v[e];
+      if (ACT != 0) s = s < 0.f ? 0.f : s;
+      o[e] = (half_t)(ACT == 4 ? s * s : s);
+    }
     return o;
   }
 };

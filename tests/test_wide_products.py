@@ -190,6 +190,30 @@ def test_wide_products_in_fp16(n, M, K, act):
 
 
 @pytest.mark.gpu
+@torch.no_grad()
+@pytest.mark.parametrize("act", ["id", "relu", "squared_relu"])
+def test_values_that_are_no_finite_numbers(act):
+    """They are where the library and a launch for the activation have them: NaN and both infinities in rows, weight and bias."""
+    from dejavu_amd import modules, ops
+
+    inf, nan = float("inf"), float("nan")
+    layer = torch.nn.Linear(2048, 8192, device="cuda", dtype=torch.float16)
+    layer.bias[17:20] = torch.tensor([nan, inf, -inf], dtype=torch.float16)
+    layer.weight[300, 5], layer.weight[301, 6], layer.weight[302, 7] = nan, inf, -inf
+    x = torch.randn(1, 400, 2048, device="cuda").half()
+    x[0, 3, 100], x[0, 130, 101], x[0, 399, 102] = nan, inf, -inf
+    y = torch.nn.functional.linear(x, layer.weight, layer.bias)
+    want = {"id": y, "relu": torch.relu(y), "squared_relu": torch.relu(y) ** 2}[act]
+    results = [ops.dense_linear_wide(x, layer.weight, layer.bias, act)]
+    if act != "id":
+        assert modules._wide_product(layer, x, act)
+        results.append(modules.decode_linear(layer, x, act))
+    for got in results:
+        assert want.isnan().sum() > 8192 and torch.equal(got.isnan(), want.isnan())
+        assert want.isinf().any() and torch.equal(got.isinf(), want.isinf()) and torch.equal(got[want.isinf()], want[want.isinf()])
+
+
+@pytest.mark.gpu
 def test_long_prompts_through_the_layers():
     """fc1 with its activation on both sides of the rule's line, and what only the library does."""
     from dejavu_amd import modules
