@@ -597,19 +597,23 @@ class ParallelMHASparseAttMlp(_MHABase):
         else:
             self.cache_offset.fill_(value)
 
-    def reset_window(self, cache_offset: Optional[int] = None):
-        """A new window; cache_offset: where it lies in the caches."""
+    def reset_window(self, cache_offset: Optional[int] = None, device=None):
+        """A new window; cache_offset: where it lies in the caches, kept on ``device`` (the tracker's)."""
         self.counter = 0
-        t = self.tracker
-        if not (t.is_cuda and t.dtype == torch.int32 and t.is_contiguous() and t.shape == (self.num_heads, self.WINDOW)):
+        t, place = self.tracker, self.cache_offset
+        device = t.device if device is None else device
+        # callers may have put tensors of their own in both places
+        plain = (results_only(t, place) and device == t.device and t.dtype == torch.int32 and t.is_contiguous() and
+                 t.shape == (self.num_heads, self.WINDOW) and (place is None or (place.dtype == torch.int32 and place.numel() == 1)))
+        if not plain:
             if cache_offset is not None:
-                self._set_cache_offset(cache_offset, t.device)
+                self._set_cache_offset(cache_offset, device)
             t.copy_(torch.arange(self.WINDOW, dtype=torch.int32, device=t.device).repeat(self.num_heads, 1))
             return
-        if cache_offset is not None and self.cache_offset is None:
-            self.cache_offset = torch.empty(1, dtype=torch.int32, device=t.device)
+        if cache_offset is not None and place is None:
+            place = self.cache_offset = torch.empty(1, dtype=torch.int32, device=device)
         # one launch (two fills, an arange and a copy: 15 to 20 us a block of a prompt)
-        check(lib.dv_window_reset(t.data_ptr(), self.num_heads, None if cache_offset is None else self.cache_offset.data_ptr(),
+        check(lib.dv_window_reset(t.data_ptr(), self.num_heads, None if cache_offset is None else place.data_ptr(),
                                   cache_offset or 0, ops._stream()), "dv_window_reset")
 
     def _sparse_decode(self, x, head_idx, inference_params):
@@ -723,7 +727,7 @@ class ParallelMHASparseAttMlp(_MHABase):
         self._streams()
         do_token_generation = x.size(1) == 1
         if x.size(1) != 1:  # prompt: remember where the decode window starts
-            self.reset_window(x.size(1))
+            self.reset_window(x.size(1), x.device)
         sparse = inference_params is not None and inference_params.sequence_len_offset > 0 and head_idx is not None
         self._side_fork(x.shape[0])
         side_done = None

@@ -222,3 +222,46 @@ def test_longest_prompts_of_the_attention_kernel(T, H, hd, ours, monkeypatch):
     s = (q[:, -3:] @ k.transpose(1, 2).contiguous()) * hd ** -0.5
     s[:, 0, -2:], s[:, 1, -1:] = -math.inf, -math.inf
     torch.testing.assert_close(got, (s.softmax(-1) @ v.contiguous()).transpose(0, 1), rtol=1e-3, atol=5e-3)
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+def test_new_windows_that_only_the_library_begins(monkeypatch):
+    """A traced reset is in the trace, and trackers and places of a caller's own, of another type, device or stride, are written as
+    ever; so are those that the kernel writes."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from dejavu_amd import modules
+
+    launches, kernel = [], modules.lib.dv_window_reset
+    monkeypatch.setattr(modules.lib, "dv_window_reset", lambda *a: [launches.append(1), kernel(*a)][1])
+    H, here = 3, torch.device("cuda", torch.cuda.current_device())
+    mha = modules.ParallelMHASparseAttMlp(192, H, None, dict(embed_dim=192, low_rank_dim=8, out_dim=H, K=1), causal=True, layer_idx=0,
+                                          device="cuda", dtype=torch.float16)
+    plain, fresh = mha.tracker, torch.arange(16).int().repeat(H, 1)
+    new = lambda value, **kw: torch.tensor([value], **{"dtype": torch.int32, "device": "cuda", **kw})  # noqa: E731
+    other = {"int64 tracker": (plain.long(), new(-1)), "strided tracker": (torch.zeros(16, H, dtype=torch.int32, device="cuda").t(), new(-1)),
+             "tracker on the CPU": (plain.cpu(), None), "int64 place": (plain, new(-1, dtype=torch.int64)),
+             "place on the CPU": (plain, new(-1, device="cpu")), "two places": (plain, new(-1).repeat(2))}
+    for name, (tracker, place) in [("plain", (plain, new(-1))), ("no place yet", (plain, None)), *other.items()]:
+        mha.tracker, mha.cache_offset = tracker.fill_(-7), place
+        launches.clear()
+        mha.reset_window(123, here)
+        assert bool(launches) == (name in ("plain", "no place yet")), name
+        assert torch.equal(mha.tracker.cpu(), fresh.to(tracker.dtype)) and (mha.cache_offset.cpu() == 123).all(), name
+        assert place is mha.cache_offset or (place is None and mha.cache_offset.device == here), name
+        mha.tracker.fill_(-7)
+        mha.reset_window()
+        assert torch.equal(mha.tracker.cpu(), fresh.to(tracker.dtype)) and (mha.cache_offset.cpu() == 123).all(), name
+
+    mha.tracker, mha.cache_offset = plain, new(-1)
+    zero = torch.zeros(1, dtype=torch.int32, device="cuda")
+    traced = make_fx(lambda t: [mha.reset_window(7, here), mha.tracker + t, mha.cache_offset + t][1:])(zero)
+    plain.fill_(-7), mha.cache_offset.fill_(-1)
+    tracker, place = traced(zero)
+    assert torch.equal(tracker.cpu(), fresh) and torch.equal(plain.cpu(), fresh) and place.item() == mha.cache_offset.item() == 7
+    with monkeypatch.context() as m:  # as on another device than the current one
+        m.setattr(modules, "results_only", lambda *tensors: False)
+        launches.clear(), plain.fill_(-7)
+        mha.reset_window(9, here)
+        assert not launches and torch.equal(plain.cpu(), fresh) and mha.cache_offset.item() == 9
