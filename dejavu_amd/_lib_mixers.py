@@ -40,7 +40,7 @@ TileArgs = _struct("TileArgs", ("x", _p), ("ldx", _l), ("W", _p), ("ldw", _l), (
 ConvGroup = _struct("ConvGroup", ("heads", _i), ("stride", _i), ("dim", _i), ("norm", _i), ("eps", _f), ("scale", _f),
                     ("out", _p), ("ld", _l))
 ConvArgs = _struct("ConvArgs", ("in_", _p), ("ldi", _l), ("n", _i), ("taps", _i), ("silu", _i), ("w", _p),
-                   ("b", _p), ("state", _p), ("g", ConvGroup * 3), ("next_state", _p))
+                   ("b", _p), ("state", _p), ("g", ConvGroup * 3))
 RmsRows = _struct("RmsRows", ("x", _p), ("dim", _i), ("padded", _i), ("w", _p), ("y", _p), ("ldy", _l))
 RingRows = _struct("RingRows", ("buf", _p), ("ldb", _l), ("ring", _p), ("ldr", _l), ("width", _i))
 HeadGroup = _struct("HeadGroup", ("heads", _i), ("stride", _i), ("dim", _i), ("w", _p), ("eps", _f), ("other", _p),
@@ -90,6 +90,7 @@ SIGNATURES = {
     "dv_mix_linear_split": (_i, [_p, _l, _p, _l, _p, _i, _i, _i, _p, _l, _p, ctypes.c_size_t, _p]),
     "dv_mix_linear_wide": (_i, [_i, _P(TileArgs), _p]),
     "dv_mix_short_conv": (_i, [_i, _i, _P(ConvArgs), _p]),
+    "dv_mix_short_conv_move": (_i, [_i, _i, _P(ConvArgs), _p, _p]),
     "dv_mix_conv_state": (_i, [_i, _p, _l, _i, _i, _i, _p, _p]),
     "dv_mix_ring_copy": (_i, [_i, _p, _l, _p, _i, _l, _i, _i, _i, _i, _p]),
     "dv_mix_ring_copy_two": (_i, [_i, _P(RingRows), _P(RingRows), _i, _i, _i, _i, _p]),

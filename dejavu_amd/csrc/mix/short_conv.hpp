@@ -5,7 +5,9 @@
 namespace dv {
 
 using ConvGroup = dvConvGroup;
-using ConvArgs = dvConvArgs;
+struct ConvArgs : dvConvArgs {
+  float* next_state;  // null, or where the state behind the last row goes (may be `state`)
+};
 
 // A lane owns eight channels of one head and walks TB consecutive tokens with the last TAPS inputs in registers; the
 // LPH lanes of a head (a power of two, 8 LPH >= stride) add up its norm.  Grid: (units of heads, token blocks).

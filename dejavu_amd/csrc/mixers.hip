@@ -178,6 +178,25 @@ int short_conv_types(const ConvArgs& a, int heads, int widest, hipStream_t s) {
   return short_conv_lanes<T, TO, 64>(a, heads, s);
 }
 
+int short_conv(int dtype, int out_f32, const dvConvArgs* a, float* next_state, void* stream) {
+  if (!dtype_ok(dtype) || !a || !a->in || a->n < 1 || a->taps < 1 || !a->w || (a->taps > 1 && !a->state))
+    return DV_ERR_INVALID_ARG;
+  int heads = 0, widest = 0;
+  for (const dvConvGroup& g : a->g) {
+    if (g.heads < 0 || (g.heads > 0 && (!g.out || g.stride < 1 || g.dim < 1))) return DV_ERR_INVALID_ARG;
+    heads += g.heads;
+    if (g.heads > 0 && g.stride > widest) widest = g.stride;
+  }
+  if (heads == 0) return DV_ERR_INVALID_ARG;
+  for (const dvConvGroup& g : a->g)
+    if (g.heads > 0 && (g.stride % 8 || g.ld % 8 || !al16(g.out))) return DV_ERR_ALIGNMENT;
+  if (a->ldi % 8 || !al16(a->in)) return DV_ERR_ALIGNMENT;
+  const ConvArgs all{*a, next_state};
+  if (dtype == DV_F32) return short_conv_types<float, float>(all, heads, widest, st(stream));
+  if (out_f32) return short_conv_types<bf16_t, float>(all, heads, widest, st(stream));
+  return short_conv_types<bf16_t, bf16_t>(all, heads, widest, st(stream));
+}
+
 // ---- attention rows --------------------------------------------------------
 template <typename T, typename TQ, int RH>
 int attn_rows_rh(const AttnArgs& a, hipStream_t s) {
@@ -585,21 +604,12 @@ int dv_mix_linear_tiles(int after, const dvTileArgs* a, void* stream) {
 }
 
 int dv_mix_short_conv(int dtype, int out_f32, const dvConvArgs* a, void* stream) {
-  if (!dtype_ok(dtype) || !a || !a->in || a->n < 1 || a->taps < 1 || !a->w || (a->taps > 1 && !a->state))
-    return DV_ERR_INVALID_ARG;
-  int heads = 0, widest = 0;
-  for (const dvConvGroup& g : a->g) {
-    if (g.heads < 0 || (g.heads > 0 && (!g.out || g.stride < 1 || g.dim < 1))) return DV_ERR_INVALID_ARG;
-    heads += g.heads;
-    if (g.heads > 0 && g.stride > widest) widest = g.stride;
-  }
-  if (heads == 0) return DV_ERR_INVALID_ARG;
-  for (const dvConvGroup& g : a->g)
-    if (g.heads > 0 && (g.stride % 8 || g.ld % 8 || !al16(g.out))) return DV_ERR_ALIGNMENT;
-  if (a->ldi % 8 || !al16(a->in)) return DV_ERR_ALIGNMENT;
-  if (dtype == DV_F32) return short_conv_types<float, float>(*a, heads, widest, st(stream));
-  if (out_f32) return short_conv_types<bf16_t, float>(*a, heads, widest, st(stream));
-  return short_conv_types<bf16_t, bf16_t>(*a, heads, widest, st(stream));
+  return short_conv(dtype, out_f32, a, nullptr, stream);
+}
+
+int dv_mix_short_conv_move(int dtype, int out_f32, const dvConvArgs* a, float* next_state, void* stream) {
+  if (!next_state && a && a->taps > 1) return DV_ERR_INVALID_ARG;
+  return short_conv(dtype, out_f32, a, next_state, stream);
 }
 
 int dv_mix_conv_state(int dtype, const void* in, int64_t ldi, int n, int channels, int taps, float* state, void* stream) {

@@ -596,12 +596,15 @@ def short_conv(x: torch.Tensor, conv_w: torch.Tensor, state: torch.Tensor, group
     the rows of x as well (``conv_state``)."""
     _f32(conv_w, conv_b)
     a = L.ConvArgs(in_=x.data_ptr(), ldi=x.stride(0), n=x.shape[0], taps=conv_w.shape[1], silu=int(silu),
-                   w=conv_w.data_ptr(), b=_ptr(conv_b), state=state.data_ptr(), next_state=state.data_ptr() if move else None)
+                   w=conv_w.data_ptr(), b=_ptr(conv_b), state=state.data_ptr())
     for i, (heads, stride, dim, norm, eps, scale, out) in enumerate(groups):
         assert out.shape == (x.shape[0], heads * stride) and out.stride(1) == 1
         a.g[i] = L.ConvGroup(heads, stride, dim, norm, eps, scale, out.data_ptr(), out.stride(0))
-    check(lib.dv_mix_short_conv(_code(x), int(groups[0][6].dtype == torch.float32), _ref(a), _stream()),
-          "dv_mix_short_conv")
+    code, f32 = _code(x), int(groups[0][6].dtype == torch.float32)
+    if move:
+        check(lib.dv_mix_short_conv_move(code, f32, _ref(a), a.state, _stream()), "dv_mix_short_conv_move")
+    else:
+        check(lib.dv_mix_short_conv(code, f32, _ref(a), _stream()), "dv_mix_short_conv")
 
 
 def conv_state(x: torch.Tensor, channels: int, taps: int, state: torch.Tensor) -> None:

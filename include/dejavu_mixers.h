@@ -136,7 +136,6 @@ typedef struct {
   const float* b;          /* [channels] or null */
   const float* state;      /* [channels][taps - 1] */
   dvConvGroup g[3];
-  float* next_state;       /* null, or where the state behind the last row goes (may be `state`) */
 } dvConvArgs;
 
 /* Rows that are RMS-normed: y = x / rms(x) * w; w has `padded` entries, the mean runs over `dim`. */
@@ -321,6 +320,8 @@ DV_API int dv_mix_linear_split(const float* x, int64_t ldx, const float* W, int6
 /* The same product for many rows (DV_OUT_T and DV_OUT_GLU). */
 DV_API int dv_mix_linear_wide(int after, const dvTileArgs* args, void* stream);
 DV_API int dv_mix_short_conv(int dtype, int out_f32, const dvConvArgs* args, void* stream);
+/* The same, and next_state <- the state behind the last row (may be args->state). */
+DV_API int dv_mix_short_conv_move(int dtype, int out_f32, const dvConvArgs* args, float* next_state, void* stream);
 DV_API int dv_mix_conv_state(int dtype, const void* in, int64_t ldi, int n, int channels, int taps, float* state,
                              void* stream);
 /* Rows of a portion's buffer <-> a ring of cap rows, token first .. first + count - 1 (count <= cap). */

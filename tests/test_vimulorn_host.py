@@ -194,6 +194,17 @@ def test_header_and_binding_agree():
         assert [n.rstrip("_") for n, *_ in py._fields_] == fields, c_name
 
 
+def test_structs_keep_their_size():
+    """A library reads no more of a caller's struct than the header said when the entry point came: what is added goes into a new one."""
+    import ctypes
+
+    from dejavu_amd import _lib_mixers as L
+
+    sizes = dict(AttnArgs=240, ConvArgs=176, ConvGroup=40, DeltaArgs=96, DeltaStepArgs=112, DynTanh=24, EmbedArgs=96, HeadArgs=240,
+                 HeadGroup=72, Hyper=48, Residual=72, RingRows=40, RmsOut=24, RmsRows=40, RowArgs=304, SsdArgs=128, SsdStepArgs=80, TileArgs=152)
+    assert {n: ctypes.sizeof(t) for n, t in vars(L).items() if isinstance(t, type) and issubclass(t, ctypes.Structure)} == sizes
+
+
 def test_host_side_argument_checks():
     """Bad sizes and null pointers are refused before anything is launched."""
     import ctypes
@@ -208,6 +219,8 @@ def test_host_side_argument_checks():
     assert L.lib.dv_mix_linear_row(0, 1, 0, ref(row), None) == -1            # norm weight missing
     assert L.lib.dv_mix_linear_row(0, 0, 3, ref(row), None) == -1            # residual missing
     assert L.lib.dv_mix_linear_tiles(0, ref(L.TileArgs(x=A + 2, ldx=64, W=A, ldw=64, n=2, M=4, K=64, out=A, ldo=4)), None) == -3
+    conv = L.ConvArgs(in_=A, ldi=64, n=3, taps=4, w=A, state=A)
+    assert L.lib.dv_mix_short_conv_move(0, 0, ref(conv), None, None) == -1   # nowhere to move to
     at = L.AttnArgs(q=A, ldq=64, k=A, ldk=64, k_head=64, v=A, ldv=64, v_head=64, n=3, H=1, G=1, dim_s=64, vdim_s=64,
                     out=A, splits=1)
     assert L.lib.dv_mix_attn_tiles(ref(at), 2, None) == -1                   # fewer keys than queries
