@@ -311,7 +311,7 @@ def _plain_layer(linear, x: torch.Tensor) -> bool:
     return (type(linear) is nn.Linear and W.dim() == 2 and x.shape[-1] == W.shape[1] and
             "forward" not in linear.__dict__ and not (linear._forward_hooks or linear._forward_pre_hooks) and
             not (nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks) and
-            results_only(x, W, b) and W.stride(1) == 1 and W.stride(0) % 8 == 0 and W.data_ptr() % 16 == 0 and
+            results_only(x, W, b) and W.stride(1) == 1 and W.stride(0) >= W.shape[1] and W.stride(0) % 8 == 0 and W.data_ptr() % 16 == 0 and
             x.data_ptr() % 16 == 0 and (b is None or (b.dtype == W.dtype and b.shape == W.shape[:1])))
 
 

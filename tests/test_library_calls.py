@@ -126,6 +126,21 @@ def test_operands_of_a_long_prompts_linear_that_only_the_library_takes(fc2):
     assert torch.equal(decode_linear(Duck(), x), x[..., :2])
 
 
+@pytest.mark.gpu
+@torch.no_grad()
+@pytest.mark.parametrize("rows,M,K,activation", [(200, 4096, 16384, "id"), (400, 8192, 2048, "relu"), (800, 5120, 20480, "id")])
+def test_weights_whose_rows_are_one_row(rows, M, K, activation):
+    """An expanded weight, whose rows begin at the same place."""
+    from dejavu_amd.modules import _long_product, _wide_product, decode_linear
+
+    layer = nn.Linear(K, M, device="cuda", dtype=torch.float16).requires_grad_(False)
+    x = torch.randn(1, rows, K, device="cuda").half()
+    assert _long_product(layer, x) or _wide_product(layer, x, activation)
+    layer.weight = nn.Parameter(layer.weight[:1].expand(M, K), requires_grad=False)
+    want = F.linear(x, layer.weight, layer.bias)
+    assert torch.equal(decode_linear(layer, x, activation), F.relu(want) if activation == "relu" else want)
+
+
 def test_modes_that_watch_library_calls():
     """A kernel's launch is invisible to dispatch and function modes, so none may stand in for a library call under one."""
     from torch.fx.experimental.proxy_tensor import make_fx
