@@ -95,6 +95,24 @@ int linear_stream(const RingPlan& p, const TileArgs& a, void* workspace, hipStre
   return gemm_ring(p, o, PlainRows{}, MixOut<AFTER>{a}, workspace, s, MixLaunch{});
 }
 
+// Rows so far apart that 32 bits do not count the bytes between them: the ring, which has an address for every row, as many rows of x at
+// a time as its grid takes.
+int linear_far(int after, const TileArgs& a, hipStream_t s) {
+  constexpr int kRows = 1 << 23;
+  for (int n0 = 0; n0 < a.n; n0 += kRows) {
+    TileArgs t = a;
+    t.n = a.n - n0 < kRows ? a.n - n0 : kRows;
+    t.x = reinterpret_cast<const bf16_t*>(a.x) + n0 * a.ldx;
+    t.out = reinterpret_cast<bf16_t*>(a.out) + n0 * a.ldo;
+    RingPlan p = plan_ring(t.n, t.M, t.K, compute_units());
+    p.splits = 1;
+    const int rc = after == DV_OUT_T ? linear_stream<DV_OUT_T>(p, t, nullptr, s) : linear_stream<DV_OUT_GLU>(p, t, nullptr, s);
+    if (rc != DV_OK) return rc;
+    if (a.n - n0 <= kRows) break;  // (n0 stays below 2^31)
+  }
+  return DV_OK;
+}
+
 // ---- fp32 rows on the bf16 instructions ----
 int linear_split(const SplitPlan& p, const SplitOperands& a, const SplitOut& out, float4_t* sums, hipStream_t s) {
   const int64_t blocks = ((int64_t)a.n + kSplitPartRows - 1) / kSplitPartRows * p.chunks;
@@ -592,11 +610,11 @@ int dv_mix_linear_split(const float* x, int64_t ldx, const float* W, int64_t ldw
 int dv_mix_linear_wide(int after, const dvTileArgs* a, void* stream) {
   const int rc = tile_args_ok(after, a);
   if (rc != DV_OK) return rc;
+  if (after != DV_OUT_T && after != DV_OUT_GLU) return DV_ERR_UNSUPPORTED;
   const int64_t tiles = ((int64_t)a->M + kWideRows - 1) / kWideRows * (((int64_t)a->n + 127) / 128);
-  if (tiles > 0x7fffffff || a->ldw >= kWideMaxStride || a->ldx >= kWideMaxStride) return DV_ERR_UNSUPPORTED;
-  if (after == DV_OUT_T) return linear_wide<DV_OUT_T>(*a, st(stream));
-  if (after == DV_OUT_GLU) return linear_wide<DV_OUT_GLU>(*a, st(stream));
-  return DV_ERR_UNSUPPORTED;
+  if (tiles > 0x7fffffff) return DV_ERR_UNSUPPORTED;
+  if (a->ldw < 0 || a->ldw >= kWideMaxStride || a->ldx < 0 || a->ldx >= kWideMaxStride) return linear_far(after, *a, st(stream));
+  return after == DV_OUT_T ? linear_wide<DV_OUT_T>(*a, st(stream)) : linear_wide<DV_OUT_GLU>(*a, st(stream));
 }
 
 int dv_mix_linear_tiles(int after, const dvTileArgs* a, void* stream) {

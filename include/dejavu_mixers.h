@@ -317,7 +317,7 @@ DV_API int dv_mix_linear_tiles_ws(int after, const dvTileArgs* args, void* works
 DV_API size_t dv_mix_linear_split_workspace_bytes(int n, int M, int K);
 DV_API int dv_mix_linear_split(const float* x, int64_t ldx, const float* W, int64_t ldw, const float* bias, int n, int M, int K,
                                float* out, int64_t ldo, void* workspace, size_t workspace_bytes, void* stream);
-/* The same product for many rows (DV_OUT_T and DV_OUT_GLU). */
+/* The same product for many rows (DV_OUT_T and DV_OUT_GLU); slower from leading dimensions of 2^25 on. */
 DV_API int dv_mix_linear_wide(int after, const dvTileArgs* args, void* stream);
 DV_API int dv_mix_short_conv(int dtype, int out_f32, const dvConvArgs* args, void* stream);
 /* The same, and next_state <- the state behind the last row (may be args->state). */

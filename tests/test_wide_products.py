@@ -143,6 +143,34 @@ def test_widths_of_the_tiles(n, M, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,M,K,x_far,w_far", [(300, 6, 136, False, True), (6, 1030, 72, True, False), (5, 12, 584, True, True),
+                                               (2 ** 23 + 5, 4, 8, False, True)])  # (as many rows as one launch takes and more)
+def test_rows_that_are_far_apart(n, M, K, x_far, w_far):
+    """Strides beyond what 32 bits count the bytes of."""
+    from dejavu_amd import _lib_mixers as L
+    from dejavu_amd import mixer_ops as ops
+
+    def far(t, yes):
+        if not yes:
+            return t
+        room = torch.empty((t.shape[0] - 1) * 2 ** 25 + t.shape[1], dtype=t.dtype, device="cuda")
+        return room.as_strided(t.shape, (2 ** 25, 1)).copy_(t)
+
+    g = torch.Generator(device="cuda").manual_seed(n + K)
+    x = torch.randn(n, K, generator=g, device="cuda").to(torch.bfloat16)
+    W = (torch.randn(M, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    prod = x.double() @ W.double().t()
+    x, W = far(x, x_far), far(W, w_far)
+    for after, want in ((L.OUT_T, prod), (L.OUT_GLU, prod[:, 0::2].clamp(min=0) * prod[:, 1::2])):
+        out = torch.full((n, want.shape[1]), 77.0, dtype=torch.bfloat16, device="cuda")
+        a = ops._tile_args(x, W)
+        a.out, a.ldo, a.act = out.data_ptr(), out.shape[1], L.GLU_RELU
+        ops.check(ops.lib.dv_mix_linear_wide(after, ops._ref(a), ops._stream()), "dv_mix_linear_wide")
+        # one rounding to bf16, 2 ** -9 at most, and fp32 sums of values of unit size
+        assert ((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-5 * K ** 0.5).all(), after
+
+
+@pytest.mark.gpu
 def test_gated_units_through_the_ops():
     """A product on each side of the rule's line (144 tiles), both with the same result."""
     from dejavu_amd import mixer_ops as ops
