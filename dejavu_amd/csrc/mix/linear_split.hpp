@@ -109,7 +109,8 @@ constexpr int64_t kSplitMaxStride = 1 << 25;  // 32 rows' bytes are counted in 3
 constexpr int kSplitMostRows = 1 << 24;       // and those of a chunk's parts
 
 // Grid: (tiles, those of W first; splits of K).  part: with several splits, the sums [split][tile][value][thread].
-template <typename Out>
+// FAR: every lane has addresses of its own, for strides and sizes beyond these two.
+template <bool FAR, typename Out>
 __global__ __launch_bounds__(kSplitThreads, 2) void linear_split_kernel(SplitOperands a, int row_tiles, Out out, float4_t* __restrict__ part) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (the loads' resources have no type on the host)
   extern __shared__ __attribute__((aligned(16))) unsigned char slots[];
@@ -132,16 +133,27 @@ __global__ __launch_bounds__(kSplitThreads, 2) void linear_split_kernel(SplitOpe
   const int w_col = (lane % PW ^ lane / PW) * 4;
   const unsigned x_at = lane / PX * (KC * 2) + (lane % PX ^ (lane / PX >> 2 & 3)) * 16;
   auto load_w = [&](int c, int slot, int i) {  // (past the end of a row its last piece: set to zero when it is used)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_ptr_t)(slots + slot * WBYTES + (wave * LW + i) * 1024), 16,
-                                             w_at + (unsigned)min(c * KC + w_col, a.K - 4) * 4u + i * w_step, 0, 0, 0);
+    const lds_ptr_t to = (lds_ptr_t)(slots + slot * WBYTES + (wave * LW + i) * 1024);
+    const int col = min(c * KC + w_col, a.K - 4);
+    if constexpr (FAR) {
+      const float* row = a.W + (int64_t)min(m0 + wave * 32 + i * (64 / PW) + lane / PW, a.M - 1) * a.ldw;
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(row + col), to, 16, 0, 0);
+    } else {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, to, 16, w_at + (unsigned)col * 4u + i * w_step, 0, 0, 0);
+    }
   };
   auto load_x = [&](int c, int slot) {
     const auto xr = __builtin_amdgcn_make_buffer_rsrc(a.parts + (int64_t)c * 3 * a.n * KC, 0, (int)((unsigned)a.n * (3u * KC * 2u)), 0x00020000);
 #pragma unroll
     for (int i = 0; i < LX; ++i) {
       const int row = (wave * LX + i) * (64 / PX), s = row / NB;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr_t)(slots + kSplitWSlots * WBYTES + slot * XBYTES + (wave * LX + i) * 1024), 16,
-                                               x_at + ((unsigned)s * a.n + n0 + row % NB) * (KC * 2u), 0, 0, 0);
+      const lds_ptr_t to = (lds_ptr_t)(slots + kSplitWSlots * WBYTES + slot * XBYTES + (wave * LX + i) * 1024);
+      if constexpr (FAR) {
+        const int64_t at = ((int64_t)c * 3 + s) * a.n + min(n0 + row % NB + lane / PX, a.n - 1);
+        __builtin_amdgcn_global_load_lds((global_ptr_t)(a.parts + at * KC + (lane % PX ^ (lane / PX >> 2 & 3)) * 8), to, 16, 0, 0);
+      } else {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, to, 16, x_at + ((unsigned)s * a.n + n0 + row % NB) * (KC * 2u), 0, 0, 0);
+      }
     }
   };
   float16_t sum[3][NT];  // of products of 1, 2^-8 and 2^-16 of the values' size

@@ -120,8 +120,10 @@ int linear_split(const SplitPlan& p, const SplitOperands& a, const SplitOut& out
   hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
   int rc = launched();
   if (rc != DV_OK) return rc;
-  const dim3 threads(kSplitThreads);
-  rc = launch_lds<linear_split_kernel<SplitOut>>(dim3((unsigned)p.tiles(), p.splits), threads, kSplitLds, s, a, p.rows, out, sums);
+  const dim3 threads(kSplitThreads), grid((unsigned)p.tiles(), p.splits);
+  const bool far = a.ldw < 0 || a.ldw >= kSplitMaxStride || a.K >= kSplitMaxStride || a.n >= kSplitMostRows;
+  rc = far ? launch_lds<linear_split_kernel<true, SplitOut>>(grid, threads, kSplitLds, s, a, p.rows, out, sums)
+           : launch_lds<linear_split_kernel<false, SplitOut>>(grid, threads, kSplitLds, s, a, p.rows, out, sums);
   if (rc != DV_OK || p.splits == 1) return rc;
   return launch_lds<linear_split_sum_kernel<SplitOut>>(dim3((unsigned)p.tiles(), kSplitCols / 8), threads, 0, s, a.n, a.M, p.rows, out,
                                                        (const float4_t*)sums, p.splits);
@@ -599,7 +601,6 @@ int dv_mix_linear_split(const float* x, int64_t ldx, const float* W, int64_t ldw
                         int64_t ldo, void* workspace, size_t workspace_bytes, void* stream) {
   if (!x || !W || !out || n < 1 || M < 1 || K < 4) return DV_ERR_INVALID_ARG;
   if (M % 4 || K % 4 || ldx % 4 || ldw % 4 || ldo % 4 || !al16(x) || !al16(W) || !al16(bias) || !al16(out)) return DV_ERR_ALIGNMENT;
-  if (ldw >= kSplitMaxStride || K >= kSplitMaxStride || n >= kSplitMostRows) return DV_ERR_UNSUPPORTED;
   const SplitPlan p = plan_split(n, M, K, compute_units());
   if (!workspace || workspace_bytes < p.workspace_bytes(n)) return DV_ERR_WORKSPACE;
   if (!al16(workspace)) return DV_ERR_ALIGNMENT;

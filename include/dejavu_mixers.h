@@ -313,7 +313,7 @@ DV_API int dv_mix_linear_tiles(int after, const dvTileArgs* args, void* stream);
 DV_API size_t dv_mix_linear_tiles_workspace_bytes(int n, int M, int K);
 DV_API int dv_mix_linear_tiles_ws(int after, const dvTileArgs* args, void* workspace, size_t workspace_bytes, void* stream);
 /* fp32 rows times an fp32 weight on the bf16 matrix instructions, every value as the sum of three bf16 parts (all 24 bits): out (n, M)
- * = x (n, K) W (M, K)^T + bias (M) or NULL.  Sizes and leading dimensions % 4 == 0; n below 2^24, K and ldw below 2^25. */
+ * = x (n, K) W (M, K)^T + bias (M) or NULL.  Sizes and leading dimensions % 4 == 0. */
 DV_API size_t dv_mix_linear_split_workspace_bytes(int n, int M, int K);
 DV_API int dv_mix_linear_split(const float* x, int64_t ldx, const float* W, int64_t ldw, const float* bias, int n, int M, int K,
                                float* out, int64_t ldo, void* workspace, size_t workspace_bytes, void* stream);

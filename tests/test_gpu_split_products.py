@@ -153,3 +153,20 @@ def test_rows_of_a_weight_that_are_far_apart(ops, stride, taken):
     assert (got is not None) == taken
     if taken:
         assert torch.equal(got, ops._split_product(x, W))
+
+
+@pytest.mark.parametrize("n,M,K,stride", [(130, 40, 68, 2 ** 25), (2 ** 24 + 131, 8, 36, 36), (5, 12, 2 ** 25 + 4, 2 ** 25 + 8)])
+def test_strides_and_sizes_beyond_32_bits(n, M, K, stride):
+    """Through the entry point itself, which takes what counts more bytes than 32 bits do.  Whole numbers: every sum is exact."""
+    from dejavu_amd import mixer_ops as o
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rand = lambda *s: torch.randint(-2, 3, s, generator=g, device="cuda").float()  # noqa: E731
+    x, W, bias = rand(n, K), rand(M, K), rand(M)
+    far = torch.empty((M - 1) * stride + K, device="cuda").as_strided((M, K), (stride, 1)).copy_(W)
+    out = torch.full((n, M), 77.0, device="cuda")
+    nbytes = o.lib.dv_mix_linear_split_workspace_bytes(n, M, K)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    o.check(o.lib.dv_mix_linear_split(x.data_ptr(), K, far.data_ptr(), stride, bias.data_ptr(), n, M, K, out.data_ptr(), M, ws.data_ptr(),
+                                      nbytes, o._stream()), "dv_mix_linear_split")
+    assert torch.equal(out, F.linear(x.double(), W.double(), bias.double()).float())
