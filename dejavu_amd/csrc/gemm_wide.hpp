@@ -23,15 +23,16 @@ constexpr int kWideRows = 256, kWideChunk = 64;
 constexpr size_t kWideLds = (size_t)5 * kWideRows * kWideChunk * 2;
 constexpr int64_t kWideMaxStride = 1 << 25;  // 64 rows' bytes are counted in 32 bits
 
-// NB whose rounds of tiles take least: a round takes as NB + 12 (256 full tiles of 128 / 160 / 192 / 224 / 256 rows with K = 4096: 58 / 69 / 84 / 99 /
-// 112 us), one that is not full half of it and half of its share (fewer compute units at work have a higher clock).  1999 rows by 18560 x
-// 4096: 301 / 289 / 314 / 273 / 281 us; 777 by 12288 x 4096: 105 / 69 / 84 / 87 / 98.
+// NB whose rounds of tiles take least: a round takes as NB + 60, one that is not full three quarters of it and a quarter of its share (fewer compute
+// units at work have a higher clock).  Over 634 products of 257..8192 rows with cold weights of 2^23 to 2^28 values and 1024 to 9216 columns, every
+// width measured, the choice takes 0.1 % longer than the best one and 6 % at most.  (NB + 12 and a half: 0.9 % and 28 %; 1024 rows by 36864 x 9216 739 us,
+// now 622, the library 584; 2048 by 28672 x 7168 802 / 718 / 672; 1152 by 27648 x 5120, gated, 379 / 323 / 295.)
 inline int plan_wide(int n, int M, int units) {
   int best = 0;
   double least = 0.0;
   for (int nb = 256; nb >= 128; nb -= 32) {
     const int64_t tiles = ((int64_t)M + kWideRows - 1) / kWideRows * (((int64_t)n + nb - 1) / nb), rest = tiles % units;
-    const double t = (nb + 12) * ((double)(tiles / units) + (rest ? 0.5 + 0.5 * rest / units : 0.0));
+    const double t = (nb + 60) * ((double)(tiles / units) + (rest ? 0.75 + 0.25 * rest / units : 0.0));
     if (best == 0 || t < least) best = nb, least = t;
   }
   return best;

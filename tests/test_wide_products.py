@@ -67,6 +67,24 @@ def kernels(tmp_path_factory):
     return found
 
 
+def test_widths_that_are_chosen(tmp_path):
+    """The sizes of the tests are of every width, and sizes for which other widths were measured to take up to a quarter longer."""
+    try:
+        hipcc = hipcc_path()
+    except RuntimeError as e:
+        pytest.skip(str(e))
+    src, exe = tmp_path / "plan.hip", tmp_path / "plan"
+    src.write_text('#include <cstdio>\n#include "gemm_wide.hpp"\nint main() { int n, M; while (scanf("%d %d", &n, &M) == 2) '
+                   'printf("%d\\n", dv::plan_wide(n, M, 256)); }\n')
+    subprocess.run([hipcc, "--offload-arch=gfx950", "-std=c++17", "-w", "-I", CSRC, "-I", os.path.join(CSRC, "..", "..", "include"),
+                    str(src), "-o", str(exe)], check=True)
+    measured = {(1024, 36864): 224, (2048, 28672): 256, (1152, 27648): 192, (2048, 22016): 256, (1999, 18560): 224, (777, 16384): 224, (400, 22016): 224,
+                (777, 12288): 160, (2048, 11264): 192}
+    asked = SIZES + list(measured)
+    out = subprocess.run([str(exe)], input="\n".join("%d %d" % q for q in asked), text=True, check=True, capture_output=True).stdout
+    assert list(map(int, out.split())) == WIDTHS + list(measured.values())
+
+
 def test_matrix_instructions_in_assembly(kernels):
     """Nothing in the hardware waits for their sums (8 states) or for operands that a vector instruction has just written (2), and
     the compiler does not see what they are."""
