@@ -59,16 +59,17 @@ HIP_PROMPT_LONG_ROWS = 256, 384
 HIP_PROMPT_LONG_WEIGHT = 1 << 23
 HIP_PROMPT_LONG_WEIGHT_ROWS = 4096, 8192
 # From 257 rows on the kernel of wide tiles (gemm_wide.hpp) takes fc1 with its activation, for which the library needs a launch more, where its tiles
-# of 128 rows by 256 weight rows are so many (below 4096 columns / from there on; the library's time over the kernel's: 8192 x 2048 with 400 / 600 /
-# 777 / 1200 / 2000 rows 1.07 / 1.18 / 1.36 / 1.28 / 1.11, 16384 x 4096 1.16 / 1.14 / 1.16 / 1.10 / 1.00, 20480 x 5120 with 400 / 600 / 777 / 1000 / 1435 / 2000 rows 1.02 / 1.27 /
-# 1.06 / 0.91 / 1.08 / 1.41; with 257 rows 0.98 to 1.01), and fc2 whose rows are the longest (5120 x 20480 with 777 / 1000 / 1200 / 1700 / 2000 rows 1.04 / 1.06 /
-# 1.17 / 1.66 / 0.96, 9216 x 36864 0.98 / 1.02 / 1.49 with 777 / 1200 / 2000, but 4096 x 16384 with 1200 0.90).  Of more than 2048 rows fc1 with up to 5120
-# columns (2100 / 2560 / 3000 / 4096 / 6000 / 8192 rows: 16384 x 4096 1.24 / 1.47 / 1.00 / 1.02 / 1.01 / 1.00, 20480 x 5120 1.01 / 1.16 / 1.06 / 1.04 / 1.04 / 1.01, 8192 x 2048
-# 1.36 / 1.19 / 1.19 / 1.07 / 1.05 / 1.04; but 36864 x 9216 1.02 / 0.90 / 0.94 / 0.93 / 0.95 / 0.93, and fc2 of 5120 x 20480 1.01 / 1.23 / 0.93 / 0.96 / 1.33 / 1.31).
+# of 128 rows by 256 weight rows are so many (below 3072 columns / from there on) and the columns up to 5120, up to 8192 rows.  The library's time over
+# the kernel's, weights cold, 385 to 2048 rows: 8192 x 2048 1.04 to 1.34, 10240 x 2560 1.05 to 1.66, 12288 x 3072 (641 rows and more) 1.04 to 1.28, 16384 x 4096
+# 1.00 to 1.25, 18432 x 4608 0.98 to 1.20, 20480 x 5120 0.98 to 1.45, 16384 x 5120 0.96 to 1.20; beyond 2048 rows the first, fourth and sixth 0.99 to 1.45.  Left to the
+# library: 22528 x 5632 0.94 to 1.46, 24576 x 6144 0.83 to 1.12, 28672 x 7168 0.93 to 1.15, 36864 x 9216 0.85 to 1.14, 12288 x 3072 with 257 to 512 rows 0.94 to 1.00 (513 to 640 1.01 to 1.11).
+# And fc2 whose rows are the longest but for those that go on from 21504 columns, of more than 768 rows and where the tiles are so many: 5120 x 20480 0.98 to
+# 1.79, 4096 x 20480 1.03 to 1.52.  Of longer rows the library has its good choices at other sizes for each weight: 5376 x 21504 0.88 to 1.76, 6144 x 24576 0.92 to 1.61, 7168 x
+# 28672 0.89 to 1.61, 9216 x 36864 0.92 to 1.61; of shorter ones mostly: 4608 x 18432 0.77 to 1.75, 4096 x 16384 0.73 to 2.01; 768 rows and fewer 0.56 to 0.87.
 HIP_PROMPT_WIDE_ROWS = 257, 2048
-HIP_PROMPT_WIDE_LONGEST = 8192, 5120   # rows, columns
-HIP_PROMPT_WIDE_COLUMNS, HIP_PROMPT_WIDE_FILL = (2048, 4096), (128, 256)
-HIP_PROMPT_WIDE_LONG = 768, 20480      # rows, columns
+HIP_PROMPT_WIDE_LONGEST = 8192, 5120   # rows, columns (with an activation)
+HIP_PROMPT_WIDE_COLUMNS, HIP_PROMPT_WIDE_FILL = (2048, 3072), (128, 256)
+HIP_PROMPT_WIDE_LONG = 769, (20480, 21504), 136  # rows, columns (from, to), tiles
 HIP_PROMPT_WIDE_STRIDE = 1 << 25
 # The package's causal-attention kernel (cache fill in the same launch) is ahead of the library's attention with the
 # permuted cache copies (40 heads of 128 and 128 / 1024 tokens: 7.5 / 47 us against 25 / 100; 32 heads and
@@ -293,15 +294,16 @@ def _long_rule(rows: int, M: int, K: int) -> bool:
 
 
 def _wide_rule(rows: int, M: int, K: int, activation: str) -> bool:
-    if rows < HIP_PROMPT_WIDE_ROWS[0] or activation not in ("id", "relu", "squared_relu"):
+    if activation not in ("id", "relu", "squared_relu"):
         return False
-    most, columns = HIP_PROMPT_WIDE_LONGEST
-    if rows > (most if activation != "id" and K <= columns else HIP_PROMPT_WIDE_ROWS[1]):
-        return False
+    tiles = -(-M // 256) * -(-rows // 128)
     if activation == "id":
-        return K >= 4 * M and K >= HIP_PROMPT_WIDE_LONG[1] and rows >= HIP_PROMPT_WIDE_LONG[0]
+        least, columns, fill = HIP_PROMPT_WIDE_LONG
+        return least <= rows <= HIP_PROMPT_WIDE_ROWS[1] and max(4 * M, columns[0]) <= K < columns[1] and tiles >= fill
+    most, columns = HIP_PROMPT_WIDE_LONGEST
     few = K < HIP_PROMPT_WIDE_COLUMNS[1]
-    return K >= HIP_PROMPT_WIDE_COLUMNS[0] and -(-M // 256) * -(-rows // 128) >= HIP_PROMPT_WIDE_FILL[0 if few else 1]
+    return (HIP_PROMPT_WIDE_ROWS[0] <= rows <= most and HIP_PROMPT_WIDE_COLUMNS[0] <= K <= columns and
+            tiles >= HIP_PROMPT_WIDE_FILL[0 if few else 1])
 
 
 def _plain_layer(linear, x: torch.Tensor) -> bool:

@@ -214,6 +214,13 @@ def test_which_products_of_a_prompt_the_wide_kernel_takes():
     for rows, M, K in ((256, 16384, 4096), (300, 16384, 4096), (257, 8192, 2048), (8193, 16384, 4096), (2049, 36864, 9216), (777, 3072, 768)):
         assert not rule(rows, M, K, "relu"), (rows, M, K)
     assert rule(777, 5120, 20480, "id") and not rule(767, 5120, 20480, "id") and not rule(1200, 4096, 16384, "id")
+    # where the library is ahead at some sizes, and on both sides of the lines
+    for rows, M, K in ((300, 36864, 9216), (1000, 36864, 9216), (640, 24576, 6144), (513, 12288, 3072), (768, 16384, 5128)):
+        assert not rule(rows, M, K, "relu"), (rows, M, K)
+    assert rule(641, 12288, 3072, "relu") and rule(257, 12288, 3064, "relu") and rule(1000, 20480, 5120, "relu")
+    for rows, M, K in ((768, 5120, 20480), (2049, 5120, 20480), (1024, 4096, 20480), (1152, 5376, 21504), (1600, 9216, 36864)):
+        assert not rule(rows, M, K, "id"), (rows, M, K)
+    assert rule(769, 5120, 20480, "id") and rule(1025, 4096, 20480, "id") and rule(2048, 5120, 20480, "id")
 
 
 @pytest.mark.gpu
