@@ -132,27 +132,40 @@ def _wide_rule(n: int, M: int, K: int) -> bool:
 
 
 # Where the library's product is followed by a launch of its own for the gated unit, and for few columns, the kernel is ahead as
-# soon as its tiles fill the chip (at least so many tiles of 128 rows by 256 weight rows, by columns): gated units of 22016 x 4096 with 400 / 777 /
-# 1200 / 1435 / 1700 rows 1.03 / 1.04 / 0.98 / 1.37 / 1.29, 18560 x 4096 1.08 / 1.04 / 1.29 / 1.10 / 1.29, 12288 x 4096 with 640 / 777 / 1435 / 1999 rows 1.08 / 1.10 / 1.18 / 0.99,
-# 8192 x 4096 with 777 / 1200 / 1999 1.16 / 1.09 / 0.99, but with 512 0.85; 11264 x 2048 with 400 / 640 / 1000 / 1700 / 1999 1.15 / 1.18 / 1.22 / 1.29 / 1.08, with 300 0.97;
-# 6144 x 2048 with 777 / 1000 1.03 / 1.14, with 640 0.92.  Plain: 11264 x 2048 with 400 / 640 / 1000 / 1700 / 1999 1.10 / 0.99 / 1.12 / 1.22 / 1.00, 9216 x 2048 with 777 / 1000 /
-# 1700 / 1999 1.06 / 1.21 / 0.95 / 1.19, 4368 x 2048 with 1200 / 1700 / 2048 1.13 / 1.19 / 1.24, with 777 0.89.
-# Gated units of 2049 to 8192 rows: 22016 x 4096 with 2100 / 2560 / 3000 / 4096 / 6000 / 8192 rows 1.50 / 0.95 / 1.20 / 1.10 / 1.04 / 1.14, 18560 x 4096 1.00 / 1.24 /
-# 1.02 / 1.28 / 1.17 / 1.03, 12288 x 4096 1.07 / 0.94 / 1.09 / 0.99 / 1.27 / 0.98, 11264 x 2048 1.08 / 0.97 / 1.10 / 1.15 / 1.27 / 1.19, but 8192 x 4096 1.15 / 1.05 / 1.09 /
-# 0.98 / 0.99 / 0.96.
-WIDE_FEW_COLUMNS, WIDE_GATED_COLUMNS = 2048, 8192
+# soon as its tiles fill the chip (at least so many tiles of 128 rows by 256 weight rows, by columns).  The library's time over the kernel's, weights
+# cold, of 37 numbers of rows from 257 to 2048 those that are taken:
+#   gated, 4096 columns: 28672 / 22016 / 20480 / 18560 / 17920 / 16384 / 14336 / 12288 / 10240 / 8192 weight rows from 0.95 / 0.96 / 0.97 / 1.05 / 0.98 / 0.98 / 0.98 / 0.99 / 0.98 / 1.03 on,
+#     up to 1.15 (8192) and 1.61; 18944 x 4608 0.97 to 1.51.  Left for their few tiles: 8192 weight rows with up to 768 rows 0.73 to 1.07.
+#   gated, 2048 columns: 11264 / 9216 / 8192 / 6144 / 4368 weight rows from 1.05 / 1.09 / 1.05 / 1.06 / 1.12 on, up to 1.5; 16384 and 8192 x 1024 from 1.04 and 1.15 on.
+#     Left: 6144 weight rows with up to 640 rows 0.92 to 1.02.
+#   gated, more columns, where tiles of 256 x 256 leave little of their last round empty: 24576 x 5120 0.97 to 1.15 (else 0.79 to 1.00), 27648 x 5120 0.96 to 1.20 (0.87 to 0.99),
+#     13696 x 5120 1.09 to 1.23 (0.77 to 1.02), 16384 x 8192 0.96 to 1.29, 22016 x 8192 1.26 to 1.31 (0.91 to 1.31).
+#   plain, where rows and weight rows leave some of such a round empty, 2048 columns: 24576 / 12288 / 11264 / 9216 / 8192 / 6144 / 4368 weight rows from 0.93 / 1.00 / 0.94 / 1.04 / 1.04 / 1.04 /
+#     1.17 on, up to 1.2 and 1.7; 5632 x 1536, 10240 x 1280, 16384 and 8192 x 1024 from 1.07, 1.03, 1.05 and 1.20 on.  Left, where the library's larger tiles fill their rounds:
+#     2048 rows by 8192 x 2048 / 24576 x 2048 / 16384 x 1024 0.94 / 0.91 / 0.90.
+# Gated units of 2049 to 8192 rows: 22016 / 18560 / 16384 / 14336 / 12288 x 4096 from 0.96 / 1.00 / 0.97 / 0.96 / 0.97 on, up to 1.54, 11264 x 2048 1.01 to 1.30, 16384 x 1024 from 1.02 on; 8192 x
+# 4096, with fewer tiles, 0.96 to 1.15.
+WIDE_FEW_COLUMNS, WIDE_GATED_COLUMNS = 2048, (4608, 8192)
 WIDE_LONG_GATED = 8192, 11264, 4096    # rows at most, weight rows at least, columns at most
 WIDE_FILL_GATED, WIDE_FILL_FEW_GATED, WIDE_FILL_FEW = 200, 144, 176
+WIDE_FULL_GATED, WIDE_FULL_FEW = 0.84, 0.83  # of the rounds of 256 x 256 tiles: tiles at least, rows by weight rows below
 
 
 def _fill_rule(n: int, M: int, K: int, gated: bool) -> bool:
-    if n <= TILE_MAX_ROWS or not 1024 <= K <= WIDE_GATED_COLUMNS or (K > WIDE_FEW_COLUMNS and not gated):
+    columns = WIDE_GATED_COLUMNS if gated else (WIDE_FEW_COLUMNS, WIDE_FEW_COLUMNS)
+    if n <= TILE_MAX_ROWS or not 1024 <= K <= columns[1]:
         return False
-    most, rows, columns = WIDE_LONG_GATED
-    if n > (most if gated and M >= rows and K <= columns else WIDE_MAX_ROWS):
+    most, rows, few = WIDE_LONG_GATED
+    if n > (most if gated and M >= rows and K <= few else WIDE_MAX_ROWS):
         return False
     fill = (WIDE_FILL_FEW_GATED if gated else WIDE_FILL_FEW) if K <= WIDE_FEW_COLUMNS else WIDE_FILL_GATED
-    return _tiles_of(n, M, 128, WIDE_TILE) >= fill
+    if _tiles_of(n, M, 128, WIDE_TILE) < fill:
+        return False
+    tiles = _tiles_of(n, M, WIDE_TILE, WIDE_TILE)
+    places = -(-tiles // WIDE_ROUND) * WIDE_ROUND
+    if not gated:
+        return n * M < WIDE_FULL_FEW * WIDE_TILE * WIDE_TILE * places
+    return K <= columns[0] or tiles >= WIDE_FULL_GATED * places
 
 
 def _tile_rule(n: int, M: int, K: int, gated: bool) -> bool:

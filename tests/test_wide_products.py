@@ -132,6 +132,13 @@ def test_which_products_the_wide_kernel_takes():
     for n, M, K in ((256, 22016, 4096), (512, 8192, 4096), (1200, 4096, 4096), (300, 11264, 2048), (640, 6144, 2048), (8193, 22016, 4096), (2049, 8192, 4096),
                     (2049, 22016, 8192), (1000, 22016, 16384)):
         assert not _fill_rule(n, M, K, True) and not _fill_rule(n, M, K, False), (n, M, K)
+    # more columns: where the last round of 256 x 256 tiles is nearly full, few columns without a unit: where it is not
+    for n, M, K, gated in ((1025, 24576, 5120, True), (777, 13696, 5120, True), (1800, 22016, 8192, True), (513, 18944, 4608, True),
+                           (1600, 8192, 2048, False), (1100, 11264, 2048, False), (1792, 24576, 1024, True)):
+        assert _fill_rule(n, M, K, gated), (n, M, K)
+    for n, M, K, gated in ((513, 24576, 5120, True), (1152, 13696, 5120, True), (1152, 22016, 8192, True), (640, 27648, 5120, True),
+                           (2048, 8192, 2048, False), (1800, 24576, 2048, False), (2048, 16384, 1024, False)):
+        assert not _fill_rule(n, M, K, gated), (n, M, K)             # 0.79 to 0.94 of the library's speed
 
 
 @pytest.mark.gpu
