@@ -482,8 +482,8 @@ int ring_scratch(const RingPlan& p, const void* workspace, size_t workspace_byte
 }
 
 // Which kernel takes a product of B rows.  From 65 rows on the ring (12288 x 4096 with 100 / 190 / 256 rows: 31 / 38 / 46 us
-// against 39 / 59 / 57; QKV of 24 heads of 9216 with 96 / 160 / 240 rows 46 / 56 / 68 against 53 / 90 / 124, of which a window's go
-// to qkv_window.hpp; 5120 x 20480 with 384 rows 134 against 245),
+// against 39 / 59 / 57; QKV of 24 heads of 9216 with 96 / 160 / 240 rows 46 / 56 / 68 against 53 / 90 / 124, 32 heads of
+// 12288 with 320 and 480 rows 191 and 195 against 208 and 214 with gemm_big.hpp, but see window_live; 5120 x 20480 with 384 rows 134 against 245),
 // but not plain products of more than 512 rows, or of more than 40960 rows of W and 256, which gemm_big.hpp takes where its
 // chunks divide N (50272 x 4096 with 300 / 400 rows: the ring 259 / 309, that 243 / 349; 36864 x 4096 199 / 237 against 195 / 242, 20480
 // x 5120 105 / 165 against 132 / 200), nor of up to 128 rows and more than 32768 of W, which are more than a round of tiles
@@ -553,14 +553,11 @@ int gemm_big(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const h
   }
 }
 
-// Windows of more than 64 rows take the rows that are live (qkv_window.hpp); up to there the weights' stream is the time whatever the rows.
-bool window_live(int tokens, int rows) { return tokens > 1 && rows > 64; }
-
 // QKV of the selected heads for B rows (see QkvScatter): M = 3 * Hk * hd output rows
 int gemm_tiled_qkv(const half_t* X, int64_t ldx, const half_t* W, const half_t* bias, int B, int d, half_t* Y,
                    const QkvScatter& qs, void* workspace, size_t workspace_bytes, hipStream_t s) {
   const int M = 3 * qs.Hk * qs.hd, Z = 3 * qs.H * qs.hd;
-  if (window_live(qs.tokens, B)) {
+  if (window_live(qs.tokens, qs.nseq, qs.hd, M, compute_units())) {
     const WindowPlan p = plan_window(B, M, d, compute_units());
     if (p.splits > 1 && (workspace == nullptr || !aligned16(workspace) || workspace_bytes < p.workspace_bytes())) return DV_ERR_WORKSPACE;
     const RingOperands<half_t> a{X, ldx, W, (int64_t)d, B, M, d};
@@ -1797,7 +1794,7 @@ size_t dv_out_proj_sparse_t_ln_workspace_bytes(int B, int nnz, int hd, int N) {
 
 size_t dv_qkv_window_batch_workspace_bytes(int tokens, int nseq, int d, int nnz, int hd) {
   if (tokens < 1 || tokens > 16 || nseq < 1 || nseq > 32 || d <= 0 || nnz <= 0 || hd <= 0) return 0;
-  if (window_live(tokens, tokens * nseq)) return plan_window(tokens * nseq, 3 * nnz * hd, d, compute_units()).workspace_bytes();
+  if (window_live(tokens, nseq, hd, 3 * nnz * hd, compute_units())) return plan_window(tokens * nseq, 3 * nnz * hd, d, compute_units()).workspace_bytes();
   return tiled_workspace_bytes(tokens * nseq, d, 3 * nnz * hd, true);
 }
 

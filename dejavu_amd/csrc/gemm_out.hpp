@@ -67,7 +67,7 @@ __device__ __forceinline__ void qkv_store4(const QkvScatter& q, half_t* __restri
 
 struct QkvRows {  // (a head out of range reads row 0 and is not stored)
   static constexpr bool kPastCaches = false;
-  static constexpr int kMostCols = 64;  // (qkv_window.hpp takes more)
+  static constexpr int kMostCols = 256;
   QkvScatter q;
   __device__ __forceinline__ int64_t operator()(int m) const {
     const int t = m / (q.Hk * q.hd), rem = m - t * q.Hk * q.hd, i = rem / q.hd, h = q.head_idx[i];

@@ -12,6 +12,9 @@ pytestmark = pytest.mark.gpu
     (17, 128, 2048, [4, 7, 8, 15, 16]),           # 68, 119, 136, 255, 272
     (13, 64, 264, [1, 5, 9, 10, 16]),             # two heads a tile; 33 pieces, no splits
     (5, 32, 520, [16, 1, 0, 13, 2, 3]),           # four heads a tile, 80 rows in all, one head without any
+    (32, 128, 264, [2, 3, 4, 5, 8, 9, 16, 1, 7, 12, 10]),   # by the rows that are live: 64, 96, 128, 160, 256, 288, 512, 32 .. rows, no splits
+    (13, 128, 2048, [4, 5, 9, 10, 16, 0, 15, 1, 2, 13, 8]),  # 52, 65, 117, 130, 208, no rows .., in splits
+    (12, 128, 2048, [4, 5, 9, 10, 16, 0, 15, 1, 2, 13, 8]),  # the last that multiplies all rows
 ])
 def test_live_rows(nseq, hd, d, counts):
     from dejavu_amd import ops

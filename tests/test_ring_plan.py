@@ -60,3 +60,20 @@ def test_a_quarter_of_the_compute_units_takes_a_quarter_of_the_rows(plan):
     asked = [(47, 16384, 4096, 256), (47, 4096, 4096, 64), (47, 4095, 4096, 64), (96, 16384, 2048, 256), (96, 16448, 2048, 256),
              (96, 8192, 2048, 128), (96, 8256, 2048, 128)]
     assert [p[0] for p in plan(asked)] == [96, 96, 64, 64, 128, 64, 128]
+
+
+def test_which_windows_multiply_live_rows_only(tmp_path):
+    """Both sides of each line: rows of the window, size of a head, chosen heads."""
+    try:
+        hipcc = hipcc_path()
+    except RuntimeError as e:
+        pytest.skip(str(e))
+    src, exe = tmp_path / "live.hip", tmp_path / "live"
+    src.write_text('#include <cstdio>\n#include "../../include/dejavu_hip.h"\n#include "qkv_window.hpp"\nint main() { int t, n, hd, h; '
+                   'while (scanf("%d %d %d %d", &t, &n, &hd, &h) == 4) printf("%d\\n", dv::window_live(t, n, hd, 3 * h * hd, 256)); }\n')
+    subprocess.run([hipcc, "--offload-arch=gfx950", "-std=c++17", "-w", "-I", CSRC, "-I", os.path.join(CSRC, "..", "..", "include"),
+                    str(src), "-o", str(exe)], check=True)
+    asked = {(13, 16, 128, 24): 1, (12, 16, 128, 24): 0, (16, 12, 128, 24): 0, (16, 13, 128, 24): 1, (16, 5, 128, 96): 0, (9, 8, 128, 24): 0,
+             (16, 32, 64, 48): 0, (16, 32, 32, 64): 0, (16, 32, 128, 10): 0, (16, 32, 128, 11): 1, (1, 32, 128, 24): 0}
+    out = subprocess.run([str(exe)], input="\n".join("%d %d %d %d" % q for q in asked), text=True, check=True, capture_output=True).stdout
+    assert list(map(int, out.split())) == list(asked.values())
