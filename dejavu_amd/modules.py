@@ -299,7 +299,8 @@ def _wide_rule(rows: int, M: int, K: int, activation: str) -> bool:
     tiles = -(-M // 256) * -(-rows // 128)
     if activation == "id":
         least, columns, fill = HIP_PROMPT_WIDE_LONG
-        return least <= rows <= HIP_PROMPT_WIDE_ROWS[1] and max(4 * M, columns[0]) <= K < columns[1] and tiles >= fill
+        # (rows of results off 16-byte boundaries are stored value by value: 780 to 1200 rows by 5124 x 20496 0.84 to 0.89)
+        return M % 8 == 0 and least <= rows <= HIP_PROMPT_WIDE_ROWS[1] and max(4 * M, columns[0]) <= K < columns[1] and tiles >= fill
     most, columns = HIP_PROMPT_WIDE_LONGEST
     few = K < HIP_PROMPT_WIDE_COLUMNS[1]
     return (HIP_PROMPT_WIDE_ROWS[0] <= rows <= most and HIP_PROMPT_WIDE_COLUMNS[0] <= K <= columns and

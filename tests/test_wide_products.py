@@ -196,6 +196,22 @@ def test_rows_that_are_far_apart(n, M, K, x_far, w_far):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,ours", [(11264, True), (11268, False)])
+def test_plain_products_whose_rows_leave_16_byte_boundaries(M, ours, monkeypatch):
+    from dejavu_amd import mixer_ops as ops
+
+    launches, kernel = [], ops.lib.dv_mix_linear_wide
+    monkeypatch.setattr(ops.lib, "dv_mix_linear_wide", lambda *a: [launches.append(1), kernel(*a)][1])
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, W = (torch.randn(s, generator=g, device="cuda").to(torch.bfloat16) for s in ((400, 2048), (M, 2048)))
+    got, want = ops.linear(x, W), x.float() @ W.float().t()
+    assert bool(launches) == ours and (got - want).norm() < 1e-2 * want.norm()
+    assert ops._fills(x, W, gated=True)
+    ops.relu_glu(x, W)
+    assert len(launches) == 1 + ours
+
+
+@pytest.mark.gpu
 def test_gated_units_through_the_ops():
     """A product on each side of the rule's line (144 tiles), both with the same result."""
     from dejavu_amd import mixer_ops as ops
@@ -225,7 +241,7 @@ def test_which_products_of_a_prompt_the_wide_kernel_takes():
     for rows, M, K in ((300, 36864, 9216), (1000, 36864, 9216), (640, 24576, 6144), (513, 12288, 3072), (768, 16384, 5128)):
         assert not rule(rows, M, K, "relu"), (rows, M, K)
     assert rule(641, 12288, 3072, "relu") and rule(257, 12288, 3064, "relu") and rule(1000, 20480, 5120, "relu")
-    for rows, M, K in ((768, 5120, 20480), (2049, 5120, 20480), (1024, 4096, 20480), (1152, 5376, 21504), (1600, 9216, 36864)):
+    for rows, M, K in ((768, 5120, 20480), (1000, 5124, 20496), (2049, 5120, 20480), (1024, 4096, 20480), (1152, 5376, 21504), (1600, 9216, 36864)):
         assert not rule(rows, M, K, "id"), (rows, M, K)
     assert rule(769, 5120, 20480, "id") and rule(1025, 4096, 20480, "id") and rule(2048, 5120, 20480, "id")
 
