@@ -63,7 +63,9 @@ def test_dense_linear_matches_fp32_reference(rows, N, M, act):
                                           (32, 2048, 4096, "id"), (32, 2048, 4104, "id"), (40, 5120, 4104, "relu"),
                                           (64, 6656, 7680, "id"), (64, 6656, 7688, "id"), (64, 264, 32770, "id"),
                                           (65, 264, 32768, "id"), (65, 264, 32770, "id"), (129, 264, 32770, "id"),
-                                          (300, 264, 40970, "id"), (300, 256, 40970, "relu")])
+                                          (300, 264, 40970, "id"), (300, 256, 40970, "relu"),
+                                          # activations that the wide tiles leave to gemm_big.hpp: 192, 256 and 128 weight rows a tile
+                                          (520, 256, 9790, "gelu"), (520, 512, 13050, "gelu_approx"), (300, 256, 40970, "gelu"), (1030, 256, 2306, "gelu")])
 def test_dense_linear_at_the_edges_of_its_rules(rows, N, M, act):
     from dejavu_amd import ops
 

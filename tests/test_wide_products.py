@@ -266,6 +266,76 @@ def test_wide_products_in_fp16(n, M, K, act):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("act", ["id", "relu", "squared_relu"])
+@pytest.mark.parametrize("n,M", SIZES)
+def test_widths_of_the_tiles_in_fp16(n, M, act):
+    from dejavu_amd import ops
+
+    K = 136
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(n, K, generator=g, device="cuda").half()
+    W = (torch.randn(M, K, generator=g, device="cuda") * K ** -0.5).half()
+    bias = torch.randn(M, generator=g, device="cuda").half()
+    want = x.double() @ W.double().t() + bias.double()
+    want = {"id": lambda t: t, "relu": lambda t: t.clamp(min=0), "squared_relu": lambda t: t.clamp(min=0) ** 2}[act](want)
+    got = ops.dense_linear_wide(x, W, bias, act).double()
+    # one rounding to fp16, 2 ** -11 at most, and fp32 sums of values of unit size
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -10 + 1e-5 * K ** 0.5).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [8, 40, 56, 64])
+def test_fewer_columns_than_a_chunk(K):
+    """The last columns are all there are: no chunk goes before them."""
+    from dejavu_amd import _lib_mixers as L
+    from dejavu_amd import mixer_ops, ops
+
+    g = torch.Generator(device="cuda").manual_seed(K)
+    n, M = 300, 1030
+    for dtype in (torch.float16, torch.bfloat16):
+        room = torch.full((n + M, K + 16), float("nan"), dtype=dtype, device="cuda")  # what lies beside the rows does not get in
+        x, W = room[:n, 8:K + 8], room[n:, 8:K + 8]
+        x.copy_(torch.randn(n, K, generator=g, device="cuda"))
+        W.copy_(torch.randn(M, K, generator=g, device="cuda") * K ** -0.5)
+        want = x.double() @ W.double().t()
+        if dtype == torch.float16:
+            got = torch.empty(n, M, dtype=dtype, device="cuda")
+            ops.check(ops.lib.dv_dense_linear_wide_f16(x.data_ptr(), x.stride(0), W.data_ptr(), W.stride(0), None, n, K, M, 0, got.data_ptr(), M,
+                                                       ops._stream()), "dv_dense_linear_wide_f16")
+        else:
+            got = torch.empty(n, M, dtype=dtype, device="cuda")
+            a = mixer_ops._tile_args(x, W)
+            a.out, a.ldo = got.data_ptr(), M
+            ops.check(mixer_ops.lib.dv_mix_linear_wide(L.OUT_T, mixer_ops._ref(a), ops._stream()), "dv_mix_linear_wide")
+        # one rounding, half of a last place, and fp32 sums of values of unit size
+        assert ((got.double() - want).abs() <= want.abs() * torch.finfo(dtype).eps + 1e-5 * K ** 0.5).all(), dtype
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+@pytest.mark.parametrize("positive", [False, True])
+def test_longest_rows_through_the_layers(positive):
+    """fc2 without an activation, whose sums are one chain over 20480 columns; of numbers of one sign they grow all the way."""
+    from dejavu_amd import modules
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    n, M, K = 769, 5120, 20480
+    layer = torch.nn.Linear(K, M, device="cuda", dtype=torch.float16)
+    x, W = torch.randn(1, n, K, generator=g, device="cuda"), torch.randn(M, K, generator=g, device="cuda") * K ** -0.5
+    if positive:
+        x, W = x.abs(), W.abs() * K ** -0.5
+    x = x.half()
+    layer.weight.copy_(W)
+    assert modules._wide_product(layer, x, "id") and not modules._wide_product(layer, x[:, :768], "id")
+    got = modules.decode_linear(layer, x)[0].double()
+    want = x[0].double() @ layer.weight.double().t() + layer.bias.double()
+    # a rounding to fp16, half of 2 ** -10, and one of 2 ** -24 of a sum at each of 640 instructions: all of one sign together, or of sums
+    # of unit size, a few times their root mean square
+    limit = want.abs() * (2.0 ** -11 + 640 * 2.0 ** -24) if positive else want.abs() * 2.0 ** -11 + 8 * 640 ** 0.5 * 2.0 ** -24
+    assert ((got - want).abs() <= limit).all()
+
+
+@pytest.mark.gpu
 @torch.no_grad()
 @pytest.mark.parametrize("act", ["id", "relu", "squared_relu"])
 def test_values_that_are_no_finite_numbers(act):
