@@ -485,7 +485,7 @@ int ring_scratch(const RingPlan& p, const void* workspace, size_t workspace_byte
 // against 39 / 59 / 57; QKV of 24 heads of 9216 with 96 / 160 / 240 rows 46 / 56 / 68 against 53 / 90 / 124, 32 heads of
 // 12288 with 320 and 480 rows 191 and 195 against 208 and 214 with gemm_big.hpp, but see window_live; 5120 x 20480 with 384 rows 134 against 245),
 // but not plain products of more than 512 rows, or of more than 40960 rows of W and 256, which gemm_big.hpp takes where its
-// chunks divide N (50272 x 4096 with 300 / 400 rows: the ring 259 / 309, that 243 / 349; 36864 x 4096 199 / 237 against 195 / 242, 20480
+// chunks divide N and the wide tiles (wide_takes) do not (50272 x 4096 with 300 / 400 rows: the ring 259 / 309, that 243 / 349; 36864 x 4096 199 / 237 against 195 / 242, 20480
 // x 5120 105 / 165 against 132 / 200), nor of up to 128 rows and more than 32768 of W, which are more than a round of tiles
 // (50272 x 4096 with 72 / 128 rows: 122 / 126 us, gemm_tiled.hpp 105 / 114).  Fewer rows are bound by the stream alone, and there
 // gemm_tiled.hpp, whose loads cover 512 bytes of a row, is ahead for large weights, the ring for small ones (us, the ring against

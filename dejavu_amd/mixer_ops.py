@@ -634,18 +634,11 @@ def _ring_rows(buf: torch.Tensor, ring: torch.Tensor) -> L.RingRows:
 
 
 def ring_copy_two(bufs, rings, first: int, to_ring: bool) -> None:
-    """``ring_copy`` of two buffers of as many rows and two rings of as many in one launch."""
+    """Rows of two buffers, tokens first, first + 1, .. in both, to two rings of as many rows, or from there, in one launch."""
     (a, b), (ra, rb) = bufs, rings
     assert a.shape[0] == b.shape[0] and ra.shape[0] == rb.shape[0] and a.dtype == b.dtype
     check(lib.dv_mix_ring_copy_two(_code(a), _ref(_ring_rows(a, ra)), _ref(_ring_rows(b, rb)), ra.shape[0], first, a.shape[0],
                                    int(to_ring), _stream()), "dv_mix_ring_copy_two")
-
-
-def ring_copy(buf: torch.Tensor, ring: torch.Tensor, first: int, to_ring: bool) -> None:
-    """Rows of buf are tokens first, first + 1, ...; ring (cap, width)."""
-    assert buf.dtype == ring.dtype and buf.shape[1] == ring.shape[1]
-    check(lib.dv_mix_ring_copy(_code(buf), _ptr(buf), buf.stride(0), _ptr(ring), ring.shape[0], ring.stride(0), first,
-                               buf.shape[0], buf.shape[1], int(to_ring), _stream()), "dv_mix_ring_copy")
 
 
 # Up to so many keys that a decode row can ever see, one launch (a workgroup per head) takes it all in bf16; beyond, splits
