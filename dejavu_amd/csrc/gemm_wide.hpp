@@ -14,6 +14,8 @@
 // 2048 rows by 22016 x 4096 338 -> 296 us, 1999 by 18560 x 4096 310 -> 276, 2048 by 8192 x 8192 233 -> 208.  Bound by power: a chunk is 2048 cycles of
 // matrix instructions and takes 2460 at 1.81 GHz with all compute units at work, at 2.1 GHz with half of them; fewer cycles come at a
 // lower clock (32 x 32 instructions: 2470 at 1.66).
+// A sum is one chain over all of K, as the library's is: of 16-bit results as many are not the nearest to 64 bits up to 8192 columns (fp16, random
+// values: 0.14 % at 2048, 0.27 % at 8192); of 20480, which the library splits, 0.32 % for its 0.24, with the same error to five digits.
 #pragma once
 #include "gemm_ring.hpp"
 
