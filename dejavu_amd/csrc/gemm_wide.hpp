@@ -26,7 +26,7 @@ constexpr size_t kWideLds = (size_t)5 * kWideRows * kWideChunk * 2;
 constexpr int64_t kWideMaxStride = 1 << 25;  // 64 rows' bytes are counted in 32 bits
 
 // NB whose rounds of tiles take least: a round takes as NB + 60, one that is not full three quarters of it and a quarter of its share (fewer compute
-// units at work have a higher clock).  Over 634 products of 257..8192 rows with cold weights of 2^23 to 2^28 values and 1024 to 9216 columns, every
+// units at work have a higher clock).  Over 634 products of 257..8192 rows with cold weights of 9 to 340 million values and 1024 to 36864 columns, every
 // width measured, the choice takes 0.1 % longer than the best one and 6 % at most.  (NB + 12 and a half: 0.9 % and 28 %; 1024 rows by 36864 x 9216 739 us,
 // now 622, the library 584; 2048 by 28672 x 7168 802 / 718 / 672; 1152 by 27648 x 5120, gated, 379 / 323 / 295.)
 inline int plan_wide(int n, int M, int units) {

@@ -147,7 +147,8 @@ DV_API int dv_dense_linear_f16(const void* x, int64_t ldx, const void* W, int64_
 
 /*
  * The same product on tiles of 256 weight rows (long prompts, where the operations bound it); act: identity, ReLU or squared
- * ReLU, others DV_ERR_UNSUPPORTED, as are row strides from 2^25 elements on.  No workspace.
+ * ReLU, which leave a NaN one (elsewhere in this library they make it zero), others DV_ERR_UNSUPPORTED, as are row strides from 2^25
+ * elements on.  No workspace.  dv_dense_linear_f16 takes these tiles for many rows too.
  */
 DV_API int dv_dense_linear_wide_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, int rows, int N,
                                     int M, int act, void* y, int64_t ldy, void* stream);
