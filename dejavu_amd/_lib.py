@@ -124,6 +124,11 @@ SIGNATURES = {
     "dv_window_step_f16": (
         _c_int, [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr]),
     "dv_window_reset": (_c_int, [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr]),
+    "dv_sparse_mlp_workspace_bytes": (_c_size, [_c_int] * 6),
+    "dv_sparse_mlp_f16": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
+         _c_ptr, _c_i64, _c_ptr, _c_i64, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr]),
     "dv_kv_append_f16": (
         _c_int,
         [_c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int,

@@ -2006,6 +2006,25 @@ int launch_ln_qkv(const QkvArgs& q, hipStream_t s) {
   return launch_status();
 }
 
+// Scratch of dv_sparse_mlp_f16: the hidden rows of the MLP and of the predictor, and what the products need in turn.
+struct MlpPlan {
+  size_t off_hidden, off_shared, shared_bytes, total;
+};
+
+MlpPlan plan_mlp(int B, int d, int n_out, int ffn, int K, int r) {
+  auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+  MlpPlan p;
+  p.off_hidden = up((size_t)B * K * sizeof(half_t));
+  p.off_shared = p.off_hidden + up((size_t)B * r * sizeof(half_t));
+  p.shared_bytes = 256;
+  // (the last: what the predictor's second product may take where it is not one of short rows)
+  for (const size_t need : {dv_gather_gemv_workspace_bytes(B, d, K), dv_gather_transposed_gemv_workspace_bytes(B, n_out, K),
+                            dv_predictor_workspace_bytes(B, d, r), B > 8 ? tiled_workspace_bytes(B, r, ffn) : 0})
+    if (need > p.shared_bytes) p.shared_bytes = need;
+  p.total = p.off_shared + up(p.shared_bytes);
+  return p;
+}
+
 // the scratch of a call is the first block's; every block of the call needs no more than it holds
 size_t layers_workspace_bytes(const dvSparseLayerArgs* layers, int n) {
   size_t need = 0;
@@ -2183,6 +2202,72 @@ int dv_sparse_layers_decode_f16(const dvSparseLayerArgs* layers, int n_layers, v
                          c.groups, 1, a.d, reinterpret_cast<half_t*>(a.hidden_out), (const half_t*)nullptr,
                          (half_t*)nullptr);
   }
+  return launch_status();
+}
+
+size_t dv_sparse_mlp_workspace_bytes(int B, int d, int n_out, int ffn, int K, int r) {
+  if (B < 1 || B > 64 || d <= 0 || n_out <= 0 || ffn <= 0 || K < 1 || r <= 0) return 0;
+  return plan_mlp(B, d, n_out, ffn, K, r).total;
+}
+
+int dv_sparse_mlp_f16(const void* x, const void* residual, const void* W1, int64_t ldw1, const void* b1, const void* W2t, int64_t ldw2,
+                      const void* b2, const void* idx, int idx_bytes, int B, int d, int n_out, int ffn, int K, int act, const void* Wa,
+                      int64_t ldwa, const void* Wb, int64_t ldwb, int r, void* y, void* logits, void* workspace, size_t workspace_bytes,
+                      void* stream) {
+  if (!x || !residual || !W1 || !W2t || !idx || !Wa || !Wb || !y || !logits || d <= 0 || n_out <= 0 || ffn <= 0 || K < 1 || r <= 0 ||
+      !idx_ok(idx_bytes) || act < DV_ACT_ID || act > DV_ACT_SQUARED_RELU)
+    return DV_ERR_INVALID_ARG;
+  if (B < 1 || B > 64) return DV_ERR_UNSUPPORTED;
+  if (d % 8 || n_out % 8 || r % 8 || ldw1 % 8 || ldw2 % 8 || ldwa % 8 || ldwb % 8 || ldw1 < d || ldw2 < n_out || ldwa < d || ldwb < r ||
+      !aligned16(x) || !aligned16(residual) || !aligned16(W1) || !aligned16(W2t) || !aligned16(Wa) || !aligned16(Wb) || !aligned16(y))
+    return DV_ERR_ALIGNMENT;
+  const MlpPlan p = plan_mlp(B, d, n_out, ffn, K, r);
+  if (!workspace || workspace_bytes < p.total || !aligned16(workspace)) return DV_ERR_WORKSPACE;
+  unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
+  half_t* h = reinterpret_cast<half_t*>(ws);
+  half_t* hidden = reinterpret_cast<half_t*>(ws + p.off_hidden);
+  void* shared = ws + p.off_shared;
+  if (B > 1 || idx_bytes != 8 || (size_t)d * sizeof(half_t) > 144 * 1024) {
+    // (several sequences' products are kernels of their own: in turn, through one piece of scratch)
+    int rc = dv_gather_gemv_ws_f16(x, W1, ldw1, b1, idx, idx_bytes, B, d, ffn, K, act, h, shared, p.shared_bytes, stream);
+    if (rc == DV_OK)
+      rc = dv_gather_transposed_gemv_f16(h, W2t, ldw2, b2, idx, idx_bytes, B, n_out, ffn, K, y, shared, p.shared_bytes, stream);
+    if (rc == DV_OK)
+      rc = dv_predictor_logits_ws_f16(residual, Wa, ldwa, Wb, ldwb, B, d, r, ffn, hidden, logits, shared, p.shared_bytes, stream);
+    return rc;
+  }
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  auto CH = [](const void* q) { return reinterpret_cast<const half_t*>(q); };
+  const int cus = compute_units();
+  auto canon_blocks = [&](int rows, int n) {
+    const int per_wave = n <= 1024 ? 4 * kCanonShortRows : 1;
+    const int blocks = ((rows + per_wave - 1) / per_wave + 3) / 4;
+    return blocks < cus * 16 ? blocks : cus * 16;
+  };
+  {
+    int nf = ((K + 1) / 2 + 3) / 4;  // two gathered rows per wavefront, as launch_gather_rows
+    if (nf > cus * 8) nf = cus * 8;
+    const CanonArgs mp0{CH(residual), CH(Wa), ldwa, r, d, hidden};
+    const int nm = canon_blocks(r, d);
+    const size_t lds = (size_t)d * sizeof(half_t);
+    auto kern = act != DV_ACT_ID ? mlp_rows_kernel<true> : mlp_rows_kernel<false>;
+    static LdsGrant grant[2];
+    if (int rc = grant[act != DV_ACT_ID].ensure(reinterpret_cast<const void*>(kern), lds); rc != DV_OK) return rc;
+    hipLaunchKernelGGL(kern, dim3(nf + nm), dim3(256), lds, s, CH(x), CH(W1), CH(b1), reinterpret_cast<const int64_t*>(idx), d, ldw1, ffn,
+                       K, h, act, nf, mp0, nm);
+  }
+  const ColsPlan c = plan_cols(n_out, K);
+  float* partial = reinterpret_cast<float*>(shared);
+  {
+    const ColsArgs cc{h, CH(W2t), ldw2, reinterpret_cast<const int64_t*>(idx), n_out, ffn, K, c.rows_per_block, c.col_tiles, c.groups,
+                      partial, reinterpret_cast<half_t*>(y), CH(b2)};
+    const CanonArgs mp1{hidden, CH(Wb), ldwb, ffn, r, reinterpret_cast<half_t*>(logits)};
+    const int nf = c.col_tiles * c.groups, nm = canon_blocks(ffn, r);
+    hipLaunchKernelGGL(layer_l8_kernel, dim3(nf + nm), dim3(256), 0, s, cc, nf, mp1, nm);
+  }
+  if (c.groups > 1)
+    hipLaunchKernelGGL(cols_reduce_kernel<false>, dim3((unsigned)((n_out + 63) / 64)), dim3(256), 0, s, partial, CH(b2), c.groups, 1,
+                       n_out, reinterpret_cast<half_t*>(y), (const half_t*)nullptr, (half_t*)nullptr);
   return launch_status();
 }
 

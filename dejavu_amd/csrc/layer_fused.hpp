@@ -296,4 +296,20 @@ __global__ __launch_bounds__(256) void layer_l8_kernel(ColsArgs c, int nblk_fc2,
   }
 }
 
+// ---- the sparse MLP by itself ------------------------------------------------
+// Roles: fc1 gather (+bias, activation) | MLP predictor fc0, both of rows that are in memory; fc2 and the predictor's second product
+// follow in layer_l8_kernel.  One sequence's step is bound by its launches (d = 768: six of 3 to 7 us for 3.5 MB, 2.5 us each the
+// launch's own), and the two chains do not depend on each other: with the split reduction three launches instead of five.
+template <bool ACT>
+__global__ __launch_bounds__(256) void mlp_rows_kernel(const half_t* __restrict__ X, const half_t* __restrict__ W, const half_t* __restrict__ bias,
+                                                       const int64_t* __restrict__ idx, int n, int64_t ldw, int Z, int M,
+                                                       half_t* __restrict__ Y, int act, int nblk_fc1, CanonArgs mp0, int nblk_mp0) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  const int bid = blockIdx.x;
+  if (bid < nblk_fc1)
+    gather_rows_body<1, 2, 4, ACT>(X, W, bias, idx, 8, n, ldw, Z, M, Y, reinterpret_cast<half_t*>(smem_raw), bid, nblk_fc1, act);
+  else
+    canonical_role(mp0, bid - nblk_fc1, nblk_mp0);
+}
+
 }  // namespace dv

@@ -16,6 +16,7 @@ the library GEMM / attention of PyTorch, as the reference's do through cuBLAS.
 """
 from __future__ import annotations
 
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -228,6 +229,48 @@ class ParallelFusedMLPDejavu(nn.Module):
         """fc2.weight as (hidden, out), contiguous; follows updates of fc2.weight."""
         return _transposed_copy(self, "fc2_weight_t", self.fc2.weight)
 
+    def _one_call(self, x, residual, idx):
+        """``forward`` of a decode step with everything in its plain form in one call of the library; None where something is not
+        (what then runs op by op converts it or says what is wrong).  The host's part of a step is what takes long: op by op, with the
+        selection before it, 55 us at d = 768 and 60 at 4096 for one sequence, 80 to 110 for 2 to 32 (the events of the side stream);
+        in one call 33, 38 and 44 to 71, whereof launches 8 to 20."""
+        # (the dictionaries, not the attributes: nn.Module looks a name up in three places, half a microsecond each)
+        fc1, fc2, sp = (self._modules.get(k) for k in ("fc1", "fc2", "sp"))
+        if type(sp) is not ParallelSP or type(fc1) is not nn.Linear or type(fc2) is not nn.Linear or _hooked(sp):
+            return None
+        W1, b1, b2 = fc1._parameters.get("weight"), fc1._parameters.get("bias"), fc2._parameters.get("bias")
+        Wa, Wb = (sp._modules[k]._parameters.get("weight") for k in ("fc0", "fc1"))
+        for t in (x, residual, W1, Wa, Wb):
+            if t is None or t.dtype != torch.float16 or not t.is_cuda or not t.is_contiguous():
+                return None
+        B, d = x.shape[0], x.shape[-1]
+        if (W1.dim() != 2 or Wa.dim() != 2 or Wb.dim() != 2 or x.dim() != 3 or not 1 <= B <= 64 or idx.dim() != 1 or
+                not idx.is_contiguous() or not idx.is_cuda or idx.dtype not in (torch.int64, torch.int32)):
+            return None
+        (ffn, d1), (r, d2), (n_logits, r2), K = W1.shape, Wa.shape, Wb.shape, idx.shape[0]
+        W2t = self.transposed_fc2()
+        n_out = W2t.shape[1]
+        if (d1 != d or d2 != d or sp.embed_dim != d or r2 != r or n_logits != ffn or W2t.shape[0] != ffn or K < 1 or W2t.dtype != torch.float16 or
+                not W2t.is_contiguous() or residual.numel() != B * d):
+            return None
+        for b, n in ((b1, ffn), (b2, n_out)):
+            if b is not None and (b.dtype != torch.float16 or not b.is_cuda or b.shape != (n,) or not b.is_contiguous()):
+                return None
+        logits = sp.logits_out
+        if logits is None:
+            logits = torch.empty(B, ffn, dtype=torch.float16, device=x.device)
+        elif logits.numel() != B * ffn or logits.dtype != torch.float16 or not logits.is_contiguous():
+            return None
+        out = torch.empty(B, 1, n_out, dtype=torch.float16, device=x.device)
+        nbytes = _one_call_bytes(torch._C._cuda_getDevice(), B, d, n_out, ffn, K, r)
+        ws = ops._workspace(x.device, nbytes)
+        if lib.dv_sparse_mlp_f16(x.data_ptr(), residual.data_ptr(), W1.data_ptr(), d, None if b1 is None else b1.data_ptr(), W2t.data_ptr(),
+                                 n_out, None if b2 is None else b2.data_ptr(), idx.data_ptr(), 8 if idx.dtype == torch.int64 else 4, B, d,
+                                 n_out, ffn, K, ops._ACT[self.activation], Wa.data_ptr(), d, Wb.data_ptr(), r, r, out.data_ptr(),
+                                 logits.data_ptr(), ws.data_ptr(), ws.numel(), ops._stream()):
+            return None
+        return out, logits.view(-1) if B == 1 else logits.view(B, ffn)
+
     def forward(self, x, residual, idx=None, defer_join=False, defer_reduce=False):
         """x, residual: (B, 1, d) at decode (or (B, s, d) for the prompt).
         idx: (K,) active neurons or None for the dense MLP.
@@ -249,6 +292,12 @@ class ParallelFusedMLPDejavu(nn.Module):
         # must be the one captured first (batch 8, OPT-175B shape: four such hand-overs per layer step).
         mlp_logit = None
         side = do_token_generation and side_stream_enabled(x.shape[0])
+        # (from a graph the products and the predictor of several sequences side by side, as below: there the host takes no part)
+        if idx is not None and do_token_generation and not (defer_reduce or USE_SIDE_STREAM or (side and (
+                defer_join or torch.cuda.is_current_stream_capturing()))):
+            done = self._one_call(x, residual, idx)
+            if done is not None:
+                return done
         if side:
             self._streams()
             curr_stream = torch.cuda.current_stream()
@@ -286,6 +335,17 @@ class ParallelFusedMLPDejavu(nn.Module):
         return out, mlp_logit
 
 
+def _hooked(module) -> bool:
+    return bool("forward" in module.__dict__ or module._forward_hooks or module._forward_pre_hooks or
+                nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks)
+
+
+@lru_cache(maxsize=4096)
+def _one_call_bytes(device: int, B: int, d: int, n_out: int, ffn: int, K: int, r: int) -> int:
+    """A function of the sizes and of the current device, whose compute units the splits are made for."""
+    return lib.dv_sparse_mlp_workspace_bytes(B, d, n_out, ffn, K, r)
+
+
 def _long_rule(rows: int, M: int, K: int) -> bool:
     if K < 4 * M or M * K < HIP_PROMPT_LONG_WEIGHT:
         return False
@@ -312,8 +372,7 @@ def _plain_layer(linear, x: torch.Tensor) -> bool:
     takes where they are, only results asked for."""
     W, b = linear.weight, linear.bias
     return (type(linear) is nn.Linear and W.dim() == 2 and x.shape[-1] == W.shape[1] and
-            "forward" not in linear.__dict__ and not (linear._forward_hooks or linear._forward_pre_hooks) and
-            not (nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks) and
+            not _hooked(linear) and
             results_only(x, W, b) and W.stride(1) == 1 and W.stride(0) >= W.shape[1] and W.stride(0) % 8 == 0 and W.data_ptr() % 16 == 0 and
             x.data_ptr() % 16 == 0 and (b is None or (b.dtype == W.dtype and b.shape == W.shape[:1])))
 

@@ -603,6 +603,23 @@ DV_API int dv_sparse_layer_decode_f16(const dvSparseLayerArgs* args, void* strea
  */
 DV_API int dv_sparse_layers_decode_f16(const dvSparseLayerArgs* layers, int n_layers, void* stream);
 
+/*
+ * The sparse MLP of a decode step together with the predictor for the next layer, ParallelFusedMLPDejavu.forward,
+ * Dejavu/src/ops/fused_dense_sparse_dejavu.py:889-951: y = fc2(act(fc1(x))) over the neurons idx and
+ * logits = Wb . fp16(Wa . residual).  The same bits as dv_gather_gemv_ws_f16, dv_gather_transposed_gemv_f16 and
+ * dv_predictor_logits_ws_f16 one after the other, which is what more than one row and 32-bit indices are; one row
+ * with 64-bit indices takes three launches.
+ *   x, residual (B, d); W1 (ffn, d); b1 (ffn,) or NULL; W2t (ffn, n_out); b2 (n_out,) or NULL; idx (K,), K >= 1;
+ *   Wa (r, d); Wb (ffn, r); y (B, n_out); logits (B, ffn); row strides ldw1, ldw2, ldwa, ldwb.  1 <= B <= 64.
+ *   workspace: dv_sparse_mlp_workspace_bytes() bytes on a 16-byte boundary, no initialisation needed.
+ */
+DV_API size_t dv_sparse_mlp_workspace_bytes(int B, int d, int n_out, int ffn, int K, int r);
+DV_API int dv_sparse_mlp_f16(const void* x, const void* residual, const void* W1, int64_t ldw1, const void* b1,
+                             const void* W2t, int64_t ldw2, const void* b2, const void* idx, int idx_bytes, int B,
+                             int d, int n_out, int ffn, int K, int act, const void* Wa, int64_t ldwa, const void* Wb,
+                             int64_t ldwb, int r, void* y, void* logits, void* workspace, size_t workspace_bytes,
+                             void* stream);
+
 #ifdef __cplusplus
 }
 #endif
