@@ -89,6 +89,8 @@ SIGNATURES = {
     "dv_mix_linear_split_workspace_bytes": (ctypes.c_size_t, [_i, _i, _i]),
     "dv_mix_linear_split": (_i, [_p, _l, _p, _l, _p, _i, _i, _i, _p, _l, _p, ctypes.c_size_t, _p]),
     "dv_mix_linear_wide": (_i, [_i, _P(TileArgs), _p]),
+    "dv_mix_linear_wide_workspace_bytes": (ctypes.c_size_t, [_i, _i, _i]),
+    "dv_mix_linear_wide_ws": (_i, [_i, _P(TileArgs), _p, ctypes.c_size_t, _p]),
     "dv_mix_short_conv": (_i, [_i, _i, _P(ConvArgs), _p]),
     "dv_mix_short_conv_move": (_i, [_i, _i, _P(ConvArgs), _p, _p]),
     "dv_mix_conv_state": (_i, [_i, _p, _l, _i, _i, _i, _p, _p]),

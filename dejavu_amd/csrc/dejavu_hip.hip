@@ -627,6 +627,12 @@ int linear_wide(const RingOperands<half_t>& a, const half_t* bias, int act, half
     default: return DV_ERR_UNSUPPORTED;
   }
 }
+template <int ACT>
+int launch_wide_parts(const WideSplit& p, const RingOperands<half_t>& a, const half_t* bias, half_t* Y, int64_t ldy, float* part, hipStream_t s) {
+  const int rc = gemm_wide(p.nb, a, WidePart{part, a.n, a.M}, s, RingLaunch{}, p.splits);
+  if (rc != DV_OK) return rc;
+  return wide_sum(p.splits, part, a.n, a.M, WideSumOut<ACT>{WidePlainOut<ACT>{bias, Y, ldy, a.M}}, s, RingLaunch{});
+}
 // Of products that gemm_big.hpp or gemm_tiled.hpp would take those whose tiles fill most of the chip (12288 / 16384 x 4096 with 777 rows
 // 161 -> 76, 211 -> 94 us, 4096 x 16384 with 1200 / 1000 rows 265 -> 199, 194 / 198).
 bool wide_takes(int B, int M, int act) {
@@ -1203,6 +1209,35 @@ int dv_dense_linear_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, 
                     reinterpret_cast<const half_t*>(bias), nullptr, 4, rows, N, M, M, act,
                     reinterpret_cast<half_t*>(y), ldy, workspace, workspace_bytes,
                     reinterpret_cast<hipStream_t>(stream));
+}
+
+size_t dv_dense_linear_wide_workspace_bytes(int rows, int N, int M) {
+  if (rows < 1 || N <= 0 || M <= 0) return 0;
+  const WideSplit p = plan_wide_split(rows, M, N, compute_units());
+  return p.splits > 1 ? p.workspace_bytes(rows, M) : 0;
+}
+
+int dv_dense_linear_wide_ws_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, int rows, int N, int M, int act,
+                                void* y, int64_t ldy, void* workspace, size_t workspace_bytes, void* stream) {
+  const WideSplit p = rows > 0 && N > 0 && M > 0 ? plan_wide_split(rows, M, N, compute_units()) : WideSplit{256, 1};
+  if (p.splits == 1 || act == DV_ACT_GELU || act == DV_ACT_GELU_APPROX)
+    return dv_dense_linear_wide_f16(x, ldx, W, ldw, bias, rows, N, M, act, y, ldy, stream);
+  if (!x || !W || !y || act < DV_ACT_ID || act > DV_ACT_SQUARED_RELU) return DV_ERR_INVALID_ARG;
+  if (N % 8 || M % 8 || ldx % 8 || ldw % 8 || ldy % 4 || ldx < N || ldw < N || ldy < M || !aligned16(x) || !aligned16(W) || !aligned8(y))
+    return DV_ERR_ALIGNMENT;
+  if (ldw >= kWideMaxStride || ldx >= kWideMaxStride) return DV_ERR_UNSUPPORTED;
+  if (!workspace || workspace_bytes < p.workspace_bytes(rows, M)) return DV_ERR_WORKSPACE;
+  if (!aligned16(workspace)) return DV_ERR_ALIGNMENT;
+  const RingOperands<half_t> a{reinterpret_cast<const half_t*>(x), ldx, reinterpret_cast<const half_t*>(W), ldw, rows, M, N};
+  const half_t* b = reinterpret_cast<const half_t*>(bias);
+  half_t* Y = reinterpret_cast<half_t*>(y);
+  float* part = reinterpret_cast<float*>(workspace);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  switch (act) {
+    case DV_ACT_ID: return launch_wide_parts<DV_ACT_ID>(p, a, b, Y, ldy, part, s);
+    case DV_ACT_RELU: return launch_wide_parts<DV_ACT_RELU>(p, a, b, Y, ldy, part, s);
+    default: return launch_wide_parts<DV_ACT_SQUARED_RELU>(p, a, b, Y, ldy, part, s);
+  }
 }
 
 int dv_dense_linear_wide_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, int rows, int N, int M, int act,

@@ -151,6 +151,17 @@ struct WidePlainOut {
   }
 };
 
+// What wide_sum_kernel stores: WidePlainOut's results, rows on 8-byte boundaries.
+template <int ACT>
+struct WideSumOut {
+  WidePlainOut<ACT> out;
+  typedef typename WidePlainOut<ACT>::Row Ready;
+  __device__ __forceinline__ Ready ready(int64_t, int m) const { return out.row(m); }
+  __device__ __forceinline__ void operator()(int64_t row, int m, const float4_t& v, const Ready& r) const {
+    *reinterpret_cast<half4_t*>(out.Y + row * out.ldy + m) = out.make(r, v);
+  }
+};
+
 struct GatheredRows {
   static constexpr bool kPastCaches = true;
   static constexpr int kMostCols = 64;

@@ -14,7 +14,9 @@
 // 2048 rows by 22016 x 4096 338 -> 296 us, 1999 by 18560 x 4096 310 -> 276, 2048 by 8192 x 8192 233 -> 208.  Bound by power: a chunk is 2048 cycles of
 // matrix instructions and takes 2460 at 1.81 GHz with all compute units at work, at 2.1 GHz with half of them; fewer cycles come at a
 // lower clock (32 x 32 instructions: 2470 at 1.66).
-// A sum is one chain over all of K, as the library's is: of 16-bit results as many are not the nearest to 64 bits up to 8192 columns (fp16, random
+// Tiles too few for the chip share a split of K each (plan_wide_split), whose sums go to memory as rows of fp32 and are added up by the
+// launch behind, together with what it is for: 777 rows by 4096 x 16384 192 us in 64 tiles, 113 in four splits (the library 146).
+// A sum is one chain over all of K (of a split's part of it), as the library's is: of 16-bit results as many are not the nearest to 64 bits up to 8192 columns (fp16, random
 // values: 0.14 % at 2048, 0.27 % at 8192); of 20480, which the library splits, 0.32 % for its 0.24, with the same error to five digits.
 #pragma once
 #include "gemm_ring.hpp"
@@ -40,6 +42,32 @@ inline int plan_wide(int n, int M, int units) {
   return best;
 }
 
+struct WideSplit {
+  int nb, splits;
+  size_t workspace_bytes(int n, int M) const { return (size_t)splits * n * M * sizeof(float); }
+};
+
+// The same with K in up to six parts, one round of workgroups at most: a chunk takes as NB + 180 (fewer columns share the chunk of W, and cold
+// weights arrive slower than they are multiplied), a workgroup's ends as 4500, a part's sums as 4.2e-4 each, to memory and back.
+// Over 96 products of 257..2048 rows (2048 to 7168 weight rows, 5632 to 28672 columns, cold), every choice measured with the launch that adds
+// up: 1.1 % longer than the best one, 14 % at most.
+inline WideSplit plan_wide_split(int n, int M, int K, int units) {
+  WideSplit best{256, 1};
+  double least = 0.0;
+  const int chunks = K / kWideChunk;
+  for (int nb = 256; nb >= 128; nb -= 32) {
+    const int64_t tiles = ((int64_t)M + kWideRows - 1) / kWideRows * (((int64_t)n + nb - 1) / nb);
+    for (int splits = 1; splits <= 6; ++splits) {
+      if (splits > 1 && (tiles * splits > units || chunks < splits * 8)) break;
+      const int64_t rest = tiles * splits % units;
+      const double rounds = (double)(tiles * splits / units) + (rest ? 0.62 + 0.38 * rest / units : 0.0);
+      const double t = rounds * (((chunks + splits - 1) / splits) * (double)(nb + 180) + 4500.0) + 4.2e-4 * splits * n * (double)M;
+      if (least == 0.0 || t < least) best = {nb, splits}, least = t;
+    }
+  }
+  return best;
+}
+
 // Four values of a vector of M from place m on (past its end: its last one), m % 4 == 0.
 template <typename T>
 struct WideBias {
@@ -57,6 +85,17 @@ struct WideBias {
   }
 };
 
+// A part's sums: rows of M floats (M % 4 == 0), one part after the other.
+struct WidePart {
+  struct Row {};
+  float* part;
+  int64_t rows;
+  int M;
+  __device__ __forceinline__ void store(int m, int row, const float4_t& v) const {
+    *reinterpret_cast<float4_t*>(part + (blockIdx.y * rows + row) * M + m) = v;
+  }
+};
+
 // The sums stay where they are: the compiler copies them from one set of registers to another when left to itself.
 template <typename T>
 __device__ __forceinline__ void wide_mfma(float4_t& acc, const ring_word_t& w, const ring_word_t& x) {
@@ -67,11 +106,13 @@ __device__ __forceinline__ void wide_mfma(float4_t& acc, const ring_word_t& w, c
 // Out: kOuts results (of type T, columns kOuts / 4 * m ..) of the sums of rows m .. m + 3, by make(row(m), sums) for any m below the
 // tile's end; row(m), what a row's results need beside their sums, is asked for before the loop (a bias read behind it: 69 instead of
 // 63 us, 2048 rows by 4096 x 4096); base, ld, columns: where they go.
+// WidePart: part blockIdx.y of gridDim.y of K.
 // Grid: row_tiles * col_tiles (256 rows of W, NB rows of X).  K, ldx, ldw % 8 == 0, X and W on 16-byte boundaries.
 template <typename T, int NB, typename Out>
 __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(RingOperands<T> a, Out out, int row_tiles, int col_tiles) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (the loads' resources have no type on the host)
   extern __shared__ __attribute__((aligned(16))) unsigned char slots[];
+  constexpr bool PART = __is_same(Out, WidePart);
   constexpr int MB = kWideRows, KC = kWideChunk, CH = KC / 8, RPL = 64 / CH, UNIT = MB * KC * 2;
   constexpr int RT = MB / 32, NT = NB / 32;                      // tiles of 16 rows a wave
   constexpr int LW = MB / RPL / 4, LX = NB / RPL / 4;            // loads of a wave
@@ -88,7 +129,9 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(RingOperands<T> a, Ou
     bm = block * 8 + at % tall;
     bn = at / tall;
   }
-  const int m0 = bm * MB, n0 = bn * NB, nch = a.K / KC;
+  const int m0 = bm * MB, n0 = bn * NB, chunks = a.K / KC;  // (the columns behind the whole chunks are the last part's)
+  const int c0 = PART ? chunks * (int)blockIdx.y / (int)gridDim.y : 0;
+  const int nch = (PART ? chunks * ((int)blockIdx.y + 1) / (int)gridDim.y : chunks) - c0;
 
   // A wave loads 64 rows of W and NB / 4 of X, eight rows at a time; rows past the end are the last one again.  A row's pieces of
   // 16 bytes lie in LDS at places exchanged by the row (place = piece ^ row): 16 rows' pieces are read from different banks.
@@ -106,15 +149,16 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(RingOperands<T> a, Ou
   for (int i = 0; i < LX; ++i)
     x_at[i] = (unsigned)(min(n0 + (wave * LX + i) * RPL + lane / CH, a.n - 1) - x_row) * (unsigned)a.ldx * 2u + piece * 16;
   auto load_w = [&](int c, int unit, int i) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_ptr_t)(slots + unit * UNIT + (wave * LW + i) * 1024), 16, w_at[i], c * KC * 2, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_ptr_t)(slots + unit * UNIT + (wave * LW + i) * 1024), 16, w_at[i], (c0 + c) * KC * 2, 0, 0);
   };
   auto load_x = [&](int c, int unit, int i) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr_t)(slots + unit * UNIT + (wave * LX + i) * 1024), 16, x_at[i], c * KC * 2, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr_t)(slots + unit * UNIT + (wave * LX + i) * 1024), 16, x_at[i], (c0 + c) * KC * 2, 0, 0);
   };
 
-  typename Out::Row rows[RT];
+  typename Out::Row rows[PART ? 1 : RT];
+  if constexpr (!PART)
 #pragma unroll
-  for (int i = 0; i < RT; ++i) rows[i] = out.row(m0 + (wm * RT + i) * 16 + g * 4);
+    for (int i = 0; i < RT; ++i) rows[i] = out.row(m0 + (wm * RT + i) * 16 + g * 4);
   ring_word_t w[2][RT], x[2][NT];
   float4_t acc[RT][NT];
 #pragma unroll
@@ -188,11 +232,11 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(RingOperands<T> a, Ou
     }
   }
   static_assert(LW == RT && LX <= RT && RT + NT <= 2 * RT, "a row of instructions has one load and two reads");
-  if (a.K % KC != 0) {  // the columns behind the whole chunks, zeros past the rows' end
+  if (a.K % KC != 0 && (!PART || blockIdx.y + 1 == gridDim.y)) {  // the columns behind the whole chunks, zeros past the rows' end
     all_here();
-    const unsigned back = max(nch * KC + piece * 8 - (a.K - 8), 0) * 2;
+    const unsigned back = max(chunks * KC + piece * 8 - (a.K - 8), 0) * 2;
 #pragma unroll
-    for (int i = 0; i < LW; ++i) w_at[i] -= back, load_w(nch, 0, i);
+    for (int i = 0; i < LW; ++i) w_at[i] -= back, load_w(nch, 0, i);  // (chunk nch of this part: c0 + nch == chunks)
 #pragma unroll
     for (int i = 0; i < LX; ++i) x_at[i] -= back, load_x(nch, 1, i);
     all_here();
@@ -201,7 +245,7 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(RingOperands<T> a, Ou
 #pragma unroll
       for (int i = 0; i < RT + NT; ++i) read(0, 1, half, i);
       reads_back();
-      if (nch * CH + half * 4 + g >= a.K / 8) {
+      if (chunks * CH + half * 4 + g >= a.K / 8) {
 #pragma unroll
         for (int i = 0; i < RT; ++i) w[half][i] = ring_word_t{0, 0, 0, 0};
 #pragma unroll
@@ -216,6 +260,17 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(RingOperands<T> a, Ou
   asm volatile("s_nop 15" ::: "memory");  // the last sums are there
   __builtin_amdgcn_sched_barrier(0);
 
+  if constexpr (PART) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int m = m0 + (wm * RT + i) * 16 + g * 4, row = n0 + (wn * NT + j) * 16 + l16;
+        if (m < a.M && row < a.n) out.store(m, row, acc[i][j]);
+      }
+    wait_loads<0>();  // no load into LDS outlives the workgroup
+    return;
+  } else {
   typedef T out_t __attribute__((ext_vector_type(Out::kOuts)));
   T* const base = out.base();
   const int64_t ld = out.ld();
@@ -262,15 +317,49 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(RingOperands<T> a, Ou
           if (row < a.n && col + k < columns) base[row * ld + col + k] = v[k];
       }
   }
-  wait_loads<0>();  // no load into LDS outlives the workgroup
+  wait_loads<0>();
+  }
 #endif
+}
+
+// Adds the parts up in their order.  done(row, m, sums of rows m .. m + 3 of W, ready(row, m)); ready asks for what is needed beside them.
+template <int SPLITS, typename Done>
+__global__ __launch_bounds__(256) void wide_sum_kernel(const float* __restrict__ part, int64_t rows, int M, Done done) {
+  const int64_t quads = rows * M / 4;
+  const float4_t* p = reinterpret_cast<const float4_t*>(part);
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < quads; q += (int64_t)gridDim.x * 256) {
+    const int64_t row = q * 4 / M;
+    const int m = (int)(q * 4 - row * M);
+    float4_t v[SPLITS];
+#pragma unroll
+    for (int k = 0; k < SPLITS; ++k) v[k] = p[k * quads + q];
+    const auto ready = done.ready(row, m);
+#pragma unroll
+    for (int k = 1; k < SPLITS; ++k) v[0] += v[k];
+    done(row, m, v[0], ready);
+  }
+}
+
+template <typename Done, typename Launch>
+int wide_sum(int splits, const float* part, int64_t rows, int M, const Done& done, hipStream_t s, const Launch& launch) {
+  const int64_t blocks = (rows * M / 4 + 255) / 256;
+  const dim3 grid((unsigned)(blocks < 8192 ? blocks : 8192)), threads(256);
+#define DV_SUM(S) launch.template operator()<wide_sum_kernel<S, Done>>(grid, threads, (size_t)0, s, part, rows, M, done)
+  switch (splits) {
+    case 2: return DV_SUM(2);
+    case 3: return DV_SUM(3);
+    case 4: return DV_SUM(4);
+    case 5: return DV_SUM(5);
+    default: return DV_SUM(6);
+  }
+#undef DV_SUM
 }
 
 // launch as for gemm_ring
 template <typename T, typename Out, typename Launch>
-int gemm_wide(int nb, const RingOperands<T>& a, const Out& out, hipStream_t s, const Launch& launch) {
+int gemm_wide(int nb, const RingOperands<T>& a, const Out& out, hipStream_t s, const Launch& launch, int splits = 1) {
   const int64_t rows = ((int64_t)a.M + kWideRows - 1) / kWideRows, cols = ((int64_t)a.n + nb - 1) / nb;
-  const dim3 grid((unsigned)(rows * cols)), threads(256);
+  const dim3 grid((unsigned)(rows * cols), (unsigned)splits), threads(256);
 #define DV_WIDE(NB) launch.template operator()<gemm_wide_kernel<T, NB, Out>>(grid, threads, kWideLds, s, a, out, (int)rows, (int)cols)
   switch (nb) {
     case 128: return DV_WIDE(128);

@@ -77,4 +77,45 @@ struct WideOut {
   }
 };
 
+// What follows a sublayer's last product behind the sums of its parts, four channels at a time (residual_norm_kernel's arithmetic on the
+// sums as they are).
+struct WideResidual {
+  dvResidual r;
+  int M;
+  struct Ready {
+    float4_t x, x0;
+  };
+  __device__ __forceinline__ Ready ready(int64_t row, int m) const {
+    Ready o;
+    o.x = *reinterpret_cast<const float4_t*>(r.x + row * M + m);
+    o.x0 = r.x0 ? *reinterpret_cast<const float4_t*>(r.x0 + row * M + m) : float4_t{0.f, 0.f, 0.f, 0.f};
+    return o;
+  }
+  __device__ __forceinline__ void operator()(int64_t row, int m, const float4_t& y, const Ready& o) const {
+    const int64_t at = row * M + m;
+    float4_t v = o.x, h;
+    const float4_t w = *reinterpret_cast<const float4_t*>(r.post.w + m), b = *reinterpret_cast<const float4_t*>(r.post.b + m);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += __builtin_fmaf(tanh_f(r.post.alpha * y[e]), w[e], b[e]);
+    if (r.x0) v += o.x0;
+    *reinterpret_cast<float4_t*>(r.x + at) = v;
+    if (!r.h) return;
+    const float4_t pw = *reinterpret_cast<const float4_t*>(r.pre.w + m), pb = *reinterpret_cast<const float4_t*>(r.pre.b + m);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = __builtin_fmaf(tanh_f(r.pre.alpha * v[e]), pw[e], pb[e]);
+    store_quad(reinterpret_cast<bf16_t*>(r.h) + at, h);
+  }
+};
+
+// The parts' sums as rows of bf16, on 8-byte boundaries.
+struct WideSumOut {
+  WideOut<DV_OUT_T> out;
+  typedef WideOut<DV_OUT_T>::Row Ready;
+  __device__ __forceinline__ Ready ready(int64_t, int m) const { return out.row(m); }
+  __device__ __forceinline__ void operator()(int64_t row, int m, const float4_t& v, const Ready& r) const {
+    typedef WideOut<DV_OUT_T>::vec_t vec_t;
+    *reinterpret_cast<vec_t*>(out.base() + row * out.ld() + m) = out.make(r, v);
+  }
+};
+
 }  // namespace dv

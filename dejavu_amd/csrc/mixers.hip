@@ -89,6 +89,15 @@ int linear_wide(const TileArgs& a, hipStream_t s) {
   return gemm_wide(nb, o, WideOut<AFTER>{a}, s, WideLaunch{});
 }
 
+// K in parts where the tiles are few.
+template <typename Done>
+int linear_wide_parts(const WideSplit& p, const TileArgs& a, float* part, const Done& done, hipStream_t s) {
+  const RingOperands<bf16_t> o{reinterpret_cast<const bf16_t*>(a.x), a.ldx, reinterpret_cast<const bf16_t*>(a.W), a.ldw, a.n, a.M, a.K};
+  const int rc = gemm_wide(p.nb, o, WidePart{part, a.n, a.M}, s, WideLaunch{}, p.splits);
+  if (rc != DV_OK) return rc;
+  return wide_sum(p.splits, part, a.n, a.M, done, s, WideLaunch{});
+}
+
 template <int AFTER>
 int linear_stream(const RingPlan& p, const TileArgs& a, void* workspace, hipStream_t s) {
   const RingOperands<bf16_t> o{reinterpret_cast<const bf16_t*>(a.x), a.ldx, reinterpret_cast<const bf16_t*>(a.W), a.ldw, a.n, a.M, a.K};
@@ -616,6 +625,34 @@ int dv_mix_linear_wide(int after, const dvTileArgs* a, void* stream) {
   if (tiles > 0x7fffffff) return DV_ERR_UNSUPPORTED;
   if (a->ldw < 0 || a->ldw >= kWideMaxStride || a->ldx < 0 || a->ldx >= kWideMaxStride) return linear_far(after, *a, st(stream));
   return after == DV_OUT_T ? linear_wide<DV_OUT_T>(*a, st(stream)) : linear_wide<DV_OUT_GLU>(*a, st(stream));
+}
+
+size_t dv_mix_linear_wide_workspace_bytes(int n, int M, int K) {
+  if (n < 1 || M < 1 || K < 8) return 0;
+  const WideSplit p = plan_wide_split(n, M, K, compute_units());
+  return p.splits > 1 ? p.workspace_bytes(n, M) : 0;
+}
+
+int dv_mix_linear_wide_ws(int after, const dvTileArgs* a, void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = tile_args_ok(after, a);
+  if (rc != DV_OK) return rc;
+  if (after != DV_OUT_T && after != DV_OUT_RESIDUAL) return DV_ERR_UNSUPPORTED;
+  const int64_t tiles = ((int64_t)a->M + kWideRows - 1) / kWideRows * (((int64_t)a->n + 127) / 128);
+  if (tiles > 0x7fffffff || a->ldw < 0 || a->ldw >= kWideMaxStride || a->ldx < 0 || a->ldx >= kWideMaxStride) return DV_ERR_UNSUPPORTED;
+  const WideSplit p = plan_wide_split(a->n, a->M, a->K, compute_units());
+  if (after == DV_OUT_RESIDUAL) {
+    if (p.splits == 1) return DV_ERR_UNSUPPORTED;
+    if (!a->res.post.b || (a->res.h && !a->res.pre.b)) return DV_ERR_INVALID_ARG;
+    if (a->M % 8 || !al16(a->res.x) || !al16(a->res.h)) return DV_ERR_ALIGNMENT;
+  } else {
+    if (p.splits == 1) return linear_wide<DV_OUT_T>(*a, st(stream));
+    if (a->M % 8 || a->ldo % 4 || !al16(a->out)) return DV_ERR_ALIGNMENT;
+  }
+  if (!workspace || workspace_bytes < p.workspace_bytes(a->n, a->M)) return DV_ERR_WORKSPACE;
+  if (!al16(workspace)) return DV_ERR_ALIGNMENT;
+  float* part = reinterpret_cast<float*>(workspace);
+  return after == DV_OUT_T ? linear_wide_parts(p, *a, part, WideSumOut{WideOut<DV_OUT_T>{*a}}, st(stream))
+                           : linear_wide_parts(p, *a, part, WideResidual{a->res, a->M}, st(stream));
 }
 
 int dv_mix_linear_tiles(int after, const dvTileArgs* a, void* stream) {

@@ -168,6 +168,45 @@ def _fill_rule(n: int, M: int, K: int, gated: bool) -> bool:
     return K <= columns[0] or tiles >= WIDE_FULL_GATED * places
 
 
+# Long rows whose tiles leave much of the chip idle: K in parts on the same tiles, the sums added up by the launch that follows (plan_wide_split),
+# with the residual in it.  The library's time over the kernels', weights cold, 16 numbers of rows from 257 to 2048 each:
+#   plain: 4096 x 11008 / 14336 1.00 to 1.17 and 1.03 to 2.09, 5120 x 13824 1.05 to 2.05, 3072 x 12288 1.14 to 1.34, 3072 / 2560 x 10240 from 385 rows on
+#     1.01 to 1.17 and 1.06 to 1.31 (fewer 0.91 to 1.18); but 4096 x 8192 0.80 to 1.18, 2048 x 8192 0.89 to 1.13, 4096 x 4096 0.78 to 1.01;
+#   with the residual: 4096 x 8192 1.06 to 1.26, 4096 x 11008 1.06 to 1.17, 4096 x 14336 1.06 to 1.95, 5120 x 13824 1.11 to 1.40, 3072 x 12288 1.14 to 1.40;
+#     but 2048 x 5632 0.95 to 1.17, 3072 x 8192 0.96 to 1.17, 4096 x 4096 0.91 to 1.04.
+#   Of more weight rows only in three parts and more: 8192 x 28672 in four 1.07 to 1.50, in two 0.87 to 1.10.
+PARTS_COLUMNS, PARTS_RESIDUAL_COLUMNS = 10240, 8192
+PARTS_WEIGHT, PARTS_LIGHT_WEIGHT, PARTS_LIGHT_ROWS = 1 << 25, 26_000_000, 385   # elements; a lighter one with so many rows at least
+PARTS_TALL = 7168, 3                                                            # weight rows, parts at least of more of them
+
+
+def _parts_rule(n: int, M: int, K: int, residual: bool, parts: int) -> bool:
+    if not TILE_MAX_ROWS < n <= WIDE_MAX_ROWS or M % 8 or parts < (PARTS_TALL[1] if M > PARTS_TALL[0] else 2):
+        return False
+    light = not residual and n >= PARTS_LIGHT_ROWS
+    return K >= (PARTS_RESIDUAL_COLUMNS if residual else PARTS_COLUMNS) and M * K >= (PARTS_LIGHT_WEIGHT if light else PARTS_WEIGHT)
+
+
+@lru_cache(maxsize=4096)
+def _parts_workspace_bytes(device: int, n: int, M: int, K: int) -> int:
+    """As ``_tile_workspace_bytes``; 0: the tiles are enough for the chip."""
+    return lib.dv_mix_linear_wide_workspace_bytes(n, M, K)
+
+
+def _parts_bytes(x: torch.Tensor, W: torch.Tensor, bias=None, residual: bool = False) -> int:
+    """What the wide kernel's parts of the product need; 0: it is not one of its products."""
+    n, (M, K) = x.shape[0], W.shape
+    if not TILE_MAX_ROWS < n <= WIDE_MAX_ROWS:
+        return 0
+    nbytes = _parts_workspace_bytes(torch._C._cuda_getDevice(), n, M, K)
+    return nbytes if _parts_rule(n, M, K, residual, nbytes // (4 * n * M)) and _wide_fits(x, W, bias) else 0
+
+
+def _parts_launch(after, a, nbytes, device) -> None:
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    check(lib.dv_mix_linear_wide_ws(after, _ref(a), _ptr(ws), nbytes, _stream()), "dv_mix_linear_wide_ws")
+
+
 def _tile_rule(n: int, M: int, K: int, gated: bool) -> bool:
     if n > TILE_MAX_ROWS:
         return False
@@ -347,6 +386,13 @@ def linear(x, W: torch.Tensor, bias: Optional[torch.Tensor] = None, f32: bool = 
         a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
         _tile_launch(L.OUT_F32 if f32 else L.OUT_T, a, x.device)
         return out
+    nbytes = 0 if f32 else _parts_bytes(x, W, bias)
+    if nbytes:
+        out = torch.empty(n, M, dtype=out_t, device=x.device)
+        a = _tile_args(x, W)
+        a.out, a.ldo, a.bias = out.data_ptr(), M, _ptr(bias)
+        _parts_launch(L.OUT_T, a, nbytes, x.device)
+        return out
     # (rows of results off 16-byte boundaries are stored value by value: 400 / 1200 rows by 11266 x 2048 0.91 / 0.88 of the library's speed, where
     # 11264 x 2048 is 1.17 / 0.97; 2048 by 22020 x 4096 343 us, 274)
     if not f32 and M % 8 == 0 and (_wide(x, W, bias) or _fills(x, W, bias)):
@@ -396,7 +442,14 @@ def linear_residual(x: torch.Tensor, W: torch.Tensor, stream: ResidualStream, po
     n = x.shape[0]
     assert stream.x.shape == (n, W.shape[0])
     if n != 1 and not _tiles(x, W, whole=W.shape[0] % 8 == 0):
-        return residual(_library_or_split(x, W), stream, post, pre, add_start)
+        nbytes = _parts_bytes(x, W, residual=True)
+        if not nbytes:
+            return residual(_library_or_split(x, W), stream, post, pre, add_start)
+        h = None if pre is None else stream.new_h()
+        a = _tile_args(x, W)
+        a.res = stream.args(post, pre, add_start, h)
+        _parts_launch(L.OUT_RESIDUAL, a, nbytes, x.device)
+        return h
     h = None if pre is None else stream.new_h()
     if n == 1:
         a = _row_args(x, W)

@@ -72,6 +72,12 @@ HIP_PROMPT_WIDE_LONGEST = 8192, 5120   # rows, columns (with an activation)
 HIP_PROMPT_WIDE_COLUMNS, HIP_PROMPT_WIDE_FILL = (2048, 3072), (128, 256)
 HIP_PROMPT_WIDE_LONG = 769, (20480, 21504), 136  # rows, columns (from, to), tiles
 HIP_PROMPT_WIDE_STRIDE = 1 << 25
+# Long rows whose tiles leave much of the chip idle: the columns in parts, the sums added up by a second launch (plan_wide_split).  What took them before (the
+# library, from 769 rows on by 20480 columns the wide tiles) over this, weights cold, 257 to 2048 rows: 2560 x 10240 1.06 to 1.30, 3072 x 12288 0.99 to 1.34,
+# 4096 x 16384 1.00 to 2.09, 4608 x 18432 1.05 to 1.92, 5120 x 20480 1.14 to 1.72, 5632 x 22528 1.32 to 1.61, 7168 x 28672 1.38 to 1.62, 9216 x 36864 1.38
+# to 1.39 (777 by 4096 x 16384 146 -> 103 us).  Of more weight rows only in three parts and more: in two 8192 x 28672 0.89 to 1.01, 12288 x 49152 0.90 to 1.00.
+HIP_PROMPT_PARTS_COLUMNS, HIP_PROMPT_PARTS_WEIGHT = 10240, 26_000_000
+HIP_PROMPT_PARTS_TALL = 7168, 3
 # The package's causal-attention kernel (cache fill in the same launch) is ahead of the library's attention with the
 # permuted cache copies (40 heads of 128 and 128 / 1024 tokens: 7.5 / 47 us against 25 / 100; 32 heads and
 # 777 / 2000 / 4000 tokens: 30 / 110 / 385 against 75 / 310 / 566; 16 sequences of 1024: 547 against 768).  Prompts of more than so
@@ -383,19 +389,41 @@ def _long_product(linear, x: torch.Tensor) -> bool:
     return W.dim() == 2 and _long_rule(x.numel() // x.shape[-1], *W.shape) and _plain_layer(linear, x)
 
 
+def _wide_fits(linear, x: torch.Tensor) -> bool:
+    W, b = linear.weight, linear.bias
+    return x.is_contiguous() and W.stride(0) < HIP_PROMPT_WIDE_STRIDE and (b is None or b.is_contiguous()) and _plain_layer(linear, x)
+
+
 def _wide_product(linear, x: torch.Tensor, activation: str) -> bool:
     """The same of ``dense_linear_wide``."""
-    W, b = linear.weight, linear.bias
-    return (W.dim() == 2 and _wide_rule(x.numel() // x.shape[-1], *W.shape, activation) and x.is_contiguous() and
-            W.stride(0) < HIP_PROMPT_WIDE_STRIDE and (b is None or b.is_contiguous()) and _plain_layer(linear, x))
+    W = linear.weight
+    return W.dim() == 2 and _wide_rule(x.numel() // x.shape[-1], *W.shape, activation) and _wide_fits(linear, x)
+
+
+def _parts_rule(rows: int, M: int, K: int, parts: int) -> bool:
+    many, least = HIP_PROMPT_PARTS_TALL
+    return (HIP_PROMPT_WIDE_ROWS[0] <= rows <= HIP_PROMPT_WIDE_ROWS[1] and K >= HIP_PROMPT_PARTS_COLUMNS and
+            M * K >= HIP_PROMPT_PARTS_WEIGHT and M % 8 == 0 and parts >= (least if M > many else 2))
+
+
+def _parts_product(linear, x: torch.Tensor) -> Optional[torch.Tensor]:
+    """The result of ``dense_linear_wide_parts`` where it is the faster one and does what ``linear(x)`` would; else None."""
+    W = linear.weight
+    rows = x.numel() // x.shape[-1]
+    if W.dim() != 2 or not HIP_PROMPT_WIDE_ROWS[0] <= rows <= HIP_PROMPT_WIDE_ROWS[1]:
+        return None
+    M, K = W.shape
+    if not _parts_rule(rows, M, K, ops.wide_parts(rows, K, M)) or not _wide_fits(linear, x):
+        return None
+    return ops.dense_linear_wide_parts(x, W, linear.bias)
 
 
 def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") -> torch.Tensor:
     """``activation(linear(x))``.  The rows of a decode step (x: (B, 1, d) with B <= 64, fp16, on the GPU)
     always go to this package's row kernels (vector ALUs for one or two rows, matrix cores above).  The
     rows of a prompt go to the matrix-core kernels that stream the weight while it is the bound (``USE_HIP_PROMPT``, up
-    to ``HIP_PROMPT_MAX_ROWS`` rows, and more of them for long-rowed weights: ``_long_product``), with an activation or the longest
-    rows to the one with wide tiles (``_wide_product``), else to the library GEMM."""
+    to ``HIP_PROMPT_MAX_ROWS`` rows, and more of them for long-rowed weights: ``_long_product``), with an activation or long
+    rows to the one with wide tiles (``_wide_product``, ``_parts_product``), else to the library GEMM."""
     on_hip = x.is_cuda and x.dtype == torch.float16 and linear.weight.dtype == torch.float16 and x.shape[-1] % 8 == 0
     if on_hip and x.dim() == 3 and x.shape[1] == 1 and x.shape[0] <= 64:
         return ops.dense_decode_linear(x, linear.weight, linear.bias, activation)
@@ -403,6 +431,9 @@ def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") ->
         rows = x.numel() // x.shape[-1]
         if rows <= HIP_PROMPT_MAX_ROWS or (rows <= HIP_PROMPT_LONG_MAX_ROWS and _long_product(linear, x)):
             return ops.dense_linear(x, linear.weight, linear.bias, activation)
+        parts = _parts_product(linear, x) if activation == "id" else None
+        if parts is not None:
+            return parts
         if _wide_product(linear, x, activation):
             return ops.dense_linear_wide(x, linear.weight, linear.bias, activation)
     y = linear(x)

@@ -14,6 +14,7 @@ kernels are enqueued on ``torch.cuda.current_stream()``.
 from __future__ import annotations
 
 import ctypes
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -281,6 +282,34 @@ def dense_linear_wide(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torc
     out = torch.empty(x2.shape[0], M, device=x.device, dtype=x.dtype)
     check(lib.dv_dense_linear_wide_f16(_ptr(x2), x2.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), x2.shape[0], N, M,
                                        _ACT[activation], _ptr(out), M, _stream()), "dv_dense_linear_wide_f16")
+    return out.view(*x.shape[:-1], M)
+
+
+@lru_cache(maxsize=4096)
+def _wide_parts_bytes(device: int, rows: int, N: int, M: int) -> int:
+    """A function of the sizes and of the current device, whose compute units the parts are made for."""
+    return lib.dv_dense_linear_wide_workspace_bytes(rows, N, M)
+
+
+def wide_parts(rows: int, N: int, M: int) -> int:
+    """Parts of the columns that ``dense_linear_wide_parts`` makes; 0: its tiles are enough for the chip."""
+    return _wide_parts_bytes(torch._C._cuda_getDevice(), rows, N, M) // (4 * rows * M)
+
+
+def dense_linear_wide_parts(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``dense_linear_wide`` without an activation and with the columns in parts (several: ``wide_parts``)."""
+    _require_device(x, weight, bias)
+    M, N = weight.shape
+    x2 = x.reshape(-1, N)
+    rows = x2.shape[0]
+    nbytes = _wide_parts_bytes(torch._C._cuda_getDevice(), rows, N, M)
+    assert nbytes and x2.dtype == weight.dtype == torch.float16 and x2.stride(1) == 1 and weight.stride(1) == 1 and M % 8 == 0
+    assert bias is None or (bias.shape == (M,) and bias.dtype == x.dtype and bias.is_contiguous())
+    out = torch.empty(rows, M, device=x.device, dtype=x.dtype)
+    # the sums of this call alone (up to 250 MB), not the stream's scratch, which is never given back
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    check(lib.dv_dense_linear_wide_ws_f16(_ptr(x2), x2.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), rows, N, M, _ACT["id"],
+                                          _ptr(out), M, _ptr(ws), nbytes, _stream()), "dv_dense_linear_wide_ws_f16")
     return out.view(*x.shape[:-1], M)
 
 

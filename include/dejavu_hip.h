@@ -152,6 +152,12 @@ DV_API int dv_dense_linear_f16(const void* x, int64_t ldx, const void* W, int64_
  */
 DV_API int dv_dense_linear_wide_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, int rows, int N,
                                     int M, int act, void* y, int64_t ldy, void* stream);
+/* The same with the columns in parts where the tiles are few; workspace: dv_dense_linear_wide_workspace_bytes (0: none is needed) on a
+ * 16-byte boundary.  With parts M % 8 == 0, ldy % 4 == 0. */
+DV_API size_t dv_dense_linear_wide_workspace_bytes(int rows, int N, int M);
+DV_API int dv_dense_linear_wide_ws_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, int rows, int N,
+                                       int M, int act, void* y, int64_t ldy, void* workspace, size_t workspace_bytes,
+                                       void* stream);
 
 /*
  * y = x . W[idx] + bias.  Replaces gather_transposed_gemv,

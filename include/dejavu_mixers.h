@@ -319,6 +319,10 @@ DV_API int dv_mix_linear_split(const float* x, int64_t ldx, const float* W, int6
                                float* out, int64_t ldo, void* workspace, size_t workspace_bytes, void* stream);
 /* The same product for many rows (DV_OUT_T and DV_OUT_GLU); slower from leading dimensions of 2^25 on. */
 DV_API int dv_mix_linear_wide(int after, const dvTileArgs* args, void* stream);
+/* The same with K in parts where the tiles are few; workspace: dv_mix_linear_wide_workspace_bytes on a 16-byte boundary (0: one part).
+ * DV_OUT_T, and of several parts DV_OUT_RESIDUAL; of those M % 8 == 0.  Leading dimensions from 2^25 on are DV_ERR_UNSUPPORTED. */
+DV_API size_t dv_mix_linear_wide_workspace_bytes(int n, int M, int K);
+DV_API int dv_mix_linear_wide_ws(int after, const dvTileArgs* args, void* workspace, size_t workspace_bytes, void* stream);
 DV_API int dv_mix_short_conv(int dtype, int out_f32, const dvConvArgs* args, void* stream);
 /* The same, and next_state <- the state behind the last row (may be args->state). */
 DV_API int dv_mix_short_conv_move(int dtype, int out_f32, const dvConvArgs* args, float* next_state, void* stream);
