@@ -47,10 +47,11 @@ struct WideSplit {
   size_t workspace_bytes(int n, int M) const { return (size_t)splits * n * M * sizeof(float); }
 };
 
-// The same with K in up to six parts, one round of workgroups at most: a chunk takes as NB + 180 (fewer columns share the chunk of W, and cold
-// weights arrive slower than they are multiplied), a workgroup's ends as 4500, a part's sums as 4.2e-4 each, to memory and back.
-// Over 96 products of 257..2048 rows (2048 to 7168 weight rows, 5632 to 28672 columns, cold), every choice measured with the launch that adds
-// up: 1.1 % longer than the best one, 14 % at most.
+// The same with K in up to six parts, one round of workgroups at most: a chunk takes as NB + 166 (fewer columns share the chunk of W, and cold
+// weights arrive slower than they are multiplied), a workgroup's ends as 7400, a part's sums as 3.6e-4 each, to memory and back.  From whole
+// prompts of 300 to 1900 tokens, every choice for their down projections or fc2 in turn (4096 x 11008, 4096 x 16384, 5120 x 20480): the prompt
+// takes 0.1 % longer than with the best one, 1.2 % at most, and 1.00 to 1.29 times less than with the library's products.  (By the products alone, back
+// to back, where the clock is lower than beside other kernels, more parts look better than they are: 0.5 % and 3.3 %.)
 inline WideSplit plan_wide_split(int n, int M, int K, int units) {
   WideSplit best{256, 1};
   double least = 0.0;
@@ -60,8 +61,8 @@ inline WideSplit plan_wide_split(int n, int M, int K, int units) {
     for (int splits = 1; splits <= 6; ++splits) {
       if (splits > 1 && (tiles * splits > units || chunks < splits * 8)) break;
       const int64_t rest = tiles * splits % units;
-      const double rounds = (double)(tiles * splits / units) + (rest ? 0.62 + 0.38 * rest / units : 0.0);
-      const double t = rounds * (((chunks + splits - 1) / splits) * (double)(nb + 180) + 4500.0) + 4.2e-4 * splits * n * (double)M;
+      const double rounds = (double)(tiles * splits / units) + (rest ? 0.5 + 0.5 * rest / units : 0.0);
+      const double t = rounds * (((chunks + splits - 1) / splits) * (double)(nb + 166) + 7400.0) + 3.6e-4 * splits * n * (double)M;
       if (least == 0.0 || t < least) best = {nb, splits}, least = t;
     }
   }

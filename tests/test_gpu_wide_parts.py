@@ -12,7 +12,7 @@ from dejavu_amd import mixer_ops, modules, ops
 pytestmark = pytest.mark.gpu
 
 # (rows, weight rows, columns): six, five, four, three and two parts on tiles of every width, which end in the middle; columns behind the last chunk
-SIZES = [(257, 1032, 4168), (300, 520, 2600), (257, 1032, 2504), (500, 3080, 4168), (500, 3080, 2120), (700, 4104, 2600), (1300, 5128, 2056)]
+SIZES = [(257, 1032, 4168), (300, 520, 2600), (383, 520, 2056), (383, 2056, 2504), (500, 2056, 4168), (700, 4104, 2600), (1300, 1032, 2504)]
 
 
 def _parts(n, M, K):
@@ -34,7 +34,7 @@ def _near(got, want, dtype, K):
 
 def test_every_number_of_parts_is_taken():
     assert {_parts(*s) for s in SIZES} == {2, 3, 4, 5, 6}
-    assert _parts(2048, 8192, 4096) == 0 and _parts(300, 512, 960) == 0  # a round of tiles; too few columns
+    assert _parts(2048, 8192, 4096) == 0 and _parts(300, 512, 960) == 0  # whole rounds of tiles; too few columns
     assert ops.wide_parts(777, 16384, 4096) == _parts(777, 4096, 16384)
 
 
