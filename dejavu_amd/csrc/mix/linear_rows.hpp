@@ -3,7 +3,8 @@
 //   before: nothing, an RMS norm of the row, a per-head RMS norm with an output gate, or an RMS norm per group;
 //   after : plain store, a gated unit, a short convolution with its state, dynamic tanh + residual add + the next
 //           dynamic tanh, or the update of several residual streams with the row that the next norm reads.
-// A wave owns R consecutive rows of W at a time; the row x is staged in LDS once per workgroup.
+// A wave owns R consecutive rows of W at a time, or KS waves do, a stretch of the columns each; the row x is staged in LDS once per
+// workgroup.
 #pragma once
 #include "elem.hpp"
 #include "hyper.hpp"
@@ -137,7 +138,7 @@ __device__ __forceinline__ void stage_row(const RowsArgs& a, T* xs, float* red) 
   __syncthreads();
 }
 
-template <typename T, int BEFORE, int AFTER, int R, int U>
+template <typename T, int BEFORE, int AFTER, int R, int U, int KS = 1>
 __global__ __launch_bounds__(256) void linear_rows_kernel(RowsArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   T* xs = reinterpret_cast<T*>(smem_raw);
@@ -159,10 +160,12 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(RowsArgs a) {
       return;
     }
   }
-  constexpr int CH = 8 * kWave;
+  constexpr int CH = 8 * kWave, TASKS = 4 / KS;
+  __shared__ float others[KS > 1 ? 4 : 1][R];
   const T* W = reinterpret_cast<const T*>(a.W);
-  const int K = a.K, ntasks = (a.M + R - 1) / R;
-  int t = blockIdx.x * 4 + wave;
+  const int K = a.K, ntasks = (a.M + R - 1) / R, rounds = (ntasks + nblocks * TASKS - 1) / (nblocks * TASKS);
+  const int part = wave % KS, per = ((K + CH - 1) / CH + KS - 1) / KS * CH, k0 = part * per, k1 = min(K, k0 + per);
+  int t = blockIdx.x * TASKS + wave / KS;
   Pack8<T> w[U][R];
   const T* wr[R];
   auto rows_of = [&](int task) {
@@ -182,12 +185,12 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(RowsArgs a) {
   };
   if (t < ntasks) {  // the first weights are requested before x is there
     rows_of(t);
-    load_w(0);
+    load_w(k0);
   }
   __shared__ float coef[DV_HYPER_ROW_MAX * (DV_HYPER_ROW_MAX + 2)];
   if constexpr (AFTER == DV_OUT_HYPER) hyper_coefficients(a.hyper, coef, threadIdx.x, 256);
   stage_row<T, BEFORE>(a, xs, red);
-  for (; t < ntasks; t += nblocks * 4) {
+  for (int round = 0; KS > 1 ? round < rounds : t < ntasks; ++round, t += nblocks * TASKS) {  // (waves that share rows stay together)
     // what the epilogue adds to is requested before the products
     float old[DV_HYPER_ROW_MAX], bias = 0.f;
     if constexpr (AFTER != DV_OUT_GLU) {
@@ -202,11 +205,11 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(RowsArgs a) {
     float acc[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.f;
-    for (int base = 0; base < K; base += U * CH) {
+    for (int base = k0; base < k1; base += U * CH) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int k = base + u * CH + lane * 8;
-        if (k < K) {
+        if (k < k1) {
           Pack8<T> xv;
           xv = *reinterpret_cast<const Pack8<T>*>(xs + k);
 #pragma unroll
@@ -215,14 +218,30 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(RowsArgs a) {
             for (int e = 0; e < 8; ++e) acc[r] = __builtin_fmaf(w[u][r].get(e), xv.get(e), acc[r]);
         }
       }
-      if (base + U * CH < K) load_w(base + U * CH);
+      if (base + U * CH < k1 && (KS == 1 || t < ntasks)) load_w(base + U * CH);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
     const int row0 = t * R;
-    if (t + nblocks * 4 < ntasks) {
-      rows_of(t + nblocks * 4);
-      load_w(0);
+    if (t + nblocks * TASKS < ntasks) {
+      rows_of(t + nblocks * TASKS);
+      load_w(k0);
+    }
+    if constexpr (KS > 1) {
+      if (round > 0) __syncthreads();
+      if (part > 0 && lane < R) {
+        float v = acc[0];
+#pragma unroll
+        for (int r = 1; r < R; ++r)
+          if (lane == r) v = acc[r];
+        others[wave][lane] = v;
+      }
+      __syncthreads();
+      if (part > 0 || t >= ntasks) continue;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int k = 1; k < KS; ++k) acc[r] += others[wave + k][r];
     }
     if constexpr (AFTER == DV_OUT_GLU) {
       static_assert(R % 2 == 0, "gate / up rows come in pairs");

@@ -143,6 +143,11 @@ template <typename T, int BEFORE, int AFTER>
 int linear_row(const RowsArgs& a, hipStream_t s) {
   constexpr int R = 2, U = sizeof(T) == 2 ? 4 : 2;
   const int ntasks = (a.M + R - 1) / R;
+  // Few long rows: two waves share a pair of rows, so that all of it is on its way at once (four waves a compute unit with three turns each
+  // leave the memory idle between them: a token of vimulorn-2k 0.9 % less, of varolorn-2k 1.1 %, whose down projections are 2048 x 5632; four waves
+  // 0.8 % and -1.3 %; 4096 x 11008, whose waves are twice as many, 0.4 to 2.7 % more).
+  if (sizeof(T) == 2 && a.K > 2048 && a.K <= 6144 && ntasks <= compute_units() * 4)
+    return launch_lds<linear_rows_kernel<T, BEFORE, AFTER, R, 6, 2>>(dim3((ntasks + 1) / 2 + (a.side_x ? 1 : 0)), dim3(256), (size_t)a.K * sizeof(T), s, a);
   int blocks = (ntasks + 3) / 4;
   if (blocks > 2048) blocks = 2048;
   if (a.side_x) ++blocks;
