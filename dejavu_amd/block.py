@@ -19,7 +19,7 @@ from torch import Tensor
 
 from . import fused_layer, ops
 from . import modules as dv_modules
-from .modules import ParallelFusedMLPDejavu, ParallelMHADejavu, ParallelMHASparseAttMlp
+from .modules import ParallelFusedMLPDejavu, ParallelMHADejavu, ParallelMHASparseAttMlp, _hooked
 
 
 # Batched sparse decode: LayerNorm 1, the window buffer's row and the tracker step in one launch
@@ -34,10 +34,10 @@ FOLD_WINDOW_STEP = True
 # next_att_idx are then good for the next block, or for anybody after modules.join_side_stream().
 # False: every module waits for its side work before it returns.
 LAZY_SIDE_JOIN = True
-# Batched sparse decode: the split reduction of out_proj, the residual add and LayerNorm 2 in one launch
-# (ops.out_proj_sparse_t_add_layer_norm).  False: out_proj with its reduction launch, then add_layer_norm.
+# Batched sparse decode and prompts: the split reduction of out_proj, the residual add and LayerNorm 2 in one launch
+# (ops.out_proj_sparse_t_add_layer_norm, modules.pending_linear).  False: out_proj with its reduction launch, then add_layer_norm.
 FOLD_NORM2 = True
-# Batched sparse decode, blocks with ``defer_mlp_reduce`` set (whoever sets it consumes the block's
+# Batched sparse decode and prompts, blocks with ``defer_mlp_reduce`` set (whoever sets it consumes the block's
 # hidden_states with ops.add_layer_norm / add_layer_norm_window, as the next block and the model's
 # final LayerNorm do): the split reduction of fc2 is left to that LayerNorm's launch; the block
 # returns ops.PendingRows as hidden_states.  False: fc2 with its reduction launch.
@@ -49,6 +49,10 @@ def _add_norm(norm: nn.LayerNorm, hidden_states: Tensor, residual: Optional[Tens
         return ops.add_layer_norm(hidden_states, residual, norm.weight, norm.bias, norm.eps)
     residual = hidden_states + residual if residual is not None else hidden_states
     return norm(residual.to(dtype=norm.weight.dtype)), residual
+
+
+def _prompt(hidden_states) -> bool:
+    return hidden_states.is_cuda and hidden_states.dtype == torch.float16 and hidden_states.size(1) > 1
 
 
 class BlockMlpAttSparse(nn.Module):
@@ -95,7 +99,8 @@ class BlockMlpAttSparse(nn.Module):
             mixer_kwargs = {}
         hidden_states, residual, window = self._norm1(hidden_states, residual, head_idx, ip)
         lazy = LAZY_SIDE_JOIN and hidden_states.is_cuda
-        post_norm = (self.norm2, residual) if (FOLD_NORM2 and window is not None) else None
+        prompt = _prompt(hidden_states)
+        post_norm = (self.norm2, residual) if FOLD_NORM2 and (window is not None or (prompt and not _hooked(self.mixer))) else None
         hidden_states, mlp_idx, next_att_idx = self.mixer(hidden_states, residual=residual, head_idx=head_idx,
                                                           mlp_sp_logit=mlp_sp_logit, window=window, defer_join=lazy,
                                                           post_norm=post_norm, **mixer_kwargs)
@@ -110,7 +115,8 @@ class BlockMlpAttSparse(nn.Module):
             hidden_states, residual = _add_norm(self.norm2, hidden_states, residual)
         hidden_states, next_mlp_sp_logit = self.mlp(
             hidden_states, residual, mlp_idx, defer_join=lazy,
-            defer_reduce=FOLD_NORM1 and self.defer_mlp_reduce and window is not None)
+            defer_reduce=FOLD_NORM1 and self.defer_mlp_reduce and
+            (window is not None or (prompt and not _hooked(self) and not _hooked(self.mlp))))
         return hidden_states, residual, next_mlp_sp_logit, next_att_idx
 
 
@@ -150,10 +156,14 @@ class BlockDejavu(nn.Module):
         if mixer_kwargs is None:
             mixer_kwargs = {}
         lazy = LAZY_SIDE_JOIN and hidden_states.is_cuda
-        hidden_states, mlp_idx = self.mixer(hidden_states, mlp_sp_logit=mlp_sp_logit, defer_join=lazy, **mixer_kwargs)
+        post_norm = (self.norm2, residual) if FOLD_NORM2 and _prompt(hidden_states) and not _hooked(self.mixer) else None
+        hidden_states, mlp_idx = self.mixer(hidden_states, mlp_sp_logit=mlp_sp_logit, defer_join=lazy, post_norm=post_norm, **mixer_kwargs)
         if lazy:
             self.mixer.join_side()  # in front of LayerNorm 2, as in BlockMlpAttSparse
-        hidden_states, residual = _add_norm(self.norm2, hidden_states, residual)
+        if isinstance(hidden_states, tuple):
+            hidden_states, residual = hidden_states
+        else:
+            hidden_states, residual = _add_norm(self.norm2, hidden_states, residual)
         hidden_states, next_mlp_sp_logit = self.mlp(hidden_states, residual, mlp_idx, defer_join=lazy)
         return hidden_states, residual, next_mlp_sp_logit
 

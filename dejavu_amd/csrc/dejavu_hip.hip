@@ -640,6 +640,7 @@ bool wide_takes(int B, int M, int act) {
 }
 
 // Y (B, M) row stride ldy = act(X (B, N) . W[idx]^T + bias[idx]); idx == nullptr: rows 0..M-1 of W.
+// Y == nullptr (idx too, dense_parts(B, N, M) > 1): the splits' sums stay in the workspace, rows of M floats, one split after the other.
 int gemm_tiled(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const half_t* bias, const void* idx,
                int idx_bytes, int B, int N, int Z, int M, int act, half_t* Y, int64_t ldy, void* workspace,
                size_t workspace_bytes, hipStream_t s) {
@@ -650,8 +651,10 @@ int gemm_tiled(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const
     return gemm_big(X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, act, s);
   if (kind == Shared::kRing) {
     const RingPlan p = plan_ring(B, M, N, compute_units());
-    if (int rc = ring_scratch(p, workspace, workspace_bytes); rc != DV_OK) return rc;
     const RingOperands<half_t> a{X, ldx, W, ldw, B, M, N};
+    if (idx == nullptr && Y == nullptr)
+      return gemm_ring(p, a, PlainRows{}, RingRowParts{reinterpret_cast<float*>(workspace), B, M}, nullptr, s, RingLaunch{});
+    if (int rc = ring_scratch(p, workspace, workspace_bytes); rc != DV_OK) return rc;
     if (idx == nullptr) return gemm_ring(p, a, PlainRows{}, PlainOut{bias, act, Y, ldy, M}, workspace, s, RingLaunch{});
     const GatheredRows rows{idx, idx_bytes, Z};
     return gemm_ring(p, a, rows, GatheredOut{rows, bias, act, Y, ldy, M}, workspace, s, RingLaunch{});
@@ -680,13 +683,20 @@ int gemm_tiled(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, const
   else if (p.bt == 4) rc = launch_tiled<4, 2, 128, 8>(p, X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, relu, partial, s);
   else rc = launch_tiled<8, 2, 128, 8>(p, X, ldx, W, ldw, bias, idx, idx_bytes, B, N, Z, M, Y, ldy, relu, partial, s);
 #undef DV_TG
-  if (rc != DV_OK) return rc;
+  if (rc != DV_OK || Y == nullptr) return rc == DV_OK ? launch_status() : rc;
   if (p.nsplit > 1) {
     const int64_t total = (int64_t)B * M;
     hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, partial,
                        p.nsplit, B, M, bias, idx, idx_bytes, Z, relu, Y, ldy);
   }
   return launch_status();
+}
+
+// Splits of K of the product that gemm_tiled makes, 1: it needs none.
+int dense_parts(int B, int N, int M) {
+  const Shared kind = shared_kernel(B, N, M, false);
+  if (kind == Shared::kBig || B > 512) return 1;
+  return kind == Shared::kRing ? plan_ring(B, M, N, compute_units()).splits : plan_tiled(B, N, M).nsplit;
 }
 
 struct ColsMfmaPlan {
@@ -1209,6 +1219,29 @@ int dv_dense_linear_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, 
                     reinterpret_cast<const half_t*>(bias), nullptr, 4, rows, N, M, M, act,
                     reinterpret_cast<half_t*>(y), ldy, workspace, workspace_bytes,
                     reinterpret_cast<hipStream_t>(stream));
+}
+
+size_t dv_dense_linear_partial_workspace_bytes(int rows, int N, int M, int wide) {
+  if (rows < 1 || N <= 0 || M <= 0) return 0;
+  const int parts = wide ? plan_wide_split(rows, M, N, compute_units()).splits : dense_parts(rows, N, M);
+  return parts > 1 ? (size_t)parts * rows * M * sizeof(float) : 0;
+}
+
+int dv_dense_linear_partial_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, int rows, int N, int M, int wide, void* partial,
+                                size_t partial_bytes, void* stream) {
+  if (!x || !W || !partial || rows < 1 || N <= 0 || M <= 0) return DV_ERR_INVALID_ARG;
+  if (N % 8 || M % 8 || ldx % 8 || ldw % 8 || ldx < N || ldw < N || !aligned16(x) || !aligned16(W) || !aligned16(partial))
+    return DV_ERR_ALIGNMENT;
+  const size_t bytes = dv_dense_linear_partial_workspace_bytes(rows, N, M, wide);
+  if (bytes == 0 || (wide && (ldw >= kWideMaxStride || ldx >= kWideMaxStride))) return DV_ERR_UNSUPPORTED;
+  if (partial_bytes < bytes) return DV_ERR_WORKSPACE;
+  const half_t* X = reinterpret_cast<const half_t*>(x);
+  const half_t* w = reinterpret_cast<const half_t*>(W);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (!wide) return gemm_tiled(X, ldx, w, ldw, nullptr, nullptr, 4, rows, N, M, M, DV_ACT_ID, nullptr, M, partial, partial_bytes, s);
+  const WideSplit p = plan_wide_split(rows, M, N, compute_units());
+  return gemm_wide(p.nb, RingOperands<half_t>{X, ldx, w, ldw, rows, M, N}, WidePart{reinterpret_cast<float*>(partial), rows, M}, s,
+                   RingLaunch{}, p.splits);
 }
 
 size_t dv_dense_linear_wide_workspace_bytes(int rows, int N, int M) {

@@ -49,6 +49,17 @@ struct PlainRows {
   __device__ __forceinline__ int64_t operator()(int m) const { return m; }
 };
 
+// As the output of a product: the splits' sums as rows of M floats (M % 4 == 0), one split after the other, for a launch that adds them up
+// with what follows, a workgroup a row.
+struct RingRowParts {
+  float* part;
+  int64_t rows;
+  int M;
+  __device__ __forceinline__ void operator()(int m, int n, const float4_t& v) const {
+    *reinterpret_cast<float4_t*>(part + (blockIdx.z * rows + n) * M + m) = v;
+  }
+};
+
 struct RingPlan {
   int mb, nb;        // tile: rows of W, rows of X
   int rows, cols;    // tiles
@@ -252,7 +263,7 @@ __device__ __forceinline__ void ring_tile(const RingOperands<T>& a, const Rows& 
     for (int i = 0; i < RT; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j) sums[0][i][j] += sums[k][i][j];
-  if (gridDim.z > 1) {
+  if (!__is_same(Out, RingRowParts) && gridDim.z > 1) {
     float4_t* p = part + threadIdx.x;
 #pragma unroll
     for (int i = 0; i < RT; ++i)
@@ -309,9 +320,13 @@ int gemm_ring_tiles(const RingPlan& p, const RingOperands<T>& a, const Rows& row
   const int rc = launch.template operator()<gemm_ring_kernel<T, MB, NB, KC, ST, WM, WN, NT_W, Rows, Out, ROUND>>(
       dim3(p.rows, p.cols, p.splits), threads, (size_t)ST * (MB + NB) * KC * 2, s, a, rows, out, part);
   if (rc != 0 || p.splits == 1) return rc;
+  if constexpr (!__is_same(Out, RingRowParts)) {
   constexpr int values = (MB / WM / 16) * (NB / WN / 16);
   return launch.template operator()<gemm_ring_sum_kernel<MB, NB, WM, WN, Out>>(dim3(p.rows, p.cols, values), threads, 0, s, a.n, a.M, out,
                                                                                (const float4_t*)part, p.splits);
+  } else {
+    return rc;
+  }
 }
 
 template <typename T, typename Rows, typename Out, typename Launch>

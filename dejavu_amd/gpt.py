@@ -168,7 +168,8 @@ class GPTModel(nn.Module):
         chain = None
         chaining = (self.chain_layers and self.att_sparse and self.record is None and input_ids.shape[1] == 1
                     and input_ids.shape[0] == 1)
-        for layer in self.layers:
+        following = list(self.layers[1:]) + [None]
+        for layer, after in zip(self.layers, following):
             if self.record is not None and input_ids.shape[1] == 1:
                 dv_modules.join_side_stream()  # the predictions of the block before may be pending on the side stream
                 self.record.append((None if next_att_idx is None else next_att_idx.clone(),
@@ -192,6 +193,9 @@ class GPTModel(nn.Module):
             else:
                 hidden_states, residual, next_mlp_sp_logit = layer(
                     hidden_states, residual, mlp_sp_logit=next_mlp_sp_logit, mixer_kwargs=mixer_kwargs)
+            if input_ids.shape[1] > 1 and isinstance(hidden_states, ops.PendingRows) and after is not None and (
+                    type(after) not in (BlockMlpAttSparse, BlockDejavu) or dv_modules._hooked(after)):
+                hidden_states = hidden_states.materialize()  # (hooks and other modules get a tensor)
             if self.record is not None and self.record_mlp_idx is not None and input_ids.shape[1] == 1:
                 idx = getattr(layer, "last_mlp_idx", None)
                 self.record_mlp_idx.append(None if idx is None else idx.clone())

@@ -281,8 +281,8 @@ class ParallelFusedMLPDejavu(nn.Module):
         """x, residual: (B, 1, d) at decode (or (B, s, d) for the prompt).
         idx: (K,) active neurons or None for the dense MLP.
         defer_reduce: the caller's next step is an ``ops.add_layer_norm`` / ``add_layer_norm_window`` of
-        ``out``; for 3..64 sequences ``out`` is then ``ops.PendingRows`` (the split reduction of fc2 runs
-        inside that LayerNorm launch).
+        ``out``; for 3..64 sequences, and for prompts whose fc2 ends in such a step, ``out`` is then ``ops.PendingRows`` (the
+        split reduction of fc2 runs inside that LayerNorm launch).
         Returns (out, mlp_logit); mlp_logit, the predictor output for the next
         layer's MLP, only when decoding one token.  defer_join: when the predictor runs on the side
         stream, the current stream does not wait for it: mlp_logit is then only good for work
@@ -325,7 +325,9 @@ class ParallelFusedMLPDejavu(nn.Module):
             if not isinstance(out, ops.PendingRows):
                 out = out.unsqueeze(1)
         else:
-            out = decode_linear(self.fc2, h)
+            out = pending_linear(self.fc2, h) if defer_reduce else None
+            if out is None:
+                out = decode_linear(self.fc2, h)
         # (tensor parallel all-reduce of `out` is the identity on one GPU)
         if side:
             if defer_join:
@@ -406,16 +408,30 @@ def _parts_rule(rows: int, M: int, K: int, parts: int) -> bool:
             M * K >= HIP_PROMPT_PARTS_WEIGHT and M % 8 == 0 and parts >= (least if M > many else 2))
 
 
-def _parts_product(linear, x: torch.Tensor) -> Optional[torch.Tensor]:
-    """The result of ``dense_linear_wide_parts`` where it is the faster one and does what ``linear(x)`` would; else None."""
+def _parts_product(linear, x: torch.Tensor) -> bool:
+    """Whether ``dense_linear_wide_parts`` is the faster one and does what ``linear(x)`` would."""
     W = linear.weight
     rows = x.numel() // x.shape[-1]
     if W.dim() != 2 or not HIP_PROMPT_WIDE_ROWS[0] <= rows <= HIP_PROMPT_WIDE_ROWS[1]:
-        return None
+        return False
     M, K = W.shape
-    if not _parts_rule(rows, M, K, ops.wide_parts(rows, K, M)) or not _wide_fits(linear, x):
+    return _parts_rule(rows, M, K, ops.wide_parts(rows, K, M)) and _wide_fits(linear, x)
+
+
+def _prompt_on_hip(linear, x: torch.Tensor) -> bool:
+    return (USE_HIP_PROMPT and x.is_cuda and x.dtype == torch.float16 and linear.weight.dtype == torch.float16 and x.shape[-1] % 8 == 0)
+
+
+def pending_linear(linear: nn.Linear, x: torch.Tensor) -> Optional[ops.PendingRows]:
+    """``decode_linear(linear, x)`` of a prompt with its last step left to the add + LayerNorm that follows, where there is such a step.
+    One launch instead of two, and the rows are not written and read between them: out_proj and fc2 of 128 tokens of the 13B
+    shape (six splits) 4.8 + 5.1 us."""
+    if not _prompt_on_hip(linear, x) or x.shape[1] == 1:
         return None
-    return ops.dense_linear_wide_parts(x, W, linear.bias)
+    rows = x.numel() // x.shape[-1]
+    if rows <= HIP_PROMPT_MAX_ROWS or (rows <= HIP_PROMPT_LONG_MAX_ROWS and _long_product(linear, x)):
+        return ops.dense_linear_pending(x, linear.weight, linear.bias)
+    return ops.dense_linear_pending(x, linear.weight, linear.bias, wide=True) if _parts_product(linear, x) else None
 
 
 def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") -> torch.Tensor:
@@ -431,9 +447,8 @@ def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") ->
         rows = x.numel() // x.shape[-1]
         if rows <= HIP_PROMPT_MAX_ROWS or (rows <= HIP_PROMPT_LONG_MAX_ROWS and _long_product(linear, x)):
             return ops.dense_linear(x, linear.weight, linear.bias, activation)
-        parts = _parts_product(linear, x) if activation == "id" else None
-        if parts is not None:
-            return parts
+        if activation == "id" and _parts_product(linear, x):
+            return ops.dense_linear_wide_parts(x, linear.weight, linear.bias)
         if _wide_product(linear, x, activation):
             return ops.dense_linear_wide(x, linear.weight, linear.bias, activation)
     y = linear(x)
@@ -446,6 +461,16 @@ def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") ->
     if activation == "squared_relu":
         return F.relu(y) ** 2
     return y
+
+
+def _project_norm(linear: nn.Linear, x: torch.Tensor, post_norm):
+    """``decode_linear(linear, x)``, or with post_norm = (LayerNorm module, residual) the pair (normed, residual_out) where the reduction
+    of the projection rides in that launch."""
+    pending = pending_linear(linear, x) if post_norm is not None else None
+    if pending is None:
+        return decode_linear(linear, x)
+    norm, residual = post_norm
+    return ops.add_layer_norm(pending, residual, norm.weight, norm.bias, norm.eps)
 
 
 def _kv_caches(inference_params, layer_idx, H, hd, dtype, device):
@@ -630,16 +655,16 @@ class ParallelMHADejavu(_MHABase):
         self._init_common(embed_dim, num_heads, process_group, bias, softmax_scale, causal, layer_idx,
                           rotary_emb_dim, device, dtype)
 
-    def forward(self, x, mlp_sp_logit=None, seqlen=None, inference_params=None, defer_join=False, **kwargs):
+    def forward(self, x, mlp_sp_logit=None, seqlen=None, inference_params=None, defer_join=False, post_norm=None, **kwargs):
         """x: (B, s, d).  Returns (out, mlp_idx).  defer_join: the caller calls ``join_side()`` itself
-        before it uses mlp_idx."""
+        before it uses mlp_idx.  post_norm: as ``ParallelMHASparseAttMlp``'s, for prompts."""
         assert seqlen is None, "sequence-parallel input layout is not used for generation"
         self._streams()
         self._side_fork(x.shape[0])
         qkv = decode_linear(self.Wqkv, x)
         qkv = qkv.view(x.shape[0], x.shape[1], 3, self.num_heads, self.head_dim)
         context = self._dense_context(qkv, inference_params)
-        out = decode_linear(self.out_proj, context)
+        out = _project_norm(self.out_proj, context, post_norm)
         mlp_idx, _ = self._side_work(mlp_sp_logit)
         if defer_join:
             self._side_keep = mlp_sp_logit
@@ -814,7 +839,7 @@ class ParallelMHASparseAttMlp(_MHABase):
         window step.  defer_join: the caller calls ``join_side()`` itself before it uses mlp_idx / att_idx
         (the block does).  post_norm = (LayerNorm module, its residual input): the caller's residual add + LayerNorm
         of `out`, done here when it can ride in the projection's reduction launch (batched sparse decode, five
-        rows and more); `out` is then the pair (normed, residual_out) instead of the projection.
+        rows and more; prompts whose projection ends in one); `out` is then the pair (normed, residual_out) instead of the projection.
         Returns (out, mlp_idx, att_idx)."""
         assert seqlen is None, "sequence-parallel input layout is not used for generation"
         self._streams()
@@ -867,7 +892,7 @@ class ParallelMHASparseAttMlp(_MHABase):
             qkv = decode_linear(self.Wqkv, x)
             qkv = qkv.view(x.shape[0], x.shape[1], 3, self.num_heads, self.head_dim)
             context = self._dense_context(qkv, inference_params)
-            out = decode_linear(self.out_proj, context)
+            out = _project_norm(self.out_proj, context, post_norm)
         if side_done is None:
             side_done = self._side_work(mlp_sp_logit, residual, self.sp if do_token_generation else None,
                                         self.att_k, self.att_idx_out)

@@ -313,6 +313,34 @@ def dense_linear_wide_parts(x: torch.Tensor, weight: torch.Tensor, bias: Optiona
     return out.view(*x.shape[:-1], M)
 
 
+@lru_cache(maxsize=4096)
+def _partial_bytes(device: int, rows: int, N: int, M: int, wide: bool) -> int:
+    """As ``_wide_parts_bytes``."""
+    return lib.dv_dense_linear_partial_workspace_bytes(rows, N, M, int(wide))
+
+
+def dense_linear_pending(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, wide: bool = False):
+    """``dense_linear`` (wide: ``dense_linear_wide_parts``) without its last step, as ``PendingRows`` of x's shape; None where the product
+    has one step only, or the operands are none that it takes where they are.  x (..., N), rows contiguous and 16-byte aligned."""
+    M, N = weight.shape
+    rows = x.numel() // N if N else 0
+    nbytes = _partial_bytes(torch._C._cuda_getDevice(), rows, N, M, wide) if rows and M % 8 == 0 else 0
+    if not nbytes or not x.is_contiguous() or x.data_ptr() % 16 or weight.stride(1) != 1 or weight.stride(0) % 8 or weight.data_ptr() % 16:
+        return None
+    _require_device(x, weight, bias)
+    assert x.shape[-1] == N and x.dtype == weight.dtype == torch.float16
+    if bias is not None:
+        bias = bias.contiguous()
+        assert bias.shape == (M,) and bias.dtype == x.dtype
+        if bias.data_ptr() % 16:
+            return None
+    out = torch.empty(rows, M, device=x.device, dtype=x.dtype)
+    partial = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    check(lib.dv_dense_linear_partial_f16(_ptr(x), N, _ptr(weight), weight.stride(0), rows, N, M, int(wide), _ptr(partial), nbytes, _stream()),
+          "dv_dense_linear_partial_f16")
+    return PendingRows(out, partial, nbytes // (4 * rows * M), bias, (*x.shape[:-1], M))
+
+
 def dense_decode_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                         activation: str = "id") -> torch.Tensor:
     """``activation(F.linear(x, weight, bias))`` for the few rows of a decode step (1..64), streamed
@@ -327,16 +355,16 @@ DEFERRED_REDUCE_MIN_ROWS = 3  # the matrix-core path of gather_transposed_gemv
 
 
 class PendingRows:
-    """The (batch, 1, N) output of a transposed product whose last step -- adding up the fp32 sums of
-    its row groups -- has not run: ``add_layer_norm`` / ``add_layer_norm_window`` take it in place of
+    """The (batch, s, N) output of a product whose last step -- adding up the fp32 sums of its row groups, or
+    of the parts of its columns -- has not run: ``add_layer_norm`` / ``add_layer_norm_window`` take it in place of
     ``hidden`` and do that step in their own launch (the fc2 of one block and LayerNorm 1 of the
     next).  ``materialize()`` runs the step alone and returns the tensor.  Shape queries answer as
-    the tensor would."""
+    the tensor would (s: 1 for a decode step)."""
 
-    def __init__(self, y: torch.Tensor, partial: torch.Tensor, groups: int, bias: Optional[torch.Tensor]):
+    def __init__(self, y: torch.Tensor, partial: torch.Tensor, groups: int, bias: Optional[torch.Tensor], shape=None):
         self.y, self.partial, self.groups, self.bias = y, partial, groups, bias
         self._reduced = groups == 1  # a single group stores the finished rows itself
-        self.shape = torch.Size((y.shape[0], 1, y.shape[1]))
+        self.shape = torch.Size((y.shape[0], 1, y.shape[1])) if shape is None else torch.Size(shape)
         self.dtype, self.device, self.is_cuda = y.dtype, y.device, True
 
     def size(self, i: Optional[int] = None):
@@ -353,7 +381,7 @@ class PendingRows:
             check(lib.dv_reduce_rows_f16(_ptr(self.partial), self.groups, _ptr(self.bias), self.y.shape[0],
                                          self.y.shape[1], _ptr(self.y), _stream()), "dv_reduce_rows_f16")
             self._reduced = True
-        return self.y.unsqueeze(1)
+        return self.y.view(self.shape)
 
 
 def _rows_source(hidden):
@@ -914,7 +942,7 @@ def _reduce_add_layer_norm(hidden: PendingRows, residual: Optional[torch.Tensor]
         assert residual.numel() == rows * d and residual.dtype == torch.float16
         residual = residual.contiguous()
     partial, groups, pbias, complete = _rows_source(hidden)
-    y = torch.empty(rows, 1, d, dtype=torch.float16, device=hidden.device)
+    y = torch.empty(hidden.shape, dtype=torch.float16, device=hidden.device)
     r_out = torch.empty_like(y)
     if window is None:
         x_cache_row = tracker = head_idx = batch_idx = None

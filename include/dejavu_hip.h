@@ -158,6 +158,15 @@ DV_API size_t dv_dense_linear_wide_workspace_bytes(int rows, int N, int M);
 DV_API int dv_dense_linear_wide_ws_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, const void* bias, int rows, int N,
                                        int M, int act, void* y, int64_t ldy, void* workspace, size_t workspace_bytes,
                                        void* stream);
+/*
+ * The product alone, its columns in parts whose fp32 sums stay in `partial` ([part][rows][M], on a 16-byte boundary): for
+ * dv_reduce_add_layer_norm_window_f16 and dv_reduce_rows_f16, which add them up (groups = bytes / (4 * rows * M)) and the bias to them.
+ * wide: dv_dense_linear_wide_ws_f16's parts instead of dv_dense_linear_f16's.  M % 8 == 0; 0 bytes: this product has no parts
+ * (DV_ERR_UNSUPPORTED).
+ */
+DV_API size_t dv_dense_linear_partial_workspace_bytes(int rows, int N, int M, int wide);
+DV_API int dv_dense_linear_partial_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, int rows, int N, int M, int wide,
+                                       void* partial, size_t partial_bytes, void* stream);
 
 /*
  * y = x . W[idx] + bias.  Replaces gather_transposed_gemv,
