@@ -124,6 +124,7 @@ def _tiles_of(n: int, M: int, rows: int, weight_rows: int) -> int:
     return -(-n // rows) * -(-M // weight_rows)
 
 
+@lru_cache(maxsize=4096)
 def _wide_rule(n: int, M: int, K: int) -> bool:
     if n > WIDE_MAX_ROWS or M > WIDE_MAX_WEIGHT_ROWS or M % NARROW_TILE == 0 or not WIDE_COLUMNS[0] <= K <= WIDE_COLUMNS[1]:
         return False
@@ -151,6 +152,7 @@ WIDE_FILL_GATED, WIDE_FILL_FEW_GATED, WIDE_FILL_FEW = 200, 144, 176
 WIDE_FULL_GATED, WIDE_FULL_FEW = 0.84, 0.83  # of the rounds of 256 x 256 tiles: tiles at least, rows by weight rows below
 
 
+@lru_cache(maxsize=4096)
 def _fill_rule(n: int, M: int, K: int, gated: bool) -> bool:
     columns = WIDE_GATED_COLUMNS if gated else (WIDE_FEW_COLUMNS, WIDE_FEW_COLUMNS)
     if n <= TILE_MAX_ROWS or not 1024 <= K <= columns[1]:
@@ -195,9 +197,10 @@ def _parts_workspace_bytes(device: int, n: int, M: int, K: int) -> int:
 
 def _parts_bytes(x: torch.Tensor, W: torch.Tensor, bias=None, residual: bool = False) -> int:
     """What the wide kernel's parts of the product need; 0: it is not one of its products."""
-    n, (M, K) = x.shape[0], W.shape
-    if not TILE_MAX_ROWS < n <= WIDE_MAX_ROWS:
+    n = x.shape[0]
+    if x.shape[1] < PARTS_RESIDUAL_COLUMNS or not TILE_MAX_ROWS < n <= WIDE_MAX_ROWS:  # (before anything that costs the host more)
         return 0
+    M, K = W.shape
     nbytes = _parts_workspace_bytes(torch._C._cuda_getDevice(), n, M, K)
     return nbytes if _parts_rule(n, M, K, residual, nbytes // (4 * n * M)) and _wide_fits(x, W, bias) else 0
 
@@ -207,6 +210,7 @@ def _parts_launch(after, a, nbytes, device) -> None:
     check(lib.dv_mix_linear_wide_ws(after, _ref(a), _ptr(ws), nbytes, _stream()), "dv_mix_linear_wide_ws")
 
 
+@lru_cache(maxsize=4096)
 def _tile_rule(n: int, M: int, K: int, gated: bool) -> bool:
     if n > TILE_MAX_ROWS:
         return False
