@@ -9,7 +9,7 @@ from ._binding import DejavuHipError, load_library
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libdejavu_mixers.so")
 
 BF16, F32 = 0, 1
-ROW_PLAIN, ROW_RMS, ROW_HEADS, ROW_GROUPS = 0, 1, 2, 3
+ROW_PLAIN, ROW_RMS, ROW_HEADS, ROW_GROUPS, ROW_SPLITS = 0, 1, 2, 3, 4
 OUT_F32, OUT_T, OUT_GLU, OUT_RESIDUAL, OUT_CONV, OUT_HYPER = 0, 1, 2, 3, 4, 5
 GLU_CLAMPED, GLU_RELU = 0, 1
 HYPER_MAX, HYPER_ROW_MAX = 16, 4
@@ -97,6 +97,7 @@ SIGNATURES = {
     "dv_mix_ring_copy": (_i, [_i, _p, _l, _p, _i, _l, _i, _i, _i, _i, _p]),
     "dv_mix_ring_copy_two": (_i, [_i, _P(RingRows), _P(RingRows), _i, _i, _i, _i, _p]),
     "dv_mix_attn_rows": (_i, [_i, _i, _P(AttnArgs), _p]),
+    "dv_mix_attn_splits": (_i, [_i, _i, _P(AttnArgs), _p]),
     "dv_mix_attn_tiles": (_i, [_P(AttnArgs), _i, _p]),
     "dv_mix_attn_tiles_f32": (_i, [_P(AttnArgs), _i, _p]),
     "dv_mix_latent_absorb": (_i, [_i, _p, _p, _i, _i, _i, _p, _p]),

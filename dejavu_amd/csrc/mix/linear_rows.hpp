@@ -1,6 +1,7 @@
 // One activation row times a weight matrix (the products of a decode step), with what comes before and after the
 // product inside the launch:
-//   before: nothing, an RMS norm of the row, a per-head RMS norm with an output gate, or an RMS norm per group;
+//   before: nothing, an RMS norm of the row, a per-head RMS norm with an output gate, an RMS norm per group, or the merge of an
+//           attention's splits with its sinks and gates;
 //   after : plain store, a gated unit, a short convolution with its state, dynamic tanh + residual add + the next
 //           dynamic tanh, or the update of several residual streams with the row that the next norm reads.
 // A wave owns R consecutive rows of W at a time, or KS waves do, a stretch of the columns each; the row x is staged in LDS once per
@@ -106,6 +107,56 @@ __device__ __forceinline__ void stage_row(const RowsArgs& a, T* xs, float* red) 
       }
     }
     for (int i = a.x_dim + tid; i < K; i += 256) xs[i] = from_f<T>(0.f);
+  } else if constexpr (BEFORE == DV_ROW_SPLITS) {
+    // eight entries of a head per thread, eight splits requested together; attn_merge_kernel's sums in the splits' order
+    constexpr int NS = 8;
+    const int vd = a.head_stride, splits = a.norm_dim;
+    const float* sums = reinterpret_cast<const float*>(a.x);
+    const float* ml = sums + (int64_t)K * splits;
+    for (int i = tid * 8; i < K; i += 2048) {
+      const int head = i / vd;
+      const float* p = sums + ((int64_t)head * splits) * vd + (i - head * vd);
+      const float* q = ml + (int64_t)head * splits * 2;
+      const float sink = a.xw ? a.xw[head] : 0.f, gate = a.gate ? a.gate[head] : 0.f;
+      float top = -1e30f, den = 0.f, t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int s0 = 0; s0 < splits; s0 += NS) {
+        Pack8<float> v[NS];
+        float m[NS], l[NS];
+#pragma unroll
+        for (int u = 0; u < NS; ++u) {
+          const int s = min(s0 + u, splits - 1);
+          v[u].load(p + (int64_t)s * vd);
+          m[u] = q[s * 2];
+          l[u] = q[s * 2 + 1];
+        }
+        float most = top;
+#pragma unroll
+        for (int u = 0; u < NS; ++u) most = fmaxf(most, s0 + u < splits ? m[u] : top);
+        const float c = exp_f(top - most);
+        top = most;
+        den *= c;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[e] *= c;
+#pragma unroll
+        for (int u = 0; u < NS; ++u) {
+          if (s0 + u < splits) {
+            const float w = exp_f(m[u] - top);
+            den = __builtin_fmaf(l[u], w, den);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) t[e] = __builtin_fmaf(v[u].get(e), w, t[e]);
+          }
+        }
+      }
+      if (a.xw) {
+        const float most = fmaxf(top, sink), c = exp_f(top - most);
+        den = __builtin_fmaf(den, c, exp_f(sink - most));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t[e] *= c;
+      }
+      const float f = a.gate ? sigmoid_f(gate) / den : 1.f / den;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xs[i + e] = from_f<T>(t[e] * f);
+    }
   } else {
     // a row of 16 lanes per head; eight channels per lane at a time, the first 128 kept in registers
     const float* x = reinterpret_cast<const float*>(a.x);

@@ -174,6 +174,12 @@ int linear_row_any(int before, int after, const RowsArgs& a, hipStream_t s) {
     return linear_row<T, DV_ROW_GROUPS, DV_OUT_HYPER>(a, s);
   } else if (before == DV_ROW_GROUPS && after == DV_OUT_T) {
     return linear_row<T, DV_ROW_GROUPS, DV_OUT_T>(a, s);
+  } else if (before == DV_ROW_SPLITS && after == DV_OUT_RESIDUAL) {
+    return linear_row<T, DV_ROW_SPLITS, DV_OUT_RESIDUAL>(a, s);
+  } else if (before == DV_ROW_SPLITS && after == DV_OUT_HYPER) {
+    return linear_row<T, DV_ROW_SPLITS, DV_OUT_HYPER>(a, s);
+  } else if (before == DV_ROW_SPLITS && after == DV_OUT_T) {
+    return linear_row<T, DV_ROW_SPLITS, DV_OUT_T>(a, s);
   } else if (before == DV_ROW_HEADS && after == DV_OUT_RESIDUAL) {
     return linear_row<T, DV_ROW_HEADS, DV_OUT_RESIDUAL>(a, s);
   }
@@ -574,6 +580,9 @@ int dv_mix_linear_row(int dtype, int before, int after, const dvRowArgs* a, void
     return DV_ERR_INVALID_ARG;
   if (before == DV_ROW_GROUPS && (!a->xw || a->x_dim < 1 || a->x_dim > a->K || a->norm_dim < 1 || a->x_dim % a->norm_dim))
     return DV_ERR_INVALID_ARG;
+  if (before == DV_ROW_SPLITS && (a->head_stride < 8 || a->head_stride % 8 || a->K % a->head_stride || a->norm_dim < 2 ||
+                                  a->norm_dim > kMaxSplits))
+    return DV_ERR_INVALID_ARG;
   if ((before == DV_ROW_RMS || before == DV_ROW_GROUPS) && !al16(a->xw)) return DV_ERR_ALIGNMENT;
   if (after == DV_OUT_HYPER && (!a->hyper.x || !a->hyper.mix || !a->hyper.out || (a->hyper.u && !a->hyper.in) ||
                                 a->hyper.streams < 1 || a->hyper.streams > DV_HYPER_ROW_MAX || a->hyper.width != a->M))
@@ -728,6 +737,15 @@ int dv_mix_attn_rows(int dtype, int q_f32, const dvAttnArgs* a, void* stream) {
   else if (q_f32) hipLaunchKernelGGL((attn_merge_kernel<bf16_t, float>), grid, dim3(256), 0, st(stream), *a, (bf16_t*)a->out);
   else hipLaunchKernelGGL((attn_merge_kernel<bf16_t, bf16_t>), grid, dim3(256), 0, st(stream), *a, (bf16_t*)a->out);
   return launched();
+}
+
+int dv_mix_attn_splits(int dtype, int q_f32, const dvAttnArgs* a, void* stream) {
+  if (!dtype_ok(dtype)) return DV_ERR_INVALID_ARG;
+  const int rc = attn_args_ok(a);
+  if (rc != DV_OK) return rc;
+  if (a->n != 1 || a->splits < 2) return DV_ERR_INVALID_ARG;
+  if (dtype == DV_F32) return attn_rows_any<float, float>(*a, st(stream));
+  return q_f32 ? attn_rows_any<bf16_t, float>(*a, st(stream)) : attn_rows_any<bf16_t, bf16_t>(*a, st(stream));
 }
 
 int dv_mix_attn_tiles_f32(const dvAttnArgs* a, int keys, void* stream) {

@@ -335,6 +335,19 @@ class GroupedRow(RmsRow):
         a.xw, a.x_dim, a.norm_dim, a.eps = self.weight.data_ptr(), self.dim, self.dim // self.groups, self.eps
 
 
+class SplitRow(RmsRow):
+    """One row of attention whose splits ``part`` still have to be merged, with the heads' sinks and gate logits."""
+
+    before = L.ROW_SPLITS
+
+    def __init__(self, part, splits: int, heads: int, vdim_s: int, sink, gate, dtype: torch.dtype):
+        self.u, self.splits, self.vdim_s, self.sink, self.gate, self.dtype = part, splits, vdim_s, sink, gate, dtype
+        self.shape, self.device = torch.Size((1, heads * vdim_s)), part.device
+
+    def fill(self, a: L.RowArgs) -> None:
+        a.xw, a.gate, a.norm_dim, a.head_stride = _ptr(self.sink), _ptr(self.gate), self.splits, self.vdim_s
+
+
 def _row_product(x, W):
     """(code, before, arguments) of the product of one row: a tensor in W's type, or an ``RmsRow``."""
     if not isinstance(x, RmsRow):
@@ -442,8 +455,9 @@ def relu_glu(x, W: torch.Tensor) -> torch.Tensor:
 
 def linear_residual(x: torch.Tensor, W: torch.Tensor, stream: ResidualStream, post, pre, add_start: bool = False):
     """``residual(x W^T, ...)``."""
-    code = _product_ok(x, W)
     n = x.shape[0]
+    if n != 1:
+        _product_ok(x, W)
     assert stream.x.shape == (n, W.shape[0])
     if n != 1 and not _tiles(x, W, whole=W.shape[0] % 8 == 0):
         nbytes = _parts_bytes(x, W, residual=True)
@@ -456,9 +470,9 @@ def linear_residual(x: torch.Tensor, W: torch.Tensor, stream: ResidualStream, po
         return h
     h = None if pre is None else stream.new_h()
     if n == 1:
-        a = _row_args(x, W)
+        code, before, a = _row_product(x, W)
         a.res = stream.args(post, pre, add_start, h)
-        _row_launch(code, L.ROW_PLAIN, L.OUT_RESIDUAL, a)
+        _row_launch(code, before, L.OUT_RESIDUAL, a)
     else:
         a = _tile_args(x, W)
         a.res = stream.args(post, pre, add_start, h)
@@ -715,6 +729,21 @@ def decode_splits(keys: int) -> int:
     return max(1, min(16, (keys + 63) // 64), min(128, keys // 128))
 
 
+# Small rows of many keys: the output projection merges the splits while it stages its row (eight at most: every workgroup reads them all, 66
+# KB of 2048 entries), so neither the launch that merges nor the one workgroup per head is waited for.  us a token, otherwise and so: vimulorn-2k
+# (16 heads of 128) at 100 / 170 / 270 / 350 / 460 / 740 / 1340 tokens 399.7 / 409.9, 414 / 423, 437 / 441, 450.6 / 446.5, 465 / 461, 468 / 462, 484 / 476, varolorn-2k at
+# 270 / 350 / 460 / 740 / 1340 462 / 465, 471 / 472, 477 / 469, 482 / 483, 506 / 496; rows of 4096 880 / 884 at 350, 901 / 899 at 460, 928 / 933 at 740, 982 / 995 at 1340.
+MERGE_KEYS, MERGE_ROW, MERGE_SPLITS = 320, 2048, 8
+
+
+def _merge_splits(keys: int) -> int:
+    return min((keys + 63) // 64, MERGE_SPLITS)
+
+
+def _merge_rule(heads: int, vdim_s: int, keys: int, dtype) -> bool:
+    return dtype == torch.bfloat16 and keys > MERGE_KEYS and heads * vdim_s <= MERGE_ROW
+
+
 def _attn_args(q, k, v, n, H, G, dim_s, vdim_s, scale, sink, gate, window, ring, base, pos_dev, pos):
     a = L.AttnArgs(q=q.data_ptr(), ldq=q.stride(0), k=k.data_ptr(), ldk=k.stride(0), k_head=dim_s, v=v.data_ptr(),
                    ldv=v.stride(0), v_head=vdim_s, n=n, H=H, G=G, dim_s=dim_s, vdim_s=vdim_s, scale=scale,
@@ -768,13 +797,13 @@ def portion_attention(q, k, v, heads: int, kv_heads: int, scale: float, first_ke
 
 
 def ring_attention_row(row, k_ring, v_ring, heads, kv_heads, dim, scale, eps, pos_dev, pos, sink=None, window=None,
-                       chunk=None, rel=None, q_weight=None, k_weight=None, mix_v=None, gate=None):
+                       chunk=None, rel=None, q_weight=None, k_weight=None, mix_v=None, gate=None, defer=False):
     """One token of attention over rings of keys and values (cap, kv_heads * stride).  row: fp32 (q, k, v); q and k
     are RMS-normed (times their weights), v mixed with ``mix_v`` = (other fp32 values, lambda), this token's k and v
-    stored.  gate: fp32 logits (heads,).  Masks and rel as in ``portion_attention``."""
+    stored.  gate: fp32 logits (heads,).  Masks and rel as in ``portion_attention``.  defer: the row goes to a product of this
+    module, which may merge the splits itself (a ``SplitRow`` is returned then)."""
     _f32(row, sink, q_weight, k_weight)
     dim_s, vdim_s, cap = k_ring.shape[1] // kv_heads, v_ring.shape[1] // kv_heads, k_ring.shape[0]
-    out = torch.empty(1, heads * vdim_s, dtype=k_ring.dtype, device=row.device)
     a = _attn_args(row, k_ring, v_ring, 1, heads, kv_heads, dim_s, vdim_s, scale, sink, None, window, cap, 0, pos_dev,
                    pos)
     _mask_args(a, window, chunk, rel)
@@ -787,10 +816,19 @@ def ring_attention_row(row, k_ring, v_ring, heads, kv_heads, dim, scale, eps, po
     if gate is not None:
         _f32(gate)
         a.gate, a.ldg = gate.data_ptr(), heads
-    a.out, a.norm_dim, a.eps = out.data_ptr(), dim, eps
+    a.norm_dim, a.eps = dim, eps
     a.fresh_k = row.data_ptr() + 4 * heads * dim_s
     a.fresh_v = row.data_ptr() + 4 * (heads + kv_heads) * dim_s
-    if k_ring.dtype != torch.bfloat16 or dim_s > 128 or vdim_s > 128 or min(cap, window or cap, chunk or cap) > ONE_LAUNCH_KEYS:
+    keys = min(cap, window or cap, chunk or cap)
+    if defer and _merge_rule(heads, vdim_s, keys, k_ring.dtype):
+        a.splits = _merge_splits(keys)
+        part = torch.empty(heads * a.splits * (vdim_s + 2), dtype=torch.float32, device=row.device)
+        a.part = part.data_ptr()
+        check(lib.dv_mix_attn_splits(_code(k_ring), 1, _ref(a), _stream()), "dv_mix_attn_splits")
+        return SplitRow(part, a.splits, heads, vdim_s, sink, gate, k_ring.dtype)
+    out = torch.empty(1, heads * vdim_s, dtype=k_ring.dtype, device=row.device)
+    a.out = out.data_ptr()
+    if k_ring.dtype != torch.bfloat16 or dim_s > 128 or vdim_s > 128 or keys > ONE_LAUNCH_KEYS:
         a.splits = decode_splits(cap)
     part = None
     if a.splits > 1:
@@ -800,8 +838,8 @@ def ring_attention_row(row, k_ring, v_ring, heads, kv_heads, dim, scale, eps, po
     return out
 
 
-def window_attention_row(row, k_ring, v_ring, heads, kv_heads, dim, scale, eps, sink, window, pos_dev, pos):
-    return ring_attention_row(row, k_ring, v_ring, heads, kv_heads, dim, scale, eps, pos_dev, pos, sink=sink, window=window)
+def window_attention_row(row, k_ring, v_ring, heads, kv_heads, dim, scale, eps, sink, window, pos_dev, pos, defer=False):
+    return ring_attention_row(row, k_ring, v_ring, heads, kv_heads, dim, scale, eps, pos_dev, pos, sink=sink, window=window, defer=defer)
 
 
 def latent_attention_row(q, k_up, v_up, cache, heads, scale, gate, pos_dev, pos):

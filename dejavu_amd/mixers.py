@@ -14,7 +14,7 @@
 
 A mixer's ``forward`` takes the normed rows h (n, width) of the next n tokens of ONE sequence (one token may come as a
 ``mixer_ops.RmsRow``, whose norm its products apply) and its state dict, moves the state on, and returns what its output
-projection is applied to (a tensor, ``mixer_ops.GatedHeads`` or ``mixer_ops.GroupedRow``); the block applies the
+projection is applied to (a tensor, ``mixer_ops.GatedHeads``, ``mixer_ops.GroupedRow`` or ``mixer_ops.SplitRow``); the block applies the
 projection together with the norm and the residual add that follow it.  One token runs the decode kernels, several
 tokens the portion kernels; a prompt may be cut anywhere.
 
@@ -30,6 +30,7 @@ import torch.nn as nn
 
 from . import mixer_ops as ops
 from .mixer_ops import padded
+from .modules import _hooked
 
 
 class StepInfo:
@@ -207,7 +208,7 @@ class WindowAttention(nn.Module):
         if n == 1:
             row = ops.row_conv(h, self.in_proj, self.conv, state["conv"], silu=False)
             return ops.window_attention_row(row, kr, vr, H, G, self.dim, self.scale, self.eps, self.sink, self.window,
-                                            step.pos_dev, step.pos)
+                                            step.pos_dev, step.pos, defer=not _hooked(self))
         p = ops.linear(h, self.in_proj)
         hist = min(step.pos, self.window - 1)  # earlier tokens that this portion can still see
         q = torch.empty(n, H * ds, dtype=h.dtype, device=h.device)
@@ -290,7 +291,7 @@ class ChunkAttention(nn.Module):
         if n == 1:
             return ops.ring_attention_row(p, kr, vr, H, G, self.dim, self.scale, self.eps, step.pos_dev, step.pos,
                                           chunk=self.chunk, rel=self.rel, q_weight=self.q_norm, k_weight=self.k_norm,
-                                          mix_v=mix, gate=gate[0])
+                                          mix_v=mix, gate=gate[0], defer=not _hooked(self))
         hist = step.pos % self.chunk if self.chunk else step.pos  # earlier tokens that this portion can still see
         q = torch.empty(n, H * ds, dtype=h.dtype, device=h.device)
         k, v = _behind_history((kr, vr), step.pos - hist, hist, n)

@@ -69,6 +69,8 @@ typedef struct {
 #define DV_ROW_RMS 1     /* x: fp32, divided by its root mean square over norm_dim, times xw              */
 #define DV_ROW_HEADS 2   /* x: fp32 heads of head_stride entries, each RMS-normed, times xw, times gate   */
 #define DV_ROW_GROUPS 3  /* x: fp32, groups of norm_dim entries (x_dim in all) each RMS-normed, times xw  */
+#define DV_ROW_SPLITS 4  /* x: what dv_mix_attn_splits leaves of K / head_stride heads, norm_dim splits of head_stride entries: their
+                            attention, with the sinks xw and the gate logits `gate` per head (either may be null) */
 #define DV_OUT_F32 0     /* fp32 store                                                                    */
 #define DV_OUT_T 1       /* store in `dtype`                                                              */
 #define DV_OUT_GLU 2     /* rows 2 i (gate) and 2 i + 1 (up) -> gated unit `act`, in `dtype`               */
@@ -336,6 +338,8 @@ DV_API int dv_mix_ring_copy_two(int dtype, const dvRingRows* a, const dvRingRows
                                 void* stream);
 /* q_f32: the queries (and gate logits) are fp32 instead of `dtype`. */
 DV_API int dv_mix_attn_rows(int dtype, int q_f32, const dvAttnArgs* args, void* stream);
+/* One decode row whose splits (two or more) stay in args->part, for a product that begins with DV_ROW_SPLITS; out, sink and gate are not used. */
+DV_API int dv_mix_attn_splits(int dtype, int q_f32, const dvAttnArgs* args, void* stream);
 /* bf16, a portion on the matrix cores; `keys` rows behind k and v (contiguous, ring = 0). */
 DV_API int dv_mix_attn_tiles(const dvAttnArgs* args, int keys, void* stream);
 /* The same in fp32. */
