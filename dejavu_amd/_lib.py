@@ -62,6 +62,9 @@ SIGNATURES = {
     "dv_dense_linear_partial_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int]),
     "dv_dense_linear_partial_f16": (
         _c_int, [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_size, _c_ptr]),
+    "dv_dense_linear_partial_sum_f16": (_c_int, [_c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr]),
+    "dv_dense_linear_partial_add_layer_norm_f16": (
+        _c_int, [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, ctypes.c_float, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr]),
     "dv_dense_linear_f16": (
         _c_int,
         [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_i64, _c_ptr, _c_size,

@@ -1244,6 +1244,15 @@ int dv_dense_linear_partial_f16(const void* x, int64_t ldx, const void* W, int64
                    RingLaunch{}, p.splits);
 }
 
+int dv_dense_linear_partial_sum_f16(const void* partial, int parts, const void* bias, int rows, int M, void* y, void* stream) {
+  if (!partial || !y || parts < 1 || rows < 1 || M <= 0) return DV_ERR_INVALID_ARG;
+  const int64_t total = (int64_t)rows * M;
+  hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                     reinterpret_cast<const float*>(partial), parts, rows, M, reinterpret_cast<const half_t*>(bias), (const void*)nullptr, 4, M,
+                     (int)DV_ACT_ID, reinterpret_cast<half_t*>(y), (int64_t)M);
+  return launch_status();
+}
+
 size_t dv_dense_linear_wide_workspace_bytes(int rows, int N, int M) {
   if (rows < 1 || N <= 0 || M <= 0) return 0;
   const WideSplit p = plan_wide_split(rows, M, N, compute_units());
@@ -1990,6 +1999,28 @@ int dv_reduce_add_layer_norm_window_f16(const void* partial, int groups, const v
   else
     DV_RLNW(1024, 4);
 #undef DV_RLNW
+  return launch_status();
+}
+
+int dv_dense_linear_partial_add_layer_norm_f16(const void* partial, int parts, const void* bias, const void* residual, const void* gamma,
+                                               const void* beta, float eps, int rows, int d, void* y, void* residual_out, void* stream) {
+  if (!partial || !gamma || !beta || !y || !residual_out || parts < 2 || rows < 1 || d <= 0) return DV_ERR_INVALID_ARG;
+  if (d % 8 || !aligned16(partial) || !aligned16(bias) || !aligned16(residual) || !aligned16(gamma) || !aligned16(beta) || !aligned16(y) ||
+      !aligned16(residual_out))
+    return DV_ERR_ALIGNMENT;
+  if (d > 1024 * 8 * 4) return DV_ERR_UNSUPPORTED;
+#define DV_RLNP(T, V)                                                                                                        \
+  hipLaunchKernelGGL((reduce_add_layer_norm_kernel<T, V, LnRowFromParts>), dim3(rows), dim3(T), 0,                           \
+                     reinterpret_cast<hipStream_t>(stream), reinterpret_cast<const float*>(partial),                         \
+                     reinterpret_cast<const half_t*>(bias), parts, rows, reinterpret_cast<const half_t*>(residual),          \
+                     reinterpret_cast<const half_t*>(gamma), reinterpret_cast<const half_t*>(beta), eps, d,                  \
+                     reinterpret_cast<half_t*>(y), reinterpret_cast<half_t*>(residual_out))
+  if (d <= 256 * 8) DV_RLNP(256, 1);
+  else if (d <= 512 * 8) DV_RLNP(512, 1);
+  else if (d <= 1024 * 8) DV_RLNP(1024, 1);
+  else if (d <= 1024 * 8 * 2) DV_RLNP(1024, 2);
+  else DV_RLNP(1024, 4);
+#undef DV_RLNP
   return launch_status();
 }
 

@@ -354,14 +354,46 @@ __global__ __launch_bounds__(THREADS) void add_layer_norm_kernel(
   add_layer_norm_body<THREADS, NV>(H, R, gamma, beta, eps, d, Y, Rout, Y2, blockIdx.x);
 }
 
-// add + LayerNorm of rows that arrive as the fp32 partial sums of a split product (LnRowFromPartials)
-template <int THREADS, int NV>
+// The same with the parts added up one after the other, as the launches do that end a dense product (gemm_ring_sum_kernel and its like).
+struct LnRowFromParts {
+  const float* __restrict__ partial;
+  const half_t* __restrict__ bias;
+  int G, d;
+  int64_t total;
+  __device__ __forceinline__ half8_t operator()(int i, int64_t row) const {
+    const float* p = partial + row * d + i * 8;
+    const half8_t bv = bias != nullptr ? load8(bias + i * 8) : zero8();
+    float4_t lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+    for (int g0 = 0; g0 < G; g0 += 4) {
+      float4_t l[4], h[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {  // (past the last part: that one again)
+        const float* at = p + (int64_t)(g0 + k < G ? g0 + k : G - 1) * total;
+        l[k] = *reinterpret_cast<const float4_t*>(at);
+        h[k] = *reinterpret_cast<const float4_t*>(at + 4);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (g0 + k < G) lo += l[k], hi += h[k];
+    }
+    half8_t y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      y[e] = (half_t)(lo[e] + (bias != nullptr ? (float)bv[e] : 0.f));
+      y[4 + e] = (half_t)(hi[e] + (bias != nullptr ? (float)bv[4 + e] : 0.f));
+    }
+    return y;
+  }
+};
+
+// add + LayerNorm of rows that arrive as the fp32 partial sums of a split product (Src: LnRowFromPartials, LnRowFromParts)
+template <int THREADS, int NV, typename Src = LnRowFromPartials>
 __global__ __launch_bounds__(THREADS) void reduce_add_layer_norm_kernel(
     const float* __restrict__ partial, const half_t* __restrict__ bias, int G, int rows,
     const half_t* __restrict__ R, const half_t* __restrict__ gamma, const half_t* __restrict__ beta, float eps,
     int d, half_t* __restrict__ Y, half_t* __restrict__ Rout) {
-  add_layer_norm_src_body<THREADS, NV, LnNoHook, LnRowFromPartials>(
-      LnRowFromPartials{partial, bias, G, d, (int64_t)rows * d}, R, gamma, beta, eps, d, Y, Rout, nullptr, blockIdx.x);
+  add_layer_norm_src_body<THREADS, NV, LnNoHook, Src>(
+      Src{partial, bias, G, d, (int64_t)rows * d}, R, gamma, beta, eps, d, Y, Rout, nullptr, blockIdx.x);
 }
 
 }  // namespace dv

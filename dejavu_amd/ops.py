@@ -359,10 +359,10 @@ class PendingRows:
     of the parts of its columns -- has not run: ``add_layer_norm`` / ``add_layer_norm_window`` take it in place of
     ``hidden`` and do that step in their own launch (the fc2 of one block and LayerNorm 1 of the
     next).  ``materialize()`` runs the step alone and returns the tensor.  Shape queries answer as
-    the tensor would (s: 1 for a decode step)."""
+    the tensor would (s: 1 for a decode step).  shape: of a dense product, whose parts are added up in their order."""
 
     def __init__(self, y: torch.Tensor, partial: torch.Tensor, groups: int, bias: Optional[torch.Tensor], shape=None):
-        self.y, self.partial, self.groups, self.bias = y, partial, groups, bias
+        self.y, self.partial, self.groups, self.bias, self.in_order = y, partial, groups, bias, shape is not None
         self._reduced = groups == 1  # a single group stores the finished rows itself
         self.shape = torch.Size((y.shape[0], 1, y.shape[1])) if shape is None else torch.Size(shape)
         self.dtype, self.device, self.is_cuda = y.dtype, y.device, True
@@ -377,6 +377,10 @@ class PendingRows:
         return self.y.numel()
 
     def materialize(self) -> torch.Tensor:
+        if not self._reduced and self.in_order:
+            check(lib.dv_dense_linear_partial_sum_f16(_ptr(self.partial), self.groups, _ptr(self.bias), *self.y.shape, _ptr(self.y), _stream()),
+                  "dv_dense_linear_partial_sum_f16")
+            self._reduced = True
         if not self._reduced:
             check(lib.dv_reduce_rows_f16(_ptr(self.partial), self.groups, _ptr(self.bias), self.y.shape[0],
                                          self.y.shape[1], _ptr(self.y), _stream()), "dv_reduce_rows_f16")
@@ -944,6 +948,12 @@ def _reduce_add_layer_norm(hidden: PendingRows, residual: Optional[torch.Tensor]
     partial, groups, pbias, complete = _rows_source(hidden)
     y = torch.empty(hidden.shape, dtype=torch.float16, device=hidden.device)
     r_out = torch.empty_like(y)
+    if hidden.in_order and not hidden._reduced:
+        assert window is None, "the parts of a dense product are a prompt's"
+        check(lib.dv_dense_linear_partial_add_layer_norm_f16(_ptr(partial), groups, _ptr(pbias), _ptr(residual), _ptr(weight.contiguous()),
+                                                             _ptr(bias.contiguous()), float(eps), rows, d, _ptr(y), _ptr(r_out), _stream()),
+              "dv_dense_linear_partial_add_layer_norm_f16")
+        return y, r_out
     if window is None:
         x_cache_row = tracker = head_idx = batch_idx = None
         nnz = H = counter = flush = 0

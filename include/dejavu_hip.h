@@ -159,14 +159,19 @@ DV_API int dv_dense_linear_wide_ws_f16(const void* x, int64_t ldx, const void* W
                                        int M, int act, void* y, int64_t ldy, void* workspace, size_t workspace_bytes,
                                        void* stream);
 /*
- * The product alone, its columns in parts whose fp32 sums stay in `partial` ([part][rows][M], on a 16-byte boundary): for
- * dv_reduce_add_layer_norm_window_f16 and dv_reduce_rows_f16, which add them up (groups = bytes / (4 * rows * M)) and the bias to them.
+ * The product alone, its columns in parts whose fp32 sums stay in `partial` ([part][rows][M], on a 16-byte boundary): parts = bytes / (4 *
+ * rows * M).  ..._sum_f16 adds them up, and the bias to them; ..._add_layer_norm_f16 (d: M) does what dv_add_layer_norm_f16 does with the result
+ * as well.  The same bits as the product, then dv_add_layer_norm_f16.
  * wide: dv_dense_linear_wide_ws_f16's parts instead of dv_dense_linear_f16's.  M % 8 == 0; 0 bytes: this product has no parts
  * (DV_ERR_UNSUPPORTED).
  */
 DV_API size_t dv_dense_linear_partial_workspace_bytes(int rows, int N, int M, int wide);
 DV_API int dv_dense_linear_partial_f16(const void* x, int64_t ldx, const void* W, int64_t ldw, int rows, int N, int M, int wide,
                                        void* partial, size_t partial_bytes, void* stream);
+DV_API int dv_dense_linear_partial_sum_f16(const void* partial, int parts, const void* bias, int rows, int M, void* y, void* stream);
+DV_API int dv_dense_linear_partial_add_layer_norm_f16(const void* partial, int parts, const void* bias, const void* residual,
+                                                      const void* gamma, const void* beta, float eps, int rows, int d, void* y,
+                                                      void* residual_out, void* stream);
 
 /*
  * y = x . W[idx] + bias.  Replaces gather_transposed_gemv,
