@@ -76,6 +76,12 @@ HIP_PROMPT_WIDE_STRIDE = 1 << 25
 # library, from 769 rows on by 20480 columns the wide tiles) over this, weights cold, 257 to 2048 rows: 2560 x 10240 1.06 to 1.30, 3072 x 12288 0.99 to 1.34,
 # 4096 x 16384 1.00 to 2.09, 4608 x 18432 1.05 to 1.92, 5120 x 20480 1.14 to 1.72, 5632 x 22528 1.32 to 1.61, 7168 x 28672 1.38 to 1.62, 9216 x 36864 1.38
 # to 1.39 (777 by 4096 x 16384 146 -> 103 us).  Of more weight rows only in three parts and more: in two 8192 x 28672 0.89 to 1.01, 12288 x 49152 0.90 to 1.00.
+# Fewer rows where one column of such tiles makes three parts (15361 to 20480 weight rows on 256 compute units): the streaming kernel over these, alone,
+# 136 / 160 / 192 rows: 16384 x 4096 1.10 / 1.10 / 1.05, 20480 x 5120 1.14 / 1.12 / 1.07, 18432 x 4608 1.03 / 1.02 / 0.99, 20480 x 2560 1.19 / 1.15 / 1.12; but
+# 16384 x 2048 0.91 to 1.01, in two parts 24576 x 6144 0.94 to 1.00, in four and five 14336 / 12288 x 4096 0.93 to 1.10.  The line in rows is by whole prompts of eight blocks
+# (us, streaming kernel or library / these), 6.7B shape 128 / 150 / 192 / 224 tokens 1309 / 1306, 1534 / 1504, 1586 / 1567, 1683 / 1695, 13B shape 1720 / 1775, 1993 /
+# 1967, 2064 / 2048, 2351 / 2366: fewer rows are as fast alone, but not beside the launches around them.
+HIP_PROMPT_FEW_PARTS, HIP_PROMPT_FEW_COLUMNS, HIP_PROMPT_FEW_ROWS = 3, 2560, (129, 192)
 HIP_PROMPT_PARTS_COLUMNS, HIP_PROMPT_PARTS_WEIGHT = 10240, 26_000_000
 HIP_PROMPT_PARTS_TALL = 7168, 3
 # The package's causal-attention kernel (cache fill in the same launch) is ahead of the library's attention with the
@@ -418,6 +424,16 @@ def _long_parts(linear, x: torch.Tensor) -> bool:
     return _parts_rule(rows, M, K, ops.wide_parts(rows, K, M)) and _wide_fits(linear, x)
 
 
+def _few_parts_product(linear, x: torch.Tensor, activation: str) -> bool:
+    """The same for a prompt of few rows, with an activation too."""
+    W = linear.weight
+    rows = x.numel() // x.shape[-1]
+    if not HIP_PROMPT_FEW_ROWS[0] <= rows <= HIP_PROMPT_FEW_ROWS[1] or W.dim() != 2 or activation not in ("id", "relu", "squared_relu"):
+        return False
+    M, K = W.shape
+    return (K >= HIP_PROMPT_FEW_COLUMNS and M % 8 == 0 and ops.wide_parts(rows, K, M) == HIP_PROMPT_FEW_PARTS and _wide_fits(linear, x))
+
+
 def _parts_product(linear, x: torch.Tensor) -> Optional[torch.Tensor]:
     return ops.dense_linear_wide_parts(x, linear.weight, linear.bias) if _long_parts(linear, x) else None
 
@@ -443,12 +459,14 @@ def decode_linear(linear: nn.Linear, x: torch.Tensor, activation: str = "id") ->
     always go to this package's row kernels (vector ALUs for one or two rows, matrix cores above).  The
     rows of a prompt go to the matrix-core kernels that stream the weight while it is the bound (``USE_HIP_PROMPT``, up
     to ``HIP_PROMPT_MAX_ROWS`` rows, and more of them for long-rowed weights: ``_long_product``), with an activation or long
-    rows to the one with wide tiles (``_wide_product``, ``_parts_product``), else to the library GEMM."""
+    rows to the one with wide tiles (``_wide_product``, ``_parts_product``, ``_few_parts_product``), else to the library GEMM."""
     on_hip = x.is_cuda and x.dtype == torch.float16 and linear.weight.dtype == torch.float16 and x.shape[-1] % 8 == 0
     if on_hip and x.dim() == 3 and x.shape[1] == 1 and x.shape[0] <= 64:
         return ops.dense_decode_linear(x, linear.weight, linear.bias, activation)
     if on_hip and USE_HIP_PROMPT:
         rows = x.numel() // x.shape[-1]
+        if _few_parts_product(linear, x, activation):
+            return ops.dense_linear_wide_parts(x, linear.weight, linear.bias, activation)
         if rows <= HIP_PROMPT_MAX_ROWS or (rows <= HIP_PROMPT_LONG_MAX_ROWS and _long_product(linear, x)):
             return ops.dense_linear(x, linear.weight, linear.bias, activation)
         parts = _parts_product(linear, x) if activation == "id" else None

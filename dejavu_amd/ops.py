@@ -296,8 +296,9 @@ def wide_parts(rows: int, N: int, M: int) -> int:
     return _wide_parts_bytes(torch._C._cuda_getDevice(), rows, N, M) // (4 * rows * M)
 
 
-def dense_linear_wide_parts(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """``dense_linear_wide`` without an activation and with the columns in parts (several: ``wide_parts``)."""
+def dense_linear_wide_parts(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                            activation: str = "id") -> torch.Tensor:
+    """``dense_linear_wide`` with the columns in parts (several: ``wide_parts``)."""
     _require_device(x, weight, bias)
     M, N = weight.shape
     x2 = x.reshape(-1, N)
@@ -308,7 +309,7 @@ def dense_linear_wide_parts(x: torch.Tensor, weight: torch.Tensor, bias: Optiona
     out = torch.empty(rows, M, device=x.device, dtype=x.dtype)
     # the sums of this call alone (up to 250 MB), not the stream's scratch, which is never given back
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    check(lib.dv_dense_linear_wide_ws_f16(_ptr(x2), x2.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), rows, N, M, _ACT["id"],
+    check(lib.dv_dense_linear_wide_ws_f16(_ptr(x2), x2.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), rows, N, M, _ACT[activation],
                                           _ptr(out), M, _ptr(ws), nbytes, _stream()), "dv_dense_linear_wide_ws_f16")
     return out.view(*x.shape[:-1], M)
 
