@@ -8,8 +8,12 @@
 // the accumulator has them (key permutation 0-3, 8-11 | 4-7, 12-15 inside 16).  Values stay in LDS as they are in memory and
 // are read transposed; pairing keys by hand took eight 4-byte stores for each 16-byte one, and with the sums rescaled for
 // every tile, not only where a maximum has grown, 32 heads of 128 and 2048 tokens took 98 us instead of 89, 4096 tokens 331
-// instead of 304 (two heads a compute unit: the last queries' 32 tiles, one after the other, are the time at 2048).
-// Two buffers with one barrier a tile were slower (96).  Bound by the chain of a tile: LDS reads, two products, the softmax.
+// instead of 304.  Two buffers with one barrier a tile were slower (96).  Bound by the chain of a tile: LDS reads, two products, the
+// softmax.  So two groups of four waves share a query tile, the even and the odd key tiles: the last queries' chain is half as long, a SIMD
+// has two waves whatever the grid (alone a wave takes 328 registers, one to a SIMD; two in a group's kernel 238), and a long workgroup and
+// a short one make the same 17 steps on every compute unit.  us, one group / two, 32 heads of 128: 300 / 777 / 2048 / 4096 / 8192
+// tokens 16.5 / 13.6, 35.1 / 25.7, 92 / 69, 308 / 217, 1172 / 713, a window of 1024 and 8 key heads 91.5 / 64.7 (2048), 352 / 251 (8192); 16 heads 33.6 / 24.3 (777),
+// 79.5 / 53.8 (2048).
 #pragma once
 #include "attn_rows.hpp"
 
@@ -18,15 +22,20 @@ namespace dv {
 constexpr int kTileQ = 128, kTileK = 64;
 
 // DT: query/key tiles of 16, VT: value tiles of 32.  Grid: H * ceil(n / 128), head fastest, last queries first.
-template <int DT, int VT>
-__global__ __launch_bounds__(256) void attn_tiles_kernel(AttnArgs a, int keys /* rows behind k and v */) {
+// KS: groups of four waves that take a query tile's key tiles in turn, each with its own softmax; their sums meet at the end.
+template <int DT, int VT, int KS>
+__global__ __launch_bounds__(256 * KS) void attn_tiles_kernel(AttnArgs a, int keys /* rows behind k and v */) {
   typedef short tr_t __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) tr_t* tr_ptr_t;
   constexpr int DL = DT * 16 + 8, VL = VT * 32;  // LDS row lengths
-  __shared__ __attribute__((aligned(16))) bf16_t ks[kTileK * DL];
-  __shared__ __attribute__((aligned(16))) bf16_t vs[kTileK * VL];
-  __shared__ float rs[kTileQ + kTileK];  // biases of a tile: entry i is the distance off + q0 - k0 - (kTileK - 1) + i
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
+  constexpr size_t KB = kTileK * DL * sizeof(bf16_t), VB = kTileK * VL * sizeof(bf16_t), MERGE = KS > 1 ? (size_t)(KS - 1) * 256 * (VT * 16 + 2) * 4 : 0;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[KS * (KB + VB) > MERGE ? KS * (KB + VB) : MERGE];
+  __shared__ float biases[KS][kTileQ + kTileK];
+  const int group = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  bf16_t* const ks = reinterpret_cast<bf16_t*>(smem + group * (KB + VB));
+  bf16_t* const vs = reinterpret_cast<bf16_t*>(smem + group * (KB + VB) + KB);
+  float* const rs = biases[group];  // biases of a tile: entry i is the distance off + q0 - k0 - (kTileK - 1) + i
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
   const int head = blockIdx.x % a.H, g = head / (a.H / a.G);
   const int nblk = (a.n + kTileQ - 1) / kTileQ;
   const int q0 = (nblk - 1 - (int)(blockIdx.x / a.H)) * kTileQ;
@@ -102,12 +111,14 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(AttnArgs a, int keys /*
   const float sc = a.scale * kLog2e;
   const int tr_row = 4 * hh + ((lane & 15) >> 2), tr_col = 16 * ((lane >> 4) & 1) + (lane & 3) * 4;
 
-  fetch(first);
-  for (int k0 = first; k0 <= last; k0 += kTileK) {
+  const int mine = first + group * kTileK;
+  fetch(mine);
+  for (int b0 = first; b0 <= last; b0 += KS * kTileK) {
+    const int k0 = b0 + group * kTileK;  // (a group may be past the last tile)
     __syncthreads();
     put();
     __syncthreads();
-    if (k0 + kTileK <= last) fetch(k0 + kTileK);
+    if (k0 + KS * kTileK <= last) fetch(k0 + KS * kTileK);
     const bool seen = k0 <= whi && k0 + kTileK - 1 >= wklo;
     if (!seen) continue;
     float16_t s[2];
@@ -184,6 +195,31 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(AttnArgs a, int keys /*
         }
         o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w.all, pf, o[t], 0, 0, 0);
       }
+    }
+  }
+  if constexpr (KS > 1) {
+    float* mg = reinterpret_cast<float*>(smem) + tid;
+    __syncthreads();
+    if (group > 0) {
+      mg += (group - 1) * 256 * (VT * 16 + 2);
+#pragma unroll
+      for (int t = 0; t < VT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mg[(t * 16 + i) * 256] = o[t][i];
+      mg[VT * 16 * 256] = m;
+      mg[(VT * 16 + 1) * 256] = l;
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int k = 1; k < KS; ++k, mg += 256 * (VT * 16 + 2)) {
+      const float mo = mg[VT * 16 * 256], m1 = fmaxf(m, mo), c0 = __builtin_amdgcn_exp2f(m - m1), c1 = __builtin_amdgcn_exp2f(mo - m1);
+      m = m1;
+      l = __builtin_fmaf(mg[(VT * 16 + 1) * 256], c1, l * c0);
+#pragma unroll
+      for (int t = 0; t < VT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[t][i] = __builtin_fmaf(mg[(t * 16 + i) * 256], c1, o[t][i] * c0);
     }
   }
   l += __shfl_xor(l, 32, kWave);

@@ -404,7 +404,18 @@ int ssd_scan_any(const SsdArgs& a, hipStream_t s) {
 
 template <int DT, int VT>
 int attn_tiles_launch(const AttnArgs& a, int keys, hipStream_t s) {
-  hipLaunchKernelGGL((attn_tiles_kernel<DT, VT>), dim3((unsigned)((int64_t)a.H * ((a.n + kTileQ - 1) / kTileQ))), dim3(256), 0, s, a, keys);
+  const dim3 grid((unsigned)((int64_t)a.H * ((a.n + kTileQ - 1) / kTileQ)));
+  // Two groups of waves from three key tiles on (us, one / two: 47 / 100 tokens after none 7.2 / 8.1, 9.9 / 10.1, 160 / 300 11.6 / 10.7, 16.5 / 13.6, 47
+  // after 1000 42 / 28).  Heads beyond 128 need more registers than two waves on a SIMD have.
+  if constexpr (DT <= 8 && VT <= 4) {
+    const int mask = a.window > 0 ? a.window : a.chunk;
+    const int64_t most = mask > 0 ? (int64_t)mask + kTileQ - 1 : keys;
+    if ((most < keys ? most : keys) > 2 * kTileK) {
+      hipLaunchKernelGGL((attn_tiles_kernel<DT, VT, 2>), grid, dim3(512), 0, s, a, keys);
+      return launched();
+    }
+  }
+  hipLaunchKernelGGL((attn_tiles_kernel<DT, VT, 1>), grid, dim3(256), 0, s, a, keys);
   return launched();
 }
 
