@@ -1485,6 +1485,20 @@ int dv_qkv_proj_batch_f16(const void* x, int64_t ldx, const void* W, const void*
   return launch_status();
 }
 
+}  // extern "C"
+namespace {
+// Tiles of 128 queries, where they are work enough for the chip and not much of the last one is empty (us, 32 queries a workgroup / tiles of 128; heads
+// of 128, 32 of them, 500 / 777 / 2000 / 4000 tokens 16.8 / 20.3, 29.9 / 27.1, 105 / 70, 353 / 227; 40 heads 400 / 500 / 2000 15.6 / 18.4, 21.4 / 20.5, 124 / 90; 96 heads 256 / 300 / 500 /
+// 1000 19.5 / 16.8, 21.8 / 24.7, 35.8 / 32.8, 94 / 69; 16 sequences of 32 heads 160 / 256 / 777 42.6 / 47.5, 71 / 58, 376 / 288; heads of 64, 12 of them, 3000 / 6000
+// 48.4 / 54.4, 141 / 115, 96 of them 400 / 500 / 777 / 1500 15.7 / 16.8, 19.6 / 18.4, 32.8 / 33.3, 88 / 64).  The line is by whole prompts of six blocks: 32 heads 777 / 1000 / 1500 tokens 2326 / 2327, 2667 / 2657, 3898 / 3814,
+// 40 heads 512 / 777 / 1000 / 1900 2546 / 2555, 3637 / 3640, 4226 / 4186, 7386 / 7185.
+bool prefill_in_tiles(int B, int T, int H, int hd) {
+  const int64_t padded = ((int64_t)T + kPtQueries - 1) / kPtQueries * kPtQueries;
+  return (int64_t)T * H * B * hd >= 32000 * 128 && (T >= 450 || 5 * (int64_t)T >= 4 * padded);
+}
+}  // namespace
+extern "C" {
+
 int dv_prefill_attention_f16(const void* qkv, int B, int T, int H, int hd, float scale, void* ctx, void* k_cache,
                              void* v_cache, int pos0, int S, void* stream) {
   if (!qkv || !ctx || B < 1 || T < 0 || H <= 0 || ((k_cache == nullptr) != (v_cache == nullptr)) ||
@@ -1497,6 +1511,15 @@ int dv_prefill_attention_f16(const void* qkv, int B, int T, int H, int hd, float
   const int64_t groups = ((int64_t)T + kPfQueries - 1) / kPfQueries * H;
   if (groups > 0x7fffffff) return DV_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)groups, B);
+  if (prefill_in_tiles(B, T, H, hd) && aligned8(ctx)) {
+    const dim3 tiles((unsigned)(((int64_t)T + kPtQueries - 1) / kPtQueries * H), B);
+#define DV_PT(HD)                                                                                                               \
+  RingLaunch{}.operator()<prefill_tiles_kernel<HD>>(tiles, dim3(512), pt_lds<HD>, s, reinterpret_cast<const half_t*>(qkv), T, H, scale, \
+                                                    reinterpret_cast<half_t*>(ctx), reinterpret_cast<half_t*>(k_cache),         \
+                                                    reinterpret_cast<half_t*>(v_cache), pos0, S)
+    return hd == 128 ? DV_PT(128) : DV_PT(64);
+#undef DV_PT
+  }
   // Two wavefronts from two workgroups a compute unit on; measured to 128 tokens, beyond which each has a block to take.
   const bool two = T <= 128 && groups * B >= 2 * compute_units();
 #define DV_PF(HD, WAVES)                                                                                       \

@@ -90,8 +90,10 @@ HIP_PROMPT_PARTS_TALL = 7168, 3
 # many tokens leave gradients, functional transforms and the like to the library.
 HIP_PROMPT_ATTN_MAX_TOKENS = 192
 # Each workgroup reads the keys and values before its 32 queries, so the L2 bounds long prompts and the library, whose tiles
-# are larger, overtakes: with 40 heads of 128 from 8192 tokens on (1759 against 1691 us; 6000 tokens 961 against 1155, 16 sequences of
-# 4096 and 32 heads 5875 against 6316), with 96 heads above 2048 (four sequences of 2048 1329 against 1404, of 4096 5184 against 4784).
+# were larger, overtook: with 40 heads of 128 from 8192 tokens on (1759 against 1691 us; 6000 tokens 961 against 1155, 16 sequences of
+# 4096 and 32 heads 5875 against 6316), with 96 heads above 2048 (four sequences of 2048 1329 against 1404, of 4096 5184 against 4784).  (Its tiles of
+# 128 queries, prefill.hpp, are ahead beyond these lines as well: 40 heads and 8192 tokens 1051 against 1738, 96 heads and 4096 690 against 1305.  The lines
+# are where they were: what prompts of each length are computed by, and their bits, are what callers know.)
 HIP_PROMPT_ATTN_LONGEST = 6144
 HIP_PROMPT_ATTN_WIDE = 5120            # heads * head_dim above which it is
 HIP_PROMPT_ATTN_WIDE_LONGEST = 2048
