@@ -109,6 +109,8 @@ SIGNATURES = {
     "dv_mix_ssd_scan": (_i, [_i, _P(SsdArgs), _p]),
     "dv_mix_ssd_step": (_i, [_P(SsdStepArgs), _p]),
     "dv_mix_greedy_advance": (_i, [_p, _i, _p, _p, _p, _p, _l, _p, _p, _l, _l, _p, _p]),
+    "dv_mix_greedy_advance_workspace_bytes": (ctypes.c_size_t, [_i]),
+    "dv_mix_greedy_advance_ws": (_i, [_p, _i, _p, _p, _p, _p, _l, _p, _p, _l, _l, _p, _p, ctypes.c_size_t, _p]),
 }
 
 lib = load_library(LIB_PATH, SIGNATURES)

@@ -930,4 +930,24 @@ int dv_mix_greedy_advance(const float* logits, int vocab, void* token, void* pos
   return launched();
 }
 
+size_t dv_mix_greedy_advance_workspace_bytes(int vocab) { return vocab < 1 ? 0 : (size_t)blocks_of(vocab, kGreedyPart) * sizeof(GreedyBest); }
+
+int dv_mix_greedy_advance_ws(const float* logits, int vocab, void* token, void* position, void* seq_pos, void* sequences,
+                             int64_t seq_capacity, void* out_index, float* scores, int64_t score_ld, int64_t score_rows,
+                             void* score_index, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!logits || vocab < 1 || !token || !position || !seq_pos || !sequences || !out_index || seq_capacity < 0 ||
+      (scores && (!score_index || score_ld < vocab || score_rows < 0)))
+    return DV_ERR_INVALID_ARG;
+  if (!workspace || workspace_bytes < dv_mix_greedy_advance_workspace_bytes(vocab)) return DV_ERR_WORKSPACE;
+  if (!al16(workspace)) return DV_ERR_ALIGNMENT;
+  const unsigned count = blocks_of(vocab, kGreedyPart);
+  GreedyBest* parts = (GreedyBest*)workspace;
+  hipLaunchKernelGGL(greedy_parts_kernel, dim3(count), dim3(256), 0, st(stream), logits, vocab, parts, scores, score_ld,
+                     (const int64_t*)score_index, score_rows);
+  hipLaunchKernelGGL(greedy_parts_advance_kernel, dim3(1), dim3(64), 0, st(stream), parts, (int)count, vocab, (int64_t*)token,
+                     (int64_t*)position, (int*)seq_pos, (int64_t*)sequences, (int64_t*)out_index, scores ? (int64_t*)score_index : nullptr,
+                     seq_capacity);
+  return launched();
+}
+
 }  // extern "C"

@@ -956,8 +956,9 @@ def greedy_advance(logits, token, position, seq_pos, sequences, out_index, score
     """``ops.greedy_advance`` for fp32 logits."""
     _f32(logits)
     assert logits.dim() == 1
-    check(lib.dv_mix_greedy_advance(_ptr(logits), logits.numel(), _ptr(token), _ptr(position), _ptr(seq_pos),
-                                    _ptr(sequences), sequences.numel(), _ptr(out_index), _ptr(scores),
-                                    0 if scores is None else scores.stride(0),
-                                    0 if scores is None else scores.shape[0], _ptr(score_index), _stream()),
-          "dv_mix_greedy_advance")
+    ws = torch.empty(lib.dv_mix_greedy_advance_workspace_bytes(logits.numel()), dtype=torch.uint8, device=logits.device)
+    check(lib.dv_mix_greedy_advance_ws(_ptr(logits), logits.numel(), _ptr(token), _ptr(position), _ptr(seq_pos),
+                                       _ptr(sequences), sequences.numel(), _ptr(out_index), _ptr(scores),
+                                       0 if scores is None else scores.stride(0),
+                                       0 if scores is None else scores.shape[0], _ptr(score_index), _ptr(ws), ws.numel(), _stream()),
+          "dv_mix_greedy_advance_ws")

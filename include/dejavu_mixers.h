@@ -364,6 +364,11 @@ DV_API int dv_mix_ssd_step(const dvSsdStepArgs* args, void* stream);
 DV_API int dv_mix_greedy_advance(const float* logits, int vocab, void* token, void* position, void* seq_pos,
                                  void* sequences, int64_t seq_capacity, void* out_index, float* scores,
                                  int64_t score_ld, int64_t score_rows, void* score_index, void* stream);
+/* The same in two launches, with scratch for both on a 16-byte boundary. */
+DV_API size_t dv_mix_greedy_advance_workspace_bytes(int vocab);
+DV_API int dv_mix_greedy_advance_ws(const float* logits, int vocab, void* token, void* position, void* seq_pos, void* sequences,
+                                    int64_t seq_capacity, void* out_index, float* scores, int64_t score_ld, int64_t score_rows,
+                                    void* score_index, void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

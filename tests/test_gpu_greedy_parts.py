@@ -1,0 +1,39 @@
+"""Argmax and bookkeeping of a generation step in two launches: ends of workgroups, ties, NaN, rows off 16-byte boundaries, full buffers."""
+import pytest
+import torch
+
+from dejavu_amd import mixer_ops as ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("vocab", [1, 3, 1023, 1024, 1025, 4099, 32768, 70001])
+@pytest.mark.parametrize("kind", ["one", "tie", "nan", "lowest"])
+@pytest.mark.parametrize("off", [0, 1])
+def test_step(vocab, kind, off):
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    logits = torch.randn(vocab + 8, device="cuda", generator=g)[off:off + vocab]
+    want = int(logits.argmax())
+    if kind == "tie":
+        top = logits.max() + 1
+        for i in (vocab // 3, vocab // 2, vocab - 1):
+            logits[i] = top
+        want = vocab // 3
+    elif kind == "nan":
+        logits[vocab // 2], logits[vocab - 1], want = float("nan"), float("nan"), vocab // 2
+    elif kind == "lowest":
+        logits.fill_(float("-inf"))
+        want = 0
+    ones = [torch.full((1,), v, dtype=t, device="cuda") for v, t in ((7, torch.int64), (8, torch.int64), (9, torch.int32), (2, torch.int64), (1, torch.int64))]
+    token, position, seq_pos, out_index, score_index = ones
+    sequences = torch.full((1, 4), -1, dtype=torch.int64, device="cuda")
+    scores = torch.full((3, vocab), 5.0, device="cuda")
+    for step in range(3):  # the third token and the third row of scores have no place
+        ops.greedy_advance(logits, token, position, seq_pos, sequences, out_index, scores, score_index)
+        assert [int(t) for t in ones] == [want, 9 + step, 10 + step, 3 + step, 2 + step]
+    assert sequences.tolist() == [[-1, -1, want, want]]
+    assert bool((scores[0] == 5).all()) and all(torch.equal(scores[i], logits) or kind == "nan" for i in (1, 2))
+    if kind == "nan":
+        assert torch.equal(scores[1].nan_to_num(3.0), logits.nan_to_num(3.0))
+    ops.greedy_advance(logits, token, position, seq_pos, sequences, out_index)
+    assert int(score_index) == 4 and int(token) == want and int(out_index) == 6
