@@ -37,10 +37,10 @@ LAZY_SIDE_JOIN = True
 # Batched sparse decode and prompts: the split reduction of out_proj, the residual add and LayerNorm 2 in one launch
 # (ops.out_proj_sparse_t_add_layer_norm, modules.pending_linear).  False: out_proj with its reduction launch, then add_layer_norm.
 FOLD_NORM2 = True
-# Batched sparse decode and prompts, blocks with ``defer_mlp_reduce`` set (whoever sets it consumes the block's
+# Batched sparse decode, blocks with ``defer_mlp_reduce`` set (whoever sets it consumes the block's
 # hidden_states with ops.add_layer_norm / add_layer_norm_window, as the next block and the model's
-# final LayerNorm do): the split reduction of fc2 is left to that LayerNorm's launch; the block
-# returns ops.PendingRows as hidden_states.  False: fc2 with its reduction launch.
+# final LayerNorm do), and prompts, of calls with ``defer_reduce`` (the same said of one call): the split reduction of fc2
+# is left to that LayerNorm's launch; the block returns ops.PendingRows as hidden_states.  False: fc2 with its reduction launch.
 FOLD_NORM1 = True
 
 
@@ -86,9 +86,10 @@ class BlockMlpAttSparse(nn.Module):
         self.defer_mlp_reduce = False
 
     def forward(self, hidden_states: Tensor, residual: Optional[Tensor] = None, mixer_subset=None,
-                mixer_kwargs=None, head_idx=None, mlp_sp_logit=None):
+                mixer_kwargs=None, head_idx=None, mlp_sp_logit=None, defer_reduce=False):
         """hidden_states: output of the previous block's MLP (or its ops.PendingRows); residual: its
-        residual stream (None for the first block).  Returns
+        residual stream (None for the first block).  defer_reduce: the caller's next step with this call's hidden_states, a prompt's,
+        is an add + LayerNorm that takes ops.PendingRows.  Returns
         (hidden_states, residual, next_mlp_sp_logit, next_att_idx)."""
         assert mixer_subset is None
         ip = None if mixer_kwargs is None else mixer_kwargs.get("inference_params")
@@ -115,8 +116,8 @@ class BlockMlpAttSparse(nn.Module):
             hidden_states, residual = _add_norm(self.norm2, hidden_states, residual)
         hidden_states, next_mlp_sp_logit = self.mlp(
             hidden_states, residual, mlp_idx, defer_join=lazy,
-            defer_reduce=FOLD_NORM1 and self.defer_mlp_reduce and
-            (window is not None or (prompt and not _hooked(self) and not _hooked(self.mlp))))
+            defer_reduce=FOLD_NORM1 and ((self.defer_mlp_reduce and window is not None) or
+                                         (defer_reduce and prompt and type(self.mlp) is ParallelFusedMLPDejavu and not _hooked(self.mlp))))
         return hidden_states, residual, next_mlp_sp_logit, next_att_idx
 
 

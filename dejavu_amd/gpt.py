@@ -124,6 +124,11 @@ class GPT2Embeddings(nn.Module):
         return embeddings + self.position_embeddings(position_ids)
 
 
+def _plain_block(block) -> bool:
+    """No wrapper, subclass or hooks, which are given tensors only."""
+    return type(block) is BlockMlpAttSparse and not dv_modules._hooked(block)
+
+
 class GPTModel(nn.Module):
     def __init__(self, config, process_group=None, device=None, dtype=None):
         super().__init__()
@@ -187,15 +192,15 @@ class GPTModel(nn.Module):
                 chain.run()
                 chain = None
             if self.att_sparse:
+                # what a prompt's block leaves to the add + LayerNorm behind it stays between plain blocks and ln_f
+                pending = {"defer_reduce": True} if input_ids.shape[1] > 1 and _plain_block(layer) and (
+                    after is None or _plain_block(after)) else {}
                 hidden_states, residual, next_mlp_sp_logit, next_att_idx = layer(
                     hidden_states, residual, head_idx=next_att_idx, mlp_sp_logit=next_mlp_sp_logit,
-                    mixer_kwargs=mixer_kwargs)
+                    mixer_kwargs=mixer_kwargs, **pending)
             else:
                 hidden_states, residual, next_mlp_sp_logit = layer(
                     hidden_states, residual, mlp_sp_logit=next_mlp_sp_logit, mixer_kwargs=mixer_kwargs)
-            if input_ids.shape[1] > 1 and isinstance(hidden_states, ops.PendingRows) and after is not None and (
-                    type(after) not in (BlockMlpAttSparse, BlockDejavu) or dv_modules._hooked(after)):
-                hidden_states = hidden_states.materialize()  # (hooks and other modules get a tensor)
             if self.record is not None and self.record_mlp_idx is not None and input_ids.shape[1] == 1:
                 idx = getattr(layer, "last_mlp_idx", None)
                 self.record_mlp_idx.append(None if idx is None else idx.clone())
