@@ -173,8 +173,7 @@ class GPTModel(nn.Module):
         chain = None
         chaining = (self.chain_layers and self.att_sparse and self.record is None and input_ids.shape[1] == 1
                     and input_ids.shape[0] == 1)
-        following = list(self.layers[1:]) + [None]
-        for layer, after in zip(self.layers, following):
+        for i, layer in enumerate(self.layers):
             if self.record is not None and input_ids.shape[1] == 1:
                 dv_modules.join_side_stream()  # the predictions of the block before may be pending on the side stream
                 self.record.append((None if next_att_idx is None else next_att_idx.clone(),
@@ -194,7 +193,7 @@ class GPTModel(nn.Module):
             if self.att_sparse:
                 # what a prompt's block leaves to the add + LayerNorm behind it stays between plain blocks and ln_f
                 pending = {"defer_reduce": True} if input_ids.shape[1] > 1 and _plain_block(layer) and (
-                    after is None or _plain_block(after)) else {}
+                    i + 1 == len(self.layers) or _plain_block(self.layers[i + 1])) else {}
                 hidden_states, residual, next_mlp_sp_logit, next_att_idx = layer(
                     hidden_states, residual, head_idx=next_att_idx, mlp_sp_logit=next_mlp_sp_logit,
                     mixer_kwargs=mixer_kwargs, **pending)
