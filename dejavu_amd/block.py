@@ -55,6 +55,11 @@ def _prompt(hidden_states) -> bool:
     return hidden_states.is_cuda and hidden_states.dtype == torch.float16 and hidden_states.size(1) > 1
 
 
+def _plain(module, cls) -> bool:
+    """A module of that class itself, whose results nobody else sees or changes."""
+    return type(module) is cls and not _hooked(module)
+
+
 class BlockMlpAttSparse(nn.Module):
     """Block whose mixer predicts heads for the next layer and whose MLP predicts
     neurons for the next layer."""
@@ -101,7 +106,9 @@ class BlockMlpAttSparse(nn.Module):
         hidden_states, residual, window = self._norm1(hidden_states, residual, head_idx, ip)
         lazy = LAZY_SIDE_JOIN and hidden_states.is_cuda
         prompt = _prompt(hidden_states)
-        post_norm = (self.norm2, residual) if FOLD_NORM2 and (window is not None or (prompt and not _hooked(self.mixer))) else None
+        post_norm = None
+        if FOLD_NORM2 and (window is not None or (prompt and _plain(self.mixer, ParallelMHASparseAttMlp))):
+            post_norm = (self.norm2, residual)
         hidden_states, mlp_idx, next_att_idx = self.mixer(hidden_states, residual=residual, head_idx=head_idx,
                                                           mlp_sp_logit=mlp_sp_logit, window=window, defer_join=lazy,
                                                           post_norm=post_norm, **mixer_kwargs)
@@ -117,7 +124,7 @@ class BlockMlpAttSparse(nn.Module):
         hidden_states, next_mlp_sp_logit = self.mlp(
             hidden_states, residual, mlp_idx, defer_join=lazy,
             defer_reduce=FOLD_NORM1 and ((self.defer_mlp_reduce and window is not None) or
-                                         (defer_reduce and prompt and type(self.mlp) is ParallelFusedMLPDejavu and not _hooked(self.mlp))))
+                                         (defer_reduce and prompt and _plain(self.mlp, ParallelFusedMLPDejavu))))
         return hidden_states, residual, next_mlp_sp_logit, next_att_idx
 
 
@@ -157,8 +164,9 @@ class BlockDejavu(nn.Module):
         if mixer_kwargs is None:
             mixer_kwargs = {}
         lazy = LAZY_SIDE_JOIN and hidden_states.is_cuda
-        post_norm = (self.norm2, residual) if FOLD_NORM2 and _prompt(hidden_states) and not _hooked(self.mixer) else None
-        hidden_states, mlp_idx = self.mixer(hidden_states, mlp_sp_logit=mlp_sp_logit, defer_join=lazy, post_norm=post_norm, **mixer_kwargs)
+        if FOLD_NORM2 and _prompt(hidden_states) and _plain(self.mixer, ParallelMHADejavu):
+            mixer_kwargs = {**mixer_kwargs, "post_norm": (self.norm2, residual)}
+        hidden_states, mlp_idx = self.mixer(hidden_states, mlp_sp_logit=mlp_sp_logit, defer_join=lazy, **mixer_kwargs)
         if lazy:
             self.mixer.join_side()  # in front of LayerNorm 2, as in BlockMlpAttSparse
         if isinstance(hidden_states, tuple):

@@ -76,3 +76,42 @@ def test_what_is_not_plain_gets_tensors(what, place):
     else:
         layers[place].mlp.__class__ = _Mlp
     assert torch.equal(_logits(model), want)
+
+
+class _Attention(modules.ParallelMHADejavu):
+    def forward(self, *args, **kwargs):
+        out, idx = super().forward(*args, **kwargs)
+        return out * 1.0, idx
+
+
+class _SparseAttention(modules.ParallelMHASparseAttMlp):
+    def forward(self, *args, **kwargs):
+        out, *rest = super().forward(*args, **kwargs)
+        return (out * 1.0, *rest)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("att_sparse", [True, False])
+def test_mixers_of_a_callers_own_get_to_see_the_projection(att_sparse):
+    model = _model(att_sparse)
+    want = _logits(model)
+    model.transformer.layers[1].mixer.__class__ = _SparseAttention if att_sparse else _Attention
+    assert torch.equal(_logits(model), want)
+
+
+@pytest.mark.parametrize("tokens", [1, 5])
+def test_a_mixer_takes_the_arguments_that_it_always_took(tokens):
+    class Mixer(nn.Module):
+        def forward(self, x, mlp_sp_logit=None, defer_join=False, inference_params=None):
+            return x * 2, None
+
+        def join_side(self):
+            pass
+
+    class Mlp(nn.Module):
+        def forward(self, x, residual, idx=None, defer_join=False):
+            return x + residual, None
+
+    block = dv_block.BlockDejavu(8, lambda d: Mixer(), lambda d: Mlp())
+    h, residual, logit = block(torch.ones(1, tokens, 8), mixer_kwargs={"inference_params": None})
+    assert h.shape == residual.shape == (1, tokens, 8) and logit is None
