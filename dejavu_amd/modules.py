@@ -252,6 +252,8 @@ class ParallelFusedMLPDejavu(nn.Module):
         fc1, fc2, sp = (self._modules.get(k) for k in ("fc1", "fc2", "sp"))
         if type(sp) is not ParallelSP or type(fc1) is not nn.Linear or type(fc2) is not nn.Linear or _hooked(sp):
             return None
+        if "bias" not in fc1._parameters or "bias" not in fc2._parameters:  # a plain tensor, as pruning leaves it
+            return None
         W1, b1, b2 = fc1._parameters.get("weight"), fc1._parameters.get("bias"), fc2._parameters.get("bias")
         Wa, Wb = (sp._modules[k]._parameters.get("weight") for k in ("fc0", "fc1"))
         for t in (x, residual, W1, Wa, Wb):

@@ -1,6 +1,7 @@
 """The sparse MLP module's decode step as one call of the library gives what its ops give one by one, bit for bit."""
 import pytest
 import torch
+from torch.nn.utils import prune
 
 from dejavu_amd.modules import ParallelFusedMLPDejavu
 
@@ -79,3 +80,17 @@ def test_replayed_from_a_graph():
         graph.replay()
         want = m(x, residual, idx)
         assert torch.equal(out[0], want[0]) and torch.equal(out[1], want[1])
+
+
+@pytest.mark.parametrize("name", ["fc1", "fc2"])
+@pytest.mark.parametrize("parameter", ["bias", "weight"])
+@torch.no_grad()
+def test_pruned_layers(monkeypatch, name, parameter):
+    """Pruning leaves the values in use as a plain attribute of the layer, not as its parameter."""
+    m = _module(256, 1024, 64, 128)
+    x, residual = (torch.randn(1, 1, 256, device="cuda").half() for _ in range(2))
+    idx = torch.arange(128, device="cuda")
+    whole = m(x, residual, idx)[0]
+    prune.random_unstructured(getattr(m, name), parameter, 0.5)
+    got = m(x, residual, idx)[0]
+    assert torch.equal(got, _ops(monkeypatch, m, x, residual, idx)[0]) and not torch.equal(got, whole)
