@@ -23,7 +23,7 @@ from .generation import CausalLMOutput, GreedyDecoding
 from .inference import InferenceParams
 from .mixer_ops import padded
 from .mixers import (ChannelDelta, ChunkAttention, ClampedGLU, DynamicTanh, HyperConnection, LatentAttention, Mamba2,
-                     ReluGLU, RMSNorm, StepInfo, WindowAttention)
+                     ReluGLU, RMSNorm, StepInfo, WindowAttention, apply_mixer)
 
 
 @dataclass
@@ -191,7 +191,7 @@ class HybridBlock(nn.Module):
     def forward(self, h, stream: ops.ResidualStream, state: dict, step: StepInfo, pre, add_start: bool = False):
         """h: norm1 of the stream.  Adds both sublayers to the stream (then, with ``add_start``, the stream's start
         once more) and returns ``pre`` of it, the input of whatever comes next (None without ``pre``)."""
-        y = self.mixer(h, state, step)
+        y = apply_mixer(self.mixer, h, state, step)
         last = self.mlp is None
         after = (self.norm1b, pre, add_start) if last else (self.norm1b, self.norm2, False)
         if isinstance(y, ops.GatedHeads):
@@ -223,7 +223,7 @@ class StreamsBlock(nn.Module):
         """h: this layer's ``entry`` of the streams.  Both sublayers join the streams; returns ``following`` of them."""
         assert not add_start
         middle = following if self.mlp is None else ops.StreamRead(self.norm2, self.hyper2.weights)
-        h = stream.update(self.mixer(h, state, step), self.mixer.out_weight, self.mixer.out_bias, self.hyper1, middle)
+        h = stream.update(apply_mixer(self.mixer, h, state, step), self.mixer.out_weight, self.mixer.out_bias, self.hyper1, middle)
         if self.mlp is None:
             return h
         return stream.update(self.mlp(h), self.mlp.out_weight, None, self.hyper2, following)

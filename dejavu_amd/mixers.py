@@ -14,7 +14,7 @@
 
 A mixer's ``forward`` takes the normed rows h (n, width) of the next n tokens of ONE sequence (one token may come as a
 ``mixer_ops.RmsRow``, whose norm its products apply) and its state dict, moves the state on, and returns what its output
-projection is applied to (a tensor, ``mixer_ops.GatedHeads``, ``mixer_ops.GroupedRow`` or ``mixer_ops.SplitRow``); the block applies the
+projection is applied to (a tensor, ``mixer_ops.GatedHeads`` or ``mixer_ops.GroupedRow``; with ``defer`` also ``mixer_ops.SplitRow``); the block applies the
 projection together with the norm and the residual add that follow it.  One token runs the decode kernels, several
 tokens the portion kernels; a prompt may be cut anywhere.
 
@@ -202,13 +202,13 @@ class WindowAttention(nn.Module):
         return dict(_rings(min(self.window, max_len), self.kv_heads * self.dim_s, self.kv_heads * self.vdim_s, w),
                     conv=torch.zeros(self.channels, max(1, self.taps - 1), dtype=torch.float32, device=w.device))
 
-    def forward(self, h, state, step: StepInfo):
+    def forward(self, h, state, step: StepInfo, defer: bool = False):
         n, H, G, ds, vs = h.shape[0], self.heads, self.kv_heads, self.dim_s, self.vdim_s
         kr, vr = state["k"], state["v"]
         if n == 1:
             row = ops.row_conv(h, self.in_proj, self.conv, state["conv"], silu=False)
             return ops.window_attention_row(row, kr, vr, H, G, self.dim, self.scale, self.eps, self.sink, self.window,
-                                            step.pos_dev, step.pos, defer=not _hooked(self))
+                                            step.pos_dev, step.pos, defer=defer)
         p = ops.linear(h, self.in_proj)
         hist = min(step.pos, self.window - 1)  # earlier tokens that this portion can still see
         q = torch.empty(n, H * ds, dtype=h.dtype, device=h.device)
@@ -278,7 +278,7 @@ class ChunkAttention(nn.Module):
         tokens = min(self.chunk, max_len) if self.chunk else max_len
         return _rings(tokens, self.kv_heads * self.dim_s, self.kv_heads * self.vdim_s, self.in_proj)
 
-    def forward(self, h, state, step: StepInfo):
+    def forward(self, h, state, step: StepInfo, defer: bool = False):
         n, H, G, ds, vs = h.shape[0], self.heads, self.kv_heads, self.dim_s, self.vdim_s
         kr, vr = state["k"], state["v"]
         p = ops.linear(h, self.in_proj, self.in_bias, f32=n == 1)
@@ -291,7 +291,7 @@ class ChunkAttention(nn.Module):
         if n == 1:
             return ops.ring_attention_row(p, kr, vr, H, G, self.dim, self.scale, self.eps, step.pos_dev, step.pos,
                                           chunk=self.chunk, rel=self.rel, q_weight=self.q_norm, k_weight=self.k_norm,
-                                          mix_v=mix, gate=gate[0], defer=not _hooked(self))
+                                          mix_v=mix, gate=gate[0], defer=defer)
         hist = step.pos % self.chunk if self.chunk else step.pos  # earlier tokens that this portion can still see
         q = torch.empty(n, H * ds, dtype=h.dtype, device=h.device)
         k, v = _behind_history((kr, vr), step.pos - hist, hist, n)
@@ -401,3 +401,11 @@ class ChannelDelta(nn.Module):
         g, beta = ops.delta_gates(z, p[:, off_b:], self.A_log, self.dt_bias, H)
         o = ops.delta_scan(q, k, v, g, beta, state["S"], H, G)
         return ops.gated_head_norm(o, ops.linear(p[:, off_g:], self.gate_up), self.norm, self.vdim, self.eps)
+
+
+def apply_mixer(mixer, h, state, step: StepInfo):
+    """``mixer(h, state, step)`` for a caller whose next step is a product of ``mixer_ops`` with what comes back: that product can
+    merge an attention's splits itself.  Subclasses, wrappers and hooks are left out of it and see tensors."""
+    if type(mixer) in (WindowAttention, ChunkAttention) and not _hooked(mixer):
+        return mixer(h, state, step, defer=True)
+    return mixer(h, state, step)
