@@ -120,11 +120,25 @@ WIDE_TILE, NARROW_TILE, WIDE_ROUND = 256, 192, 256
 WIDE_TILES = 2 * WIDE_ROUND + 1, 3 * WIDE_ROUND - 10  # (a third round that is all but full is the library's again)
 
 
+def _remembered(rule):
+    """A rule's answers are kept by its sizes, but those of symbolic sizes, which have no hash (to look at the types first costs
+    0.3 us a product, which is as much as a rule)."""
+    known = lru_cache(maxsize=4096)(rule)
+
+    def ask(n, M, K, *more):
+        try:
+            return known(n, M, K, *more)
+        except TypeError:
+            return rule(n, M, K, *more)
+
+    return ask
+
+
 def _tiles_of(n: int, M: int, rows: int, weight_rows: int) -> int:
     return -(-n // rows) * -(-M // weight_rows)
 
 
-@lru_cache(maxsize=4096)
+@_remembered
 def _wide_rule(n: int, M: int, K: int) -> bool:
     if n > WIDE_MAX_ROWS or M > WIDE_MAX_WEIGHT_ROWS or M % NARROW_TILE == 0 or not WIDE_COLUMNS[0] <= K <= WIDE_COLUMNS[1]:
         return False
@@ -152,7 +166,7 @@ WIDE_FILL_GATED, WIDE_FILL_FEW_GATED, WIDE_FILL_FEW = 200, 144, 176
 WIDE_FULL_GATED, WIDE_FULL_FEW = 0.84, 0.83  # of the rounds of 256 x 256 tiles: tiles at least, rows by weight rows below
 
 
-@lru_cache(maxsize=4096)
+@_remembered
 def _fill_rule(n: int, M: int, K: int, gated: bool) -> bool:
     columns = WIDE_GATED_COLUMNS if gated else (WIDE_FEW_COLUMNS, WIDE_FEW_COLUMNS)
     if n <= TILE_MAX_ROWS or not 1024 <= K <= columns[1]:
@@ -182,8 +196,8 @@ PARTS_WEIGHT, PARTS_LIGHT_WEIGHT, PARTS_LIGHT_ROWS = 1 << 25, 26_000_000, 385   
 PARTS_TALL = 7168, 3                                                            # weight rows, parts at least of more of them
 
 
-def _parts_rule(n: int, M: int, K: int, residual: bool, parts: int) -> bool:
-    if not TILE_MAX_ROWS < n <= WIDE_MAX_ROWS or M % 8 or parts < (PARTS_TALL[1] if M > PARTS_TALL[0] else 2):
+def _parts_rule(n: int, M: int, K: int, residual: bool) -> bool:
+    if not TILE_MAX_ROWS < n <= WIDE_MAX_ROWS or M % 8:
         return False
     light = not residual and n >= PARTS_LIGHT_ROWS
     return K >= (PARTS_RESIDUAL_COLUMNS if residual else PARTS_COLUMNS) and M * K >= (PARTS_LIGHT_WEIGHT if light else PARTS_WEIGHT)
@@ -201,8 +215,10 @@ def _parts_bytes(x: torch.Tensor, W: torch.Tensor, bias=None, residual: bool = F
     if x.shape[1] < PARTS_RESIDUAL_COLUMNS or not TILE_MAX_ROWS < n <= WIDE_MAX_ROWS:  # (before anything that costs the host more)
         return 0
     M, K = W.shape
+    if not _parts_rule(n, M, K, residual) or not _wide_fits(x, W, bias):  # (tracers go no further)
+        return 0
     nbytes = _parts_workspace_bytes(torch._C._cuda_getDevice(), n, M, K)
-    return nbytes if _parts_rule(n, M, K, residual, nbytes // (4 * n * M)) and _wide_fits(x, W, bias) else 0
+    return nbytes if nbytes >= (PARTS_TALL[1] if M > PARTS_TALL[0] else 2) * 4 * n * M else 0
 
 
 def _parts_launch(after, a, nbytes, device) -> None:
@@ -210,7 +226,7 @@ def _parts_launch(after, a, nbytes, device) -> None:
     check(lib.dv_mix_linear_wide_ws(after, _ref(a), _ptr(ws), nbytes, _stream()), "dv_mix_linear_wide_ws")
 
 
-@lru_cache(maxsize=4096)
+@_remembered
 def _tile_rule(n: int, M: int, K: int, gated: bool) -> bool:
     if n > TILE_MAX_ROWS:
         return False

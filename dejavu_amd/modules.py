@@ -412,20 +412,21 @@ def _wide_product(linear, x: torch.Tensor, activation: str) -> bool:
     return W.dim() == 2 and _wide_rule(x.numel() // x.shape[-1], *W.shape, activation) and _wide_fits(linear, x)
 
 
-def _parts_rule(rows: int, M: int, K: int, parts: int) -> bool:
-    many, least = HIP_PROMPT_PARTS_TALL
+def _parts_rule(rows: int, M: int, K: int) -> bool:
     return (HIP_PROMPT_WIDE_ROWS[0] <= rows <= HIP_PROMPT_WIDE_ROWS[1] and K >= HIP_PROMPT_PARTS_COLUMNS and
-            M * K >= HIP_PROMPT_PARTS_WEIGHT and M % 8 == 0 and parts >= (least if M > many else 2))
+            M * K >= HIP_PROMPT_PARTS_WEIGHT and M % 8 == 0)
 
 
 def _long_parts(linear, x: torch.Tensor) -> bool:
     """Whether ``dense_linear_wide_parts`` is the faster one and does what ``linear(x)`` would."""
     W = linear.weight
     rows = x.numel() // x.shape[-1]
-    if W.dim() != 2 or not HIP_PROMPT_WIDE_ROWS[0] <= rows <= HIP_PROMPT_WIDE_ROWS[1]:
+    # (the number of parts is asked for last: tracers, which only the library's product is for, do not get that far)
+    if W.dim() != 2 or not _parts_rule(rows, *W.shape) or not _wide_fits(linear, x):
         return False
     M, K = W.shape
-    return _parts_rule(rows, M, K, ops.wide_parts(rows, K, M)) and _wide_fits(linear, x)
+    many, least = HIP_PROMPT_PARTS_TALL
+    return ops.wide_parts(rows, K, M) >= (least if M > many else 2)
 
 
 def _few_parts_product(linear, x: torch.Tensor, activation: str) -> bool:

@@ -293,7 +293,8 @@ def _wide_parts_bytes(device: int, rows: int, N: int, M: int) -> int:
 
 def wide_parts(rows: int, N: int, M: int) -> int:
     """Parts of the columns that ``dense_linear_wide_parts`` makes; 0: its tiles are enough for the chip."""
-    return _wide_parts_bytes(torch._C._cuda_getDevice(), rows, N, M) // (4 * rows * M)
+    nbytes = _wide_parts_bytes(torch._C._cuda_getDevice(), rows, N, M)
+    return nbytes and nbytes // (4 * rows * M)
 
 
 def dense_linear_wide_parts(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,

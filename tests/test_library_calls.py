@@ -280,3 +280,46 @@ def test_new_windows_that_only_the_library_begins(monkeypatch):
         launches.clear(), plain.fill_(-7)
         mha.reset_window(9, here)
         assert not launches and torch.equal(plain.cpu(), fresh) and mha.cache_offset.item() == 9
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+@pytest.mark.parametrize("rows,M,K,kind", [(300, 4096, 16384, "linear"), (300, 2560, 10240, "linear"), (300, 16384, 4096, "linear"),
+                                           (100, 4096, 4096, "portion"), (300, 4096, 11008, "portion"), (2048, 22016, 4096, "portion")])
+def test_products_in_traced_programs(rows, M, K, kind):
+    """Whole graphs and symbolic sizes: what a kernel's rule asks for may not get in the way of the library's product."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from dejavu_amd import mixer_ops
+    from dejavu_amd.modules import decode_linear
+
+    dtype = torch.float16 if kind == "linear" else torch.bfloat16
+    layer = nn.Linear(K, M, bias=False, device="cuda", dtype=dtype).requires_grad_(False)
+    x = torch.randn(1, rows, K, device="cuda").to(dtype)
+    if kind == "portion":
+        x = x[0]
+    want = F.linear(x, layer.weight)
+
+    def f(t, W):
+        return decode_linear(layer, t) if kind == "linear" else mixer_ops.linear(t, W)
+
+    torch._dynamo.reset()
+    whole = torch.compile(f, backend="eager", fullgraph=True)(x, layer.weight)
+    torch.testing.assert_close(whole, want, rtol=2e-2, atol=2e-2)  # (one rounding of each side: 2^-8 and less)
+    if kind == "portion":  # (a module's own weight is no input of the graph, and symbolic graphs take such ones only)
+        traced = make_fx(f, tracing_mode="symbolic")(x, layer.weight)
+        torch.testing.assert_close(traced(x, layer.weight), want, rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+def test_layers_without_results():
+    from dejavu_amd import mixer_ops, ops
+    from dejavu_amd.modules import decode_linear
+
+    for K in (4096, 16384):
+        layer = nn.Linear(K, 0, device="cuda", dtype=torch.float16)
+        assert decode_linear(layer, torch.zeros(1, 300, K, device="cuda").half()).shape == (1, 300, 0)
+    W = torch.zeros(0, 11008, device="cuda").bfloat16()
+    assert mixer_ops.linear(torch.zeros(300, 11008, device="cuda").bfloat16(), W).shape == (300, 0)
+    assert ops.wide_parts(150, 4096, 0) == 0
