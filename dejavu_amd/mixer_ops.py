@@ -749,15 +749,23 @@ def decode_splits(keys: int) -> int:
 # KB of 2048 entries), so neither the launch that merges nor the one workgroup per head is waited for.  us a token, otherwise and so: vimulorn-2k
 # (16 heads of 128) at 100 / 170 / 270 / 350 / 460 / 740 / 1340 tokens 399.7 / 409.9, 414 / 423, 437 / 441, 450.6 / 446.5, 465 / 461, 468 / 462, 484 / 476, varolorn-2k at
 # 270 / 350 / 460 / 740 / 1340 462 / 465, 471 / 472, 477 / 469, 482 / 483, 506 / 496; rows of 4096 880 / 884 at 350, 901 / 899 at 460, 928 / 933 at 740, 982 / 995 at 1340.
+# Beyond eight tiles of 64 keys a workgroup walks over several, and more splits with a launch that merges them are ahead: with a window, which stays
+# full, from there on, with a chunk or a whole sequence, of which half is seen on average, from twice as many.  us a token that the merge saves at 460 / 740 / 1000 /
+# 1340 / 1900 tokens (three such layers, 16 heads on 4 key heads): windows of 512 3.2 / 4.9 / 5.2 / 5.5 / 5.8, 1024 4.6 / -1.8 / -2.8 / -2.8 / -2.1, 2048 5.0 / -1.6 /
+# -1.9 / -1.7 / -9.7; chunks of 1024 5.8 / -0.3 / 1.8 / 4.1 / -1.6, 2048 4.3 / -1.3 / -2.7 / -2.0 / -9.0, 4096 6.2 / -0.5 / -1.2 / -1.6 / -10.1.  A row with its projection,
+# all keys seen, so many keys possible, 2048 / 4096 / 8192 / 32768: 19.9 / 23.9, 20.5 / 34.5, 21.6 / 56, 36.8 / 201.
 MERGE_KEYS, MERGE_ROW, MERGE_SPLITS = 320, 2048, 8
+MERGE_WINDOW, MERGE_CHUNK = 512, 1024
 
 
 def _merge_splits(keys: int) -> int:
     return min((keys + 63) // 64, MERGE_SPLITS)
 
 
-def _merge_rule(heads: int, vdim_s: int, keys: int, dtype) -> bool:
-    return dtype == torch.bfloat16 and keys > MERGE_KEYS and heads * vdim_s <= MERGE_ROW
+def _merge_rule(heads: int, vdim_s: int, keys: int, dtype, full: bool) -> bool:
+    """full: all of the keys are seen from some token on (a window's)."""
+    most = MERGE_WINDOW if full else MERGE_CHUNK
+    return dtype == torch.bfloat16 and MERGE_KEYS < keys <= most and heads * vdim_s <= MERGE_ROW
 
 
 def _attn_args(q, k, v, n, H, G, dim_s, vdim_s, scale, sink, gate, window, ring, base, pos_dev, pos):
@@ -836,7 +844,7 @@ def ring_attention_row(row, k_ring, v_ring, heads, kv_heads, dim, scale, eps, po
     a.fresh_k = row.data_ptr() + 4 * heads * dim_s
     a.fresh_v = row.data_ptr() + 4 * (heads + kv_heads) * dim_s
     keys = min(cap, window or cap, chunk or cap)
-    if defer and _merge_rule(heads, vdim_s, keys, k_ring.dtype):
+    if defer and _merge_rule(heads, vdim_s, keys, k_ring.dtype, keys == window):
         a.splits = _merge_splits(keys)
         part = torch.empty(heads * a.splits * (vdim_s + 2), dtype=torch.float32, device=row.device)
         a.part = part.data_ptr()
