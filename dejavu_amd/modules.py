@@ -39,8 +39,14 @@ USE_SIDE_STREAM = False
 # From this many sequences on the side stream is used regardless: a batched layer step goes module by
 # module, its predictors and top-ks are a dozen short launches beside kernels of 50-170 us, and
 # overlapping them pays (OPT-175B shape: 279.9 -> 255.3 us/layer at batch 8, 425.1 -> 385.0 us at
-# batch 32).  None: never.
+# batch 32).  None: never.  (The sparse MLP called by itself, without a graph, first up to ``ONE_CALL_PRODUCTS``: the host is what it waits for.)
 SIDE_STREAM_MIN_BATCH = 2
+# A decode step of the sparse MLP alone is one call of the library, with everything on the current stream, up to so many products of the neurons' two
+# rows; beyond, where a side stream is used, the kernels are longer than the host's part and the predictor runs beside them.  us a step among others / waited for, op by
+# op with the side stream and in one call: 16 / 32 / 64 sequences, 4096 wide and 4096 neurons 76.7, 44.5 / 93.5, 68.6, 94.4, 52.8 / 105.8, 78.5, 104, 83 / 126, 110; 7168
+# wide 64 sequences (3.8e9 products) 114, 104 / 134, 130; 9216 wide 32 (2.4e9) 95, 80 / 117, 106, 64 (4.8e9) 115, 122 / 146, 147; 12288 wide 8 / 32 (3.2e9) / 64 (6.4e9) 97.7, 92.6 /
+# 117.1, 116.9, 103, 95 / 127, 121, 134, 140 / 162, 166; 12288 wide and 16384 neurons 8 (3.2e9) / 16 (6.4e9) / 32 / 64 206, 202 / 238, 228, 206, 204 / 227, 230, 196, 205 / 224, 231, 222, 241 / 250, 268.
+ONE_CALL_PRODUCTS = 1 << 32
 
 # Prompt phase on this package's own kernels (dense products: dv_dense_linear_f16; causal attention
 # + cache fill: dv_prefill_attention_f16).  False: PyTorch's library GEMM and attention.
@@ -310,7 +316,7 @@ class ParallelFusedMLPDejavu(nn.Module):
         side = do_token_generation and side_stream_enabled(x.shape[0])
         # (from a graph the products and the predictor of several sequences side by side, as below: there the host takes no part)
         if idx is not None and do_token_generation and not (defer_reduce or USE_SIDE_STREAM or (side and (
-                defer_join or torch.cuda.is_current_stream_capturing()))):
+                defer_join or 2 * x.numel() * idx.numel() > ONE_CALL_PRODUCTS or torch.cuda.is_current_stream_capturing()))):
             done = self._one_call(x, residual, idx)
             if done is not None:
                 return done

@@ -94,3 +94,28 @@ def test_pruned_layers(monkeypatch, name, parameter):
     prune.random_unstructured(getattr(m, name), parameter, 0.5)
     got = m(x, residual, idx)[0]
     assert torch.equal(got, _ops(monkeypatch, m, x, residual, idx)[0]) and not torch.equal(got, whole)
+
+
+@pytest.mark.parametrize("batch,K,one", [(1, 512, True), (2, 512, True), (2, 513, False), (32, 32, True), (33, 32, False)])
+@torch.no_grad()
+def test_long_steps_use_the_side_stream(monkeypatch, batch, K, one):
+    """Both sides of the line, laid where small sizes reach it; one sequence has no side stream."""
+    m = _module(256, 1024, 64, 128)
+    x, residual = (torch.randn(batch, 1, 256, device="cuda").half() for _ in range(2))
+    idx = torch.arange(K, device="cuda")
+    monkeypatch.setattr("dejavu_amd.modules.ONE_CALL_PRODUCTS", 2 * 2 * 256 * 512 if batch <= 2 else 2 * 32 * 256 * 32)
+    calls, call = [], ParallelFusedMLPDejavu._one_call
+    monkeypatch.setattr(ParallelFusedMLPDejavu, "_one_call", lambda *a: [calls.append(1), call(*a)][1])
+    got = m(x, residual, idx)
+    assert bool(calls) == one
+    monkeypatch.undo()
+    assert all(torch.equal(a, b) for a, b in zip(got, _ops(monkeypatch, m, x, residual, idx)))
+
+
+def test_the_line_by_its_sizes():
+    """9216 wide with 32 / 64 sequences, 12288 wide with 32 / 64, the same with four times the neurons and 8 / 16."""
+    from dejavu_amd import modules
+
+    sizes = ((9216, 4096, 32, 64), (12288, 4096, 32, 64), (12288, 16384, 8, 16))
+    for d, K, below, above in sizes:
+        assert 2 * d * K * below <= modules.ONE_CALL_PRODUCTS < 2 * d * K * above
