@@ -460,6 +460,8 @@ def pending_linear(linear: nn.Linear, x: torch.Tensor) -> Optional[ops.PendingRo
     if not _prompt_on_hip(linear, x) or x.shape[1] == 1:
         return None
     rows = x.numel() // x.shape[-1]
+    if _few_parts_product(linear, x, "id"):  # (in decode_linear's order: the same kernels, the same sums)
+        return ops.dense_linear_pending(x, linear.weight, linear.bias, wide=True)
     if rows <= HIP_PROMPT_MAX_ROWS or (rows <= HIP_PROMPT_LONG_MAX_ROWS and _long_product(linear, x)):
         return ops.dense_linear_pending(x, linear.weight, linear.bias)
     return ops.dense_linear_pending(x, linear.weight, linear.bias, wide=True) if _long_parts(linear, x) else None

@@ -36,7 +36,7 @@ def test_pending_product_and_norm(rows, M, K, wide):
     assert torch.equal(alone + res, r)
     if not wide:
         assert torch.equal(alone, ops.dense_linear(x, W, b))
-    elif K % 64 == 0:
+    else:
         assert torch.equal(alone, ops.dense_linear_wide_parts(x, W, b))
     assert all(torch.equal(p, q) for p, q in zip(ops.add_layer_norm(alone, res, gamma, beta, 1e-5), (y, r)))
 
@@ -92,3 +92,13 @@ def test_hooked_blocks_get_tensors():
         h.remove()
     assert len(seen) == 3 and all(isinstance(t, torch.Tensor) and t.shape == (1, 100, 1024) for t in seen)
     assert torch.equal(plain, hooked)
+
+
+@pytest.mark.parametrize("rows,M,K", [(2, 1024, 4096), (128, 5120, 5120), (150, 16384, 2560), (192, 20480, 5120), (193, 4096, 16384), (300, 4096, 16384), (777, 5120, 20480)])
+@torch.no_grad()
+def test_pending_linear_is_decode_linear(rows, M, K):
+    """Which kernel takes a product, and so its bits, does not depend on what follows."""
+    lin = torch.nn.Linear(K, M, device="cuda", dtype=torch.float16).requires_grad_(False)
+    x = torch.randn(1, rows, K, device="cuda").half()
+    pending = modules.pending_linear(lin, x)
+    assert pending is not None and torch.equal(pending.materialize(), modules.decode_linear(lin, x))
