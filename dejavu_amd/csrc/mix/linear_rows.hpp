@@ -4,8 +4,8 @@
 //           attention's splits with its sinks and gates;
 //   after : plain store, a gated unit, a short convolution with its state, dynamic tanh + residual add + the next
 //           dynamic tanh, or the update of several residual streams with the row that the next norm reads.
-// A wave owns R consecutive rows of W at a time, or KS waves do, a stretch of the columns each; the row x is staged in LDS once per
-// workgroup.
+// A wave owns R consecutive rows of W at a time, or KS waves do, a stretch of the columns each (a grid of all rows then); the row x is staged in
+// LDS once per workgroup.
 #pragma once
 #include "elem.hpp"
 #include "hyper.hpp"
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(RowsArgs a) {
   constexpr int CH = 8 * kWave, TASKS = 4 / KS;
   __shared__ float others[KS > 1 ? 4 : 1][R];
   const T* W = reinterpret_cast<const T*>(a.W);
-  const int K = a.K, ntasks = (a.M + R - 1) / R, rounds = (ntasks + nblocks * TASKS - 1) / (nblocks * TASKS);
+  const int K = a.K, ntasks = (a.M + R - 1) / R;
   const int part = wave % KS, per = ((K + CH - 1) / CH + KS - 1) / KS * CH, k0 = part * per, k1 = min(K, k0 + per);
   int t = blockIdx.x * TASKS + wave / KS;
   Pack8<T> w[U][R];
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(RowsArgs a) {
   __shared__ float coef[DV_HYPER_ROW_MAX * (DV_HYPER_ROW_MAX + 2)];
   if constexpr (AFTER == DV_OUT_HYPER) hyper_coefficients(a.hyper, coef, threadIdx.x, 256);
   stage_row<T, BEFORE>(a, xs, red);
-  for (int round = 0; KS > 1 ? round < rounds : t < ntasks; ++round, t += nblocks * TASKS) {  // (waves that share rows stay together)
+  for (bool any = KS > 1 || t < ntasks; any; t += nblocks * TASKS, any = KS == 1 && t < ntasks) {  // (waves that share rows: one turn, all of them)
     // what the epilogue adds to is requested before the products
     float old[DV_HYPER_ROW_MAX], bias = 0.f;
     if constexpr (AFTER != DV_OUT_GLU) {
@@ -274,12 +274,11 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(RowsArgs a) {
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
     const int row0 = t * R;
-    if (t + nblocks * TASKS < ntasks) {
+    if (KS == 1 && t + nblocks * TASKS < ntasks) {
       rows_of(t + nblocks * TASKS);
       load_w(k0);
     }
     if constexpr (KS > 1) {
-      if (round > 0) __syncthreads();
       if (part > 0 && lane < R) {
         float v = acc[0];
 #pragma unroll
@@ -288,7 +287,7 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(RowsArgs a) {
         others[wave][lane] = v;
       }
       __syncthreads();
-      if (part > 0 || t >= ntasks) continue;
+      if (part > 0 || t >= ntasks) return;
 #pragma unroll
       for (int r = 0; r < R; ++r)
 #pragma unroll

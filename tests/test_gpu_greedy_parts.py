@@ -37,3 +37,27 @@ def test_step(vocab, kind, off):
         assert torch.equal(scores[1].nan_to_num(3.0), logits.nan_to_num(3.0))
     ops.greedy_advance(logits, token, position, seq_pos, sequences, out_index)
     assert int(score_index) == 4 and int(token) == want and int(out_index) == 6
+
+
+@pytest.mark.parametrize("vocab", [1, 7, 1025, 32768, 50272])
+@pytest.mark.parametrize("off", [0, 1])
+def test_entry_without_scratch(vocab, off):
+    """The one launch that callers of the C library without scratch have does the same."""
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    logits = torch.randn(vocab + 8, device="cuda", generator=g)[off:off + vocab]
+    logits[vocab // 2] = logits.max() + 1
+    logits[vocab - 1] = logits[vocab // 2]  # a tie: the first
+    got = []
+    for scratch in (True, False):
+        ones = [torch.full((1,), v, dtype=t, device="cuda") for v, t in ((7, torch.int64), (8, torch.int64), (9, torch.int32), (2, torch.int64), (1, torch.int64))]
+        token, position, seq_pos, out_index, score_index = ones
+        sequences, scores = torch.full((1, 4), -1, dtype=torch.int64, device="cuda"), torch.full((3, vocab), 5.0, device="cuda")
+        for _ in range(3):
+            if scratch:
+                ops.greedy_advance(logits, token, position, seq_pos, sequences, out_index, scores, score_index)
+            else:
+                assert ops.lib.dv_mix_greedy_advance(logits.data_ptr(), vocab, token.data_ptr(), position.data_ptr(), seq_pos.data_ptr(),
+                                                     sequences.data_ptr(), 4, out_index.data_ptr(), scores.data_ptr(), vocab, 3, score_index.data_ptr(),
+                                                     ops._stream()) == 0
+        got.append([t.clone() for t in (*ones, sequences, scores)])
+    assert int(got[0][0]) == vocab // 2 and all(torch.equal(a, b) for a, b in zip(*got))
