@@ -9,7 +9,7 @@
 // are read transposed; pairing keys by hand took eight 4-byte stores for each 16-byte one, and with the sums rescaled for
 // every tile, not only where a maximum has grown, 32 heads of 128 and 2048 tokens took 98 us instead of 89, 4096 tokens 331
 // instead of 304.  Two buffers with one barrier a tile were slower (96).  Bound by the chain of a tile: LDS reads, two products, the
-// softmax.  So two groups of four waves share a query tile, the even and the odd key tiles: the last queries' chain is half as long, a SIMD
+// softmax.  So two groups of four waves share a query tile (where two_groups says), the even and the odd key tiles: the last queries' chain is half as long, a SIMD
 // has two waves whatever the grid (alone a wave takes 328 registers, one to a SIMD; two in a group's kernel 238), and a long workgroup and
 // a short one make the same 17 steps on every compute unit.  us, one group / two, 32 heads of 128: 300 / 777 / 2048 / 4096 / 8192
 // tokens 16.5 / 13.6, 35.1 / 25.7, 92 / 69, 308 / 217, 1172 / 713, a window of 1024 and 8 key heads 91.5 / 64.7 (2048), 352 / 251 (8192); 16 heads 33.6 / 24.3 (777),

@@ -402,15 +402,35 @@ int ssd_scan_any(const SsdArgs& a, hipStream_t s) {
   return DV_ERR_UNSUPPORTED;
 }
 
+// Whether two groups of waves share a query tile's key tiles.  One group has a wave on each SIMD where values are wider than 64, two workgroups of it on a compute
+// unit where they are not.  The time of one group over that of two, 150 to 4096 tokens, 8 to 64 heads:
+//   wider values: from four key tiles on, or three without a mask, 1.04 to 1.62 (us: 160 / 300 tokens 11.6 / 10.7, 16.5 / 13.6, 47 after 1000 42 / 28); fewer
+//     do not pay for the sums that meet: windows of 16 to 64 and chunks of 64 and 128 0.92 to 1.02, 47 / 100 tokens 7.2 / 8.1, 9.9 / 10.1 us;
+//   values up to 64, no more workgroups than compute units: 1.04 to 1.68 from three key tiles on, windows and chunks of 128 and less 0.98 to 1.30; twice as many: more than
+//     ten key tiles 0.92 to 1.56, ten 0.86 to 1.22, fewer 0.69 to 0.96; beyond, 0.64 to 1.13.
+// Heads beyond 128 need more registers than two waves on a SIMD have.
+bool two_groups(const AttnArgs& a, int keys, int vt, int64_t workgroups) {
+  if (keys <= 2 * kTileK) return false;
+  if (vt <= 2 && workgroups <= compute_units()) return true;
+  if (vt <= 2 && workgroups > 2 * compute_units()) return false;
+  const int off = a.pos_host - a.base;
+  int most = 0;       // key tiles of a query tile
+  bool cut = false;   // a mask leaves keys out
+  for (int64_t q0 = 0; q0 < a.n; q0 += kTileQ) {
+    const int64_t pos = a.pos_host + q0, oldest = (a.window > 0 ? pos - a.window + 1 : a.chunk > 0 ? pos - pos % a.chunk : 0) - a.base;
+    const int64_t first = oldest > 0 ? oldest : 0, end = (q0 + kTileQ < a.n ? q0 + kTileQ : a.n) + off;
+    const int tiles = (int)((end - 1) / kTileK - first / kTileK + 1);
+    if (tiles > most) most = tiles;
+    cut |= oldest > 0;
+  }
+  return vt <= 2 ? most > 10 : most > 3 || (most == 3 && !cut);
+}
+
 template <int DT, int VT>
 int attn_tiles_launch(const AttnArgs& a, int keys, hipStream_t s) {
   const dim3 grid((unsigned)((int64_t)a.H * ((a.n + kTileQ - 1) / kTileQ)));
-  // Two groups of waves from three key tiles on (us, one / two: 47 / 100 tokens after none 7.2 / 8.1, 9.9 / 10.1, 160 / 300 11.6 / 10.7, 16.5 / 13.6, 47
-  // after 1000 42 / 28).  Heads beyond 128 need more registers than two waves on a SIMD have.
   if constexpr (DT <= 8 && VT <= 4) {
-    const int mask = a.window > 0 ? a.window : a.chunk;
-    const int64_t most = mask > 0 ? (int64_t)mask + kTileQ - 1 : keys;
-    if ((most < keys ? most : keys) > 2 * kTileK) {
+    if (two_groups(a, keys, VT, grid.x)) {
       hipLaunchKernelGGL((attn_tiles_kernel<DT, VT, 2>), grid, dim3(512), 0, s, a, keys);
       return launched();
     }

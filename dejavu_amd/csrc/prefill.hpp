@@ -22,7 +22,8 @@
 // 40 heads of 128 and 128 tokens: 7.5 us (one wavefront for 16 queries and all their keys: 27); 32 heads
 // and 777 tokens 30 us (215, and 75 with the library's attention and the copies into the caches).  Short
 // prompts are bound by one block's chain of loads and exchanges, long ones by L2: each workgroup reads
-// the keys and values before its 32 queries, 160 MB at 777 tokens (from there on prefill_tiles_kernel, below).  Where short prompts make workgroups enough, two
+// the keys and values before its 32 queries, 160 MB at 777 tokens (prefill_tiles_kernel, below, takes those of 1000 on,
+// 800 with 40 heads; the line is prefill_in_tiles').  Where short prompts make workgroups enough, two
 // wavefronts do: of four, some have no block at all, yet hold their registers and LDS (16 sequences of 16 / 33 / 128
 // tokens and 96 heads of 64: 9.4 / 17.4 / 38 us with four, 7.0 / 13.8 / 33 with two; of 128: 16 / 35 / 107 and 15 / 25 / 97).
 //

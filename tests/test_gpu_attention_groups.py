@@ -56,3 +56,18 @@ def test_large_scores_in_one_group_only():
     got = ops.portion_attention(q, k, v, H, H, 128 ** -0.5, 0, 0)
     want = _reference(q, k, v, H, H, 128 ** -0.5, 0, None, None, None, None, None)
     assert bool(torch.isfinite(got).all()) and (got.double() - want).norm() <= 2 ** -8 * want.norm()
+
+
+# around one and two workgroups a compute unit (256 of them), key tiles a query tile on both sides of the lines
+@pytest.mark.parametrize("H,n", [(64, 500), (72, 500), (128, 500), (136, 500), (40, 1500), (4, 400)])
+@pytest.mark.parametrize("mask", [{}, {"window": 64}, {"window": 66}, {"window": 130}, {"chunk": 64}, {"chunk": 128}, {"chunk": 700}])
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 128), (64, 72)])
+def test_many_workgroups(H, n, mask, dim, vdim):
+    G = 4
+    g = torch.Generator(device="cuda").manual_seed(H + n)
+    q, k, v = (torch.randn(n, h * d, device="cuda", generator=g).bfloat16() for h, d in ((H, dim), (G, dim), (G, vdim)))
+    got = ops.portion_attention(q, k, v, H, G, dim ** -0.5, 0, 0, **mask).view(n, H, vdim)
+    some = [0, H // 4, 3 * H // 4 - 1, H - 1]  # a head of each key head
+    want = _reference(q.view(n, H, dim)[:, some].reshape(n, -1), k, v, G, G, dim ** -0.5, 0, mask.get("window"), mask.get("chunk"), None, None, None)
+    got = got[:, some].reshape(n, -1).double()
+    assert (got - want).norm() <= 2 ** -8 * want.norm() and (got - want).abs().max() <= 2 ** -6 * want.abs().max()
