@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256) void gated_head_norm_kernel(const float* __res
 // First index of the largest of `vocab` fp32 logits (NaN ranks highest), and the bookkeeping of a generation loop (one
 // workgroup): token <- argmax, sequences[out_index++] <- token, position++, seq_pos++, scores[score_index++] <- logits.
 // Bound by the latency of its loads: eight of 16 bytes per thread are on their way at once, and the row of scores is stored
-// from registers (32768 logits: 11 us; one load at a time 17).  For callers without scratch.
+// from registers (32768 logits: 11 us; one load at a time 17).  For few logits, and for callers without scratch.
 __global__ __launch_bounds__(1024) void greedy_advance_f32_kernel(
     const float* __restrict__ logits, int vocab, int64_t* __restrict__ token, int64_t* __restrict__ position,
     int* __restrict__ seq_pos, int64_t* __restrict__ sequences, int64_t* __restrict__ out_index,

@@ -406,6 +406,6 @@ class ChannelDelta(nn.Module):
 def apply_mixer(mixer, h, state, step: StepInfo):
     """``mixer(h, state, step)`` for a caller whose next step is a product of ``mixer_ops`` with what comes back: that product can
     merge an attention's splits itself.  Subclasses, wrappers and hooks are left out of it and see tensors."""
-    if type(mixer) in (WindowAttention, ChunkAttention) and not _hooked(mixer):
+    if h.shape[0] == 1 and type(mixer) in (WindowAttention, ChunkAttention) and not _hooked(mixer):
         return mixer(h, state, step, defer=True)
     return mixer(h, state, step)

@@ -5,6 +5,13 @@ import torch
 from dejavu_amd import mixer_ops as ops
 
 pytestmark = pytest.mark.gpu
+LINE = ops.GREEDY_PARTS
+
+
+@pytest.fixture(params=[1, 1 << 30], ids=["two launches", "one launch"], autouse=True)
+def launches(request, monkeypatch):
+    """Both forms at every size, whichever the line between them would choose."""
+    monkeypatch.setattr(ops, "GREEDY_PARTS", request.param)
 
 
 @pytest.mark.parametrize("vocab", [1, 3, 1023, 1024, 1025, 4099, 32768, 70001])
@@ -61,3 +68,19 @@ def test_entry_without_scratch(vocab, off):
                                                      ops._stream()) == 0
         got.append([t.clone() for t in (*ones, sequences, scores)])
     assert int(got[0][0]) == vocab // 2 and all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("vocab,count", [(5, 1), (8191, 1), (8192, 2), (50272, 2)])
+def test_few_logits_take_one_launch(vocab, count, monkeypatch):
+    called = []
+    monkeypatch.setattr(ops, "GREEDY_PARTS", LINE)
+    for name, n in (("dv_mix_greedy_advance", 1), ("dv_mix_greedy_advance_ws", 2)):
+        entry = getattr(ops.lib, name)
+        monkeypatch.setattr(ops.lib, name, lambda *a, entry=entry, n=n: [called.append(n), entry(*a)][1])
+    logits = torch.randn(vocab, device="cuda")
+    logits[vocab - 2] = 9.0
+    token, position, out_index = (torch.zeros(1, dtype=torch.int64, device="cuda") for _ in range(3))
+    seq_pos, sequences = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.zeros(1, 4, dtype=torch.int64, device="cuda")
+    ops.greedy_advance(logits, token, position, seq_pos, sequences, out_index)
+    assert called == [count] and int(token) == int(sequences[0, 0]) == vocab - 2
+    assert int(position) == int(seq_pos) == int(out_index) == 1
