@@ -82,12 +82,16 @@ HIP_PROMPT_WIDE_STRIDE = 1 << 25
 # library, from 769 rows on by 20480 columns the wide tiles) over this, weights cold, 257 to 2048 rows: 2560 x 10240 1.06 to 1.30, 3072 x 12288 0.99 to 1.34,
 # 4096 x 16384 1.00 to 2.09, 4608 x 18432 1.05 to 1.92, 5120 x 20480 1.14 to 1.72, 5632 x 22528 1.32 to 1.61, 7168 x 28672 1.38 to 1.62, 9216 x 36864 1.38
 # to 1.39 (777 by 4096 x 16384 146 -> 103 us).  Of more weight rows only in three parts and more: in two 8192 x 28672 0.89 to 1.01, 12288 x 49152 0.90 to 1.00.
-# Fewer rows where one column of such tiles makes three parts (15361 to 20480 weight rows on 256 compute units): the streaming kernel over these, alone,
-# 136 / 160 / 192 rows: 16384 x 4096 1.10 / 1.10 / 1.05, 20480 x 5120 1.14 / 1.12 / 1.07, 18432 x 4608 1.03 / 1.02 / 0.99, 20480 x 2560 1.19 / 1.15 / 1.12; but
-# 16384 x 2048 0.91 to 1.01, in two parts 24576 x 6144 0.94 to 1.00, in four and five 14336 / 12288 x 4096 0.93 to 1.10.  The line in rows is by whole prompts of eight blocks
+# Fewer rows where one column of such tiles makes three parts (15361 to 20480 weight rows on 256 compute units).  The streaming kernel over these, alone, 129 / 160 / 192
+# rows: above 16384 weight rows (17408 to 20480), where the streaming kernel's tiles leave some of its round empty, 2560 columns 1.06 to 1.09 / 1.00 to 1.12 / 0.99 to 1.03, 2816 to 3584
+# 1.09 to 1.18 / 1.04 to 1.12 / 1.00 to 1.08, 4096 1.15 to 1.20 / 1.11 to 1.15 / 1.07 to 1.10, 4608 and 5120 1.03 to 1.08 / 1.01 to 1.05 / 0.98 to 1.03, 5632 to 8192 1.10 to 1.23 / 1.06 to 1.19 / 1.01 to
+# 1.13, 10240 and 12288 1.05 to 1.07 / 1.02 to 1.05 / 0.97 to 1.04, but 6144 0.94 to 0.98 / 0.93 to 0.95 / 0.89 to 0.93; of 16384 and fewer, which it has in a round, those whose rows lie a power of
+# two apart: 4096 1.09 to 1.15 / 1.09 to 1.14 / 1.02 to 1.09, 8192 1.19 / 1.15 to 1.17 / 1.13 to 1.15, but 2560 to 3584 0.93 to 1.03 / 0.88 to 1.01 / 0.88 to 0.97, 4608 to 12288 0.84 to 1.03 / 0.82 to 1.00 /
+# 0.80 to 0.97.  16384 x 2048 0.91 to 1.01, in two parts 24576 x 6144 0.94 to 1.00, in four and five 14336 / 12288 x 4096 0.93 to 1.10.  The line in rows is by whole prompts of eight blocks
 # (us, streaming kernel or library / these), 6.7B shape 128 / 150 / 192 / 224 tokens 1309 / 1306, 1534 / 1504, 1586 / 1567, 1683 / 1695, 13B shape 1720 / 1775, 1993 /
 # 1967, 2064 / 2048, 2351 / 2366: fewer rows are as fast alone, but not beside the launches around them.
-HIP_PROMPT_FEW_PARTS, HIP_PROMPT_FEW_COLUMNS, HIP_PROMPT_FEW_ROWS = 3, 2560, (129, 192)
+HIP_PROMPT_FEW_PARTS, HIP_PROMPT_FEW_COLUMNS, HIP_PROMPT_FEW_ROWS = 3, (2560, 12288), (129, 192)
+HIP_PROMPT_FEW_WEIGHT_ROWS, HIP_PROMPT_FEW_BUT = 16384, 6144   # weight rows above which any columns but these
 HIP_PROMPT_PARTS_COLUMNS, HIP_PROMPT_PARTS_WEIGHT = 10240, 26_000_000
 HIP_PROMPT_PARTS_TALL = 7168, 3
 # The package's causal-attention kernel (cache fill in the same launch) is ahead of the library's attention with the
@@ -98,8 +102,8 @@ HIP_PROMPT_ATTN_MAX_TOKENS = 192
 # Each workgroup reads the keys and values before its 32 queries, so the L2 bounds long prompts and the library, whose tiles
 # were larger, overtook: with 40 heads of 128 from 8192 tokens on (1759 against 1691 us; 6000 tokens 961 against 1155, 16 sequences of
 # 4096 and 32 heads 5875 against 6316), with 96 heads above 2048 (four sequences of 2048 1329 against 1404, of 4096 5184 against 4784).  (Its tiles of
-# 128 queries, prefill.hpp, are ahead beyond these lines as well: 40 heads and 8192 tokens 1051 against 1738, 96 heads and 4096 690 against 1305.  The lines
-# are where they were: what prompts of each length are computed by, and their bits, are what callers know.)
+# 128 queries, prefill.hpp, which take prompts of a thousand tokens and more since, are ahead beyond these lines alone: 40 heads and 8192 tokens 1051 against
+# 1738, 96 heads and 4096 690 against 1305.  The lines are the older kernel's still: whole prompts of such lengths have not been measured on both sides.)
 HIP_PROMPT_ATTN_LONGEST = 6144
 HIP_PROMPT_ATTN_WIDE = 5120            # heads * head_dim above which it is
 HIP_PROMPT_ATTN_WIDE_LONGEST = 2048
@@ -435,6 +439,12 @@ def _long_parts(linear, x: torch.Tensor) -> bool:
     return ops.wide_parts(rows, K, M) >= (least if M > many else 2)
 
 
+def _few_rule(M: int, K: int) -> bool:
+    least, most = HIP_PROMPT_FEW_COLUMNS
+    return (least <= K <= most and M % 8 == 0 and
+            (K & (K - 1) == 0 if M <= HIP_PROMPT_FEW_WEIGHT_ROWS else K != HIP_PROMPT_FEW_BUT))
+
+
 def _few_parts_product(linear, x: torch.Tensor, activation: str) -> bool:
     """The same for a prompt of few rows, with an activation too."""
     W = linear.weight
@@ -442,7 +452,7 @@ def _few_parts_product(linear, x: torch.Tensor, activation: str) -> bool:
     if not HIP_PROMPT_FEW_ROWS[0] <= rows <= HIP_PROMPT_FEW_ROWS[1] or W.dim() != 2 or activation not in ("id", "relu", "squared_relu"):
         return False
     M, K = W.shape
-    return (K >= HIP_PROMPT_FEW_COLUMNS and M % 8 == 0 and ops.wide_parts(rows, K, M) == HIP_PROMPT_FEW_PARTS and _wide_fits(linear, x))
+    return _few_rule(M, K) and ops.wide_parts(rows, K, M) == HIP_PROMPT_FEW_PARTS and _wide_fits(linear, x)
 
 
 def _parts_product(linear, x: torch.Tensor) -> Optional[torch.Tensor]:

@@ -26,13 +26,16 @@ def test_few_rows_in_parts(rows, M, K, activation):
 
 
 def test_what_the_modules_send_there():
-    taken = [(rows, M, K) for M, K in ((15368, 2560), (20480, 2560), (20488, 2560), (15360, 2560), (16384, 2552)) for rows in (128, 129, 192, 193)
+    # (columns, and weight rows up to 16384, by what was measured on both sides of each line)
+    taken = [(rows, M, K) for M, K in ((15368, 4096), (20480, 2560), (20488, 2560), (15360, 4096), (20480, 2552), (15368, 2560), (16384, 5120), (16392, 5120),
+                                       (20480, 6144), (16384, 6144), (16384, 8192)) for rows in (128, 129, 192, 193)
              if modules._few_parts_product(nn.Linear(K, M, device="cuda", dtype=torch.float16).requires_grad_(False),
                                            torch.zeros(1, rows, K, device="cuda", dtype=torch.float16), "relu")]
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
-        assert taken == [(129, 15368, 2560), (192, 15368, 2560), (129, 20480, 2560), (192, 20480, 2560)]
-    lin = nn.Linear(2560, 16384, device="cuda", dtype=torch.float16).requires_grad_(False)
+        assert taken == [(rows, M, K) for M, K in ((15368, 4096), (20480, 2560), (16392, 5120), (16384, 8192)) for rows in (129, 192)]
+    lin = nn.Linear(2560, 16392, device="cuda", dtype=torch.float16).requires_grad_(False)
     x = torch.randn(1, 150, 2560, device="cuda").half()
+    assert modules._few_parts_product(lin, x, "relu") or torch.cuda.get_device_properties(0).multi_processor_count != 256
     assert not modules._few_parts_product(lin, x, "gelu") and not modules._few_parts_product(lin, torch.cat([x, x])[:, ::2], "relu")
     y = modules.decode_linear(lin, x, "relu")
     want = torch.relu(x.double() @ lin.weight.double().t() + lin.bias.double())
