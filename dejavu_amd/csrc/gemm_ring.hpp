@@ -78,7 +78,8 @@ struct RingPlan {
 // More rows: 128 rows of W, so that X is fetched less often (5120 x 20480 with 96 rows: 53 us, 60 with 64 rows of W),
 // where that leaves 32 tiles and K is long enough to split (but 64 where these make one round and K is short: 16384 x 4096 with
 // 72 / 128 rows 41.5 / 45 us, in two splits 47.5 / 48; and for small weights, of whose K tiles of 128 have an eighth each: 4096 x 4096 with 72 / 100 /
-// 128 rows 13.5 / 14.0 / 14.5, 16.9 / 17.9 / 18.2, a prompt of 68 to 127 tokens with such a product a layer 1 to 2 % less; 4096 x 8192 25.4 either way); 192 where they fill the chip better (20480 x 5120 with 96 rows:
+// 128 rows 13.5 / 14.0 / 14.5, 16.9 / 17.9 / 18.2, a prompt of 68 to 127 tokens with such a product a layer 1 to 2 % less; 4096 x
+// 4608 / 5632 1.04 / 1.00 to 1.04 times the speed, but 6144 0.98 to 1.01, 6656 to 8064 0.93 to 1.00); 192 where they fill the chip better (20480 x 5120 with 96 rows:
 // 107 tiles in 2 splits take 53 us, 160 tiles of 128 rows 59) or spare a round of it (36864 x 12288 with 128 rows: 192
 // tiles against 288).  257 to 384 rows are two tiles of 192, not of 256 (320 rows: QKV of 24 heads of 9216 97 against 147 us, of
 // 32 heads of 12288 141 against 195).
@@ -103,7 +104,7 @@ inline RingPlan plan_ring(int n, int M, int K, int units) {
     else if (p.nb == 64 && M >= units * 64) lay((M + 95) / 96 > units && (M + 127) / 128 <= units ? 128 : 96);
     else lay(taller && (p.nb == 32 || M <= units * 60) ? 128 : 64);  // (33 to 64 rows: not where 64 make a round)
   } else if (M < 32 * 128 || K < 2048 || (p.nb == 128 && K <= 4096 && M > units * 56 && M <= units * 64) ||
-             (p.nb == 128 && K >= 4096 && K < 8192 && M <= units * 16)) {
+             (p.nb == 128 && K >= 4096 && K < 6144 && M <= units * 16)) {
     lay(64);
   } else {
     const bool tall = p.nb < 256 && K >= 4096;

@@ -62,6 +62,12 @@ def test_a_quarter_of_the_compute_units_takes_a_quarter_of_the_rows(plan):
     assert [p[0] for p in plan(asked)] == [96, 96, 64, 64, 128, 64, 128]
 
 
+def test_small_weights_of_65_to_128_rows(plan):
+    """Tiles of 64 weight rows from 4096 to below 6144 columns, where those of 128 would have an eighth of the columns each."""
+    asked = [(n, 4096, K, 256) for n in (65, 128) for K in (4088, 4096, 6136, 6144, 8184)] + [(100, 4224, 4096, 256), (64, 4096, 4096, 256)]
+    assert [p[0] for p in plan(asked)] == [128, 64, 64, 128, 128] * 2 + [128, 64]
+
+
 def test_which_windows_multiply_live_rows_only(tmp_path):
     """Both sides of each line: rows of the window, size of a head, chosen heads."""
     try:
