@@ -1492,9 +1492,15 @@ namespace {
 // 1000 19.5 / 16.8, 21.8 / 24.7, 35.8 / 32.8, 94 / 69; 16 sequences of 32 heads 160 / 256 / 777 42.6 / 47.5, 71 / 58, 376 / 288; heads of 64, 12 of them, 3000 / 6000
 // 48.4 / 54.4, 141 / 115, 96 of them 400 / 500 / 777 / 1500 15.7 / 16.8, 19.6 / 18.4, 32.8 / 33.3, 88 / 64).  The line is by whole prompts of six blocks: 32 heads 777 / 1000 / 1500 tokens 2326 / 2327, 2667 / 2657, 3898 / 3814,
 // 40 heads 512 / 777 / 1000 / 1900 2546 / 2555, 3637 / 3640, 4226 / 4186, 7386 / 7185.
+// Shorter prompts, the one over the other's time by how much of their tiles is queries and by workgroups: seven eighths and more 0.97 to 1.28 (340 to 449 tokens, heads of 64 and 128), of two
+// tiles 1.0 to 1.24 but between one and one and a half workgroups a compute unit 0.93 to 1.02; four fifths, heads of 128, 205 / 308 / 410 tokens 0.96 to 1.13, 1.00 to 1.12, 1.01 to 1.15
+// from 600 workgroups on and 0.92 to 1.17, 0.95 to 1.03, 0.97 to 1.07 below, heads of 64 0.96 to 1.07, 0.91 to 1.00, 0.86 to 1.04.
 bool prefill_in_tiles(int B, int T, int H, int hd) {
-  const int64_t padded = ((int64_t)T + kPtQueries - 1) / kPtQueries * kPtQueries;
-  return (int64_t)T * H * B * hd >= 32000 * 128 && (T >= 450 || 5 * (int64_t)T >= 4 * padded);
+  const int64_t tiles = ((int64_t)T + kPtQueries - 1) / kPtQueries, groups = tiles * H * B, units = compute_units();
+  if ((int64_t)T * H * B * hd < 32000 * 128) return false;
+  if (T >= 450) return true;
+  if (8 * (int64_t)T >= 7 * tiles * kPtQueries) return tiles > 2 || groups <= units || 2 * groups >= 3 * units;
+  return hd == 128 && 5 * (int64_t)T >= 4 * tiles * kPtQueries && 3 * groups >= 7 * units;
 }
 }  // namespace
 extern "C" {

@@ -31,3 +31,10 @@ def test_tiles(B, T, H, hd, pos0, more):
     # weights and results are rounded to fp16, 2^-12 each
     assert (got - want).norm() <= 2 ** -10 * want.norm() and (got - want).abs().max() <= 2 ** -9 * want.abs().max()
     assert torch.equal(ops.prefill_attention(qkv).view(B, T, H, hd)[:, :, ::7].double(), got)  # without caches
+
+
+# short prompts on both sides of the lines in full tiles and in workgroups (288, 384; 588, 600 of 256 compute units)
+@pytest.mark.parametrize("B,T,H,hd", [(2, 224, 72, 128), (2, 224, 96, 128), (1, 256, 128, 128), (2, 308, 98, 128), (2, 308, 100, 128), (4, 307, 50, 128), (4, 410, 50, 64),
+                                      (4, 448, 40, 64), (4, 447, 40, 64)])
+def test_short_prompts(B, T, H, hd):
+    test_tiles(B, T, H, hd, 0, 3)
