@@ -308,7 +308,7 @@ def dense_linear_wide_parts(x: torch.Tensor, weight: torch.Tensor, bias: Optiona
     assert nbytes and x2.dtype == weight.dtype == torch.float16 and x2.stride(1) == 1 and weight.stride(1) == 1 and M % 8 == 0
     assert bias is None or (bias.shape == (M,) and bias.dtype == x.dtype and bias.is_contiguous())
     out = torch.empty(rows, M, device=x.device, dtype=x.dtype)
-    # the sums of this call alone (up to 250 MB), not the stream's scratch, which is never given back
+    # the sums of this call alone (up to 64 MiB: 256 by 256 of them a compute unit), not the stream's scratch, which is never given back
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     check(lib.dv_dense_linear_wide_ws_f16(_ptr(x2), x2.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), rows, N, M, _ACT[activation],
                                           _ptr(out), M, _ptr(ws), nbytes, _stream()), "dv_dense_linear_wide_ws_f16")
